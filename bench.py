@@ -338,7 +338,7 @@ def main():
             _, psec = g.prefill(ptoks, want_logits=False)
             out["prefill"] = {"positions": int(n_pre), "positions_per_s": round(n_pre / psec, 1), "ms": round(psec * 1e3, 3),
                               "ms_per_32_positions": round(psec * 1e3 / ((n_pre + 31) // 32), 4),
-                              "note": "l2j_prefill: the forward passes of consecutive positions of one sequence, 32 per step on the "
+                              "note": "l2j_prefill: the forward passes of consecutive positions of one sequence, up to 1024 per pass on the "
                                       "matrix cores, into the KV cache of the single-sequence path (device time)"}
             g.reset()
         except l2j.L2JError as e:

@@ -97,12 +97,12 @@ int l2j_device_count(void);
  * sampling step of a vocabulary of at most 36864 is one launch of a workgroup per 256 probabilities with grid barriers; a
  * bounded wait of it that runs out is L2J_E_HIP, and the context sets the option to 0 itself: seed the sampler again and go on;
  * 0: one launch per stage, as larger vocabularies always take), "prefill" (0, the default: the decode loops take the prompt
- * positions one by one, as the reference does; 1: the first whole steps of 32 prompt positions go through l2j_prefill, the
- * loop goes on behind them: the same tokens but where two logits lie within rounding of each other; shapes l2j_prefill
- * does not take run as with 0), "prefill_flash" (the attention of l2j_prefill's steps: 1, the default: 16 positions at a time on
- * the fp32 matrix cores from position 64 on, where that is the faster form, every position for itself below; 2: always;
+ * positions one by one, as the reference does; 1: a prompt of eight ids or more goes through l2j_prefill, the
+ * loop goes on behind it: the same tokens but where two logits lie within rounding of each other; shapes l2j_prefill
+ * does not take run as with 0), "prefill_flash" (the attention of l2j_prefill: 1, the default: the keys of a head and 16 positions are
+ * shared by the waves of a workgroup where a wave per 16 positions would leave compute units idle; 2: always;
  * 0: never), "prefill_split" (workgroups that share the keys of a head and 16 positions there: 1 to 4; 0, the default:
- * one below position 192, then as many of up to four as the GPU has compute units for).  l2j_get_option reads the value in force
+ * one below 192 keys, then as many of up to four as the GPU has compute units for).  l2j_get_option reads the value in force
  * ("fuse" reads 0 after such a switch; "wall_clock_khz", read-only: the rate of the device clock that l2j_decode_greedy
  * times itself with, 0 when the device does not tell it). */
 int l2j_set_option(l2j_ctx *ctx, const char *name, int32_t value);
@@ -155,17 +155,19 @@ int l2j_decode_greedy(l2j_ctx *ctx, const int32_t *prompt, int32_t n_prompt, int
  * the token loop of l2j_decode_greedy (BOS first, its own prompt ids forced, first-maximum argmax afterwards) for
  * exactly `steps` positions; a sequence that emits token 1 keeps running and the caller cuts it there.  prompts: n_seq
  * rows of prompt_stride ids, n_prompt[b] of them used; out_tokens: n_seq rows of `steps` ids.  The products of the
- * quantized matrices run on the bf16 matrix cores with the arithmetic of K/MatMul.java:117-151 kept: a code is a bf16
- * exactly, an fp32 activation is cut exactly into three bf16, the products are exact and the sums fp32 (the fp32
- * classifier runs on the fp32 matrix cores); sums are formed in another order than in the single-sequence path, so
- * logits agree to rounding, not bit for bit.  The first call makes a second copy of the quantized matrices on the
+ * quantized matrices run on the int8 matrix cores: a code less 128 is a signed byte, an fp32 activation a 31-bit fixed-point
+ * number relative to the largest of its group of 256 (four signed digits to the base 256), the sums over a group are exact
+ * and the groups are added in fp32 with their scales and offsets as in K/MatMul.java:117-151 (the fp32 classifier runs on the
+ * fp32 matrix cores); sums are formed in another order than in the single-sequence path, so logits agree to rounding, not
+ * bit for bit.  The positions whose input tokens all sequences know (up to the shortest prompt) are taken at once.  The first call makes a second copy of the quantized matrices on the
  * device, in the order this path reads them (as large as the matrices themselves: 6.9 GB at the 7B shape), its
  * activation buffers, a KV cache of n_seq x steps rows per layer and the captured graph of a step; the context keeps
  * them until l2j_destroy, so later calls allocate and capture nothing unless they ask for another n_seq, more steps or
  * longer prompts (then the set is replaced).  The context's own cache is not touched.  L2J_E_OOM when the device
  * memory does not suffice (n_seq x n_layers x steps x kv_dim x 8 bytes of cache).
  * Needs dim and hidden_dim in whole groups of 256 and head_size 64, 128 or 256.
- * *seconds (may be NULL): GPU time from the end of the first step to the end of the last. */
+ * *seconds (may be NULL): GPU time from the end of the first step to the end of the last (from the start of the pass over the
+ * known positions, where there is one). */
 int l2j_decode_greedy_batch(l2j_ctx *ctx, const int32_t *prompts, const int32_t *n_prompt, int32_t n_seq,
                             int32_t prompt_stride, int32_t steps, int32_t *out_tokens, double *seconds);
 /* Gives back what the calls for several sequences at once keep on the device (l2j_decode_greedy_batch,
@@ -253,8 +255,8 @@ int l2j_get_config(l2j_ctx *ctx, l2j_config *cfg);
 /* The forward passes of n consecutive positions pos0 .. pos0 + n - 1 of one sequence, tokens[i] being the input token of
  * position pos0 + i: what n calls of l2j_forward(tokens[i], pos0 + i) leave in the KV cache and return for the last of
  * them, i.e. the prompt positions of the token loop (J/Run.java:623-640: the reference runs them one by one through
- * Run.transformer), 32 positions per step through the batched products on the matrix cores (every weight read once per
- * 32 positions).  logits (null: not wanted): the vocab_size logits of the last position; they are also what l2j_sample
+ * Run.transformer), up to 1024 positions per pass through the batched products on the matrix cores (every weight read once per
+ * pass).  logits (null: not wanted): the vocab_size logits of the last position; they are also what l2j_sample
  * samples from next.  seconds (null: not wanted): device time of the steps.  The sums are formed in another order than
  * l2j_forward's, so cache rows and logits agree with its to rounding (1e-6 of the largest), not bit for bit.  Shapes as for
  * l2j_decode_greedy_batch (else L2J_E_SIZE: take l2j_forward); its buffers and its copy of the matrices are shared. */
@@ -295,10 +297,9 @@ int l2j_decode_greedy_batch_logits(l2j_ctx *ctx, const int32_t *prompts, const i
 /* Measurement and test of the matrix-core kernel for several sequences at once (the reference has none: "parallel
  * processing of multiple queries" is on its wish-list, README.md:347): y[b][r] = sum_k dequant(W[r][k]) * x[b][k] for
  * sixteen activation vectors x (16 x K floats) against one layer's matrix of a quantized matrix tensor (L2J_WQ..L2J_W3;
- * K a multiple of 256), in the arithmetic of K/MatMul.java:117-151 (exact products, fp32 sums, group scale and offset;
- * see l2j_decode_greedy_batch).  y: 16 x rows floats.  groups_per_slice is ignored (a slice of K is four groups of 256
- * codes since the kernel keeps the activations in its waves' registers; the argument remains for callers built against
- * the earlier kernel).  The call makes the tile-ordered copy of the tensor if the context has none yet.  *mean_us (may be
+ * K a multiple of 256), in the arithmetic of K/MatMul.java:117-151 (exact sums over a group, group scale and offset;
+ * see l2j_decode_greedy_batch).  y: 16 x rows floats.  groups_per_slice is ignored (the product picks its slices of
+ * K by the shape; the argument remains for callers built against an earlier kernel).  The call makes the tile-ordered copy of the tensor if the context has none yet.  *mean_us (may be
  * NULL): mean time of `rounds` launches of the product kernel. */
 int l2j_batch_matmul(l2j_ctx *ctx, int tensor, int layer, const float *x, float *y, int32_t groups_per_slice,
                      int32_t rounds, double *mean_us);

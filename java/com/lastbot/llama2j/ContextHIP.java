@@ -282,8 +282,8 @@ public final class ContextHIP implements AutoCloseable {
     }
 
     /**
-     * Run.transformer(tokens[i], pos0 + i, ...) for every i (the prompt positions of Run.main's loop), 32 positions per
-     * step on the matrix cores (l2j_prefill); logits (may be null) receives those of the last position.  The token loop
+     * Run.transformer(tokens[i], pos0 + i, ...) for every i (the prompt positions of Run.main's loop), up to 1024 positions per
+     * pass on the matrix cores (l2j_prefill); logits (may be null) receives those of the last position.  The token loop
      * then goes on at position pos0 + tokens.length with forwardArgmax / forward.
      */
     public void prefill(int[] tokens, int pos0, float[] logits) {

@@ -382,7 +382,7 @@ class Transformer:
         return logits
 
     def prefill(self, tokens, pos0=0, want_logits=True):
-        """forward(tokens[i], pos0 + i) for every i, 32 positions per step on the matrix cores: (logits of the last
+        """forward(tokens[i], pos0 + i) for every i, up to 1024 positions per pass on the matrix cores: (logits of the last
         position or None, device seconds)."""
         tokens = np.ascontiguousarray(tokens, dtype=np.int32)
         logits = np.empty(self.config.vocab_size, dtype=np.float32) if want_logits else None

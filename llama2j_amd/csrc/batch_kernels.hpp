@@ -1,13 +1,12 @@
 // Several sequences per pass over the weights ("parallel processing of multiple queries", the reference's README
-// wish-list): with sixteen activation vectors per weight matrix the multiply-adds are a 16-wide GEMM and run on the
-// matrix cores.  The arithmetic of the single-sequence path is kept (byte code -> float, fp32 activations, fp32 sums,
-// rm * sum(code * x) + min * sum(x) per group of 256; K/MatMul.java:117-151 is the loop it restates) although the
-// products run on the bf16 cores, sixteen times as fast as the fp32 ones: a code (0..255) is a bf16 exactly, and an
-// fp32 activation is the sum of three bf16 (its 24 significant bits cut into 8 + 8 + 8), so code * x is the sum of
-// three products that v_mfma_f32_16x16x32_bf16 forms exactly and accumulates in fp32.  The vector units only convert
-// the codes.  The fp32 classifier keeps the fp32 cores (v_mfma_f32_16x16x4_f32).
+// wish-list): the copy of the matrices in tile order that their products read (digit_gemm.hpp), the classifier for sixteen
+// or thirty-two vectors, the attention of a decode step, and the waves of the one-launch step (batch_step.hpp), whose
+// products run on the bf16 cores: a code less 128 is a bf16 exactly, and an fp32 activation is the sum of three bf16 (its
+// 24 significant bits cut into 8 + 8 + 8), so code * x is the sum of three products that v_mfma_f32_16x16x32_bf16 forms
+// exactly and accumulates in fp32.  The fp32 classifier keeps the fp32 cores (v_mfma_f32_16x16x4_f32).
 #pragma once
 
+#include "digit_gemm.hpp"
 #include "kernels.hpp"
 #include "phase_kernels.hpp"   // grid barrier, device-coherent loads and stores
 
@@ -73,7 +72,8 @@ __host__ __device__ inline int bg_slices(int K) { return ((K >> 8) + kBgGroups -
 // codes of a (tile of 16 rows, group) block are 4 KB in a row, [T][lane][16 codes] with lane = r + 16 s holding row r of
 // the tile at k = 64 T + 16 s + j, so that each of a wave's four load instructions per block reads 1 KB in one piece
 // (row by row a wave's instruction touches 16 rows, 64 bytes each: a third slower, measured); the blocks of a tile
-// follow each other group by group, then come those of the next tile.  The scales likewise: 16 (rm, min) per block.
+// follow each other group by group, then come those of the next tile.  The codes are stored less 128, as the signed bytes the
+// int8 matrix cores take (code * rm + min = (code - 128) * rm + (min + 128 rm)), and the scales likewise: 16 (rm, min + 128 rm) per block.
 // One thread per 16 codes of the whole tensor (layers x rows x K); rows % 16 == 0, K % 256 == 0.
 static __global__ void __launch_bounds__(256) k_btile(const uint8_t *__restrict__ codes, const float2 *__restrict__ gs, long n16, int rows, int K,
                                                uint8_t *__restrict__ tcodes, float2 *__restrict__ tgs)
@@ -86,9 +86,13 @@ static __global__ void __launch_bounds__(256) k_btile(const uint8_t *__restrict_
     const int block = (int)(w >> 8), in = (int)(w & 255), T = in >> 6, lane = in & 63, r = lane & 15, sq = lane >> 4;
     const int tile = block / ngroups, g = block - tile * ngroups;
     const long src = layer * (long)rows * K + (long)(16 * tile + r) * K + (g << 8) + 64 * T + 16 * sq;
-    reinterpret_cast<uint4 *>(tcodes)[o] = *reinterpret_cast<const uint4 *>(codes + src);
-    if (in < 16)   // the block's 16 scales: rows 16 tile + in
-        tgs[(layer * (long)rows * K >> 8) + (long)block * 16 + in] = gs[((layer * (long)rows * K + (long)(16 * tile + in) * K) >> 8) + g];
+    uint4 v = *reinterpret_cast<const uint4 *>(codes + src);
+    v.x ^= 0x80808080u; v.y ^= 0x80808080u; v.z ^= 0x80808080u; v.w ^= 0x80808080u;
+    reinterpret_cast<uint4 *>(tcodes)[o] = v;
+    if (in < 16) {   // the block's 16 scales: rows 16 tile + in
+        const float2 m = gs[((layer * (long)rows * K + (long)(16 * tile + in) * K) >> 8) + g];
+        tgs[(layer * (long)rows * K >> 8) + (long)block * 16 + in] = make_float2(m.x, fmaf(128.0f, m.x, m.y));
+    }
 }
 
 // LDS of k_bgemm: the sums of a batch of tiles (as many tiles as the workgroup has waves; per tile, wave and column block
@@ -99,14 +103,15 @@ __host__ __device__ inline size_t bg_lds_bytes(int nseq, int hv)
     return waves * waves * nb * 1024 + waves * nseq * sizeof(float);
 }
 
-// eight codes (two words of a row) as eight bf16: the upper halves of the codes' floats, two to a register
+// eight codes less 128 (two words of a row) as eight bf16: the upper halves of their floats, two to a register
 __device__ __forceinline__ v8bf16 codes_bf16(uint32_t d0, uint32_t d1)
 {
+    auto f = [](uint32_t w, int b) { return __float_as_uint((float)(int8_t)(w >> (8 * b))); };
     uint4 o;
-    o.x = __builtin_amdgcn_perm(__float_as_uint(ubyte_f(d0, 1)), __float_as_uint(ubyte_f(d0, 0)), 0x07060302u);
-    o.y = __builtin_amdgcn_perm(__float_as_uint(ubyte_f(d0, 3)), __float_as_uint(ubyte_f(d0, 2)), 0x07060302u);
-    o.z = __builtin_amdgcn_perm(__float_as_uint(ubyte_f(d1, 1)), __float_as_uint(ubyte_f(d1, 0)), 0x07060302u);
-    o.w = __builtin_amdgcn_perm(__float_as_uint(ubyte_f(d1, 3)), __float_as_uint(ubyte_f(d1, 2)), 0x07060302u);
+    o.x = __builtin_amdgcn_perm(f(d0, 1), f(d0, 0), 0x07060302u);
+    o.y = __builtin_amdgcn_perm(f(d0, 3), f(d0, 2), 0x07060302u);
+    o.z = __builtin_amdgcn_perm(f(d1, 1), f(d1, 0), 0x07060302u);
+    o.w = __builtin_amdgcn_perm(f(d1, 3), f(d1, 2), 0x07060302u);
     return __builtin_bit_cast(v8bf16, o);
 }
 
@@ -355,16 +360,6 @@ struct BgWave {
     }
 };
 
-// grid (workgroups per slice, slices of K), 256 HV threads; dynamic LDS: bg_lds_bytes(16 NB, HV)
-template <int NB, int HV>
-__global__ void __launch_bounds__(kBgThreads * HV) k_bgemm(const BGemm a)
-{
-    extern __shared__ __align__(16) float bg_lds[];
-    BgWave<NB, HV> w(a);
-    w.begin(blockIdx.x, blockIdx.y, gridDim.x, false);
-    w.template run<false>(bg_lds, false);
-}
-
 // ---- the classifier: fp32 weights (K/MatMul.java:37-60), the same tiling -------------------------------------------
 
 struct BGemmF32 {
@@ -499,137 +494,72 @@ static __global__ void __launch_bounds__(1024) k_brms(const float *__restrict__ 
     }
 }
 
-// x[b] += the slices of a product summed in order (K/Accum.java:26-30), then xn[b] as k_brms does: the
-// hand-over from Wo to W1/W3 and from W2 to the next layer's Wq/Wk/Wv (or to the classifier) in one kernel.
-static __global__ void __launch_bounds__(1024) k_bres_rms(const float *__restrict__ part, int slices, float *__restrict__ x, const float *__restrict__ w,
-                                                   float *__restrict__ xn, int n)
-{
-    __shared__ float red[16];
-    const int b = blockIdx.x, tid = threadIdx.x, n4 = n >> 2;
-    const long stride4 = (long)gridDim.x * n4;   // 16-byte words between two slices (one workgroup per sequence)
-    const float4 *pp = reinterpret_cast<const float4 *>(part) + (long)b * n4;
-    float4 *xp = reinterpret_cast<float4 *>(x + (long)b * n);
-    float ssq = 0.0f;
-    for (int i = tid; i < n4; i += 1024) {
-        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 8
-        for (int s = 0; s < slices; s++) {   // (independent loads, added in slice order)
-            const float4 v = pp[(long)s * stride4 + i];
-            t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
-        }
-        float4 v = xp[i];
-        v.x = __fadd_rn(v.x, t.x); v.y = __fadd_rn(v.y, t.y); v.z = __fadd_rn(v.z, t.z); v.w = __fadd_rn(v.w, t.w);
-        xp[i] = v;
-        ssq += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-    }
-    ssq = block_sum(ssq, red, 16);   // (its barriers also order the stores above before the loads below)
-    const float ss = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ssq, (float)n), 1e-5f)));
-    const float4 *wp = reinterpret_cast<const float4 *>(w);
-    float4 *op = reinterpret_cast<float4 *>(xn + (long)b * n);
-    for (int i = tid; i < n4; i += 1024) {
-        float4 v = xp[i];   // (written by this same thread)
-        const float4 wv = wp[i];
-        v.x = __fmul_rn(wv.x, __fmul_rn(ss, v.x));
-        v.y = __fmul_rn(wv.y, __fmul_rn(ss, v.y));
-        v.z = __fmul_rn(wv.z, __fmul_rn(ss, v.z));
-        v.w = __fmul_rn(wv.w, __fmul_rn(ss, v.w));
-        op[i] = v;
-    }
-}
-
-// hb[b][r] = silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74), h1 and h3 the slices summed in order.
-// grid (hidden / 256, sequences), 256 threads.
-static __global__ void __launch_bounds__(256) k_bepi_swiglu(const float *__restrict__ p1, const float *__restrict__ p3, int slices, int hidden,
-                                                     const float *__restrict__ silu, int exact, float *__restrict__ hb)
-{
-    const int b = blockIdx.y, rix = blockIdx.x * 256 + threadIdx.x;
-    const long n = (long)gridDim.y * hidden, i = (long)b * hidden + rix;
-    float h1 = 0.0f, h3 = 0.0f;
-#pragma unroll 8
-    for (int s = 0; s < slices; s++) { h1 += p1[(long)s * n + i]; h3 += p3[(long)s * n + i]; }
-    const float sg = silu_sigma(silu, h1, exact);
-    hb[i] = __fmul_rn(h1, __fmul_rn(sg, h3));
-}
-
 struct BAttn {
-    const float *pq, *pk, *pv;   // partial products of Wq, Wk, Wv: (slices, sequences, dim | kv_dim)
+    const float *part;           // (slices, sequences, dim + 2 kv_dim): the products of Wq, Wk, Wv
     int slices;
     const float2 *rope;          // (seq_len, head_size / 2) cos, sin
     float *kc, *vc;              // this layer's part of the batch cache, head-major: + b * seq_stride + (kv head * cap + pos) * head_size
     long seq_stride;             // floats between two sequences
     int cap;                     // positions the cache holds
-    float *out;                  // (sequences, dim)
+    Digits out;                  // the attention output of every sequence, as digits
     const BatchState *st;
-    int n_heads, kv_mul, head_size, kv_dim, dim;
+    int kv_mul, kv_dim, dim;
     float sqrt_hs;
-    // MODE 1, 2 (the rows are consecutive positions of ONE sequence, st->pos + b, in one cache):
-    long head_stride;            // floats between two kv heads of a position's row
-    int row_stride;              // and between two positions
-    int nrows;                   // rows in use: the others neither store nor attend
-    int nseq;                    // rows of the products' partial sums (k_pflash; k_battn has them as its grid)
-    // k_pflash with the keys of a (head, 16 queries) pair split over gridDim.z workgroups:
-    float *pf_part;              // (head, half, z) x (16 maxima, 16 sums, 16 x head_size values): what each leaves for the last one
-    unsigned *pf_cnt;            // (head, half): how many have; zero between launches
 };
 
-// Attention of one head of one sequence over positions 0..pos (K/AttentionLoop.java:29-54, K/ExpSumNormalize.java:25-38,
-// K/AccumWeightedValue.java).  First q of the head and k, v of its kv head at this position: the slices of the products
+// Attention of one sequence over positions 0..pos (K/AttentionLoop.java:29-54, K/ExpSumNormalize.java:25-38,
+// K/AccumWeightedValue.java), for the 256 / head_size heads whose outputs are one group of 256 of the next product's input:
+// 256 threads per head.  First q of the head and k, v of its kv head at this position: the slices of the products
 // summed in order, RoPE on the pairs of q and k (K/ApplyRope.java:74-90), k and v into the cache row (J/Run.java:95-99; by
 // the first head of the kv group).  Then LPR lanes per cache row (four floats of the head each): the row slots of the
-// workgroup take the positions in turn with an online softmax, and the slots are folded at the end.  grid (n_heads, sequences).
+// head take the positions in turn with an online softmax, and the slots are folded at the end; sixteen threads write the
+// group's digits.  grid (dim / 256, sequences), 256 * 256 / head_size threads.
 constexpr int kBattnRows = 4;
 
-// MODE 0: the sequences of a batch, all at position st->pos, each with a cache of its own (head-major).  MODE 1 and 2: the
-// rows are the positions st->pos + b of one sequence sharing one cache (any layout: head_stride, row_stride): 1 only stores
-// k and v of its position, 2 only attends (over the rows below its own position, which a launch in MODE 1 has stored,
-// and its own).
-template <int LPR, int MODE = 0>
-__global__ void __launch_bounds__(256) k_battn(const BAttn a)
+template <int LPR>
+__global__ void __launch_bounds__(16384 / LPR) k_battn(const BAttn a)
 {
-    constexpr int RPW = 64 / LPR, NSLOT = 4 * RPW;
-    __shared__ float sm_m[NSLOT], sm_l[NSLOT];
-    __shared__ float4 sm_acc[NSLOT * LPR];
-    __shared__ __align__(16) float sm_qkv[3][4 * LPR];
-    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    constexpr int RPW = 64 / LPR, NSLOT = 4 * RPW, HS = 4 * LPR, HPG = 256 / HS;   // HPG heads per workgroup
+    __shared__ float sm_m_[HPG][NSLOT], sm_l_[HPG][NSLOT];
+    __shared__ float4 sm_acc_[HPG][NSLOT * LPR];
+    __shared__ __align__(16) float sm_qkv_[HPG][3][HS];
+    __shared__ __align__(16) float sm_out[256];
+    const int sub = threadIdx.x >> 8, h = blockIdx.x * HPG + sub, b = blockIdx.y, tid = threadIdx.x & 255, lane = tid & 63;
+    float *sm_m = sm_m_[sub], *sm_l = sm_l_[sub];
+    float4 *sm_acc = sm_acc_[sub];
+    float(*sm_qkv)[HS] = sm_qkv_[sub];
     const int j = lane % LPR, slot = (tid >> 6) * RPW + lane / LPR;
-    if (MODE != 0 && b >= a.nrows) return;
-    if (MODE == 1 && h % a.kv_mul != 0) return;   // (one head of a group stores its kv head)
-    const int pos = a.st->pos + (MODE != 0 ? b : 0), len = pos + 1, hs = a.head_size, kvh = h / a.kv_mul;
-    const long hstride = MODE != 0 ? a.head_stride : (long)a.cap * hs;
-    const int rs = MODE != 0 ? a.row_stride : hs;
-    const int half = hs >> 1;
+    const int pos = a.st->pos, len = pos + 1, kvh = h / a.kv_mul;
+    const long hstride = (long)a.cap * HS;
+    constexpr int half = HS >> 1;
+    const int cols = a.dim + 2 * a.kv_dim;
     for (int p = tid; p < 3 * half; p += 256) {   // one thread per pair of q, k, v
         const int which = p / half, idx = p - which * half;
-        {
-            const int rows = which == 0 ? a.dim : a.kv_dim, row = (which == 0 ? h : kvh) * hs + 2 * idx;
-            const float *part = which == 0 ? a.pq : which == 1 ? a.pk : a.pv;
-            float v0 = 0.0f, v1 = 0.0f;
+        const int col = (which == 0 ? h * HS : which == 1 ? a.dim + kvh * HS : a.dim + a.kv_dim + kvh * HS) + 2 * idx;
+        float v0 = 0.0f, v1 = 0.0f;
 #pragma unroll 8
-            for (int s = 0; s < a.slices; s++) {   // (independent loads, added in slice order)
-                const float2 t = *reinterpret_cast<const float2 *>(part + ((long)s * gridDim.y + b) * rows + row);
-                v0 += t.x; v1 += t.y;
-            }
-            if (which < 2) {
-                const float2 cs = a.rope[(long)pos * half + idx];
-                const float r0 = __fsub_rn(__fmul_rn(v0, cs.x), __fmul_rn(v1, cs.y));
-                const float r1 = __fadd_rn(__fmul_rn(v0, cs.y), __fmul_rn(v1, cs.x));
-                v0 = r0; v1 = r1;
-            }
-            sm_qkv[which][2 * idx] = v0;
-            sm_qkv[which][2 * idx + 1] = v1;
-            if (MODE != 2 && which > 0 && h % a.kv_mul == 0)
-                *reinterpret_cast<float2 *>((which == 1 ? a.kc : a.vc) + (long)b * a.seq_stride + kvh * hstride + (long)pos * rs + 2 * idx) =
-                    make_float2(v0, v1);
+        for (int s = 0; s < a.slices; s++) {   // (independent loads, added in slice order)
+            const float2 t = *reinterpret_cast<const float2 *>(a.part + ((long)s * gridDim.y + b) * cols + col);
+            v0 += t.x; v1 += t.y;
         }
+        if (which < 2) {
+            const float2 cs = a.rope[(long)pos * half + idx];
+            const float r0 = __fsub_rn(__fmul_rn(v0, cs.x), __fmul_rn(v1, cs.y));
+            const float r1 = __fadd_rn(__fmul_rn(v0, cs.y), __fmul_rn(v1, cs.x));
+            v0 = r0; v1 = r1;
+        }
+        sm_qkv[which][2 * idx] = v0;
+        sm_qkv[which][2 * idx + 1] = v1;
+        if (which > 0 && h % a.kv_mul == 0)
+            *reinterpret_cast<float2 *>((which == 1 ? a.kc : a.vc) + (long)b * a.seq_stride + kvh * hstride + (long)pos * HS + 2 * idx) =
+                make_float2(v0, v1);
     }
-    if (MODE == 1) return;
     __syncthreads();
-    const bool on = 4 * j < hs;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 q4 = on ? *reinterpret_cast<const float4 *>(&sm_qkv[0][4 * j]) : zero;
-    const float4 kp = on ? *reinterpret_cast<const float4 *>(&sm_qkv[1][4 * j]) : zero;   // the row of this position
-    const float4 vp = on ? *reinterpret_cast<const float4 *>(&sm_qkv[2][4 * j]) : zero;
-    const long base = (long)b * a.seq_stride + kvh * hstride + 4 * j;   // (MODE 0: the head's rows lie one after the other)
+    const float4 q4 = *reinterpret_cast<const float4 *>(&sm_qkv[0][4 * j]);
+    const float4 kp = *reinterpret_cast<const float4 *>(&sm_qkv[1][4 * j]);   // the row of this position
+    const float4 vp = *reinterpret_cast<const float4 *>(&sm_qkv[2][4 * j]);
+    const long base = (long)b * a.seq_stride + kvh * hstride + 4 * j;   // (the head's rows lie one after the other)
     float m = -3.0e38f, l = 0.0f;
     float4 acc = zero;
     constexpr int R = kBattnRows;   // rows in flight per slot
@@ -640,7 +570,7 @@ __global__ void __launch_bounds__(256) k_battn(const BAttn a)
         float4 kk[R], vv[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const long at = base + (long)min(tb + r * NSLOT, last) * rs;
+            const long at = base + (long)min(tb + r * NSLOT, last) * HS;
             kk[r] = *reinterpret_cast<const float4 *>(a.kc + at);
             vv[r] = *reinterpret_cast<const float4 *>(a.vc + at);
         }
@@ -648,7 +578,7 @@ __global__ void __launch_bounds__(256) k_battn(const BAttn a)
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int t = tb + r * NSLOT;
-            const bool cached = on && t < pos;
+            const bool cached = t < pos;
             // (component by component: a choice between whole float4s went through scratch memory)
             kk[r].x = t == pos ? kp.x : cached ? kk[r].x : 0.0f; kk[r].y = t == pos ? kp.y : cached ? kk[r].y : 0.0f;
             kk[r].z = t == pos ? kp.z : cached ? kk[r].z : 0.0f; kk[r].w = t == pos ? kp.w : cached ? kk[r].w : 0.0f;
@@ -681,7 +611,7 @@ __global__ void __launch_bounds__(256) k_battn(const BAttn a)
     if (j == 0) { sm_m[slot] = m; sm_l[slot] = l; }
     sm_acc[slot * LPR + j] = acc;
     __syncthreads();
-    if (tid < LPR && 4 * tid < hs) {
+    if (tid < LPR) {
         float M = sm_m[0];
 #pragma unroll
         for (int e = 1; e < NSLOT; e++) M = fmaxf(M, sm_m[e]);
@@ -695,7 +625,17 @@ __global__ void __launch_bounds__(256) k_battn(const BAttn a)
             o.x += w * v.x; o.y += w * v.y; o.z += w * v.z; o.w += w * v.w;
         }
         o.x = __fdiv_rn(o.x, L); o.y = __fdiv_rn(o.y, L); o.z = __fdiv_rn(o.z, L); o.w = __fdiv_rn(o.w, L);
-        *reinterpret_cast<float4 *>(a.out + (long)b * a.dim + h * hs + 4 * tid) = o;
+        *reinterpret_cast<float4 *>(&sm_out[sub * HS + 4 * tid]) = o;
+    }
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        float v[16];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 f = *reinterpret_cast<const float4 *>(&sm_out[16 * threadIdx.x + 4 * q]);
+            v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+        }
+        quantize_group(a.out, b, a.dim >> 8, blockIdx.x, threadIdx.x, v);
     }
 }
 
@@ -753,197 +693,6 @@ static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *
 }
 
 // y[b][r] = sum over the slices, in slice order
-// Attention of 16 consecutive positions of one sequence for one head on the fp32 matrix cores (after k_battn<LPR, 1> has
-// stored their k and v): every cache row is fetched once for the 16 queries, instead of once per query.
-//   scores, transposed: S^T (16 keys x 16 queries) = K (16 keys x HS) . Q^T (HS x 16 queries), HS / 4 v_mfma_f32_16x16x4_f32;
-//     a lane (c = lane % 16, g = lane / 16) then holds S^T[key 4 g + e][query c], e = 0..3: the keys of a query lie in four
-//     lanes, so a query's maximum is two cross-lane steps, and the same registers are the B operand of
-//   values, transposed: O^T (HS x 16 queries) += V^T (HS x 16 keys) . P^T (16 keys x 16 queries), HS / 4 more;
-//   online softmax over the tiles of 16 keys (K/AttentionLoop.java:29-54, K/ExpSumNormalize.java:25-38,
-//     K/AccumWeightedValue.java restated as in k_battn), a query seeing the keys up to its own position.
-// The waves of the workgroup take every WAVES-th tile of keys and merge their (maximum, sum, values) through LDS.
-// The k index of a product may be permuted if both operands are: lane group g supplies the dimensions 16 u + 4 g + e
-// (one 16-byte load per u) and the keys 4 g + e.
-// grid: (n_heads, 2, 1..4): z splits the tiles of keys over that many workgroups, the last of which to finish merges what the
-// others left in device memory.  64 * WAVES threads; dynamic LDS: (16 (HS + 4) + 32 WAVES + 16 WAVES HS) floats.
-template <int HS, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) k_pflash(const BAttn a)
-{
-    constexpr int U = HS / 16;
-    extern __shared__ __align__(16) float pf_lds[];
-    constexpr int SQ = HS + 4;           // (a row of q four floats longer: the sixteen rows a wave reads together start in different banks)
-    float *sq = pf_lds;                  // [16 queries][SQ]
-    float *wm = pf_lds + 16 * SQ;        // [WAVES][16]
-    float *wl = wm + WAVES * 16;         // [WAVES][16]
-    float *wo = wl + WAVES * 16;         // [WAVES][HS / 4][16 queries][4]: dimension d of query q at (d / 4) * 64 + 4 q + d % 4
-    __shared__ float ww[WAVES * 16], wM[16];
-    __shared__ int s_last;
-    const int h = blockIdx.x, qb = blockIdx.y * 16, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = lane & 15, g = lane >> 4;
-    if (qb >= a.nrows) return;
-    const int vrows = min(16, a.nrows - qb);   // (rows past the end repeat the last one: their output is not used)
-    const int pos0 = a.st->pos + qb, kvh = h / a.kv_mul, half = HS / 2;
-    for (int p = tid; p < 16 * half; p += 64 * WAVES) {   // q of the rows: the slices of the product added up, RoPE at the row's position
-        const int r = p / half, idx = p - r * half, b = qb + min(r, vrows - 1);
-        float v0 = 0.0f, v1 = 0.0f;
-#pragma unroll 8
-        for (int s = 0; s < a.slices; s++) {
-            const float2 t = *reinterpret_cast<const float2 *>(a.pq + ((long)s * a.nseq + b) * a.dim + h * HS + 2 * idx);
-            v0 += t.x; v1 += t.y;
-        }
-        const float2 cs = a.rope[(long)(a.st->pos + b) * half + idx];
-        sq[r * SQ + 2 * idx] = __fsub_rn(__fmul_rn(v0, cs.x), __fmul_rn(v1, cs.y));
-        sq[r * SQ + 2 * idx + 1] = __fadd_rn(__fmul_rn(v0, cs.y), __fmul_rn(v1, cs.x));
-    }
-    __syncthreads();
-    float4 qv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) qv[u] = *reinterpret_cast<const float4 *>(&sq[c * SQ + 16 * u + 4 * g]);
-    const int qpos = pos0 + min(c, vrows - 1), lastkey = pos0 + vrows - 1, ntiles = lastkey / 16 + 1;
-    const float *kc = a.kc + kvh * a.head_stride, *vc = a.vc + kvh * a.head_stride;
-    const long rs = a.row_stride;
-    v4f32 o[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) o[u] = v4f32{0.f, 0.f, 0.f, 0.f};
-    float m = -3.0e38f, l = 0.0f;
-    // tile t of the keys goes to workgroup t % NS (z) and there to wave (t / NS) % WAVES: few tiles spread over the workgroups first
-    const int NS = gridDim.z;
-    const int mytiles = (ntiles - (int)blockIdx.z + NS - 1) / NS;   // of this workgroup
-    const int nw = min(WAVES, mytiles);                              // waves that have any
-    for (int t = blockIdx.z + NS * wave; t < ntiles; t += NS * WAVES) {
-        const int k0 = t * 16;
-        const float *krow = kc + (long)min(k0 + c, lastkey) * rs + 4 * g;   // (past the last key: that key again, left out below)
-        float4 kf[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) kf[u] = *reinterpret_cast<const float4 *>(krow + 16 * u);
-        v4f32 st = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].x, qv[u].x, st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].y, qv[u].y, st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].z, qv[u].z, st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].w, qv[u].w, st, 0, 0, 0);
-        }
-        float sv[4], tmax = -3.0e38f;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            sv[e] = k0 + 4 * g + e <= qpos ? __fdiv_rn(st[e], a.sqrt_hs) : -3.0e38f;   // (a query sees the keys up to its own position)
-            tmax = fmaxf(tmax, sv[e]);
-        }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float mb = fmaxf(m, tmax), sc = expf(m - mb);
-        float pr[4];
-        l *= sc;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            pr[e] = k0 + 4 * g + e <= qpos ? expf(sv[e] - mb) : 0.0f;
-            l += pr[e];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) o[u] *= sc;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + c;
-#pragma unroll
-            for (int u = 0; u < U; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * u], pr[e], o[u], 0, 0, 0);
-        }
-        m = mb;
-    }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    if (g == 0) { wm[wave * 16 + c] = m; wl[wave * 16 + c] = l; }
-    if (wave < nw) {   // (the waves without a tile have nothing to add)
-#pragma unroll
-        for (int u = 0; u < U; u++)   // (a lane's four dimensions 16 u + 4 g + e of query c as one 16-byte store, a wave's stores 1 KB in a row)
-            *reinterpret_cast<v4f32 *>(&wo[wave * HS * 16 + (4 * u + g) * 64 + 4 * c]) = o[u];
-    }
-    __syncthreads();
-    if (tid < 16 * WAVES) {   // weight of wave w's part in query q's sum: tid = w * 16 + q (a workgroup without any tile leaves
-        const int q = tid & 15;   // maximum -3e38, sum 0 and values 0)
-        float M = wm[q];
-#pragma unroll
-        for (int w = 1; w < WAVES; w++) M = fmaxf(M, wm[w * 16 + q]);
-        ww[tid] = expf(wm[tid] - M);
-        if (tid < 16) wM[tid] = M;
-    }
-    __syncthreads();
-    if (NS == 1) {
-        for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {   // the waves' parts of a query merged
-            const int d = (idx >> 6) * 4 + (idx & 3), q = (idx >> 2) & 15;   // (neighbouring lanes read neighbouring words of LDS)
-            float L = 0.0f, O = 0.0f;
-#pragma unroll
-            for (int w = 0; w < WAVES; w++) {
-                if (w < nw) {
-                    const float wt = ww[w * 16 + q];
-                    L += wt * wl[w * 16 + q];
-                    O += wt * wo[w * HS * 16 + idx];
-                }
-            }
-            if (q < vrows) a.out[(long)(qb + q) * a.dim + h * HS + d] = __fdiv_rn(O, L);
-        }
-        return;
-    }
-    // The keys are split over NS workgroups: each leaves its maxima, sums and values (not yet divided) in device memory, and
-    // the last one to do so merges them all.
-    constexpr int PER = 32 + 16 * HS;
-    const int pair = h * gridDim.y + blockIdx.y;
-    float *mine = a.pf_part + ((long)pair * NS + blockIdx.z) * PER;
-    for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {   // (values in the order they have in LDS)
-        const int d = (idx >> 6) * 4 + (idx & 3), q = (idx >> 2) & 15;
-        float L = 0.0f, O = 0.0f;
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            if (w < nw) {
-                const float wt = ww[w * 16 + q];
-                L += wt * wl[w * 16 + q];
-                O += wt * wo[w * HS * 16 + idx];
-            }
-        }
-        st_coh(mine + 32 + idx, O);
-        if (d == 0) { st_coh(mine + q, wM[q]); st_coh(mine + 16 + q, L); }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (this thread's stores have arrived where the other workgroups read)
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned old = __hip_atomic_fetch_add(a.pf_cnt + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = old + 1u == (unsigned)NS;
-        if (s_last) __hip_atomic_store(a.pf_cnt + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (for the next launch)
-    }
-    __syncthreads();
-    if (!s_last) return;
-    const float *all = a.pf_part + (long)pair * NS * PER;
-    for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {
-        const int q = (idx >> 2) & 15;
-        float mz[4], M = -3.0e38f;
-#pragma unroll
-        for (int z = 0; z < 4; z++) {
-            mz[z] = z < NS ? ld_coh(all + (long)z * PER + q) : -3.0e38f;
-            M = fmaxf(M, mz[z]);
-        }
-        float L = 0.0f, O = 0.0f;
-#pragma unroll
-        for (int z = 0; z < 4; z++) {
-            if (z < NS) {
-                const float wt = expf(mz[z] - M);
-                L += wt * ld_coh(all + (long)z * PER + 16 + q);
-                O += wt * ld_coh(all + (long)z * PER + 32 + idx);
-            }
-        }
-        if (q < vrows) a.out[(long)(qb + q) * a.dim + h * HS + (idx >> 6) * 4 + (idx & 3)] = __fdiv_rn(O, L);
-    }
-}
-
-// y[0..rows) = row `row` of the product whose slices lie in part, (slices, nseq, rows)
-static __global__ void __launch_bounds__(256) k_brow(const float *__restrict__ part, float *__restrict__ y, int rows, int slices, int nseq, int row)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += gridDim.x * blockDim.x) {
-        float t = 0.0f;
-        for (int sl = 0; sl < slices; sl++) t += part[((long)sl * nseq + row) * rows + i];
-        y[i] = t;
-    }
-}
-
 static __global__ void __launch_bounds__(256) k_breduce(const float *__restrict__ part, float *__restrict__ y, int rows, int slices)
 {
     const long n = (long)kBatch * rows;

@@ -9,17 +9,17 @@ obj="$here/build"
 mkdir -p "$obj"
 FLAGS="-O3 -std=c++17 --offload-arch=gfx950 -fPIC -Xclang -target-feature -Xclang -packed-fp32-ops -Wall -Wno-unused-function $L2J_EXTRA_FLAGS"
 pids=""
-for f in l2j_context.hip l2j_forward.hip l2j_sampler.hip l2j_batch.hip host_io.cpp host_tokenizer.cpp; do
+for f in l2j_context.hip l2j_forward.hip l2j_sampler.hip l2j_batch.hip l2j_rows.hip host_io.cpp host_tokenizer.cpp; do
     ( hipcc $FLAGS -c "$here/$f" -o "$obj/${f%.*}.o" 2> "$obj/${f%.*}.log"; echo $? > "$obj/${f%.*}.rc" ) &
     pids="$pids $!"
 done
 wait $pids
 rc=0
-for f in l2j_context l2j_forward l2j_sampler l2j_batch host_io host_tokenizer; do
+for f in l2j_context l2j_forward l2j_sampler l2j_batch l2j_rows host_io host_tokenizer; do
     grep -v "'-packed-fp32-ops' is not a recognized feature for this target" "$obj/$f.log" >&2
     [ "$(cat "$obj/$f.rc")" = "0" ] || rc=1
 done
 [ $rc = 0 ] || { echo "build failed" >&2; exit 1; }
-hipcc --offload-arch=gfx950 -shared -fPIC -o "$out" "$obj"/l2j_context.o "$obj"/l2j_forward.o "$obj"/l2j_sampler.o "$obj"/l2j_batch.o \
+hipcc --offload-arch=gfx950 -shared -fPIC -o "$out" "$obj"/l2j_context.o "$obj"/l2j_forward.o "$obj"/l2j_sampler.o "$obj"/l2j_batch.o "$obj"/l2j_rows.o \
     "$obj"/host_io.o "$obj"/host_tokenizer.o -lpthread || exit 1
 echo "built $out"

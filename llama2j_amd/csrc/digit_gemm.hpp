@@ -1,0 +1,424 @@
+// Products of the quantized matrices with many activation vectors on the int8 matrix cores.
+//
+// An fp32 activation is written as a fixed-point number: per vector and group of 256 (the weights' groups) a power of two
+// 2^s brings the largest magnitude of the group into [2^29, 2^30), x = q * 2^-s with an integer q, and q is four signed
+// digits to the base 256, which v_mfma_i32_16x16x64_i8 multiplies by the codes (less 128: signed bytes) and adds up
+// exactly.  Every activation that is not 64 times smaller than the largest of its group keeps all 24 bits of its
+// significand, and none is off by more than 2^-30 of that largest one; the sum over a group is exact, where a sum of fp32
+// products rounds at every addition (K/MatMul.java:117-151 is the loop this restates).  Groups are added in fp32.
+// Against three bf16 planes per activation (the exact cut this replaces): four products at twice the rate instead of
+// three, and no conversion of the codes, whose bytes go into the matrix cores as they lie in memory.
+#pragma once
+
+#include "kernels.hpp"
+
+namespace l2j {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kRowTile = 32;                       // activation vectors per tile: two MFMAs of 16
+constexpr int kDigitBytes = 4 * 4 * 2 * 64 * 16;   // digits of a (tile, group): [digit][64 k][half of the tile][lane][16], most significant digit first
+
+// The digits of `rows` activation vectors of length K, in the order the matrix cores take them, with the groups' scales
+// 2^-s and sums.  Tiles of 32 vectors; the vectors past the last one hold anything finite.
+struct Digits {
+    uint4 *d;      // (tile, group) x kDigitBytes; lane l of a block of 64 k: vector l % 16 of the half, k = 16 (l / 16) + 0..15
+    float *sx;     // (tile, group, 32): 2^-s (NaN: the group holds a NaN or an infinity)
+    float *sum;    // (tile, group, 32): the sum of the group's activations
+};
+
+__host__ __device__ inline size_t digit_tiles(int rows) { return (size_t)(rows + kRowTile - 1) / kRowTile; }
+
+// The exponent s for a group whose largest magnitude has the bits `amax` (sign cleared), and 2^-s.
+__device__ __forceinline__ int digit_shift(unsigned amax, float *inv)
+{
+    // 2^e <= amax < 2^(e+1): s = 29 - e, no larger than 126 (below 2^-97 the step stays at 2^-126)
+    const int e = (int)(amax >> 23) - 127;
+    const int s = min(29 - e, 126);
+    *inv = amax >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : ldexpf(1.0f, -s);
+    return s;
+}
+
+// Sixteen consecutive activations of one vector (k = 16 c .. 16 c + 15 of group g) as digits; s: the group's exponent.
+__device__ __forceinline__ void store_digits(const Digits &o, int row, int ngroups, int g, int c, const float (&v)[16], int s)
+{
+    unsigned w[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        // (a group with a NaN or an infinity: any digits, its scale is a NaN)
+        const int q = (int)rintf(ldexpf(v[i], s));
+        w[i] = ((unsigned)q + 0x80808080u) ^ 0x80808080u;   // byte d: digit d, -128 .. 127
+    }
+    uint4 *p = o.d + ((size_t)(row >> 5) * ngroups + g) * (kDigitBytes / 16) + (2 * (c >> 2) + ((row >> 4) & 1)) * 64 + (row & 15) + 16 * (c & 3);
+#pragma unroll
+    for (int d = 0; d < 4; d++) {   // byte 3 - d of every word
+        unsigned t[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const unsigned sel = 0x0c0c0400u + (unsigned)((3 - d) * 0x0101u);
+            const unsigned lo = __builtin_amdgcn_perm(w[4 * i + 1], w[4 * i], sel), hi = __builtin_amdgcn_perm(w[4 * i + 3], w[4 * i + 2], sel);
+            t[i] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        }
+        p[d * 8 * 64] = make_uint4(t[0], t[1], t[2], t[3]);
+    }
+}
+
+// max and sum over the sixteen lanes that hold a group (lanes 16 n .. 16 n + 15)
+__device__ __forceinline__ unsigned amax16(const float (&v)[16])
+{
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) m = max(m, __float_as_uint(v[i]) & 0x7fffffffu);
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
+    return m;
+}
+
+__device__ __forceinline__ float sum16(const float (&v)[16])
+{
+    float t = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) t += (v[i] + v[i + 1]) + (v[i + 2] + v[i + 3]);
+    return row16_sum(t);
+}
+
+// A group of vector `row` held by sixteen lanes, sixteen activations each (lane % 16 = c): digits, scale and sum.
+__device__ __forceinline__ void quantize_group(const Digits &o, int row, int ngroups, int g, int c, const float (&v)[16])
+{
+    float inv;
+    const int s = digit_shift(amax16(v), &inv);
+    const float t = sum16(v);
+    store_digits(o, row, ngroups, g, c, v, s);
+    if (c == 0) {
+        const size_t at = ((size_t)(row >> 5) * ngroups + g) * 32 + (row & 31);
+        o.sx[at] = inv;
+        o.sum[at] = t;
+    }
+}
+
+struct DGemm {
+    const uint8_t *codes[3];   // the matrices of one layer in tile order (k_btile): codes less 128
+    const float2 *gs[3];       // (rm, min + 128 rm) in tile order
+    int tiles[3];              // 16-row tiles of each; the matrices' rows follow each other in the output
+    int ntiles;                // all of them
+    int ngroups;               // K / 256
+    int gps;                   // groups per slice of K
+    Digits x;
+    int npos;                  // vectors
+    float *out;                // (slice, npos, 16 * ntiles)
+    int ncol, nrow;            // tiles of the grid: vectors, matrix rows
+};
+
+constexpr int kDgWaveRows = 64;   // matrix rows per wave
+
+template <int PT> __host__ __device__ constexpr size_t dgemm_lds() { return (size_t)2 * PT * (kDigitBytes + 128); }
+
+// A workgroup takes 64 NW rows of the matrix x 32 PT vectors x one slice of K.  A wave holds the codes of its 64 rows of a
+// group in registers (read once from memory, 1 KB per load) and multiplies them by the digits of the vectors, which the
+// workgroup stages in LDS a group ahead; the digits of an output are summed 256 * first + second in one accumulator, and
+// then third and fourth.  (16 x 16 tiles: v_mfma_i32_16x16x64_i8 sustains 3.75 POP/s on such data, v_mfma_i32_32x32x32_i8 3.3:
+// the clock drops under the matrix cores' load.)
+template <int PT, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
+{
+    extern __shared__ __align__(16) v4i dg_lds[];
+    constexpr int STAGE = PT * kDigitBytes / 16;            // 16-byte words of a group's digits
+    constexpr int NT = 64 * NW, NST = STAGE / NT, NQ = NST / (2 * PT);   // words a thread stages per group, and per half of a tile of vectors
+    float *lsx = reinterpret_cast<float *>(dg_lds + 2 * STAGE);   // [2][32 PT]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
+    // The workgroups of an XCD (blockIdx % 8) take the same rows of the matrix against all vectors, one after the other.
+    const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int tile = (i / a.ncol) * 8 + xcd, col = i % a.ncol;    // (tile: of rows and slices)
+    const int nslice = (a.ngroups + a.gps - 1) / a.gps;
+    if (tile >= a.nrow * nslice) return;
+    const int rt = tile / nslice, slice = tile % nslice;
+    const int g0 = slice * a.gps, g1 = min(g0 + a.gps, a.ngroups);
+    // The wave's 64 rows lie in one matrix (with several matrices: rows % 64 == 0): its address is uniform.  (Rows past the
+    // matrix's last tile of 16 repeat that tile and are not stored.)
+    const int row0 = (rt * NW + wave) * kDgWaveRows;
+    int t = min(row0 >> 4, a.ntiles - 1), m = 0, nt = a.tiles[0];
+    if (t >= nt) { t -= nt; m = 1; nt = a.tiles[1]; if (t >= nt) { t -= nt; m = 2; nt = a.tiles[2]; } }
+    const uint8_t *cm = m == 0 ? a.codes[0] : m == 1 ? a.codes[1] : a.codes[2];
+    const float2 *sm = m == 0 ? a.gs[0] : m == 1 ? a.gs[1] : a.gs[2];
+    const uint8_t *cp[4];
+    const float2 *sp[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const size_t blk = (size_t)min(t + r, nt - 1) * a.ngroups + g0;
+        cp[r] = cm + blk * 4096;
+        sp[r] = sm + blk * 16;
+    }
+    const unsigned co = lane * 16;
+    const v4i *xd = reinterpret_cast<const v4i *>(a.x.d) + ((size_t)col * PT * a.ngroups + g0) * (kDigitBytes / 16);
+    const size_t xstep = (size_t)a.ngroups * (kDigitBytes / 16);   // 16-byte words between two tiles of vectors
+    const float *xs = a.x.sx + ((size_t)col * PT * a.ngroups + g0) * 32;
+    const int xt = tid & (32 * PT - 1);   // (every wave stages the scales: no branch in the loop)
+    const unsigned xso = (xt >> 5) * a.ngroups * 32 + (xt & 31);
+
+    // codes of the first group
+    v4i cw[4][4];
+#pragma unroll
+    for (int T = 0; T < 4; T++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) cw[r][T] = *reinterpret_cast<const v4i *>(cp[r] + co + 1024 * T);
+    // digits of the first group
+    {
+        v4i st[NST];
+#pragma unroll
+        for (int q = 0; q < NST; q++) st[q] = (xd + (q * NT / 2048) * xstep + q * NT % 2048)[(unsigned)tid];
+        lsx[xt] = xs[xso];
+#pragma unroll
+        for (int q = 0; q < NST; q++) dg_lds[q * NT + tid] = st[q];
+    }
+    // the groups' offsets times the sums of the activations: fp32 matrix cores, four groups at a time
+    v4f f0[PT][2][4];
+#pragma unroll
+    for (int p = 0; p < PT; p++)
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) f0[p][mt][r] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int g = g0; g < g1; g += 4) {
+        const bool on = g + s4 < g1;
+        const int gg = on ? s4 : 0;
+        float b[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) { const float v = (sp[r] + (size_t)(g - g0) * 16)[gg * 16 + n].y; b[r] = on ? v : 0.0f; }
+#pragma unroll
+        for (int p = 0; p < PT; p++)
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                const float v = (a.x.sum + ((size_t)(col * PT + p) * a.ngroups + g) * 32 + 16 * mt)[gg * 32 + n];
+                const float s = on ? v : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; r++) f0[p][mt][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(s, b[r], f0[p][mt][r], 0, 0, 0);
+            }
+    }
+    float f[PT][2][4][4];
+#pragma unroll
+    for (int p = 0; p < PT; p++)
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[p][mt][r][e] = f0[p][mt][r][e];
+    float rm[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) rm[r] = sp[r][n].x;
+    __syncthreads();
+
+    const int ng = g1 - g0;
+    for (int g = 0; g < ng; g++) {
+        const v4i *cur = dg_lds + (g & 1) * STAGE;
+        v4i *nxt = dg_lds + ((g + 1) & 1) * STAGE;
+        const float *csx = lsx + (g & 1) * 32 * PT;
+        const int gn = min(g + 1, ng - 1);                    // (past the last group: that group again, not used)
+        const v4i *xn = xd + (size_t)gn * (kDigitBytes / 16);
+        float rm_lo[4], rm_hi[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) { rm_lo[r] = rm[r]; rm_hi[r] = rm[r] * 65536.0f; }
+        const float nsx = (xs + gn * 32)[xso];
+#pragma unroll
+        for (int r = 0; r < 4; r++) rm[r] = (sp[r] + (size_t)gn * 16)[n].x;
+#pragma unroll
+        for (int p = 0; p < PT; p++) {
+#pragma unroll
+            for (int pair = 0; pair < 2; pair++) {
+                v4i st[NQ];
+                const int q0 = (2 * p + pair) * NQ;
+#pragma unroll
+                for (int q = 0; q < NQ; q++) st[q] = (xn + ((q0 + q) * NT / 2048) * xstep + (q0 + q) * NT % 2048)[(unsigned)tid];
+                const v4i *fr = cur + p * (kDigitBytes / 16) + pair * 2 * 512 + lane;
+                v4i acc[2][4];
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[mt][r] = v4i{0, 0, 0, 0};
+#pragma unroll
+                for (int T = 0; T < 4; T++)
+#pragma unroll
+                    for (int mt = 0; mt < 2; mt++) {
+                        const v4i x = fr[(2 * T + mt) * 64];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[mt][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, cw[r][T], acc[mt][r], 0, 0, 0);
+                    }
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[mt][r] <<= 8;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int T = 0; T < 4; T++) {
+#pragma unroll
+                    for (int mt = 0; mt < 2; mt++) {
+                        const v4i x = fr[512 + (2 * T + mt) * 64];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[mt][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, cw[r][T], acc[mt][r], 0, 0, 0);
+                    }
+                    if (p == PT - 1 && pair == 1) {   // (the last use of these codes: the next group's in their place)
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) cw[r][T] = *reinterpret_cast<const v4i *>(cp[r] + (size_t)gn * 4096 + co + 1024 * T);
+                    }
+                }
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++) {
+                    const v4f sx = *reinterpret_cast<const v4f *>(csx + 32 * p + 16 * mt + 4 * s4);
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            f[p][mt][r][e] = fmaf((float)acc[mt][r][e], (pair ? rm_lo[r] : rm_hi[r]) * sx[e], f[p][mt][r][e]);
+                }
+#pragma unroll
+                for (int q = 0; q < NQ; q++) nxt[(q0 + q) * NT + tid] = st[q];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        lsx[((g + 1) & 1) * 32 * PT + xt] = nsx;
+        __syncthreads();
+    }
+    const int ldo = 16 * a.ntiles;
+#pragma unroll
+    for (int p = 0; p < PT; p++)
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int pos = (col * PT + p) * 32 + 16 * mt + 4 * s4 + e;
+                if (pos < a.npos) {
+                    float *o = a.out + ((size_t)slice * a.npos + pos) * ldo;
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[p][mt][r][e];
+                }
+            }
+}
+
+// ---- at most 32 vectors: a decode step of a batch ---------------------------------------------------------------------
+
+constexpr int kStreamWaves = 8, kStreamGroups = kStreamWaves / 2;   // groups per slice of K: two waves each
+template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (size_t)2 * kStreamWaves * NB * 512 * sizeof(float); }
+
+// With at most 32 vectors a product is bound by the codes' way from memory, and the digits are what is reused: a wave owns
+// half a group of the slice (128 k) and keeps its digits of all 16 NB vectors in registers for the whole launch, while the
+// codes of 32 matrix rows after another stream past, requested a tile ahead.  The waves' sums of a tile meet in LDS (two
+// buffers in turn, one barrier per tile).
+// Workgroup (blockIdx.x, slice blockIdx.y) of gridDim.x per slice: every gridDim.x-th tile of 32 rows (rows % 32 == 0).
+template <int NB>
+static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
+{
+    constexpr int NT = 2;   // blocks of 64 k per wave
+    extern __shared__ __align__(16) float ds_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
+    const int slice = blockIdx.y, g0 = slice * a.gps, ng = min(a.gps, a.ngroups - g0);
+    const bool on = wave < 2 * ng;       // (a wave without a group multiplies the slice's last one by zero scales: no branch around loads)
+    const int g = g0 + min(wave >> 1, ng - 1), hf = wave & 1, ntile = a.ntiles >> 1, step = gridDim.x;
+    // this wave's k of the first tile of the first matrix, and how far from there the others lie (differences of addresses:
+    // a choice between pointers would turn the loads into flat ones)
+    const uint8_t *cb = a.codes[0] + (size_t)g * 4096 + 1024 * NT * hf;
+    const float2 *sb = a.gs[0] + (size_t)g * 16;
+    const long cd1 = a.codes[1] - a.codes[0], cd2 = a.codes[2] - a.codes[0], sd1 = a.gs[1] - a.gs[0], sd2 = a.gs[2] - a.gs[0];
+    const int nt0 = a.tiles[0], nt1 = a.tiles[1];
+
+    struct Codes { v4i w[2][NT]; float2 s[2]; };
+    // the codes of this wave's k of tile t (past the end: the last tile again, not used), and the rows' scales
+    auto request = [&](int t, Codes &c) {
+        t = 2 * min(t, ntile - 1);
+        long cd = 0, sd = 0;
+        if (t >= nt0) { t -= nt0; cd = cd1; sd = sd1; if (t >= nt1) { t -= nt1; cd = cd2; sd = sd2; } }
+#pragma unroll
+        for (int r = 0; r < 2; r++) c.s[r] = (sb + ((long)(t + r) * a.ngroups * 16 + sd))[n];
+#pragma unroll
+        for (int T = 0; T < NT; T++)
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+                c.w[r][T] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(cb + ((long)(t + r) * a.ngroups * 4096 + cd) + 1024 * T + (unsigned)lane * 16));
+    };
+
+    Codes c0, c1;
+    const int t0 = blockIdx.x;
+    request(t0, c0);
+    v4i dg[4][NB][NT];
+    {
+        const v4i *xp = reinterpret_cast<const v4i *>(a.x.d) + (size_t)g * (kDigitBytes / 16) + hf * NT * 128;
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+#pragma unroll
+            for (int T = 0; T < NT; T++)
+#pragma unroll
+                for (int mt = 0; mt < NB; mt++) dg[d][mt][T] = (xp + ((d * 4 + T) * 2 + mt) * 64)[(unsigned)lane];
+    }
+    v4f sx[NB], sm[NB];
+#pragma unroll
+    for (int mt = 0; mt < NB; mt++) {
+        sx[mt] = *reinterpret_cast<const v4f *>(a.x.sx + (size_t)g * 32 + 16 * mt + 4 * s4);
+        sm[mt] = *reinterpret_cast<const v4f *>(a.x.sum + (size_t)g * 32 + 16 * mt + 4 * s4);
+        if (!on) sx[mt] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (!on || hf) sm[mt] = v4f{0.f, 0.f, 0.f, 0.f};   // (the group's offset: by the first of its waves)
+    }
+    const int ldo = 16 * a.ntiles;
+    float *out = a.out + (size_t)slice * a.npos * ldo;
+
+    auto tile = [&](int buf, const Codes &c) {
+        float *red = ds_lds + buf * kStreamWaves * NB * 512;
+#pragma unroll
+        for (int mt = 0; mt < NB; mt++)
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                v4i hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
+#pragma unroll
+                for (int T = 0; T < NT; T++) {
+                    hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(dg[0][mt][T], c.w[r][T], hi, 0, 0, 0);
+                    lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(dg[2][mt][T], c.w[r][T], lo, 0, 0, 0);
+                }
+                hi <<= 8; lo <<= 8;
+#pragma unroll
+                for (int T = 0; T < NT; T++) {
+                    hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(dg[1][mt][T], c.w[r][T], hi, 0, 0, 0);
+                    lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(dg[3][mt][T], c.w[r][T], lo, 0, 0, 0);
+                }
+                v4f y;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    y[e] = fmaf(fmaf((float)hi[e], 65536.0f, (float)lo[e]), c.s[r].x * sx[mt][e], c.s[r].y * sm[mt][e]);
+                *reinterpret_cast<v4f *>(red + (((wave * NB + mt) * 2 + r) * 64 + lane) * 4) = y;
+            }
+    };
+    // the tile's sums: NB x 2 blocks of 64 lanes x 4: NB values per thread
+    auto finish = [&](int tt, int buf) {
+        const int at = tid * NB, blk = at >> 8, l = (at >> 2) & 63, e = at & 3;
+        const float *red = ds_lds + buf * kStreamWaves * NB * 512 + at;
+        float v[kStreamWaves][NB];   // (all reads in flight together)
+#pragma unroll
+        for (int w = 0; w < kStreamWaves; w++)
+#pragma unroll
+            for (int k = 0; k < NB; k++) v[w][k] = red[w * NB * 512 + k];
+        const int row = 16 * (blk >> 1) + 4 * (l >> 4) + e;
+        float *o = out + (size_t)row * ldo + 32 * tt + 16 * (blk & 1) + (l & 15);
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            float y = v[0][k];
+#pragma unroll
+            for (int w = 1; w < kStreamWaves; w++) y += v[w][k];
+            if (row + k < a.npos) o[(size_t)k * ldo] = y;
+        }
+    };
+    for (int t = t0; t < ntile; t += 2 * step) {
+        request(t + step, c1);
+        __builtin_amdgcn_sched_barrier(0);   // (not moved behind the products, where it would find its registers free)
+        tile(0, c0);
+        __syncthreads();
+        finish(t, 0);
+        request(t + 2 * step, c0);
+        __builtin_amdgcn_sched_barrier(0);
+        tile(1, c1);
+        __syncthreads();
+        if (t + step < ntile) finish(t + step, 1);
+    }
+}
+
+}  // namespace l2j

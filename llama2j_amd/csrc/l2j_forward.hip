@@ -359,20 +359,22 @@ int decode_loop(l2j_ctx *c, const int32_t *prompt, int32_t n_prompt, int32_t ste
     }
     if ((rc = set_state(c, 1, 0, np))) return rc;  // token 1 = BOS at pos 0 (J/Run.java:614)
 
-    // Option prefill: the first P prompt positions (whole steps of 32; their outputs are the prompt's own ids, J/Run.java:635-637)
-    // through the batched products, the loop then goes on at position P.  Not when one of those ids is 1 (the loop would
-    // have stopped there, J/Run.java:670-672), nor for shapes the batched products do not take.
+    // Option prefill: the first P prompt positions (their outputs are the prompt's own ids, J/Run.java:635-637) at once
+    // (l2j_prefill), the loop then goes on at position P.  From kPrefillFrom ids on: a pass over few positions costs what
+    // three to four single ones do.  Not when one of those ids is 1 (the loop would have stopped there,
+    // J/Run.java:670-672), nor for shapes the batched products do not take.
+    constexpr int kPrefillFrom = 8;
     int P = 0;
     double prefill_s = 0.0;
-    if (c->opt[OPT_PREFILL] != 0 && np >= 32 && steps > 32) {
-        P = std::min(np, steps - 1) / 32 * 32;
+    if (c->opt[OPT_PREFILL] != 0 && np >= kPrefillFrom && steps > kPrefillFrom) {
+        P = std::min(np, steps - 1);
         for (int i = 0; i < P; i++)
             if (prompt[i] == 1) P = 0;
         if (P > 0) {
             std::vector<int32_t> in((size_t)P);
             in[0] = 1;
             for (int i = 1; i < P; i++) in[i] = prompt[i - 1];
-            rc = prefill_positions(c, in.data(), P, 0, nullptr, &prefill_s);
+            rc = prefill_positions(c, in.data(), P, 0, nullptr, &prefill_s, false);
             if (rc == L2J_E_SIZE) {
                 P = 0;   // (a shape for l2j_forward only)
             } else if (rc) {

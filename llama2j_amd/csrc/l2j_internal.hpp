@@ -3,8 +3,10 @@
 //   l2j_forward.hip   launch shapes, hipGraph capture, forward passes, the decode loops, kernel timing
 //   l2j_sampler.hip   the device sampler's host side, running sums
 //   l2j_batch.hip     several sequences at once
+//   l2j_rows.hip      many positions at once (l2j_prefill), the products with many activation vectors
 #pragma once
 
+#include "digit_gemm.hpp"
 #include "kernels.hpp"
 #include "phase_kernels.hpp"
 #include "sampler_state.hpp"
@@ -86,9 +88,9 @@ inline const OptionDef kOptions[OPT_COUNT] = {
     {"fallback", 1, true},             // a whole-token kernel whose bounded wait ran out: switch to one launch per phase and repeat
     {"batch_fuse", 0, true},           // batched decode: 1: the layers of a step in one launch with grid barriers (slower, measured); 0: eight launches per layer
     {"sampler_wide", 1, true},         // sampling step: 1: one launch over many workgroups (vocabularies that fit in LDS), 0: one launch per stage
-    {"prefill_flash", 1, true},        // l2j_prefill's attention: 1: 16 positions at a time on the fp32 matrix cores from position 64 on, every position for itself before; 2: always; 0: never
-    {"prefill", 0, true},              // decode loops: 1: the prompt positions 32 at a time through the batched products (l2j_prefill), 0: one by one as the reference
-    {"prefill_split", 0, true},        // workgroups that share the keys of one head and 16 positions in that attention: 1..4, 0: one below position 192, then as many as the GPU has compute units for
+    {"prefill_flash", 1, true},        // l2j_prefill's attention: 1: the keys of 16 positions shared by the waves of a workgroup where a wave per 16 positions would leave compute units idle; 2: always; 0: never
+    {"prefill", 0, true},              // decode loops: 1: the prompt positions at once (l2j_prefill), 0: one by one as the reference
+    {"prefill_split", 0, true},        // workgroups that share the keys of one head and 16 positions there: 1..4, 0: one below 192 keys, then as many as the GPU has compute units for
 };
 
 inline int option_from_env(int i)
@@ -102,6 +104,19 @@ inline int option_from_env(int i)
 }
 
 struct BatchBufs;   // l2j_batch.hip
+
+// What a forward pass of up to `cap` rows (positions, sequences) works in (l2j_rows.hip).
+struct RowBufs {
+    int cap = 0;
+    float *x = nullptr, *part = nullptr, *q = nullptr, *xb = nullptr, *xn = nullptr;
+    Digits dig{};
+    int *tokens = nullptr;
+    float *pf_part = nullptr;      // k_pflash with the keys of a block split over several workgroups: what each leaves for the one
+    unsigned *pf_cnt = nullptr;    // that merges, and how many have (zero between launches);
+    int pf_blocks = 0;             // room for this many blocks of 16 positions
+    hipError_t alloc(l2j_ctx *c, int rows, bool attention);
+    void release();
+};
 
 }  // namespace l2j
 
@@ -188,7 +203,8 @@ struct l2j_ctx {
     float *sort_k[2] = {nullptr, nullptr};   // intermediate runs of the sort (padded to whole runs of 4096)
     int *sort_v[2] = {nullptr, nullptr};
     float *sample_exp = nullptr;   // exp(logit / temperature - max) of one sampling step (k_sample_exp)
-    bool pflash_ready = false;           // k_pflash's LDS attributes are set
+    bool dgemm_ready = false;            // the LDS attributes of k_dgemm and k_pflash are set
+    RowBufs rows;                        // l2j_prefill and the prompts of a batch, made by the first call and replaced by a longer one
     unsigned char *wide_mem = nullptr;   // what the workgroups of the one-launch sampling step hand each other (k_sample_wide)
 };
 
@@ -265,8 +281,9 @@ void free_batch_samplers(BatchSamplers *bs);
 // top-p step left), on the rows of logits; the tokens go to token[s] and out[s * out_stride].
 hipError_t launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned active, unsigned cur, float *logits, float temperature,
                            float topp, int *token, int *out, long out_stride);
-// l2j_batch.hip: l2j_prefill without the lock (the decode loops call it holding it)
-int prefill_positions(l2j_ctx *c, const int32_t *tokens, int32_t n, int32_t pos0, float *logits, double *seconds);
+// l2j_rows.hip: l2j_prefill without the lock (the decode loops call it holding it)
+// keep_logits: leave the last position's logits in the context, as l2j_prefill does
+int prefill_positions(l2j_ctx *c, const int32_t *tokens, int32_t n, int32_t pos0, float *logits, double *seconds, bool keep_logits = true);
 int check_sampler_status(l2j_ctx *c);
 int check_sampler_args(float temperature, float topp);
 

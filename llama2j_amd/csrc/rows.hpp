@@ -1,0 +1,53 @@
+// The forward pass of many positions at once: what l2j_rows.hip offers to the batched path.
+#pragma once
+
+#include <initializer_list>
+
+#include "l2j_internal.hpp"
+#include "digit_gemm.hpp"
+
+namespace l2j {
+
+constexpr int kRowsMax = 1024;   // rows of a pass
+
+struct DgPlan {
+    int variant = 0, gps = 0, slices = 0, nrow = 0, ncol = 0;
+};
+
+struct RowNorm;
+
+// k_dstream takes the products with at most 32 vectors (rows of the matrices in whole tiles of 32), k_dgemm the others.
+inline bool streams(int tiles16, int rows) { return rows <= kRowTile && tiles16 % 2 == 0; }
+inline int stream_slices(int ngroups) { return (ngroups + kStreamGroups - 1) / kStreamGroups; }
+
+// Most slices of K k_dgemm cuts a product into: their sums are written and read again.
+inline int max_slices(int rows) { return std::min(16, std::max(4, 1024 / std::max(1, rows))); }
+// Most (slice, row) pairs of products of up to `cap` rows with rows of up to `ngroups` groups.
+inline int max_slice_rows(int cap, int ngroups) { return std::max({std::min(16 * cap, 1024), 4 * cap, stream_slices(ngroups) * std::min(cap, kRowTile)}); }
+
+DgPlan dgemm_plan(int n_cu, int tiles16, int ngroups, int rows);
+hipError_t prepare_dgemm(l2j_ctx *c);
+int product_slices(l2j_ctx *c, int tiles16, int ngroups, int rows);
+void launch_norm(l2j_ctx *c, const RowNorm &n, int rows);
+int launch_dgemm(l2j_ctx *c, std::initializer_list<int> tensors, int layer, const Digits &x, int rows, float *part);
+
+struct RowJob {
+    int nseg, T, pos0;                                        // T positions from pos0 on of nseg sequences; b.tokens: their tokens
+    float *kc, *vc;
+    long seq_stride, layer_stride, head_stride, row_stride;   // of the cache, floats
+    int norm_from;                                            // rows from here on are wanted after the final norm
+};
+int ensure_rows(l2j_ctx *c, int rows);
+hipError_t launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job);
+
+// l2j_batch.hip
+bool matrix_shape(const l2j_config &cf, int tensor, int *rows, int *K);
+int ensure_batch_tiles(l2j_ctx *c);   // the tile-ordered copy of every matrix
+
+// k_pflash (the keys of 16 positions shared by the waves of a workgroup) from this many keys on, while a wave per block of 16
+// positions would leave the compute units with fewer than kSharedKeysBelow waves each; and the keys split over several
+// workgroups from kSplitKeysFrom on.
+constexpr int kSharedKeysFrom = 128, kSharedKeysBelow = 4, kSplitKeysFrom = 192, kPflashMaxSplit = 4;
+inline size_t pflash_lds(int hs, int waves) { return (size_t)(32 * waves + 16 * waves * hs) * sizeof(float); }
+
+}  // namespace l2j

@@ -1,0 +1,448 @@
+// Many positions in one pass over the weights: the kernels between the products of digit_gemm.hpp.  A row is one position
+// of one sequence: row = t * nseg + seg is position pos0 + t of sequence seg (a prompt: nseg = 1; the prompts of a batch
+// side by side: nseg sequences).
+#pragma once
+
+#include "batch_kernels.hpp"
+#include "digit_gemm.hpp"
+
+namespace l2j {
+
+// The sum of a product's slices at four consecutive columns, added in slice order (the loads are independent).
+__device__ __forceinline__ v4f slices4(const float *__restrict__ part, int slices, size_t stride)
+{
+    v4f t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < slices; s++) t += *reinterpret_cast<const v4f *>(part + s * stride);
+    return t;
+}
+
+__device__ __forceinline__ void load16(const float *p, float (&v)[16])
+{
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const v4f f = reinterpret_cast<const v4f *>(p)[q];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[4 * q + e] = f[e];
+    }
+}
+
+struct RowNorm {
+    const float *emb;       // with tokens: the row's x is its token's row of the table (J/Run.java:72)
+    const int *tokens;
+    const float *part;      // else: x += the slices of a product (K/Accum.java:26-30)
+    int slices, nrows;      // nrows: rows of the product's output
+    float *x;               // (rows, dim)
+    const float *w;         // norm weights
+    int dim;
+    Digits dig;             // the normed row as digits,
+    float *xn;              // or, not null, as floats
+};
+
+// x, then w * (ss * x), ss = 1 / sqrt(sum(x^2) / n + 1e-5) (K/RootMeanSquare.java:25-35, K/WeightNormalizeAndScale.java:73).
+// One workgroup per row, four values per thread and step of 4096, which meet in LDS (dim floats) for the digits: sixteen
+// threads write a group's, sixteen values each.
+static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
+{
+    extern __shared__ __align__(16) float ln[];
+    __shared__ float red[16];
+    const int row = blockIdx.x, tid = threadIdx.x, n4 = a.dim >> 2, nt = blockDim.x;
+    v4f *x = reinterpret_cast<v4f *>(a.x + (size_t)row * a.dim), *l4 = reinterpret_cast<v4f *>(ln);
+    const v4f *e = a.tokens ? reinterpret_cast<const v4f *>(a.emb + (size_t)a.tokens[row] * a.dim) : nullptr;
+    const float *part = a.part + (size_t)row * a.dim;
+    const size_t stride = (size_t)a.nrows * a.dim;
+    float ssq = 0.0f;
+    for (int i = tid; i < n4; i += nt) {
+        v4f v;
+        if (e) {
+            v = e[i];
+        } else {
+            const v4f t = slices4(part + 4 * i, a.slices, stride);
+            v = x[i];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = __fadd_rn(v[k], t[k]);
+        }
+        x[i] = v;
+        l4[i] = v;
+        ssq += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+    }
+    ssq = block_sum(ssq, red, nt >> 6);
+    const float ss = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ssq, (float)a.dim), 1e-5f)));
+    for (int i = tid; i < n4; i += nt) {   // (each thread its own values)
+        const v4f w = reinterpret_cast<const v4f *>(a.w)[i];
+        v4f v = l4[i];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = __fmul_rn(w[k], __fmul_rn(ss, v[k]));
+        if (a.xn) reinterpret_cast<v4f *>(a.xn + (size_t)row * a.dim)[i] = v;
+        else l4[i] = v;
+    }
+    if (a.xn) return;
+    __syncthreads();
+    for (int c = tid; c < (a.dim >> 4); c += nt) {
+        float v[16];
+        load16(ln + 16 * c, v);
+        quantize_group(a.dig, row, a.dim >> 8, c >> 4, c & 15, v);
+    }
+}
+
+struct RowQkv {
+    const float *part;       // (slices, rows, dim + 2 kv_dim)
+    int slices, nrows, nseg, pos0;
+    const float2 *rope;      // (seq_len, head_size / 2) cos, sin
+    float *q;                // (rows, dim)
+    float *kc, *vc;          // + seg * seq_stride + kv head * head_stride + position * row_stride
+    long seq_stride, head_stride, row_stride;
+    int dim, kv_dim, head_size;
+};
+
+// q, k and v of a row: the slices added up, RoPE on the pairs of q and k (K/ApplyRope.java:74-90), k and v into the cache row
+// (J/Run.java:95-99).  One workgroup per row, two pairs per thread and step.
+static __global__ void __launch_bounds__(256) k_rows_qkv(const RowQkv a)
+{
+    const int row = blockIdx.x, seg = row % a.nseg, pos = a.pos0 + row / a.nseg, cols = a.dim + 2 * a.kv_dim, hs = a.head_size;
+    const size_t stride = (size_t)a.nrows * cols;
+    const float *part = a.part + (size_t)row * cols;
+    const float4 *rope = reinterpret_cast<const float4 *>(a.rope + (size_t)pos * (hs >> 1));
+    for (int c = 4 * threadIdx.x; c < cols; c += 1024) {
+        const v4f t = slices4(part + c, a.slices, stride);
+        float4 v = make_float4(t[0], t[1], t[2], t[3]);
+        const bool isq = c < a.dim, isk = !isq && c < a.dim + a.kv_dim;
+        const int at = isq ? c : c - a.dim - (isk ? 0 : a.kv_dim);
+        const int head = at / hs, idx = at - head * hs;
+        if (isq || isk) {
+            const float4 cs = rope[idx >> 2];
+            const float r0 = __fsub_rn(__fmul_rn(v.x, cs.x), __fmul_rn(v.y, cs.y)), r1 = __fadd_rn(__fmul_rn(v.x, cs.y), __fmul_rn(v.y, cs.x));
+            const float r2 = __fsub_rn(__fmul_rn(v.z, cs.z), __fmul_rn(v.w, cs.w)), r3 = __fadd_rn(__fmul_rn(v.z, cs.w), __fmul_rn(v.w, cs.z));
+            v = make_float4(r0, r1, r2, r3);
+        }
+        float *o = isq ? a.q + (size_t)row * a.dim + c
+                       : (isk ? a.kc : a.vc) + seg * a.seq_stride + head * a.head_stride + pos * a.row_stride + idx;
+        *reinterpret_cast<float4 *>(o) = v;
+    }
+}
+
+// (rows, K) floats as digits: sixteen values per thread.
+static __global__ void __launch_bounds__(256) k_rows_digits(const float *__restrict__ x, Digits o, int rows, int K)
+{
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const int nc = K >> 4;
+    if (i >= (long)rows * nc) return;   // (whole groups: sixteen lanes leave together)
+    const int row = (int)(i / nc), c = (int)(i - (long)row * nc);
+    float v[16];
+    load16(x + (size_t)row * K + 16 * c, v);
+    quantize_group(o, row, K >> 8, c >> 4, c & 15, v);
+}
+
+// silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74) as digits; part: (slices, rows, 2 hidden), h1 | h3.
+// Workgroup (x, row): four groups of 256, four values per thread; the values meet in LDS for the digits.
+static __global__ void __launch_bounds__(256) k_rows_swiglu(const float *__restrict__ part, int slices, Digits o, int rows, int hidden,
+                                                     const float *__restrict__ silu, int exact)
+{
+    __shared__ __align__(16) float lh[1024];
+    const int row = blockIdx.y, tid = threadIdx.x, col = blockIdx.x * 1024 + 4 * tid;
+    if (col < hidden) {
+        const size_t stride = (size_t)rows * 2 * hidden;
+        const float *p = part + (size_t)row * 2 * hidden + col;
+        const v4f h1 = slices4(p, slices, stride), h3 = slices4(p + hidden, slices, stride);
+        v4f y;
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = __fmul_rn(h1[e], __fmul_rn(silu_sigma(silu, h1[e], exact), h3[e]));
+        *reinterpret_cast<v4f *>(lh + 4 * tid) = y;
+    }
+    __syncthreads();
+    const int g = 4 * blockIdx.x + (tid >> 4);
+    if (tid < 64 && g < (hidden >> 8)) {
+        float v[16];
+        load16(lh + 16 * tid, v);
+        quantize_group(o, row, hidden >> 8, g, tid & 15, v);
+    }
+}
+
+struct RowAttn {
+    const float *q;          // (rows, dim), RoPE applied
+    const float *kc, *vc;    // as RowQkv; the rows of this pass are stored
+    long seq_stride, head_stride, row_stride;
+    float *out;              // (rows, dim)
+    int nseg, T, pos0;       // rows: T positions of nseg sequences
+    int n_heads, kv_mul, dim;
+    float sqrt_hs;
+    int nqb;                 // blocks of 16 positions
+    // k_pflash with the keys of a (head, block) pair split over gridDim.z workgroups (nseg = 1):
+    float *pf_part;          // (head, block, z) x (16 maxima, 16 sums, 16 x head_size values): what each leaves for the last one
+    unsigned *pf_cnt;        // (head, block): how many have; zero between launches
+};
+
+// Causal attention of 16 positions of one head of one sequence per wave on the fp32 matrix cores, as k_pflash multiplies
+// them, without a split of the keys: a wave goes through the cache rows up to its last position (online softmax per tile
+// of 16 keys), up to four waves of neighbouring blocks of the same head per workgroup, so that they find each other's
+// cache rows in the compute unit's cache.  The blocks with the most keys come first.  64 * min(4, nqb) threads, grid:
+// (nqb / 4 rounded up) * nseg * n_heads.
+// Tile u of the values holds the dimensions 64 (u / 4) + 4 m + u % 4, m = 0..15, so that a lane's four values of a cache
+// row are one 16-byte load, and the keys of the next tile are requested before this tile's are multiplied.
+template <int HS>
+static __global__ void __launch_bounds__(256, HS > 128 ? 1 : 2) k_rows_attn(const RowAttn a)
+{
+    constexpr int U = HS / 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int units = a.n_heads * a.nseg, nblk = gridDim.x / units;
+    const int qb = (nblk - 1 - (int)blockIdx.x / units) * nw + wave, u0 = blockIdx.x % units;
+    if (qb >= a.nqb) return;
+    const int h = u0 % a.n_heads, seg = u0 / a.n_heads, kvh = h / a.kv_mul;
+    const int t0 = 16 * qb, tlast = min(t0 + 15, a.T - 1);        // (past the last position: that one again, not stored)
+    const int tq = min(t0 + c, tlast), qpos = a.pos0 + tq, lastkey = a.pos0 + tlast, ntiles = lastkey / 16 + 1;
+    const float *qp = a.q + (size_t)(tq * a.nseg + seg) * a.dim + h * HS + 4 * g;
+    v4f qv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) qv[u] = *reinterpret_cast<const v4f *>(qp + 16 * u);
+    const float *kc = a.kc + seg * a.seq_stride + kvh * a.head_stride, *vc = a.vc + seg * a.seq_stride + kvh * a.head_stride;
+    const long rs = a.row_stride;
+    v4f o[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) o[u] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m = -3.0e38f, l = 0.0f;
+    v4f kf[U];
+    auto keys = [&](int t) {
+        const float *krow = kc + (long)min(16 * t + c, lastkey) * rs + 4 * g;
+#pragma unroll
+        for (int u = 0; u < U; u++) kf[u] = *reinterpret_cast<const v4f *>(krow + 16 * u);
+    };
+    keys(0);
+    for (int t = 0; t < ntiles; t++) {
+        const int k0 = t * 16;
+        v4f vf[4][U / 4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + 4 * c;
+#pragma unroll
+            for (int w = 0; w < U / 4; w++) vf[e][w] = *reinterpret_cast<const v4f *>(vrow + 64 * w);
+        }
+        v4f st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][e], qv[u][e], st, 0, 0, 0);
+        keys(min(t + 1, ntiles - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        float sv[4], tmax = -3.0e38f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            sv[e] = k0 + 4 * g + e <= qpos ? __fdiv_rn(st[e], a.sqrt_hs) : -3.0e38f;
+            tmax = fmaxf(tmax, sv[e]);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        const float mb = fmaxf(m, tmax), sc = expf(m - mb);
+        float pr[4];
+        l *= sc;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            pr[e] = k0 + 4 * g + e <= qpos ? expf(sv[e] - mb) : 0.0f;
+            l += pr[e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) o[u] *= sc;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int u = 0; u < U; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e][u / 4][u % 4], pr[e], o[u], 0, 0, 0);
+        m = mb;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (t0 + c <= tlast) {   // (element i of o[u]: m = 4 g + i)
+        float *op = a.out + (size_t)((t0 + c) * a.nseg + seg) * a.dim + h * HS + 16 * g;
+#pragma unroll
+        for (int w = 0; w < U / 4; w++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                *reinterpret_cast<v4f *>(op + 64 * w + 4 * i) = v4f{__fdiv_rn(o[4 * w][i], l), __fdiv_rn(o[4 * w + 1][i], l), __fdiv_rn(o[4 * w + 2][i], l), __fdiv_rn(o[4 * w + 3][i], l)};
+    }
+}
+
+// Attention of 16 consecutive positions of one sequence for one head on the fp32 matrix cores (after k_rows_qkv has stored
+// their k and v): every cache row is fetched once for the 16 queries, instead of once per query.
+//   scores, transposed: S^T (16 keys x 16 queries) = K (16 keys x HS) . Q^T (HS x 16 queries), HS / 4 v_mfma_f32_16x16x4_f32;
+//     a lane (c = lane % 16, g = lane / 16) then holds S^T[key 4 g + e][query c], e = 0..3: the keys of a query lie in four
+//     lanes, so a query's maximum is two cross-lane steps, and the same registers are the B operand of
+//   values, transposed: O^T (HS x 16 queries) += V^T (HS x 16 keys) . P^T (16 keys x 16 queries), HS / 4 more;
+//   online softmax over the tiles of 16 keys (K/AttentionLoop.java:29-54, K/ExpSumNormalize.java:25-38,
+//     K/AccumWeightedValue.java restated as in k_battn), a query seeing the keys up to its own position.
+// The waves of the workgroup take every WAVES-th tile of keys and merge their (maximum, sum, values) through LDS.
+// The k index of a product may be permuted if both operands are: lane group g supplies the dimensions 16 u + 4 g + e
+// (one 16-byte load per u) and the keys 4 g + e.
+// grid: (n_heads, blocks of 16 positions, 1..4): z splits the tiles of keys over that many workgroups, the last of which to finish merges what the
+// others left in device memory.  64 * WAVES threads; dynamic LDS: (32 WAVES + 16 WAVES HS) floats.
+template <int HS, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) k_pflash(const RowAttn a)
+{
+    constexpr int U = HS / 16;
+    extern __shared__ __align__(16) float pf_lds[];
+    float *wm = pf_lds;                  // [WAVES][16]
+    float *wl = wm + WAVES * 16;         // [WAVES][16]
+    float *wo = wl + WAVES * 16;         // [WAVES][HS / 4][16 queries][4]: dimension d of query q at (d / 4) * 64 + 4 q + d % 4
+    __shared__ float ww[WAVES * 16], wM[16];
+    __shared__ int s_last;
+    const int h = blockIdx.x, qb = blockIdx.y * 16, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int vrows = min(16, a.T - qb);   // (rows past the end repeat the last one: their output is not used)
+    const int pos0 = a.pos0 + qb, kvh = h / a.kv_mul;
+    const float *qp = a.q + (size_t)(qb + min(c, vrows - 1)) * a.dim + h * HS + 4 * g;
+    float4 qv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) qv[u] = *reinterpret_cast<const float4 *>(qp + 16 * u);
+    const int qpos = pos0 + min(c, vrows - 1), lastkey = pos0 + vrows - 1, ntiles = lastkey / 16 + 1;
+    const float *kc = a.kc + kvh * a.head_stride, *vc = a.vc + kvh * a.head_stride;
+    const long rs = a.row_stride;
+    v4f32 o[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) o[u] = v4f32{0.f, 0.f, 0.f, 0.f};
+    float m = -3.0e38f, l = 0.0f;
+    // tile t of the keys goes to workgroup t % NS (z) and there to wave (t / NS) % WAVES: few tiles spread over the workgroups first
+    const int NS = gridDim.z;
+    const int mytiles = (ntiles - (int)blockIdx.z + NS - 1) / NS;   // of this workgroup
+    const int nw = min(WAVES, mytiles);                              // waves that have any
+    for (int t = blockIdx.z + NS * wave; t < ntiles; t += NS * WAVES) {
+        const int k0 = t * 16;
+        const float *krow = kc + (long)min(k0 + c, lastkey) * rs + 4 * g;   // (past the last key: that key again, left out below)
+        float4 kf[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) kf[u] = *reinterpret_cast<const float4 *>(krow + 16 * u);
+        v4f32 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].x, qv[u].x, st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].y, qv[u].y, st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].z, qv[u].z, st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u].w, qv[u].w, st, 0, 0, 0);
+        }
+        float sv[4], tmax = -3.0e38f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            sv[e] = k0 + 4 * g + e <= qpos ? __fdiv_rn(st[e], a.sqrt_hs) : -3.0e38f;   // (a query sees the keys up to its own position)
+            tmax = fmaxf(tmax, sv[e]);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        const float mb = fmaxf(m, tmax), sc = expf(m - mb);
+        float pr[4];
+        l *= sc;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            pr[e] = k0 + 4 * g + e <= qpos ? expf(sv[e] - mb) : 0.0f;
+            l += pr[e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) o[u] *= sc;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + c;
+#pragma unroll
+            for (int u = 0; u < U; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * u], pr[e], o[u], 0, 0, 0);
+        }
+        m = mb;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) { wm[wave * 16 + c] = m; wl[wave * 16 + c] = l; }
+    if (wave < nw) {   // (the waves without a tile have nothing to add)
+#pragma unroll
+        for (int u = 0; u < U; u++)   // (a lane's four dimensions 16 u + 4 g + e of query c as one 16-byte store, a wave's stores 1 KB in a row)
+            *reinterpret_cast<v4f32 *>(&wo[wave * HS * 16 + (4 * u + g) * 64 + 4 * c]) = o[u];
+    }
+    __syncthreads();
+    if (tid < 16 * WAVES) {   // weight of wave w's part in query q's sum: tid = w * 16 + q (a workgroup without any tile leaves
+        const int q = tid & 15;   // maximum -3e38, sum 0 and values 0)
+        float M = wm[q];
+#pragma unroll
+        for (int w = 1; w < WAVES; w++) M = fmaxf(M, wm[w * 16 + q]);
+        ww[tid] = expf(wm[tid] - M);
+        if (tid < 16) wM[tid] = M;
+    }
+    __syncthreads();
+    if (NS == 1) {
+        for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {   // the waves' parts of a query merged
+            const int d = (idx >> 6) * 4 + (idx & 3), q = (idx >> 2) & 15;   // (neighbouring lanes read neighbouring words of LDS)
+            float L = 0.0f, O = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                if (w < nw) {
+                    const float wt = ww[w * 16 + q];
+                    L += wt * wl[w * 16 + q];
+                    O += wt * wo[w * HS * 16 + idx];
+                }
+            }
+            if (q < vrows) a.out[(long)(qb + q) * a.dim + h * HS + d] = __fdiv_rn(O, L);
+        }
+        return;
+    }
+    // The keys are split over NS workgroups: each leaves its maxima, sums and values (not yet divided) in device memory, and
+    // the last one to do so merges them all.
+    constexpr int PER = 32 + 16 * HS;
+    const int pair = h * gridDim.y + blockIdx.y;
+    float *mine = a.pf_part + ((long)pair * NS + blockIdx.z) * PER;
+    for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {   // (values in the order they have in LDS)
+        const int d = (idx >> 6) * 4 + (idx & 3), q = (idx >> 2) & 15;
+        float L = 0.0f, O = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            if (w < nw) {
+                const float wt = ww[w * 16 + q];
+                L += wt * wl[w * 16 + q];
+                O += wt * wo[w * HS * 16 + idx];
+            }
+        }
+        st_coh(mine + 32 + idx, O);
+        if (d == 0) { st_coh(mine + q, wM[q]); st_coh(mine + 16 + q, L); }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (this thread's stores have arrived where the other workgroups read)
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned old = __hip_atomic_fetch_add(a.pf_cnt + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = old + 1u == (unsigned)NS;
+        if (s_last) __hip_atomic_store(a.pf_cnt + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (for the next launch)
+    }
+    __syncthreads();
+    if (!s_last) return;
+    const float *all = a.pf_part + (long)pair * NS * PER;
+    for (int idx = tid; idx < HS * 16; idx += 64 * WAVES) {
+        const int q = (idx >> 2) & 15;
+        float mz[4], M = -3.0e38f;
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            mz[z] = z < NS ? ld_coh(all + (long)z * PER + q) : -3.0e38f;
+            M = fmaxf(M, mz[z]);
+        }
+        float L = 0.0f, O = 0.0f;
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            if (z < NS) {
+                const float wt = expf(mz[z] - M);
+                L += wt * ld_coh(all + (long)z * PER + 16 + q);
+                O += wt * ld_coh(all + (long)z * PER + 32 + idx);
+            }
+        }
+        if (q < vrows) a.out[(long)(qb + q) * a.dim + h * HS + (idx >> 6) * 4 + (idx & 3)] = __fdiv_rn(O, L);
+    }
+}
+
+// logits = W x for one row x (K/MatMul.java:37-60): a wave per row of the classifier.
+static __global__ void __launch_bounds__(256) k_rows_logits(const float *__restrict__ w, const float *__restrict__ x, float *__restrict__ logits,
+                                                     int dim, int vocab)
+{
+    extern __shared__ __align__(16) float lx[];
+    const int n4 = dim >> 2, lane = threadIdx.x & 63;
+    float4 *l4 = reinterpret_cast<float4 *>(lx);
+    for (int i = threadIdx.x; i < n4; i += 256) l4[i] = reinterpret_cast<const float4 *>(x)[i];
+    __syncthreads();
+    for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < vocab; r += 4 * gridDim.x) {
+        const float4 *wr = reinterpret_cast<const float4 *>(w + (size_t)r * dim);
+        float t = 0.0f;
+#pragma unroll 8
+        for (int i = lane; i < n4; i += 64) t += dot4(load_stream(wr + i), l4[i]);
+        t = wave_sum(t);
+        if (lane == 0) logits[r] = t;
+    }
+}
+
+}  // namespace l2j

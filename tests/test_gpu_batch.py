@@ -338,3 +338,40 @@ def test_release_batch_gives_the_memory_back_and_the_next_call_makes_it_again():
     g.reset()
     np.testing.assert_array_equal(g.decode_greedy(prompts[0], 24)[0], single)   # the single-sequence path: untouched
     g.close()
+
+
+@pytest.mark.parametrize("n_seq,shortest,longest", [(16, 1, 1), (16, 2, 5), (32, 15, 18), (32, 33, 40), (16, 66, 70)])
+def test_common_prompt_positions_taken_at_once(orc, n_seq, shortest, longest):
+    """Prompts for every sequence: the positions whose inputs all sequences know (up to the shortest prompt) are one pass, or
+    several (1024 rows each), the loop goes on behind them.  Tokens as every sequence decodes alone, with and without the
+    logits kept, and the logits of every step the oracle's."""
+    shape = SHAPES[1][:6] + (80,) + SHAPES[1][7:]
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    rng = np.random.default_rng(n_seq + shortest)
+    lengths = rng.integers(shortest, longest + 1, size=n_seq)
+    lengths[1], lengths[2] = shortest, longest
+    prompts = [rng.integers(2, shape[5], size=int(n)).astype(np.int32) for n in lengths]
+    for steps in (longest + 6, max(1, shortest - 1)):        # on behind the prompts; inside them
+        got, sec = g.decode_greedy_batch(prompts, steps, n_seq=n_seq)
+        assert sec >= 0
+        kept, logits = g.decode_greedy_batch(prompts, steps, n_seq=n_seq, want_logits=True)
+        np.testing.assert_array_equal(kept, got)
+        m = oracle_of(orc, shape, 9)
+        for b in range(n_seq):
+            g.reset()
+            want, _ = g.decode_greedy(prompts[b], steps)
+            same_until_a_tie(got[b, :len(want)], want, logits[:, b], "sequence %d" % b)
+            if b < 4:
+                check_against_oracle(m, prompts[b], steps, got[b], logits[:, b], "sequence %d against the oracle" % b)
+        m.close()
+        seeds = rng.integers(0, 2**40, size=n_seq).astype(np.int64)
+        sampled, _, lg = g.decode_sample_batch(prompts, steps, 0.9, 0.9, seeds, n_seq=n_seq, want_logits=True)
+        again, _ = g.decode_sample_batch(prompts, steps, 0.9, 0.9, seeds, n_seq=n_seq)
+        np.testing.assert_array_equal(again, sampled)
+        for b in (0, 1, 2, n_seq - 1):
+            s = orc.Sampler(int(seeds[b]), shape[5])
+            want = [int(prompts[b][pos]) if pos < lengths[b] else s.step(lg[pos, b], 0.9, 0.9)[0] for pos in range(steps)]
+            np.testing.assert_array_equal(sampled[b], np.array(want, dtype=np.int32), err_msg="sequence %d" % b)
+    g.close()

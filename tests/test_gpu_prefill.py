@@ -221,3 +221,35 @@ def test_the_keys_of_a_head_split_over_one_to_four_workgroups(shape):
         assert rel_err(got, want.astype(np.float64)) < CLOSE, split
         assert rel_err(got_k, want_k.astype(np.float64)) < CLOSE and rel_err(got_v, want_v.astype(np.float64)) < CLOSE, split
     g.close()
+
+
+@pytest.mark.parametrize("shape", [
+    (512, 1024, 2, 8, 2, 1008, 1104, 0),     # head 64, grouped-query attention: a wave per 16 positions and shared keys
+    (256, 768, 2, 1, 1, 512, 304, 1),        # head 256, one head: one group per row, three per hidden row
+])
+def test_passes_of_many_positions(shape):
+    """Edges of the tiles of 32 and 64 positions, of a pass (1024 positions; one more makes two passes of half), and a second
+    call behind cached positions, against position by position: logits of the last position and the cache rows."""
+    seq_len, kvd = shape[6], shape[0] // shape[3] * shape[4]
+    rng = np.random.default_rng(shape[0])
+    g = model(shape)
+    tokens = np.concatenate([[1], rng.integers(2, shape[5], size=seq_len - 1)]).astype(np.int32)
+    sizes = [n for n in (2, 63, 64, 65, 129, 257, 300, 1024, 1025, 1104) if n <= seq_len]
+    want = {}
+    for i, t in enumerate(tokens):
+        lg = g.forward(int(t), i, want_logits=i + 1 in sizes)
+        if i + 1 in sizes:
+            want[i + 1] = lg
+    want_k, want_v = (x.reshape(shape[2], seq_len, kvd) for x in caches(g, shape))
+    for n in sizes:
+        for first in ((0,) if n < 65 else (0, n // 3)):
+            g.reset()
+            if first:
+                g.prefill(tokens[:first], want_logits=False)
+            got, _ = g.prefill(tokens[first:n], pos0=first)
+            assert rel_err(got, want[n].astype(np.float64)) < CLOSE, (n, first)
+            k, v = (x.reshape(shape[2], seq_len, kvd) for x in caches(g, shape))
+            assert rel_err(k[:, :n], want_k[:, :n].astype(np.float64)) < CLOSE, (n, first)
+            assert rel_err(v[:, :n], want_v[:, :n].astype(np.float64)) < CLOSE, (n, first)
+            assert not k[:, n:].any() and not v[:, n:].any(), (n, first)
+    g.close()
