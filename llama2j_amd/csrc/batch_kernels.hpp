@@ -448,11 +448,14 @@ __global__ void __launch_bounds__(kBgThreads) k_bgemm_f32(const BGemmF32 a)
 
 // ---- the element-wise kernels between the products --------------------------------------------------------------
 
+constexpr int kLogSlots = 32;   // steps whose logits are on their way to the caller while the next ones are computed
+
 // Loop state of a batched decode, on the device.
 struct BatchState {
     int pos;              // position of the step being computed
     int token[kMaxBatch];    // input token of every sequence at this position
     int n_prompt[kMaxBatch];
+    float *log;           // null, or kLogSlots x (sequences, vocab): the logits of step pos also go to slot pos % kLogSlots
 };
 
 // x[b] = row token[b] of the embedding table (J/Run.java:72).  As the first kernel of a step it also clears the
@@ -659,6 +662,8 @@ static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *
     __shared__ int bidx[16];
     const int b = blockIdx.x, tid = threadIdx.x;
     const long n = (long)gridDim.x * a.vocab;
+    const int pos = a.st->pos;
+    float *log = a.st->log ? a.st->log + (pos % kLogSlots) * n + (long)b * a.vocab : nullptr;
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
     for (int i = tid; i < a.vocab; i += 1024) {
@@ -666,6 +671,7 @@ static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *
 #pragma unroll 8
         for (int s = 0; s < a.slices; s++) t += a.part[(long)s * n + (long)b * a.vocab + i];
         a.logits[(long)b * a.vocab + i] = t;
+        if (log) log[i] = t;
         if (better(t, i, bv, bi)) { bv = t; bi = i; }
     }
 #pragma unroll
@@ -680,7 +686,6 @@ static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *
         for (int w = 1; w < 16; w++)
             if (better(bval[w], bidx[w], bv, bi)) { bv = bval[w]; bi = bidx[w]; }
         if (bi == 0x7fffffff) bi = 0;
-        const int pos = a.st->pos;
         const int next = pos < a.st->n_prompt[b] ? a.prompts[(long)b * a.prompt_stride + pos] : bi;
         a.out_tokens[(long)b * a.out_stride + pos] = next;
         a.st->token[b] = next;

@@ -5,6 +5,9 @@
 #include "rows_kernels.hpp"
 #include "rows.hpp"
 
+#include <condition_variable>
+#include <thread>
+
 using namespace l2j;
 
 bool l2j::matrix_shape(const l2j_config &cf, int tensor, int *rows, int *K)
@@ -143,12 +146,32 @@ struct l2j::BatchBufs {
     int fuse_opt = 0;              // option batch_fuse when the step was planned
     int h_fault = 0;
     int *h_pin = nullptr;   // pinned: every transfer of a call goes through it, as in the single-sequence loops
+    // the logits of every step for a caller that wants them: kept here while later steps are computed, made by the first such call
+    float *log_dev = nullptr, *log_pin = nullptr;   // kLogSlots steps on the device, one pinned
+    hipStream_t log_stream = nullptr;
+    hipEvent_t log_step[kLogSlots] = {};            // the slot holds its step's logits
     BatchSamplers samplers;   // l2j_decode_sample_batch: a sampler per sequence (made by its first call)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    hipError_t ensure_log(size_t step_floats)
+    {
+        if (log_step[kLogSlots - 1]) return hipSuccess;
+        hipError_t e = hipSuccess;
+        if (!log_dev) e = hipMalloc(reinterpret_cast<void **>(&log_dev), kLogSlots * step_floats * sizeof(float));
+        if (e == hipSuccess && !log_pin) e = hipHostMalloc(reinterpret_cast<void **>(&log_pin), step_floats * sizeof(float), hipHostMallocDefault);
+        if (e == hipSuccess && !log_stream) e = hipStreamCreateWithFlags(&log_stream, hipStreamNonBlocking);
+        for (int i = 0; i < kLogSlots; i++)
+            if (e == hipSuccess && !log_step[i]) e = hipEventCreateWithFlags(&log_step[i], hipEventDisableTiming);
+        return e;
+    }
     void release()
     {
+        for (hipEvent_t ev : log_step)
+            if (ev) (void)hipEventDestroy(ev);
+        if (log_stream) (void)hipStreamDestroy(log_stream);
+        (void)hipFree(log_dev);
+        if (log_pin) (void)hipHostFree(log_pin);
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         if (e0) (void)hipEventDestroy(e0);
@@ -418,6 +441,87 @@ int seed_batch_samplers(l2j_ctx *c, BatchBufs &b, const int64_t *seeds)
     return L2J_OK;
 }
 
+// Brings the logits of the steps of one call to the caller's memory while later steps are computed, in a thread of its own:
+// the copy into memory the caller has just been given (page faults included) takes about as long as a step of a small
+// model.  The thread waits for a step on the host: a queue that waits for another one on the device (hipStreamWaitEvent) made the
+// 100 kernels of a step 1 us longer each (1745 -> 1853 us per replay of a graph of 100 kernels, 1757 us with the copies alone).
+class LogTaker {
+public:
+    LogTaker(const BatchBufs &b_, float *out_, size_t step_floats_, int device_) : b(b_), out(out_), step_floats(step_floats_), device(device_)
+    {
+        if (out) th = std::thread([this] { run(); });
+    }
+    ~LogTaker()
+    {
+        if (!th.joinable()) return;
+        {
+            std::lock_guard<std::mutex> l(mu);
+            stop = true;
+        }
+        cv.notify_all();
+        th.join();
+    }
+    // the slot of step `pos` is free (or a copy has failed)
+    void wait_slot(int pos)
+    {
+        std::unique_lock<std::mutex> l(mu);
+        cv.wait(l, [&] { return err != hipSuccess || pos - taken < kLogSlots; });
+    }
+    // log_step of step `pos` has been recorded
+    void offer(int pos)
+    {
+        {
+            std::lock_guard<std::mutex> l(mu);
+            offered = pos + 1;
+        }
+        cv.notify_all();
+    }
+    hipError_t wait_all()
+    {
+        std::unique_lock<std::mutex> l(mu);
+        cv.wait(l, [&] { return err != hipSuccess || taken == offered; });
+        return err;
+    }
+
+private:
+    const BatchBufs &b;
+    float *out;
+    size_t step_floats;
+    int device;
+    std::mutex mu;
+    std::condition_variable cv;
+    int offered = 0, taken = 0;
+    bool stop = false;
+    hipError_t err = hipSuccess;
+    std::thread th;
+
+    void run()
+    {
+        hipError_t e = hipSetDevice(device);
+        for (int i = 0; ; i++) {
+            {
+                std::unique_lock<std::mutex> l(mu);
+                if (e != hipSuccess) err = e;
+                else cv.wait(l, [&] { return stop || offered > i; });
+                if (err != hipSuccess || offered <= i) {
+                    cv.notify_all();
+                    return;
+                }
+            }
+            const int slot = i % kLogSlots;
+            e = hipEventSynchronize(b.log_step[slot]);
+            if (e == hipSuccess) e = hipMemcpyAsync(b.log_pin, b.log_dev + slot * step_floats, step_floats * sizeof(float), hipMemcpyDeviceToHost, b.log_stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(b.log_stream);
+            if (e == hipSuccess) memcpy(out + (size_t)i * step_floats, b.log_pin, step_floats * sizeof(float));
+            {
+                std::lock_guard<std::mutex> l(mu);
+                if (e == hipSuccess) taken = i + 1;
+            }
+            cv.notify_all();
+        }
+    }
+};
+
 // logits_log: null, or steps x n_seq x vocab_size floats of the caller that receive the logits of every step.
 // seeds: null (every unforced token is the argmax), or the seed of every sequence's sampler: unforced tokens are sampled as
 // l2j_sample does at this temperature (not 0) and topp.
@@ -451,14 +555,14 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     const size_t state_ints = sizeof(BatchState) / sizeof(int);
     unsigned cur = 0;   // bit s: the copy of its ProbIndex array that sequence s's last top-p step left
     if (seeds && (rc = seed_batch_samplers(c, b, seeds))) return rc;
-    float *dlog = nullptr;
+    const size_t step_floats = (size_t)nseq * vocab;
     if (logits_log) {
-        hipError_t me = hipMalloc(reinterpret_cast<void **>(&dlog), (size_t)steps * nseq * vocab * sizeof(float));
-        if (me != hipSuccess) return hip_rc(me, "logits of every step");
+        const hipError_t le = b.ensure_log(step_floats);
+        if (le != hipSuccess) return hip_rc(le, "logits of every step");
     }
     auto fail_hip = [&](hipError_t e, const char *what) {
         (void)hipStreamSynchronize(c->stream);
-        (void)hipFree(dlog);
+        if (b.log_stream) (void)hipStreamSynchronize(b.log_stream);
         return hip_rc(e, what);
     };
     // The positions whose input tokens are known for every sequence (BOS and the shortest prompt) are taken at once, nseq
@@ -467,10 +571,11 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     for (int i = 0; i < nseq; i++) known = std::min(known, n_prompt[i] + 1);
     if (known < 2 || b.step_grid > 0) known = 0;
     const int per = std::min(known, kRowsMax / nseq);
-    if (known > 0 && (rc = ensure_rows(c, per * nseq))) { (void)hipFree(dlog); return rc; }
+    if (known > 0 && (rc = ensure_rows(c, per * nseq))) return rc;
     BatchState h{};
-    h.pos = known > 0 && !dlog ? known - 1 : 0;
+    h.pos = known > 0 && !logits_log ? known - 1 : 0;
     for (int i = 0; i < nseq; i++) { h.token[i] = 1; h.n_prompt[i] = n_prompt[i]; }   // BOS first (J/Run.java:612)
+    h.log = logits_log ? b.log_dev : nullptr;
     memcpy(b.h_pin, &h, sizeof(h));
     memset(b.h_pin + state_ints, 0, (size_t)nseq * pcap * sizeof(int));
     for (int s = 0; s < nseq && prompt_stride > 0; s++)
@@ -482,11 +587,14 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     if (e == hipSuccess) e = hipMemcpyAsync(b.prompts, b.h_pin + state_ints, (size_t)nseq * pcap * sizeof(int), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(b.done, 0, sizeof(unsigned), c->stream);
     if (e != hipSuccess) return fail_hip(e, "state upload");
+    LogTaker taker(b, logits_log, step_floats, cf.device);
     // after the logits of a position: kept for the caller, and J/Run.java:643-665 for the sequences whose prompt is used up
     // (the sampled token replaces the argmax k_bnext stored)
     auto after_logits = [&](int pos) {
-        if (dlog && e == hipSuccess)
-            e = hipMemcpyAsync(dlog + (size_t)pos * nseq * vocab, b.logits, (size_t)nseq * vocab * sizeof(float), hipMemcpyDeviceToDevice, c->stream);
+        if (logits_log && e == hipSuccess) {
+            e = hipEventRecord(b.log_step[pos % kLogSlots], c->stream);
+            if (e == hipSuccess) taker.offer(pos);
+        }
         if (seeds && e == hipSuccess) {
             unsigned active = 0;
             for (int s = 0; s < nseq; s++) active |= pos >= n_prompt[s] ? 1u << s : 0u;
@@ -505,17 +613,19 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
         for (int t0 = 0; t0 < known && e == hipSuccess; t0 += per) {
             job.pos0 = t0; job.T = std::min(per, known - t0);
             const bool last = t0 + job.T == known;
-            job.norm_from = dlog ? 0 : last ? (job.T - 1) * nseq : job.T * nseq;
+            job.norm_from = logits_log ? 0 : last ? (job.T - 1) * nseq : job.T * nseq;
             e = hipMemcpyAsync(c->rows.tokens, h_rows + (size_t)t0 * nseq, (size_t)job.T * nseq * sizeof(int), hipMemcpyHostToDevice, c->stream);
             if (e == hipSuccess) e = launch_rows(c, c->rows, job);
-            for (int t = dlog ? 0 : job.T - 1; t < job.T && (dlog || last) && e == hipSuccess; t++) {
-                launch_batch_tokens(c, b, c->rows.xn + (dlog ? (size_t)t * nseq * cf.dim : 0));
+            for (int t = logits_log ? 0 : job.T - 1; t < job.T && (logits_log || last) && e == hipSuccess; t++) {
+                if (logits_log) taker.wait_slot(t0 + t);
+                launch_batch_tokens(c, b, c->rows.xn + (logits_log ? (size_t)t * nseq * cf.dim : 0));
                 e = hipGetLastError();
                 after_logits(t0 + t);
             }
         }
     }
     for (int pos = known; pos < steps && e == hipSuccess; pos++) {
+        if (logits_log) taker.wait_slot(pos);
         if (b.exec) {
             e = hipGraphLaunch(b.exec, c->stream);
         } else {
@@ -527,18 +637,13 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     }
     if (e == hipSuccess) e = hipEventRecord(b.e1, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(b.h_pin, b.out, (size_t)nseq * cap * sizeof(int), hipMemcpyDeviceToHost, c->stream);
+    if (logits_log && e == hipSuccess) e = taker.wait_all();
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return fail_hip(e, "step");
     for (int s = 0; s < nseq; s++) {
         memcpy(out_tokens + (size_t)s * steps, b.h_pin + (size_t)s * cap, (size_t)steps * sizeof(int));
         if (known > 1 && !logits_log)   // (the outputs of the known positions but the last are the prompt's ids)
             memcpy(out_tokens + (size_t)s * steps, prompts + (size_t)s * prompt_stride, (size_t)(known - 1) * sizeof(int));
-    }
-    if (dlog) {
-        e = hipMemcpy(logits_log, dlog, (size_t)steps * nseq * vocab * sizeof(float), hipMemcpyDeviceToHost);
-        (void)hipFree(dlog);
-        dlog = nullptr;
-        if (e != hipSuccess) return hip_rc(e, "logits read-back");
     }
     if (seeds) {   // the reference's exceptions, as in l2j_sample
         SamplerState h[kMaxBatch] = {};
