@@ -9,19 +9,19 @@ using namespace l2j;
 namespace {
 
 // The two shapes of k_dgemm: 256 rows of the matrix x 32 vectors per workgroup, two of which share a compute unit, and
-// 512 x 64, one per compute unit.  Microseconds per group of 256: a workgroup in a round of workgroups that leaves compute
-// units idle (alone), in one that just fills its slots (last), in the rounds before the last (full); before the first and after the last group
-// (start).  Fitted to 424 launches at the products of Llama-2-7B with 32 to 1024 vectors and 1 to 16 slices (10 % root mean
-// square; the pick is 5 % slower than the best of the launches on average, 20 % at most), the full rounds to the same
-// products inside a forward pass of 1024 positions, where the clock is lower than in a short burst.
-struct Variant { int pt, nw, per_cu; double alone, last, full, start; };
-constexpr Variant kVariants[2] = {{1, 4, 2, 2.44, 6.2, 4.2, 4.3}, {2, 8, 1, 4.9, 7.2, 7.2, 7.7}};
+// 512 x 64, one per compute unit.  Microseconds per group of 256: the only workgroup of its compute unit (alone), in a round that
+// fills the slots (shared), in the rounds before the last (full); before the first and after the last group (start).  Fitted
+// to 800 launches at the products of Llama-2-7B with 32 to 1024 vectors and 1 to 16 slices (9 % root mean square; the
+// pick is 3 % slower than the best of the launches on average, 11 % at most), the full rounds to the same products inside
+// a forward pass of 1024 positions, where the clock is lower than in a short burst.
+struct Variant { int pt, nw, per_cu; double alone, shared, full, start; };
+constexpr Variant kVariants[2] = {{1, 4, 2, 2.3, 3.8, 4.2, 4.3}, {2, 8, 1, 4.9, 7.2, 7.2, 7.7}};
 
 }  // namespace
 
 // How the product of `tiles16` 16-row tiles (rows of K = 256 ngroups) with `rows` vectors is launched: the variant and the
 // groups per slice of K with the smallest estimate: rounds of workgroups over the compute units, and the slices' sums
-// written and read again (0.25 us per MB).  It depends on the shape alone, so a shape always adds up in the same order.
+// written and read again (0.2 us per MB).  It depends on the shape alone, so a shape always adds up in the same order.
 DgPlan l2j::dgemm_plan(int n_cu, int tiles16, int ngroups, int rows)
 {
     DgPlan best;
@@ -34,11 +34,9 @@ DgPlan l2j::dgemm_plan(int n_cu, int tiles16, int ngroups, int rows)
             if ((ngroups + gps - 1) / gps != s) continue;
             const long wgs = (long)nrow * ncol * s, slots = (long)n_cu * k.per_cu;
             const long full = wgs / slots, rest = wgs % slots;
-            double us = full * (gps * k.full + k.start) + 0.25e-6 * s * rows * tiles16 * 64;
+            double us = full * (gps * k.full + k.start) + 0.2e-6 * s * rows * tiles16 * 64;
             if (rest > 0) {
-                const double fill = (double)rest / slots;
-                const double group = full > 0 ? k.alone + (k.full - k.alone) * fill
-                                              : k.alone + (k.last - k.alone) * (k.per_cu == 2 ? std::max(0.0, 2.0 * fill - 1.0) : fill);
+                const double group = k.per_cu == 2 ? (rest <= n_cu ? k.alone : k.shared) : k.alone + (k.shared - k.alone) * rest / slots;
                 us += gps * group + k.start;
             }
             if (best_us == 0.0 || us < best_us) {
@@ -57,6 +55,10 @@ hipError_t l2j::prepare_dgemm(l2j_ctx *c)
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dgemm<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)dgemm_lds<2>());
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_norm), hipFuncAttributeMaxDynamicSharedMemorySize, 128 << 10);
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_logits), hipFuncAttributeMaxDynamicSharedMemorySize, 128 << 10);
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<64, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(64, 2));
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<128, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(128, 1));
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<128, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(128, 2));
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<256, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(256, 1));
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_pflash<64, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)pflash_lds(64, 16));
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_pflash<128, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)pflash_lds(128, 16));
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_pflash<256, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)pflash_lds(256, 8));
@@ -144,6 +146,21 @@ hipError_t RowBufs::alloc(l2j_ctx *c, int rows, bool attention)
     return e;
 }
 
+// Blocks of 32 positions (the cache rows loaded once for 32) from where their pairs still fill the compute units; pairs of blocks
+// unless one block per workgroup already leaves compute units idle.
+template <int HS>
+static void launch_attn(l2j_ctx *c, RowAttn t)
+{
+    const int units = c->cfg.n_heads / (256 / HS) * t.nseg;
+    auto blocks = [&](int q) { return (t.T + q - 1) / q; };
+    const bool two = HS < 256 && (blocks(32) + 1) / 2 * units >= c->n_cu;
+    const int n = blocks(two ? 32 : 16);
+    t.paired = n * units > c->n_cu;
+    const dim3 g((t.paired ? (n + 1) / 2 : n) * units), blk(64 * attn_waves(HS));
+    if (two) hipLaunchKernelGGL((k_rows_attn<HS, HS < 256 ? 2 : 1>), g, blk, attn_lds(HS, 2), c->stream, t);
+    else hipLaunchKernelGGL((k_rows_attn<HS, 1>), g, blk, attn_lds(HS, 1), c->stream, t);
+}
+
 // The forward passes of job.T positions of job.nseg sequences: their k and v rows are left in the cache and, from row
 // job.norm_from on, the rows after the final norm in b.xn.
 hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
@@ -155,7 +172,9 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
     // Few blocks of 16 positions over many keys: the keys of a block dealt to the waves of a workgroup (and to several
     // workgroups), else a wave per block.
     const int flash = c->opt[OPT_PREFILL_FLASH], keys = job.pos0 + job.T;
-    const bool shared_keys = job.nseg == 1 && flash != 0 && (flash == 2 || (keys >= kSharedKeysFrom && cf.n_heads * nqb < kSharedKeysBelow * c->n_cu));
+    const long waves = (long)cf.n_heads * job.nseg * nqb;   // of a wave per block
+    const bool far = (long)keys * job.row_stride > UINT32_MAX;   // (past the 32-bit offsets of k_rows_attn)
+    const bool shared_keys = job.nseg == 1 && (far || (flash != 0 && (flash == 2 || (keys >= kSharedKeysFrom && waves < kSharedKeysBelow * c->n_cu))));
     int split = 1;
     if (shared_keys) {
         const int opt = c->opt[OPT_PREFILL_SPLIT];
@@ -171,6 +190,7 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
             b.pf_blocks = nqb;
         }
     }
+    const int qkv_parts = std::min((dim + 2 * kvd + 1023) / 1024, std::max(1, 4 * c->n_cu / rows));   // (few rows: their columns over several workgroups)
     RowNorm n{};
     n.emb = c->emb; n.nrows = rows; n.x = b.x; n.dim = dim; n.dig = b.dig;
     n.tokens = b.tokens; n.w = c->rmsw;
@@ -184,25 +204,24 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
         k.kc = job.kc + l * job.layer_stride; k.vc = job.vc + l * job.layer_stride;
         k.seq_stride = job.seq_stride; k.head_stride = job.head_stride; k.row_stride = job.row_stride;
         k.dim = dim; k.kv_dim = kvd; k.head_size = hs;
-        hipLaunchKernelGGL(k_rows_qkv, dim3(rows), dim3(256), 0, s, k);
+        hipLaunchKernelGGL(k_rows_qkv, dim3(rows, qkv_parts), dim3(256), 0, s, k);
         RowAttn t{};
         t.q = b.q; t.kc = k.kc; t.vc = k.vc; t.seq_stride = k.seq_stride; t.head_stride = k.head_stride; t.row_stride = k.row_stride;
         t.out = b.xb; t.nseg = job.nseg; t.T = job.T; t.pos0 = job.pos0; t.n_heads = cf.n_heads; t.kv_mul = c->kv_mul; t.dim = dim;
-        t.sqrt_hs = sqrtf((float)hs); t.nqb = nqb; t.pf_part = b.pf_part; t.pf_cnt = b.pf_cnt;
+        t.dig = b.dig; t.sqrt_hs = sqrtf((float)hs); t.nqb = nqb; t.pf_part = b.pf_part; t.pf_cnt = b.pf_cnt;
         if (shared_keys) {
             const dim3 g(cf.n_heads, nqb, split);
             if (hs == 64) hipLaunchKernelGGL((k_pflash<64, 16>), g, dim3(1024), pflash_lds(64, 16), s, t);
             else if (hs == 128) hipLaunchKernelGGL((k_pflash<128, 16>), g, dim3(1024), pflash_lds(128, 16), s, t);
             else hipLaunchKernelGGL((k_pflash<256, 8>), g, dim3(512), pflash_lds(256, 8), s, t);
+            hipLaunchKernelGGL(k_rows_digits, dim3((unsigned)(((long)rows * (dim / 16) + 255) / 256)), dim3(256), 0, s, b.xb, b.dig, rows, dim);
+        } else if (hs == 64) {
+            launch_attn<64>(c, t);
+        } else if (hs == 128) {
+            launch_attn<128>(c, t);
         } else {
-            const int nw = std::min(4, nqb);
-            const dim3 g((unsigned)((nqb + nw - 1) / nw * cf.n_heads * job.nseg)), blk(64 * nw);
-            if (hs == 64) hipLaunchKernelGGL(k_rows_attn<64>, g, blk, 0, s, t);
-            else if (hs == 128) hipLaunchKernelGGL(k_rows_attn<128>, g, blk, 0, s, t);
-            else hipLaunchKernelGGL(k_rows_attn<256>, g, blk, 0, s, t);
+            launch_attn<256>(c, t);
         }
-        const unsigned chunks = (unsigned)(((long)rows * (dim / 16) + 255) / 256);
-        hipLaunchKernelGGL(k_rows_digits, dim3(chunks), dim3(256), 0, s, b.xb, b.dig, rows, dim);
         n.slices = launch_dgemm(c, {L2J_WO}, l, b.dig, rows, b.part);
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, rows);

@@ -96,14 +96,14 @@ struct RowQkv {
 };
 
 // q, k and v of a row: the slices added up, RoPE on the pairs of q and k (K/ApplyRope.java:74-90), k and v into the cache row
-// (J/Run.java:95-99).  One workgroup per row, two pairs per thread and step.
+// (J/Run.java:95-99).  grid (rows, parts of the columns), two pairs per thread and step.
 static __global__ void __launch_bounds__(256) k_rows_qkv(const RowQkv a)
 {
     const int row = blockIdx.x, seg = row % a.nseg, pos = a.pos0 + row / a.nseg, cols = a.dim + 2 * a.kv_dim, hs = a.head_size;
     const size_t stride = (size_t)a.nrows * cols;
     const float *part = a.part + (size_t)row * cols;
     const float4 *rope = reinterpret_cast<const float4 *>(a.rope + (size_t)pos * (hs >> 1));
-    for (int c = 4 * threadIdx.x; c < cols; c += 1024) {
+    for (int c = 4 * (threadIdx.x + 256 * blockIdx.y); c < cols; c += 1024 * gridDim.y) {
         const v4f t = slices4(part + c, a.slices, stride);
         float4 v = make_float4(t[0], t[1], t[2], t[3]);
         const bool isq = c < a.dim, isk = !isq && c < a.dim + a.kv_dim;
@@ -162,101 +162,150 @@ struct RowAttn {
     const float *q;          // (rows, dim), RoPE applied
     const float *kc, *vc;    // as RowQkv; the rows of this pass are stored
     long seq_stride, head_stride, row_stride;
-    float *out;              // (rows, dim)
+    float *out;              // (rows, dim): k_pflash
+    Digits dig;              // k_rows_attn
     int nseg, T, pos0;       // rows: T positions of nseg sequences
     int n_heads, kv_mul, dim;
     float sqrt_hs;
-    int nqb;                 // blocks of 16 positions
+    int nqb;                 // blocks of 16 positions (k_pflash)
+    int paired;              // k_rows_attn: two blocks per workgroup
     // k_pflash with the keys of a (head, block) pair split over gridDim.z workgroups (nseg = 1):
     float *pf_part;          // (head, block, z) x (16 maxima, 16 sums, 16 x head_size values): what each leaves for the last one
     unsigned *pf_cnt;        // (head, block): how many have; zero between launches
 };
 
-// Causal attention of 16 positions of one head of one sequence per wave on the fp32 matrix cores, as k_pflash multiplies
-// them, without a split of the keys: a wave goes through the cache rows up to its last position (online softmax per tile
-// of 16 keys), up to four waves of neighbouring blocks of the same head per workgroup, so that they find each other's
-// cache rows in the compute unit's cache.  The blocks with the most keys come first.  64 * min(4, nqb) threads, grid:
-// (nqb / 4 rounded up) * nseg * n_heads.
+// Waves of a workgroup of k_rows_attn, and its dynamic LDS: per wave 16 QPW rows of HS floats (rows a bank apart), maxima and sums.
+__host__ __device__ constexpr int attn_waves(int hs) { return hs == 256 ? 4 : 8; }
+__host__ __device__ constexpr size_t attn_lds(int hs, int qpw) { return (size_t)attn_waves(hs) * 16 * qpw * (hs + 4 + 2) * sizeof(float); }
+
+// Causal attention on the fp32 matrix cores, as k_pflash multiplies them.  A workgroup takes the HPG = 256 / HS heads whose
+// outputs are one group of 256 of the next product's input, and two blocks of 16 QPW positions of one sequence, one after the
+// other: block i from the front and block i from the back, so that every workgroup has as many keys to go through (a wave
+// per block left the compute units of the first blocks idle behind the last: 142 us at 1024 positions of the 7B shape,
+// head size 128, and 16 for the digits as a kernel of their own; now 117, of which the matrix cores need 65).  The KS = waves / HPG waves of a head take every KS-th tile of 16 keys
+// with an online softmax each; their parts meet in LDS, where sixteen threads per position merge them into digits.
+// QPW = 2: two positions per lane share every cache row loaded, where there are workgroups enough.
+// grid: blocks (paired: half of them, rounded up) * nseg * n_heads / HPG.
 // Tile u of the values holds the dimensions 64 (u / 4) + 4 m + u % 4, m = 0..15, so that a lane's four values of a cache
-// row are one 16-byte load, and the keys of the next tile are requested before this tile's are multiplied.
-template <int HS>
-static __global__ void __launch_bounds__(256, HS > 128 ? 1 : 2) k_rows_attn(const RowAttn a)
+// row are one 16-byte load; the keys of the next tile are requested before this tile's are used up.
+template <int HS, int QPW>
+static __global__ void __launch_bounds__(64 * attn_waves(HS), HS > 128 ? 1 : 2) k_rows_attn(const RowAttn a)
 {
-    constexpr int U = HS / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    constexpr int U = HS / 16, HPG = 256 / HS, NW = attn_waves(HS), KS = NW / HPG, LD = HS + 4, Q = 16 * QPW;
+    extern __shared__ __align__(16) float at_lds[];
+    float *lm = at_lds + NW * Q * LD, *ll = lm + NW * Q;   // [wave][Q]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int units = a.n_heads * a.nseg, nblk = gridDim.x / units;
-    const int qb = (nblk - 1 - (int)blockIdx.x / units) * nw + wave, u0 = blockIdx.x % units;
-    if (qb >= a.nqb) return;
-    const int h = u0 % a.n_heads, seg = u0 / a.n_heads, kvh = h / a.kv_mul;
-    const int t0 = 16 * qb, tlast = min(t0 + 15, a.T - 1);        // (past the last position: that one again, not stored)
-    const int tq = min(t0 + c, tlast), qpos = a.pos0 + tq, lastkey = a.pos0 + tlast, ntiles = lastkey / 16 + 1;
-    const float *qp = a.q + (size_t)(tq * a.nseg + seg) * a.dim + h * HS + 4 * g;
-    v4f qv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) qv[u] = *reinterpret_cast<const v4f *>(qp + 16 * u);
+    const int units = a.n_heads / HPG * a.nseg, u0 = blockIdx.x % units;
+    const int nblk = (a.T + Q - 1) / Q, front = (int)blockIdx.x / units, back = nblk - 1 - front;
+    const int hg = u0 % (a.n_heads / HPG), seg = u0 / (a.n_heads / HPG), h = hg * HPG + wave / KS, kvh = h / a.kv_mul;
     const float *kc = a.kc + seg * a.seq_stride + kvh * a.head_stride, *vc = a.vc + seg * a.seq_stride + kvh * a.head_stride;
-    const long rs = a.row_stride;
-    v4f o[U];
+    const unsigned rs = (unsigned)a.row_stride;   // (uniform addresses and 32-bit offsets, in floats)
+    for (int which = 0; which < (a.paired && front != back ? 2 : 1); which++) {
+        const int qb = which ? front : back;
+        int qpos[QPW];
+        v4f qv[QPW][U], o[QPW][U];
+        float m[QPW], l[QPW];
 #pragma unroll
-    for (int u = 0; u < U; u++) o[u] = v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -3.0e38f, l = 0.0f;
-    v4f kf[U];
-    auto keys = [&](int t) {
-        const float *krow = kc + (long)min(16 * t + c, lastkey) * rs + 4 * g;
+        for (int p = 0; p < QPW; p++) {
+            const int tq = min(Q * qb + 16 * p + c, a.T - 1);        // (past the last position: that one again, not stored)
+            qpos[p] = a.pos0 + tq;
+            const float *qp = a.q + (size_t)(tq * a.nseg + seg) * a.dim + h * HS + 4 * g;
 #pragma unroll
-        for (int u = 0; u < U; u++) kf[u] = *reinterpret_cast<const v4f *>(krow + 16 * u);
-    };
-    keys(0);
-    for (int t = 0; t < ntiles; t++) {
-        const int k0 = t * 16;
-        v4f vf[4][U / 4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + 4 * c;
-#pragma unroll
-            for (int w = 0; w < U / 4; w++) vf[e][w] = *reinterpret_cast<const v4f *>(vrow + 64 * w);
+            for (int u = 0; u < U; u++) { qv[p][u] = *reinterpret_cast<const v4f *>(qp + 16 * u); o[p][u] = v4f{0.f, 0.f, 0.f, 0.f}; }
+            m[p] = -3.0e38f; l[p] = 0.0f;
         }
-        v4f st = {0.f, 0.f, 0.f, 0.f};
+        const int lastkey = a.pos0 + min(Q * (qb + 1) - 1, a.T - 1), ntiles = lastkey / 16 + 1;
+        v4f kf[U];
+        auto keys = [&](int t) {
+            const unsigned off = (unsigned)min(16 * t + c, lastkey) * rs + 4 * g;
 #pragma unroll
-        for (int u = 0; u < U; u++)
+            for (int u = 0; u < U; u++) kf[u] = *reinterpret_cast<const v4f *>(kc + 16 * u + off);
+        };
+        keys(wave % KS);
+        for (int t = wave % KS; t < ntiles; t += KS) {
+            const int k0 = t * 16;
+            v4f vf[4][U / 4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][e], qv[u][e], st, 0, 0, 0);
-        keys(min(t + 1, ntiles - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        float sv[4], tmax = -3.0e38f;
+            for (int e = 0; e < 4; e++) {
+                const unsigned off = (unsigned)min(k0 + 4 * g + e, lastkey) * rs + 4 * c;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            sv[e] = k0 + 4 * g + e <= qpos ? __fdiv_rn(st[e], a.sqrt_hs) : -3.0e38f;
-            tmax = fmaxf(tmax, sv[e]);
+                for (int w = 0; w < U / 4; w++) vf[e][w] = *reinterpret_cast<const v4f *>(vc + 64 * w + off);
+            }
+            v4f st[QPW];
+#pragma unroll
+            for (int p = 0; p < QPW; p++) st[p] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int p = 0; p < QPW; p++) st[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][e], qv[p][u][e], st[p], 0, 0, 0);
+            keys(min(t + KS, ntiles - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            float pr[QPW][4];
+#pragma unroll
+            for (int p = 0; p < QPW; p++) {
+                float sv[4], tmax = -3.0e38f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    sv[e] = k0 + 4 * g + e <= qpos[p] ? __fdiv_rn(st[p][e], a.sqrt_hs) : -3.0e38f;
+                    tmax = fmaxf(tmax, sv[e]);
+                }
+                tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+                tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+                const float mb = fmaxf(m[p], tmax), sc = expf(m[p] - mb);
+                l[p] *= sc;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    pr[p][e] = k0 + 4 * g + e <= qpos[p] ? expf(sv[e] - mb) : 0.0f;
+                    l[p] += pr[p][e];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) o[p][u] *= sc;
+                m[p] = mb;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int p = 0; p < QPW; p++) o[p][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e][u / 4][u % 4], pr[p][e], o[p][u], 0, 0, 0);
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float mb = fmaxf(m, tmax), sc = expf(m - mb);
-        float pr[4];
-        l *= sc;
+        if (which) __syncthreads();   // (the block before has been read)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            pr[e] = k0 + 4 * g + e <= qpos ? expf(sv[e] - mb) : 0.0f;
-            l += pr[e];
+        for (int p = 0; p < QPW; p++) {
+            l[p] += __shfl_xor(l[p], 16);
+            l[p] += __shfl_xor(l[p], 32);
+            if (g == 0) { lm[wave * Q + 16 * p + c] = m[p]; ll[wave * Q + 16 * p + c] = l[p]; }
+            float *op = at_lds + (wave * Q + 16 * p + c) * LD + 16 * g;   // (element i of o[u]: m = 4 g + i)
+#pragma unroll
+            for (int w = 0; w < U / 4; w++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    *reinterpret_cast<v4f *>(op + 64 * w + 4 * i) = v4f{o[p][4 * w][i], o[p][4 * w + 1][i], o[p][4 * w + 2][i], o[p][4 * w + 3][i]};
         }
+        __syncthreads();
+        // position q, values 16 cc .. 16 cc + 15 of the group: of one head, whose KS parts are merged
+        for (int i = threadIdx.x; i < Q * 16; i += 64 * NW) {
+            const int q = i >> 4, cc = i & 15, t = Q * qb + q, w0 = 16 * cc / HS * KS, at = 16 * cc % HS;
+            if (t >= a.T) continue;   // (sixteen threads at a time)
+            float M = lm[w0 * Q + q], L = 0.0f, v[16] = {};
 #pragma unroll
-        for (int u = 0; u < U; u++) o[u] *= sc;
+            for (int w = 1; w < KS; w++) M = fmaxf(M, lm[(w0 + w) * Q + q]);
 #pragma unroll
-        for (int e = 0; e < 4; e++)
+            for (int w = 0; w < KS; w++) {   // (a wave without a tile has left maximum -3e38, sum 0 and values 0)
+                const float wt = expf(lm[(w0 + w) * Q + q] - M);
+                float x[16];
+                load16(at_lds + ((w0 + w) * Q + q) * LD + at, x);
+                L += wt * ll[(w0 + w) * Q + q];
 #pragma unroll
-            for (int u = 0; u < U; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e][u / 4][u % 4], pr[e], o[u], 0, 0, 0);
-        m = mb;
-    }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    if (t0 + c <= tlast) {   // (element i of o[u]: m = 4 g + i)
-        float *op = a.out + (size_t)((t0 + c) * a.nseg + seg) * a.dim + h * HS + 16 * g;
+                for (int k = 0; k < 16; k++) v[k] += wt * x[k];
+            }
 #pragma unroll
-        for (int w = 0; w < U / 4; w++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                *reinterpret_cast<v4f *>(op + 64 * w + 4 * i) = v4f{__fdiv_rn(o[4 * w][i], l), __fdiv_rn(o[4 * w + 1][i], l), __fdiv_rn(o[4 * w + 2][i], l), __fdiv_rn(o[4 * w + 3][i], l)};
+            for (int k = 0; k < 16; k++) v[k] = __fdiv_rn(v[k], L);
+            quantize_group(a.dig, t * a.nseg + seg, a.dim >> 8, hg, cc, v);
+        }
     }
 }
 
