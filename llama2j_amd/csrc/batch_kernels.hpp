@@ -536,15 +536,26 @@ __global__ void __launch_bounds__(16384 / LPR) k_battn(const BAttn a)
     const long hstride = (long)a.cap * HS;
     constexpr int half = HS >> 1;
     const int cols = a.dim + 2 * a.kv_dim;
+    const long base = (long)b * a.seq_stride + kvh * hstride + 4 * j;   // (the head's rows lie one after the other)
+    constexpr int R = kBattnRows;   // rows in flight per slot
+    const int last = max(pos - 1, 0);
+    // (unconditional loads from the global address space: a row past the cache's last is that last row again and is left
+    // out below; a load chosen by a condition became a flat load from one of two addresses)
+    float4 kk[R], vv[R];
+    auto rows = [&](int tb) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const long at = base + (long)min(tb + r * NSLOT, last) * HS;
+            kk[r] = *reinterpret_cast<const float4 *>(a.kc + at);
+            vv[r] = *reinterpret_cast<const float4 *>(a.vc + at);
+        }
+    };
+    rows(slot);   // on their way while q, k and v are formed
     for (int p = tid; p < 3 * half; p += 256) {   // one thread per pair of q, k, v
         const int which = p / half, idx = p - which * half;
         const int col = (which == 0 ? h * HS : which == 1 ? a.dim + kvh * HS : a.dim + a.kv_dim + kvh * HS) + 2 * idx;
-        float v0 = 0.0f, v1 = 0.0f;
-#pragma unroll 8
-        for (int s = 0; s < a.slices; s++) {   // (independent loads, added in slice order)
-            const float2 t = *reinterpret_cast<const float2 *>(a.part + ((long)s * gridDim.y + b) * cols + col);
-            v0 += t.x; v1 += t.y;
-        }
+        const v2f t = sum_slices<v2f>(a.part + (long)b * cols + col, a.slices, (size_t)gridDim.y * cols);
+        float v0 = t[0], v1 = t[1];
         if (which < 2) {
             const float2 cs = a.rope[(long)pos * half + idx];
             const float r0 = __fsub_rn(__fmul_rn(v0, cs.x), __fmul_rn(v1, cs.y));
@@ -562,21 +573,10 @@ __global__ void __launch_bounds__(16384 / LPR) k_battn(const BAttn a)
     const float4 q4 = *reinterpret_cast<const float4 *>(&sm_qkv[0][4 * j]);
     const float4 kp = *reinterpret_cast<const float4 *>(&sm_qkv[1][4 * j]);   // the row of this position
     const float4 vp = *reinterpret_cast<const float4 *>(&sm_qkv[2][4 * j]);
-    const long base = (long)b * a.seq_stride + kvh * hstride + 4 * j;   // (the head's rows lie one after the other)
     float m = -3.0e38f, l = 0.0f;
     float4 acc = zero;
-    constexpr int R = kBattnRows;   // rows in flight per slot
-    const int last = max(pos - 1, 0);
     for (int tb = slot; tb < len; tb += R * NSLOT) {
-        // (unconditional loads from the global address space: a row past the cache's last is that last row again and is
-        // left out below; a load chosen by a condition became a flat load from one of two addresses)
-        float4 kk[R], vv[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const long at = base + (long)min(tb + r * NSLOT, last) * HS;
-            kk[r] = *reinterpret_cast<const float4 *>(a.kc + at);
-            vv[r] = *reinterpret_cast<const float4 *>(a.vc + at);
-        }
+        if (tb != slot) rows(tb);
         float sv[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -631,15 +631,7 @@ __global__ void __launch_bounds__(16384 / LPR) k_battn(const BAttn a)
         *reinterpret_cast<float4 *>(&sm_out[sub * HS + 4 * tid]) = o;
     }
     __syncthreads();
-    if (threadIdx.x < 16) {
-        float v[16];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 f = *reinterpret_cast<const float4 *>(&sm_out[16 * threadIdx.x + 4 * q]);
-            v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
-        }
-        quantize_group(a.out, b, a.dim >> 8, blockIdx.x, threadIdx.x, v);
-    }
+    if (threadIdx.x < 64) quantize_wave(a.out, b, a.dim >> 8, blockIdx.x, threadIdx.x, *reinterpret_cast<const v4f *>(&sm_out[4 * threadIdx.x]));
 }
 
 struct BNext {
@@ -649,30 +641,36 @@ struct BNext {
     BatchState *st;
     const int *prompts;   // (sequences, prompt_stride)
     int prompt_stride;
-    int *out_tokens;      // (sequences, out_stride): `next` of every step
+    int *out_tokens;      // (sequences, out_stride)
     int out_stride;
+    unsigned long long *best;   // (sequences, kNextParts): each workgroup's first maximum, value bits | index
+    unsigned *done;       // [0] sequences, [1 + b] workgroups of sequence b that have finished; zero between launches
 };
 
+constexpr int kNextParts = 8;   // workgroups per sequence of k_bnext
+
 // Logits of every sequence (the slices summed in order), first index of the maximum (J/Sampler.java:46-57) and the step of
-// the token loop (J/Run.java:635-642, 668, 680): forced prompt id or argmax.  One workgroup per sequence; the last
-// workgroup to finish advances the position.
-static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *done)
+// the token loop (J/Run.java:635-642, 668, 680): forced prompt id or argmax.  A workgroup takes an eighth of a sequence's
+// vocabulary (32000 ids of 13 sequences 27 -> 11 us, of 32 sequences behind 8 slices 26 -> 20, against one workgroup, whose
+// compute unit read a sequence's slices alone); the last of a
+// sequence to finish folds the maxima, the last of all advances the position.  grid (kNextParts, sequences).
+static __global__ void __launch_bounds__(512) k_bnext(const BNext a)
 {
-    __shared__ float bval[16];
-    __shared__ int bidx[16];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const long n = (long)gridDim.x * a.vocab;
+    __shared__ float bval[8];
+    __shared__ int bidx[8];
+    const int b = blockIdx.y, tid = threadIdx.x;
+    const long n = (long)gridDim.y * a.vocab;
     const int pos = a.st->pos;
     float *log = a.st->log ? a.st->log + (pos % kLogSlots) * n + (long)b * a.vocab : nullptr;
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
-    for (int i = tid; i < a.vocab; i += 1024) {
-        float t = 0.0f;
-#pragma unroll 8
-        for (int s = 0; s < a.slices; s++) t += a.part[(long)s * n + (long)b * a.vocab + i];
-        a.logits[(long)b * a.vocab + i] = t;
-        if (log) log[i] = t;
-        if (better(t, i, bv, bi)) { bv = t; bi = i; }
+    for (int i = 4 * (tid + 512 * blockIdx.x); i < a.vocab; i += 4 * 512 * kNextParts) {   // (vocab % 16 == 0)
+        const v4f t = sum_slices<v4f>(a.part + (long)b * a.vocab + i, a.slices, n);
+        *reinterpret_cast<v4f *>(a.logits + (long)b * a.vocab + i) = t;
+        if (log) *reinterpret_cast<v4f *>(log + i) = t;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (better(t[e], i + e, bv, bi)) { bv = t[e]; bi = i + e; }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -682,18 +680,29 @@ static __global__ void __launch_bounds__(1024) k_bnext(const BNext a, unsigned *
     }
     if ((tid & 63) == 0) { bval[tid >> 6] = bv; bidx[tid >> 6] = bi; }
     __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < 16; w++)
-            if (better(bval[w], bidx[w], bv, bi)) { bv = bval[w]; bi = bidx[w]; }
-        if (bi == 0x7fffffff) bi = 0;
-        const int next = pos < a.st->n_prompt[b] ? a.prompts[(long)b * a.prompt_stride + pos] : bi;
-        a.out_tokens[(long)b * a.out_stride + pos] = next;
-        a.st->token[b] = next;
-        __threadfence();
-        if (atomicAdd(done, 1u) == gridDim.x - 1) {   // every sequence has its token: the step is over
-            *done = 0u;
-            a.st->pos = pos + 1;
-        }
+    if (tid != 0) return;
+    for (int w = 1; w < 8; w++)
+        if (better(bval[w], bidx[w], bv, bi)) { bv = bval[w]; bi = bidx[w]; }
+    unsigned long long *best = a.best + b * kNextParts;
+    st_coh(best + blockIdx.x, ((unsigned long long)__float_as_uint(bv) << 32) | (unsigned)bi);
+    __threadfence();
+    if (atomicAdd(a.done + 1 + b, 1u) != kNextParts - 1) return;
+    a.done[1 + b] = 0u;
+    __threadfence();
+    for (int w = 0; w < kNextParts; w++) {
+        const unsigned long long o = ld_coh(best + w);
+        const float ov = __uint_as_float((unsigned)(o >> 32));
+        const int oi = (int)(unsigned)o;
+        if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+    }
+    if (bi == 0x7fffffff) bi = 0;
+    const int next = pos < a.st->n_prompt[b] ? a.prompts[(long)b * a.prompt_stride + pos] : bi;
+    a.out_tokens[(long)b * a.out_stride + pos] = next;
+    a.st->token[b] = next;
+    __threadfence();
+    if (atomicAdd(a.done, 1u) == gridDim.y - 1) {   // every sequence has its token: the step is over
+        a.done[0] = 0u;
+        a.st->pos = pos + 1;
     }
 }
 

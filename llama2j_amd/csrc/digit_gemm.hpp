@@ -15,8 +15,7 @@
 namespace l2j {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 
 constexpr int kRowTile = 32;                       // activation vectors per tile: two MFMAs of 16
 constexpr int kDigitBytes = 4 * 4 * 2 * 64 * 16;   // digits of a (tile, group): [digit][64 k][half of the tile][lane][16], most significant digit first
@@ -96,6 +95,65 @@ __device__ __forceinline__ void quantize_group(const Digits &o, int row, int ngr
         o.sx[at] = inv;
         o.sum[at] = t;
     }
+}
+
+// A group of vector `row` held by the whole wave, four consecutive activations per lane (k = 4 lane ..): digits, scale and sum.
+__device__ __forceinline__ void quantize_wave(const Digits &o, int row, int ngroups, int g, int lane, const v4f &v)
+{
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) m = max(m, __float_as_uint(v[i]) & 0x7fffffffu);   // (as bits: a NaN is the largest)
+    m = max(m, dpp_u<0xB1>(m));
+    m = max(m, dpp_u<0x4E>(m));
+    m = max(m, dpp_u<0x124>(m));
+    m = max(m, dpp_u<0x128>(m));
+    auto at = [&](int l) { return (unsigned)__builtin_amdgcn_readlane((int)m, l); };
+    m = max(max(at(0), at(16)), max(at(32), at(48)));
+    float inv;
+    const int s = digit_shift(m, &inv);
+    const float t = wave_sum((v[0] + v[1]) + (v[2] + v[3]));
+    unsigned w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = ((unsigned)(int)rintf(ldexpf(v[i], s)) + 0x80808080u) ^ 0x80808080u;   // (as store_digits)
+    const int c = lane >> 2;
+    unsigned *p = reinterpret_cast<unsigned *>(o.d + ((size_t)(row >> 5) * ngroups + g) * (kDigitBytes / 16) + (2 * (c >> 2) + ((row >> 4) & 1)) * 64 + (row & 15) + 16 * (c & 3)) + (lane & 3);
+    // (a transpose within four lanes, for one 16-byte store per lane instead of four of 4 bytes, gains nothing)
+#pragma unroll
+    for (int d = 0; d < 4; d++) {   // byte 3 - d of every word
+        const unsigned sel = 0x0c0c0400u + (unsigned)((3 - d) * 0x0101u);
+        p[d * 8 * 64 * 4] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(w[3], w[2], sel), __builtin_amdgcn_perm(w[1], w[0], sel), 0x05040100u);
+    }
+    if (lane == 0) {
+        const size_t q = ((size_t)(row >> 5) * ngroups + g) * 32 + (row & 31);
+        o.sx[q] = inv;
+        o.sum[q] = t;
+    }
+}
+
+// The sum of a product's slices at consecutive columns (V: float2, v4f), added in slice order: up to four, or eight at a time,
+// with all loads in flight (past the last slice: that one again, not added).
+template <int N, class V>
+__device__ __forceinline__ void add_slices(V &t, const float *__restrict__ part, int s0, int slices, size_t stride)
+{
+    V v[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = *reinterpret_cast<const V *>(part + min(s0 + i, slices - 1) * stride);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        if (s0 + i < slices) t += v[i];
+}
+
+template <class V>
+__device__ __forceinline__ V sum_slices(const float *__restrict__ part, int slices, size_t stride)
+{
+    V t = {};
+    if (slices == 1) return t + *reinterpret_cast<const V *>(part);   // (-0 + 0 = +0, as the sum of several)
+    if (slices <= 4) {
+        add_slices<4>(t, part, 0, slices, stride);
+    } else {
+        for (int s = 0; s < slices; s += 8) add_slices<8>(t, part, s, slices, stride);
+    }
+    return t;
 }
 
 struct DGemm {

@@ -137,7 +137,8 @@ struct l2j::BatchBufs {
     float *kc = nullptr, *vc = nullptr;             // (sequence, layer, kv head, cap_steps, head_size)
     BatchState *st = nullptr;
     int *prompts = nullptr, *out = nullptr;         // (sequence, cap_pstride), (sequence, cap_steps)
-    unsigned *done = nullptr;
+    unsigned *done = nullptr;             // (1 + nseq) counters and
+    unsigned long long *best = nullptr;   // (nseq, kNextParts) maxima of k_bnext
     unsigned *bar_ctr = nullptr;   // k_bstep: the counters of its grid barrier,
     int *fault = nullptr;          // the flag a bounded wait sets when it runs out,
     float *ssq = nullptr;          // the sums of squares behind the two norms of a layer,
@@ -176,7 +177,7 @@ struct l2j::BatchBufs {
         if (graph) (void)hipGraphDestroy(graph);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
-        void *ps[] = {xb, hb, logits, cls_part, part[0], part[1], part[2], kc, vc, st, prompts, out, done, bar_ctr, fault, ssq, step_args};
+        void *ps[] = {xb, hb, logits, cls_part, part[0], part[1], part[2], kc, vc, st, prompts, out, done, best, bar_ctr, fault, ssq, step_args};
         for (void *p : ps) (void)hipFree(p);
         r.release();
         free_batch_samplers(&samplers);
@@ -300,7 +301,8 @@ void launch_batch_tokens(l2j_ctx *c, BatchBufs &b, const float *xn)
     BNext n{};
     n.part = b.cls_part; n.slices = cls_slices(cf.dim); n.vocab = cf.vocab_size; n.logits = b.logits; n.st = b.st; n.prompts = b.prompts;
     n.prompt_stride = b.cap_pstride; n.out_tokens = b.out; n.out_stride = b.cap_steps;
-    hipLaunchKernelGGL(k_bnext, dim3(b.nseq), dim3(1024), 0, s, n, b.done);
+    n.best = b.best; n.done = b.done;
+    hipLaunchKernelGGL(k_bnext, dim3(kNextParts, b.nseq), dim3(512), 0, s, n);
 }
 
 // One position of all sequences: embedding, the layers, the classifier, the next tokens.
@@ -380,7 +382,8 @@ int ensure_batch(l2j_ctx *c, int nseq, int steps, int pstride)
     if (e == hipSuccess) e = b->r.alloc(c, nseq, false);
     alloc(&b->logits, (size_t)nseq * vocab); alloc(&b->cls_part, (size_t)nseq * cls_slices(dim) * vocab);
     alloc(&b->kc, cache_floats); alloc(&b->vc, cache_floats);
-    alloc(&b->st, 1); alloc(&b->prompts, (size_t)nseq * pstride); alloc(&b->out, (size_t)nseq * steps); alloc(&b->done, 1);
+    alloc(&b->st, 1); alloc(&b->prompts, (size_t)nseq * pstride); alloc(&b->out, (size_t)nseq * steps); alloc(&b->done, 1 + nseq);
+    alloc(&b->best, (size_t)nseq * kNextParts);
     if (e == hipSuccess) e = plan_bstep(c, *b, nseq);
     if (e == hipSuccess && b->step_grid > 0) {
         const size_t part_floats = (size_t)nseq * std::max((size_t)batch_slices(dim) * hidden, (size_t)batch_slices(hidden) * dim);
@@ -585,7 +588,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
         for (int s = 0; s < nseq; s++) h_rows[t * nseq + s] = t == 0 ? 1 : prompts[(size_t)s * prompt_stride + t - 1];
     hipError_t e = hipMemcpyAsync(b.st, b.h_pin, sizeof(h), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(b.prompts, b.h_pin + state_ints, (size_t)nseq * pcap * sizeof(int), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(b.done, 0, sizeof(unsigned), c->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b.done, 0, (1 + b.nseq) * sizeof(unsigned), c->stream);
     if (e != hipSuccess) return fail_hip(e, "state upload");
     LogTaker taker(b, logits_log, step_floats, cf.device);
     // after the logits of a position: kept for the caller, and J/Run.java:643-665 for the sequences whose prompt is used up

@@ -8,15 +8,6 @@
 
 namespace l2j {
 
-// The sum of a product's slices at four consecutive columns, added in slice order (the loads are independent).
-__device__ __forceinline__ v4f slices4(const float *__restrict__ part, int slices, size_t stride)
-{
-    v4f t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int s = 0; s < slices; s++) t += *reinterpret_cast<const v4f *>(part + s * stride);
-    return t;
-}
-
 __device__ __forceinline__ void load16(const float *p, float (&v)[16])
 {
 #pragma unroll
@@ -40,8 +31,11 @@ struct RowNorm {
 };
 
 // x, then w * (ss * x), ss = 1 / sqrt(sum(x^2) / n + 1e-5) (K/RootMeanSquare.java:25-35, K/WeightNormalizeAndScale.java:73).
-// One workgroup per row, four values per thread and step of 4096, which meet in LDS (dim floats) for the digits: sixteen
-// threads write a group's, sixteen values each.
+// One workgroup per row, four values per thread and step of 4096, kept in LDS (dim floats, each thread its own): a wave
+// holds whole groups of 256 and writes their digits.  Bound by its chain of latencies (slices, sum over the workgroup,
+// digits): the loads of the slices and of the first weights go out together.  32 rows of 4096 behind 4 or 11 slices
+// 6.7 us, 13 of 768 behind 1 or 2 slices 3.5 (7.4 and 4.0 when sixteen lanes per group wrote the digits behind another barrier
+// and the slices came four at a time).
 static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
 {
     extern __shared__ __align__(16) float ln[];
@@ -51,14 +45,16 @@ static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
     const v4f *e = a.tokens ? reinterpret_cast<const v4f *>(a.emb + (size_t)a.tokens[row] * a.dim) : nullptr;
     const float *part = a.part + (size_t)row * a.dim;
     const size_t stride = (size_t)a.nrows * a.dim;
+    const v4f *w = reinterpret_cast<const v4f *>(a.w);
+    v4f w0 = w[tid];   // (no more threads than n4)
     float ssq = 0.0f;
     for (int i = tid; i < n4; i += nt) {
         v4f v;
         if (e) {
             v = e[i];
         } else {
-            const v4f t = slices4(part + 4 * i, a.slices, stride);
             v = x[i];
+            const v4f t = sum_slices<v4f>(part + 4 * i, a.slices, stride);
 #pragma unroll
             for (int k = 0; k < 4; k++) v[k] = __fadd_rn(v[k], t[k]);
         }
@@ -68,20 +64,13 @@ static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
     }
     ssq = block_sum(ssq, red, nt >> 6);
     const float ss = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(ssq, (float)a.dim), 1e-5f)));
-    for (int i = tid; i < n4; i += nt) {   // (each thread its own values)
-        const v4f w = reinterpret_cast<const v4f *>(a.w)[i];
+    for (int i = tid; i < n4; i += nt) {   // (each thread its own values; whole waves leave together: n4 % 64 == 0)
+        if (i != tid) w0 = w[i];
         v4f v = l4[i];
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = __fmul_rn(w[k], __fmul_rn(ss, v[k]));
+        for (int k = 0; k < 4; k++) v[k] = __fmul_rn(w0[k], __fmul_rn(ss, v[k]));
         if (a.xn) reinterpret_cast<v4f *>(a.xn + (size_t)row * a.dim)[i] = v;
-        else l4[i] = v;
-    }
-    if (a.xn) return;
-    __syncthreads();
-    for (int c = tid; c < (a.dim >> 4); c += nt) {
-        float v[16];
-        load16(ln + 16 * c, v);
-        quantize_group(a.dig, row, a.dim >> 8, c >> 4, c & 15, v);
+        else quantize_wave(a.dig, row, a.dim >> 8, i >> 6, tid & 63, v);
     }
 }
 
@@ -104,7 +93,7 @@ static __global__ void __launch_bounds__(256) k_rows_qkv(const RowQkv a)
     const float *part = a.part + (size_t)row * cols;
     const float4 *rope = reinterpret_cast<const float4 *>(a.rope + (size_t)pos * (hs >> 1));
     for (int c = 4 * (threadIdx.x + 256 * blockIdx.y); c < cols; c += 1024 * gridDim.y) {
-        const v4f t = slices4(part + c, a.slices, stride);
+        const v4f t = sum_slices<v4f>(part + c, a.slices, stride);
         float4 v = make_float4(t[0], t[1], t[2], t[3]);
         const bool isq = c < a.dim, isk = !isq && c < a.dim + a.kv_dim;
         const int at = isq ? c : c - a.dim - (isk ? 0 : a.kv_dim);
@@ -134,28 +123,19 @@ static __global__ void __launch_bounds__(256) k_rows_digits(const float *__restr
 }
 
 // silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74) as digits; part: (slices, rows, 2 hidden), h1 | h3.
-// Workgroup (x, row): four groups of 256, four values per thread; the values meet in LDS for the digits.
+// Workgroup (x, row): four groups of 256, one per wave, four values per thread.
 static __global__ void __launch_bounds__(256) k_rows_swiglu(const float *__restrict__ part, int slices, Digits o, int rows, int hidden,
                                                      const float *__restrict__ silu, int exact)
 {
-    __shared__ __align__(16) float lh[1024];
-    const int row = blockIdx.y, tid = threadIdx.x, col = blockIdx.x * 1024 + 4 * tid;
-    if (col < hidden) {
-        const size_t stride = (size_t)rows * 2 * hidden;
-        const float *p = part + (size_t)row * 2 * hidden + col;
-        const v4f h1 = slices4(p, slices, stride), h3 = slices4(p + hidden, slices, stride);
-        v4f y;
+    const int row = blockIdx.y, col = blockIdx.x * 1024 + 4 * threadIdx.x;
+    if (col >= hidden) return;   // (whole waves: hidden % 256 == 0)
+    const size_t stride = (size_t)rows * 2 * hidden;
+    const float *p = part + (size_t)row * 2 * hidden + col;
+    const v4f h1 = sum_slices<v4f>(p, slices, stride), h3 = sum_slices<v4f>(p + hidden, slices, stride);
+    v4f y;
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = __fmul_rn(h1[e], __fmul_rn(silu_sigma(silu, h1[e], exact), h3[e]));
-        *reinterpret_cast<v4f *>(lh + 4 * tid) = y;
-    }
-    __syncthreads();
-    const int g = 4 * blockIdx.x + (tid >> 4);
-    if (tid < 64 && g < (hidden >> 8)) {
-        float v[16];
-        load16(lh + 16 * tid, v);
-        quantize_group(o, row, hidden >> 8, g, tid & 15, v);
-    }
+    for (int e = 0; e < 4; e++) y[e] = __fmul_rn(h1[e], __fmul_rn(silu_sigma(silu, h1[e], exact), h3[e]));
+    quantize_wave(o, row, hidden >> 8, col >> 8, threadIdx.x & 63, y);
 }
 
 struct RowAttn {
