@@ -216,7 +216,7 @@ int cls_slices(int K) { return (K / 256 + kClsGps - 1) / kClsGps; }
 size_t step_lds(int nseq) { return bg_lds_bytes(nseq, nseq / kBatch); }       // k_bstep: 256 threads per 16 sequences
 size_t batch_lds_f32(int nseq) { return (size_t)nseq * (kClsGps * 256 + kXPad) * sizeof(float); }   // k_bgemm_f32: floats
 
-// The product of one layer's matrices `tensors` (the same input, the same row length) as one k_bgemm argument.
+// The product of one layer's matrices `tensors` (the same input, the same row length) as one argument of the one-launch step.
 BGemm bgemm_args(l2j_ctx *c, std::initializer_list<int> tensors, int layer, const float *x, float *const *part)
 {
     BGemm a{};
@@ -448,11 +448,16 @@ int seed_batch_samplers(l2j_ctx *c, BatchBufs &b, const int64_t *seeds)
 // the copy into memory the caller has just been given (page faults included) takes about as long as a step of a small
 // model.  The thread waits for a step on the host: a queue that waits for another one on the device (hipStreamWaitEvent) made the
 // 100 kernels of a step 1 us longer each (1745 -> 1853 us per replay of a graph of 100 kernels, 1757 us with the copies alone).
+// A process that may not start another thread (std::thread throws) has each step copied by offer() itself.
 class LogTaker {
 public:
     LogTaker(const BatchBufs &b_, float *out_, size_t step_floats_, int device_) : b(b_), out(out_), step_floats(step_floats_), device(device_)
     {
-        if (out) th = std::thread([this] { run(); });
+        if (!out) return;
+        try {
+            th = std::thread([this] { run(); });
+        } catch (const std::exception &) {
+        }
     }
     ~LogTaker()
     {
@@ -473,6 +478,11 @@ public:
     // log_step of step `pos` has been recorded
     void offer(int pos)
     {
+        if (!th.joinable()) {
+            if (err == hipSuccess) err = take(pos);
+            offered = taken = pos + 1;
+            return;
+        }
         {
             std::lock_guard<std::mutex> l(mu);
             offered = pos + 1;
@@ -498,6 +508,16 @@ private:
     hipError_t err = hipSuccess;
     std::thread th;
 
+    hipError_t take(int pos)
+    {
+        const int slot = pos % kLogSlots;
+        hipError_t e = hipEventSynchronize(b.log_step[slot]);
+        if (e == hipSuccess) e = hipMemcpyAsync(b.log_pin, b.log_dev + slot * step_floats, step_floats * sizeof(float), hipMemcpyDeviceToHost, b.log_stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(b.log_stream);
+        if (e == hipSuccess) memcpy(out + (size_t)pos * step_floats, b.log_pin, step_floats * sizeof(float));
+        return e;
+    }
+
     void run()
     {
         hipError_t e = hipSetDevice(device);
@@ -511,11 +531,7 @@ private:
                     return;
                 }
             }
-            const int slot = i % kLogSlots;
-            e = hipEventSynchronize(b.log_step[slot]);
-            if (e == hipSuccess) e = hipMemcpyAsync(b.log_pin, b.log_dev + slot * step_floats, step_floats * sizeof(float), hipMemcpyDeviceToHost, b.log_stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(b.log_stream);
-            if (e == hipSuccess) memcpy(out + (size_t)i * step_floats, b.log_pin, step_floats * sizeof(float));
+            e = take(i);
             {
                 std::lock_guard<std::mutex> l(mu);
                 if (e == hipSuccess) taken = i + 1;
