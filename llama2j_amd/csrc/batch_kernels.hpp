@@ -95,7 +95,7 @@ static __global__ void __launch_bounds__(256) k_btile(const uint8_t *__restrict_
     }
 }
 
-// LDS of k_bgemm: the sums of a batch of tiles (as many tiles as the workgroup has waves; per tile, wave and column block
+// LDS of the one-launch step's products: the sums of a batch of tiles (as many tiles as the workgroup has waves; per tile, wave and column block
 // 64 lanes x 16 bytes), then every wave's sums of its activations per sequence
 __host__ __device__ inline size_t bg_lds_bytes(int nseq, int hv)
 {
@@ -370,7 +370,7 @@ struct BGemmF32 {
     int gps;
 };
 
-// As k_bgemm with float weights on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), rows as they lie in memory: a lane
+// The classifier for 16 NB vectors: float weights on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), rows as they lie in memory: a lane
 // (r, s) holds row r at k = 64 T + 16 q + 4 s + e as four 16-byte loads (q) per block of 64 k, so that the four lanes of a
 // row read 64 bytes in one piece per load; step (q, e) multiplies the 16 rows by 16 sequences over the four k of the four s.
 // NB = 2: two column blocks of 16 sequences share the weights.  256 threads, 32 rows per wave.

@@ -1,5 +1,5 @@
 // All layers of a batched step in one launch (option batch_fuse; slower than the eight launches per layer it replaces,
-// measured, and off by default): the four products of a layer (k_bgemm's waves) and what lies between them (attention,
+// measured, and off by default): the four products of a layer (BgWave) and what lies between them (attention,
 // residual + rmsnorm, SwiGLU) as eight phases with a grid barrier after each, all workgroups resident.  The first codes
 // of a product are requested before the barrier that precedes it, and the phases between the products spread over all
 // workgroups: the rmsnorm scalar is deferred (sum_k w_k (g_k ss x_k) = ss sum_k w_k g_k x_k), so a norm is no pass of one
@@ -274,7 +274,7 @@ __device__ __forceinline__ void bstep_swiglu(const BStep &a, const float *ss_lds
     }
 }
 
-// grid: as many workgroups of 256 NB threads as are resident at once (one per compute unit); dynamic LDS as k_bgemm.
+// grid: as many workgroups of 256 NB threads as are resident at once (one per compute unit); dynamic LDS: step_lds.
 // Before: x = the embeddings, xn = their rmsnorm (normalized: the first attention multiplies by no ss), the barrier
 // counters zero.  After: x = the residual stream after the last layer (the final norm is the caller's).
 template <int NB>

@@ -309,7 +309,7 @@ void launch_batch_tokens(l2j_ctx *c, BatchBufs &b, const float *xn)
 void launch_batch_step(l2j_ctx *c, BatchBufs &b)
 {
     const l2j_config &cf = c->cfg;
-    const int dim = cf.dim, hidden = cf.hidden_dim, L = cf.n_layers, hs = c->head_size, kvd = c->kv_dim, nseq = b.nseq, cap = b.cap_steps;
+    const int dim = cf.dim, L = cf.n_layers, hs = c->head_size, kvd = c->kv_dim, nseq = b.nseq, cap = b.cap_steps;
     hipStream_t s = c->stream;
     if (b.step_grid > 0) {
         hipLaunchKernelGGL(k_bembed, dim3(nseq), dim3(256), 0, s, c->emb, b.st, b.r.x, dim, b.bar_ctr);
@@ -340,8 +340,7 @@ void launch_batch_step(l2j_ctx *c, BatchBufs &b)
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, nseq);
         const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, l, b.r.dig, nseq, b.r.part);
-        hipLaunchKernelGGL(k_rows_swiglu, dim3((hidden + 1023) / 1024, nseq), dim3(256), 0, s, b.r.part, s13, b.r.dig, nseq, hidden,
-                           c->silu, (cf.flags & L2J_F_EXACT_SILU) ? 1 : 0);
+        launch_swiglu(c, b.r.part, s13, b.r.dig, nseq);
         n.slices = launch_dgemm(c, {L2J_W2}, l, b.r.dig, nseq, b.r.part);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         n.w = c->rmsw + (l + 1 < L ? (size_t)(l + 1) * dim : (size_t)2 * L * dim);

@@ -110,7 +110,16 @@ int l2j::product_slices(l2j_ctx *c, int tiles16, int ngroups, int rows)
 void l2j::launch_norm(l2j_ctx *c, const RowNorm &n, int rows)
 {
     const int threads = std::min(1024, std::max(64, n.dim / 4));
-    hipLaunchKernelGGL(k_rows_norm, dim3(rows), dim3(threads), (size_t)n.dim * sizeof(float), c->stream, n);
+    RowNorm a = n;
+    a.together = rows >= kTogetherFrom && !n.xn ? rows : 0;
+    hipLaunchKernelGGL(k_rows_norm, dim3(a.together ? together_grid(rows, 1) : rows), dim3(threads), (size_t)n.dim * sizeof(float), c->stream, a);
+}
+
+void l2j::launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows)
+{
+    const int hidden = c->cfg.hidden_dim, parts = (hidden + 1023) / 1024, together = rows >= kTogetherFrom;
+    const dim3 grid = together ? dim3(together_grid(rows, parts)) : dim3(parts, rows);
+    hipLaunchKernelGGL(k_rows_swiglu, grid, dim3(256), 0, c->stream, part, slices, o, rows, hidden, c->silu, (c->cfg.flags & L2J_F_EXACT_SILU) ? 1 : 0, together);
 }
 
 void RowBufs::release()
@@ -166,7 +175,7 @@ static void launch_attn(l2j_ctx *c, RowAttn t)
 hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
 {
     const l2j_config &cf = c->cfg;
-    const int dim = cf.dim, hidden = cf.hidden_dim, L = cf.n_layers, hs = c->head_size, kvd = c->kv_dim, rows = job.nseg * job.T;
+    const int dim = cf.dim, L = cf.n_layers, hs = c->head_size, kvd = c->kv_dim, rows = job.nseg * job.T;
     const int nqb = (job.T + 15) / 16;
     hipStream_t s = c->stream;
     // Few blocks of 16 positions over many keys: the keys of a block dealt to the waves of a workgroup (and to several
@@ -226,8 +235,7 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, rows);
         const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, l, b.dig, rows, b.part);
-        hipLaunchKernelGGL(k_rows_swiglu, dim3((hidden + 1023) / 1024, rows), dim3(256), 0, s, b.part, s13, b.dig, rows, hidden,
-                           c->silu, (cf.flags & L2J_F_EXACT_SILU) ? 1 : 0);
+        launch_swiglu(c, b.part, s13, b.dig, rows);
         n.slices = launch_dgemm(c, {L2J_W2}, l, b.dig, rows, b.part);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         if (l + 1 < L) {

@@ -9,6 +9,7 @@
 namespace l2j {
 
 constexpr int kRowsMax = 1024;   // rows of a pass
+constexpr int kTogetherFrom = 256;   // rows from which on the rows of a line of digits share an XCD (together_row): below, too few units of eight rows to keep eight XCDs evenly busy
 
 struct DgPlan {
     int variant = 0, gps = 0, slices = 0, nrow = 0, ncol = 0;
@@ -29,6 +30,7 @@ DgPlan dgemm_plan(int n_cu, int tiles16, int ngroups, int rows);
 hipError_t prepare_dgemm(l2j_ctx *c);
 int product_slices(l2j_ctx *c, int tiles16, int ngroups, int rows);
 void launch_norm(l2j_ctx *c, const RowNorm &n, int rows);
+void launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows);
 int launch_dgemm(l2j_ctx *c, std::initializer_list<int> tensors, int layer, const Digits &x, int rows, float *part);
 
 struct RowJob {

@@ -234,7 +234,7 @@ def test_passes_of_many_positions(shape):
     rng = np.random.default_rng(shape[0])
     g = model(shape)
     tokens = np.concatenate([[1], rng.integers(2, shape[5], size=seq_len - 1)]).astype(np.int32)
-    sizes = [n for n in (2, 63, 64, 65, 129, 257, 300, 1024, 1025, 1104) if n <= seq_len]
+    sizes = [n for n in (2, 63, 64, 65, 129, 255, 256, 257, 300, 1024, 1025, 1104) if n <= seq_len]
     want = {}
     for i, t in enumerate(tokens):
         lg = g.forward(int(t), i, want_logits=i + 1 in sizes)
