@@ -294,7 +294,7 @@ def main():
 
     if (not a.no_batched or a.prefill_only) and not long_context:
         # Not the metric either: 32 (and 16) sequences decoded at once (every weight read once per step for all of them, the
-        # products on the bf16 matrix cores); sequence 0 has the prompt of the timed run and must repeat its tokens.
+        # products on the int8 matrix cores); sequence 0 has the prompt of the timed run and must repeat its tokens.
         try:
             bsteps = min(steps, 288)
             n0 = min(bsteps, len(tokens))
@@ -326,7 +326,7 @@ def main():
                 out["batched_decode"]["sixteen_sequences"] = {k: runs[16][k] for k in ("tok_s", "ms_per_step", "sequence_0_equals_the_single_decode")}
         except l2j.L2JError as e:  # shapes the batched path does not take (rows that are not whole groups of 256)
             out["batched_decode"] = {"error": str(e)}
-        # Nor this: the forward passes of 1024 consecutive positions of one sequence, 32 at a time through the same products
+        # Nor this: the forward passes of 1024 consecutive positions of one sequence, in one pass through the same products
         # (l2j_prefill), as a prompt of that length would be taken instead of one position per launch.
         try:
             n_pre = min(1024, shape[6] - 1)
