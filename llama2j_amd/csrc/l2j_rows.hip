@@ -155,14 +155,16 @@ hipError_t RowBufs::alloc(l2j_ctx *c, int rows, bool attention)
     return e;
 }
 
-// Blocks of 32 positions (the cache rows loaded once for 32) from where their pairs still fill the compute units; pairs of blocks
-// unless one block per workgroup already leaves compute units idle.
+// Blocks of 32 positions (the cache rows loaded once for 32) where pairs of blocks of 16 are an eighth more workgroups than compute
+// units: a last round of them costs more than half-filled compute units do.  7B shape, us a launch with blocks of 16 -> 32: 520
+// positions 58.6 -> 71.0 (272 pairs of blocks of 16: just past the 256 units), 560 76.4 -> 69.0 (288), 700 88.2 -> 79.5, 900 110.8 ->
+// 100.1.  Pairs of blocks unless one block per workgroup already leaves compute units idle.
 template <int HS>
 static void launch_attn(l2j_ctx *c, RowAttn t)
 {
     const int units = c->cfg.n_heads / (256 / HS) * t.nseg;
     auto blocks = [&](int q) { return (t.T + q - 1) / q; };
-    const bool two = HS < 256 && (blocks(32) + 1) / 2 * units >= c->n_cu;
+    const bool two = HS < 256 && t.T > 16 && 8L * ((blocks(16) + 1) / 2) * units >= 9L * c->n_cu;
     const int n = blocks(two ? 32 : 16);
     t.paired = n * units > c->n_cu;
     const dim3 g((t.paired ? (n + 1) / 2 : n) * units), blk(64 * attn_waves(HS));
