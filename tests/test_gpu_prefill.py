@@ -1,5 +1,5 @@
 """l2j_prefill: the prompt positions of the token loop (J/Run.java:623-640, one Run.transformer call per position in the
-reference) 32 at a time through the batched products.  It must leave in the KV cache, and return for the last position,
+reference) many at once through the batched products.  It must leave in the KV cache, and return for the last position,
 what l2j_forward position by position does (to rounding: the sums are formed in another order), and both must be what the
 CPU oracle computes."""
 import numpy as np
