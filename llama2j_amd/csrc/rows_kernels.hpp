@@ -176,6 +176,21 @@ struct RowAttn {
     unsigned *pf_cnt;        // (head, block): how many have; zero between launches
 };
 
+// Keys behind a query's position have weight 0, and 0 times a NaN or an infinity is a NaN.  Where a tile of 16 keys holds such
+// values and reaches behind the position of some query of the block, the values go into the product as 0, and the sums of the
+// queries that see one are set to NaN by this: flag[e]: 1 where the lane's value of key k0 + 4 g + e (one tile of the
+// dimensions) is not finite, else 0.  (An infinity leaves a NaN as well: the norms and digits behind make it one in any case.)
+__device__ __forceinline__ void see_not_finite(v4f &o, const float (&flag)[4], int key0, int qpos)
+{
+    v4f t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(flag[e], key0 + e <= qpos ? 1.0f : 0.0f, t, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = t[i] > 0.0f ? __builtin_nanf("") : o[i];
+}
+
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+
 // Waves of a workgroup of k_rows_attn, and its dynamic LDS: per wave 16 QPW rows of HS floats (rows a bank apart), maxima and sums.
 __host__ __device__ constexpr int attn_waves(int hs) { return hs == 256 ? 4 : 8; }
 __host__ __device__ constexpr size_t attn_lds(int hs, int qpw) { return (size_t)attn_waves(hs) * 16 * qpw * (hs + 4 + 2) * sizeof(float); }
@@ -267,6 +282,28 @@ static __global__ void __launch_bounds__(64 * attn_waves(HS), HS > 128 ? 1 : 2) 
                 for (int u = 0; u < U; u++) o[p][u] *= sc;
                 m[p] = mb;
             }
+            if (k0 + 15 > a.pos0 + Q * qb) {   // (a key behind a position of the block)
+                v4f z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) z[e] = fmaf(vf[e][u / 4][u % 4], 0.0f, z[e]);
+                if (__any(!((z[0] + z[1]) + (z[2] + z[3]) == 0.0f))) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        float flag[4];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const bool ok = finite(vf[e][u / 4][u % 4]);
+                            flag[e] = ok ? 0.0f : 1.0f;
+                            vf[e][u / 4][u % 4] = ok ? vf[e][u / 4][u % 4] : 0.0f;
+                        }
+#pragma unroll
+                        for (int p = 0; p < QPW; p++) see_not_finite(o[p][u], flag, k0 + 4 * g, qpos[p]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
@@ -345,9 +382,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_pflash(const RowAttn a)
     const int qpos = pos0 + min(c, vrows - 1), lastkey = pos0 + vrows - 1, ntiles = lastkey / 16 + 1;
     const float *kc = a.kc + kvh * a.head_stride, *vc = a.vc + kvh * a.head_stride;
     const long rs = a.row_stride;
-    v4f32 o[U];
+    v4f o[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) o[u] = v4f32{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < U; u++) o[u] = v4f{0.f, 0.f, 0.f, 0.f};
     float m = -3.0e38f, l = 0.0f;
     // tile t of the keys goes to workgroup t % NS (z) and there to wave (t / NS) % WAVES: few tiles spread over the workgroups first
     const int NS = gridDim.z;
@@ -385,13 +422,37 @@ __global__ void __launch_bounds__(64 * WAVES) k_pflash(const RowAttn a)
         }
 #pragma unroll
         for (int u = 0; u < U; u++) o[u] *= sc;
+        m = mb;
+        bool clean = true;
+        if (k0 + 15 > pos0) {   // (as in k_rows_attn)
+            float z = 0.0f;
+#pragma unroll 1
+            for (int e = 0; e < 4; e++) {
+                const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + c;
+#pragma unroll
+                for (int u = 0; u < U; u++) z = fmaf(vrow[16 * u], 0.0f, z);
+            }
+            clean = !__any(!(z == 0.0f));
+            if (!clean) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    float flag[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) flag[e] = finite(vc[(long)min(k0 + 4 * g + e, lastkey) * rs + c + 16 * u]) ? 0.0f : 1.0f;
+                    see_not_finite(o[u], flag, k0 + 4 * g, qpos);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const float *vrow = vc + (long)min(k0 + 4 * g + e, lastkey) * rs + c;
 #pragma unroll
-            for (int u = 0; u < U; u++) o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * u], pr[e], o[u], 0, 0, 0);
+            for (int u = 0; u < U; u++) {
+                const float v = vrow[16 * u];
+                o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(clean || finite(v) ? v : 0.0f, pr[e], o[u], 0, 0, 0);
+            }
         }
-        m = mb;
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -399,7 +460,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_pflash(const RowAttn a)
     if (wave < nw) {   // (the waves without a tile have nothing to add)
 #pragma unroll
         for (int u = 0; u < U; u++)   // (a lane's four dimensions 16 u + 4 g + e of query c as one 16-byte store, a wave's stores 1 KB in a row)
-            *reinterpret_cast<v4f32 *>(&wo[wave * HS * 16 + (4 * u + g) * 64 + 4 * c]) = o[u];
+            *reinterpret_cast<v4f *>(&wo[wave * HS * 16 + (4 * u + g) * 64 + 4 * c]) = o[u];
     }
     __syncthreads();
     if (tid < 16 * WAVES) {   // weight of wave w's part in query q's sum: tid = w * 16 + q (a workgroup without any tile leaves

@@ -375,3 +375,27 @@ def test_common_prompt_positions_taken_at_once(orc, n_seq, shortest, longest):
             want = [int(prompts[b][pos]) if pos < lengths[b] else s.step(lg[pos, b], 0.9, 0.9)[0] for pos in range(steps)]
             np.testing.assert_array_equal(sampled[b], np.array(want, dtype=np.int32), err_msg="sequence %d" % b)
     g.close()
+
+
+@pytest.mark.parametrize("n_seq", [16, 32])
+def test_a_sequence_that_is_not_finite_leaves_earlier_positions_and_the_others_alone(n_seq):
+    """A token whose embedding holds a NaN inside the common prompt: the logits of every other sequence, and of the positions before
+    it of its own, are the bits they are with another token there."""
+    shape = SHAPES[1]
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    rng = np.random.default_rng(n_seq)
+    emb = (0.02 * rng.standard_normal((shape[5], shape[0]))).astype(np.float32)
+    emb[5, 3] = np.nan
+    g.upload_f32(TENSOR.TOK_EMB, emb)
+    g.finalize()
+    prompts = [rng.integers(6, shape[5], size=24).astype(np.int32) for _ in range(n_seq)]
+    _, want = g.decode_greedy_batch(prompts, 25, n_seq=n_seq, want_logits=True)
+    bad = [p.copy() for p in prompts]
+    bad[3][9] = 5                                         # the input of position 10
+    _, got = g.decode_greedy_batch(bad, 25, n_seq=n_seq, want_logits=True)
+    others = [b for b in range(n_seq) if b != 3]
+    np.testing.assert_array_equal(got[:, others].view(np.uint32), want[:, others].view(np.uint32))
+    np.testing.assert_array_equal(got[:10, 3].view(np.uint32), want[:10, 3].view(np.uint32))
+    assert np.isnan(got[10:, 3]).all()
+    g.close()

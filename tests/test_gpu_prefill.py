@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import llama2j_amd as l2j
-from llama2j_amd.binding import BUFFER, L2JError
+from llama2j_amd.binding import BUFFER, TENSOR, L2JError
 from tests.test_gpu_batch import LOGIT_TOL, oracle_of, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -252,4 +252,39 @@ def test_passes_of_many_positions(shape):
             assert rel_err(k[:, :n], want_k[:, :n].astype(np.float64)) < CLOSE, (n, first)
             assert rel_err(v[:, :n], want_v[:, :n].astype(np.float64)) < CLOSE, (n, first)
             assert not k[:, n:].any() and not v[:, n:].any(), (n, first)
+    g.close()
+
+
+@pytest.mark.parametrize("shape,n,flash,split", [
+    ((512, 1024, 2, 8, 2, 1008, 64, 0), 40, 1, 0),        # head 64: blocks of 16 positions
+    ((4096, 512, 2, 32, 8, 512, 608, 0), 600, 1, 0),      # head 128: pairs of blocks of 32
+    ((4096, 512, 2, 16, 16, 512, 304, 0), 300, 1, 0),     # head 256: pairs of blocks of 16
+    ((512, 1024, 2, 8, 2, 1008, 64, 0), 40, 2, 1),        # the keys shared by the waves of a workgroup,
+    ((1024, 512, 2, 8, 4, 512, 64, 0), 50, 2, 4),         # and by four workgroups
+    ((512, 768, 2, 2, 2, 512, 40, 1), 38, 2, 1),
+])
+def test_values_that_are_not_finite_stay_behind_the_causal_mask(shape, n, flash, split):
+    """A token whose embedding holds a NaN, in the middle of a tile of keys: the positions before it attend to none of its
+    rows and keep theirs, to the bit, and all positions from it on are NaN from the second layer's rows on."""
+    kvd = shape[0] // shape[3] * shape[4]
+    rng = np.random.default_rng(n)
+    g = l2j.Transformer(l2j.Config(*shape), options={"prefill_flash": flash, "prefill_split": split})
+    g.fill_synthetic(9, 0.02)
+    emb = (0.02 * rng.standard_normal((shape[5], shape[0]))).astype(np.float32)
+    emb[5, 3] = np.nan
+    g.upload_f32(TENSOR.TOK_EMB, emb)
+    g.finalize()
+    tokens = np.concatenate([[1], rng.integers(6, shape[5], size=n - 1)]).astype(np.int32)
+    g.prefill(tokens, want_logits=False)
+    want_k, want_v = (x.reshape(shape[2], shape[6], kvd) for x in caches(g, shape))
+    for t in (n - 1, n // 2 + 3, 5, 0):
+        g.reset()
+        bad = tokens.copy()
+        bad[t] = 5
+        logits, _ = g.prefill(bad)
+        assert np.isnan(logits).all(), t
+        for got, want in zip(caches(g, shape), (want_k, want_v)):
+            got = got.reshape(shape[2], shape[6], kvd)
+            np.testing.assert_array_equal(got[:, :t].view(np.uint32), want[:, :t].view(np.uint32), err_msg=str(t))
+            assert np.isnan(got[1, t:n]).all(), t
     g.close()
