@@ -33,10 +33,10 @@ __host__ __device__ inline size_t digit_tiles(int rows) { return (size_t)(rows +
 // The exponent s for a group whose largest magnitude has the bits `amax` (sign cleared), and 2^-s.
 __device__ __forceinline__ int digit_shift(unsigned amax, float *inv)
 {
-    // 2^e <= amax < 2^(e+1): s = 29 - e, no larger than 126 (below 2^-97 the step stays at 2^-126)
+    // 2^e <= amax < 2^(e+1): s = 29 - e, no larger than 149 (below 2^-120 every float is a multiple of the step 2^-149)
     const int e = (int)(amax >> 23) - 127;
-    const int s = min(29 - e, 126);
-    *inv = amax >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : ldexpf(1.0f, -s);
+    const int s = min(29 - e, 149);
+    *inv = amax >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : amax == 0u ? 1.0f : ldexpf(1.0f, -s);
     return s;
 }
 
@@ -222,11 +222,12 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
 #pragma unroll
         for (int r = 0; r < 4; r++) cw[r][T] = *reinterpret_cast<const v4i *>(cp[r] + co + 1024 * T);
     // digits of the first group
+    float sx0;
     {
         v4i st[NST];
 #pragma unroll
         for (int q = 0; q < NST; q++) st[q] = (xd + (q * NT / 2048) * xstep + q * NT % 2048)[(unsigned)tid];
-        lsx[xt] = xs[xso];
+        sx0 = xs[xso];
 #pragma unroll
         for (int q = 0; q < NST; q++) dg_lds[q * NT + tid] = st[q];
     }
@@ -263,6 +264,35 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
             for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) f[p][mt][r][e] = f0[p][mt][r][e];
+    // Where 2^-s of some vector is so small that its product with a matrix's scale would lose bits (below 2^-126), all sums are kept
+    // times 2^48 from that group on, unless a group of some vector is so large that this might carry its sum past the largest
+    // float.  (2^-s into the sum of digits instead, as k_dstream has it, is one product more behind the matrix cores: W1 and W3
+    // of the 7B shape with 1024 vectors 330 -> 336 us; the vectors looked through ahead 330 -> 335.)  Every wave holds the 2^-s of all
+    // the workgroup's vectors, so all come to the same power.
+    const bool live = col * PT * 32 + xt < a.npos;
+    float up = 1.0f;
+    bool large = false;
+    auto keep = [&](float x) {
+        x = live ? x : 1.0f;
+        if (__any(!(x >= 0x1p-64f && x <= 0x1p20f))) {
+            large |= __any(x > 0x1p20f) != 0;
+            const float k = large ? 1.0f : __any(x < 0x1p-64f) ? 0x1p48f : up;
+            if (k != up) {
+                const float by = k > up ? 0x1p48f : 0x1p-48f;
+#pragma unroll
+                for (int p = 0; p < PT; p++)
+#pragma unroll
+                    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) f[p][mt][r][e] *= by;
+                up = k;
+            }
+        }
+        return x * up;
+    };
+    lsx[xt] = keep(sx0);
     float rm[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) rm[r] = sp[r][n].x;
@@ -336,10 +366,11 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        lsx[((g + 1) & 1) * 32 * PT + xt] = nsx;
+        lsx[((g + 1) & 1) * 32 * PT + xt] = keep(nsx);
         __syncthreads();
     }
     const int ldo = 16 * a.ntiles;
+    const float down = up == 1.0f ? 1.0f : 0x1p-48f;
 #pragma unroll
     for (int p = 0; p < PT; p++)
 #pragma unroll
@@ -351,7 +382,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
                     float *o = a.out + ((size_t)slice * a.npos + pos) * ldo;
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[p][mt][r][e];
+                        if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[p][mt][r][e] * down;
                 }
             }
 }
@@ -441,8 +472,8 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
                 }
                 v4f y;
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    y[e] = fmaf(fmaf((float)hi[e], 65536.0f, (float)lo[e]), c.s[r].x * sx[mt][e], c.s[r].y * sm[mt][e]);
+                for (int e = 0; e < 4; e++)   // (the power of two into the sum, which takes it exactly: times the scale a small one would lose bits)
+                    y[e] = fmaf(fmaf((float)hi[e], 65536.0f, (float)lo[e]) * sx[mt][e], c.s[r].x, c.s[r].y * sm[mt][e]);
                 *reinterpret_cast<v4f *>(red + (((wave * NB + mt) * 2 + r) * 64 + lane) * 4) = y;
             }
     };
