@@ -588,8 +588,14 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     int known = steps;
     for (int i = 0; i < nseq; i++) known = std::min(known, n_prompt[i] + 1);
     if (known < 2 || b.step_grid > 0) known = 0;
-    const int per = std::min(known, kRowsMax / nseq);
-    if (known > 0 && (rc = ensure_rows(c, per * nseq))) return rc;
+    int per = std::min(known, kRowsMax / nseq);
+    if (known > 0) {
+        int got = 0;
+        rc = ensure_rows(c, per * nseq, 2 * nseq, &got);
+        if (rc == L2J_E_OOM) known = 0;   // (the loop takes these positions as well)
+        else if (rc) return rc;
+        per = got / nseq;
+    }
     BatchState h{};
     h.pos = known > 0 && !logits_log ? known - 1 : 0;
     for (int i = 0; i < nseq; i++) { h.token[i] = 1; h.n_prompt[i] = n_prompt[i]; }   // BOS first (J/Run.java:612)

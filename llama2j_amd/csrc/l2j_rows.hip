@@ -197,8 +197,14 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
             hipError_t e = hipMalloc(reinterpret_cast<void **>(&b.pf_part), (size_t)cf.n_heads * nqb * kPflashMaxSplit * (32 + 16 * hs) * sizeof(float));
             if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&b.pf_cnt), (size_t)cf.n_heads * nqb * sizeof(unsigned));
             if (e == hipSuccess) e = hipMemsetAsync(b.pf_cnt, 0, (size_t)cf.n_heads * nqb * sizeof(unsigned), s);
-            if (e != hipSuccess) return e;
-            b.pf_blocks = nqb;
+            if (e == hipErrorOutOfMemory) {   // (the keys of a block in one workgroup then)
+                (void)hipGetLastError();
+                split = 1;
+            } else if (e != hipSuccess) {
+                return e;
+            } else {
+                b.pf_blocks = nqb;
+            }
         }
     }
     const int qkv_parts = std::min((dim + 2 * kvd + 1023) / 1024, std::max(1, 4 * c->n_cu / rows));   // (few rows: their columns over several workgroups)
@@ -253,8 +259,9 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
     return hipGetLastError();
 }
 
-// Room in the context's buffers for passes of `rows` rows.
-int l2j::ensure_rows(l2j_ctx *c, int rows)
+// Room in the context's buffers for passes of `rows` rows, or, where the device memory does not suffice, of half as many and so
+// on down to `least` (passes of many rows are faster, but nothing needs them): *got, at most rows.
+int l2j::ensure_rows(l2j_ctx *c, int rows, int least, int *got)
 {
     const int rc = ensure_batch_tiles(c);
     if (rc) return rc;
@@ -262,8 +269,14 @@ int l2j::ensure_rows(l2j_ctx *c, int rows)
     if (c->rows.cap < rows) {
         HIPCHK(hipStreamSynchronize(c->stream));
         c->rows.release();
-        HIPCHK(c->rows.alloc(c, rows, true));
+        hipError_t e;
+        for (int n = rows; (e = c->rows.alloc(c, n, true)) == hipErrorOutOfMemory; n = std::max(least, n / 2)) {
+            (void)hipGetLastError();   // (or the next launch would report it)
+            if (n <= least) break;
+        }
+        HIPCHK(e);
     }
+    *got = std::min(rows, c->rows.cap);
     return L2J_OK;
 }
 
@@ -283,9 +296,11 @@ int l2j::prefill_positions(l2j_ctx *c, const int32_t *tokens, int32_t n, int32_t
         if (tokens[i] < 0 || tokens[i] >= cf.vocab_size) return fail(L2J_E_ARG, "token id out of range");
     HIPCHK(hipSetDevice(cf.device));
     // passes of at most kRowsMax positions, as even as they come
-    const int npass = (n + kRowsMax - 1) / kRowsMax, per = (n + npass - 1) / npass;
-    const int rc = ensure_rows(c, per);
+    auto even = [&](int most) { const int npass = (n + most - 1) / most; return (n + npass - 1) / npass; };
+    int got = 0;
+    const int rc = ensure_rows(c, even(kRowsMax), std::min(n, kRowTile), &got);
     if (rc) return rc;
+    const int per = even(got);
     RowBufs &b = c->rows;
     while ((int)c->events.size() < 2) {
         hipEvent_t ev;

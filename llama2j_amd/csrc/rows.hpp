@@ -39,7 +39,7 @@ struct RowJob {
     long seq_stride, layer_stride, head_stride, row_stride;   // of the cache, floats
     int norm_from;                                            // rows from here on are wanted after the final norm
 };
-int ensure_rows(l2j_ctx *c, int rows);
+int ensure_rows(l2j_ctx *c, int rows, int least, int *got);
 hipError_t launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job);
 
 // l2j_batch.hip

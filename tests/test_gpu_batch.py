@@ -429,3 +429,48 @@ def test_a_product_keeps_its_precision_at_every_magnitude(shape, tensor, rows, K
     zero, _ = g.batch_matmul(tensor, 1, np.zeros((16, K), dtype=np.float32), rows)
     assert not zero.any()
     g.close()
+
+
+class FullDevice:
+    """All of the device's free memory but `leave` bytes, held for the duration of a with block."""
+
+    def __init__(self, leave):
+        import ctypes as C
+        self.C, self.hip, self.leave, self.held = C, C.CDLL("libamdhip64.so"), leave, []
+
+    def free_bytes(self):
+        free, total = self.C.c_size_t(0), self.C.c_size_t(0)
+        assert self.hip.hipMemGetInfo(self.C.byref(free), self.C.byref(total)) == 0
+        return free.value
+
+    def __enter__(self):
+        while self.free_bytes() > self.leave + (4 << 20):
+            p = self.C.c_void_p()
+            n = min(self.free_bytes() - self.leave, 32 << 30) & ~((2 << 20) - 1)
+            assert self.hip.hipMalloc(self.C.byref(p), self.C.c_size_t(n)) == 0
+            self.held.append(p)
+        return self
+
+    def __exit__(self, *a):
+        for p in self.held:
+            self.hip.hipFree(p)
+
+
+def test_known_positions_go_through_the_loop_where_the_memory_for_their_pass_is_missing():
+    """The pass over the known prompt positions is a shortcut: with room for half its rows it runs in smaller passes, with room for
+    none the loop takes every position.  The tokens are those of the run with all the memory."""
+    shape = (256, 28672, 1, 1, 1, 512, 64, 1)         # a row's hidden products are large: 205 MB for the step's 32 rows, 630 for 672
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    rng = np.random.default_rng(5)
+    prompts = [rng.integers(2, shape[5], size=20).astype(np.int32) for _ in range(32)]
+    want, logits = g.decode_greedy_batch(prompts, 30, n_seq=32, want_logits=True)
+    for leave in (420 << 20, 120 << 20):
+        g.release_batch()
+        g.decode_greedy_batch([p[:0] for p in prompts[:31]] + [prompts[31]], 30, n_seq=32)     # the step's buffers, prompts of this length
+        with FullDevice(leave):
+            got, _ = g.decode_greedy_batch(prompts, 30, n_seq=32)
+        for b in range(32):
+            same_until_a_tie(got[b], want[b], logits[:, b], "sequence %d, %d MB" % (b, leave >> 20))
+    g.close()

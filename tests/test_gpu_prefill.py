@@ -7,7 +7,7 @@ import pytest
 
 import llama2j_amd as l2j
 from llama2j_amd.binding import BUFFER, TENSOR, L2JError
-from tests.test_gpu_batch import LOGIT_TOL, oracle_of, rel_err
+from tests.test_gpu_batch import FullDevice, LOGIT_TOL, oracle_of, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -287,4 +287,28 @@ def test_values_that_are_not_finite_stay_behind_the_causal_mask(shape, n, flash,
             got = got.reshape(shape[2], shape[6], kvd)
             np.testing.assert_array_equal(got[:, :t].view(np.uint32), want[:, :t].view(np.uint32), err_msg=str(t))
             assert np.isnan(got[1, t:n]).all(), t
+    g.close()
+
+
+def test_a_prompt_goes_through_in_smaller_passes_where_the_memory_for_a_large_one_is_missing():
+    """1100 positions with room for passes of 275 instead of 550, the decode loop with option prefill likewise; other calls go on
+    as before, and so does the prompt once there is room."""
+    shape = (256, 28672, 1, 1, 1, 512, 1104, 1)       # (a pass of 550 rows takes 570 MB, of 275 rows 290)
+    rng = np.random.default_rng(6)
+    g = model(shape)
+    tokens = np.concatenate([[1], rng.integers(2, shape[5], size=1099)]).astype(np.int32)
+    want, _ = g.prefill(tokens)
+    want_k, _ = caches(g, shape)
+    single, _ = g.decode_greedy(tokens[1:], 1104)
+    g.release_batch()
+    g.prefill(tokens[:8])                              # the copy of the matrices and the buffers of eight rows (205 MB)
+    with FullDevice(200 << 20):
+        g.reset()
+        got, _ = g.prefill(tokens)
+        got_k, _ = caches(g, shape)
+        assert rel_err(got, want.astype(np.float64)) < CLOSE and rel_err(got_k, want_k.astype(np.float64)) < CLOSE
+        g.set_option("prefill", 1)
+        np.testing.assert_array_equal(g.decode_greedy(tokens[1:], 1104)[0], single)
+    again, _ = g.prefill(tokens)
+    np.testing.assert_array_equal(again.view(np.uint32), want.view(np.uint32))
     g.close()
