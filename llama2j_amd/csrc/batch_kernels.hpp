@@ -448,14 +448,15 @@ __global__ void __launch_bounds__(kBgThreads) k_bgemm_f32(const BGemmF32 a)
 
 // ---- the element-wise kernels between the products --------------------------------------------------------------
 
-constexpr int kLogSlots = 32;   // steps whose logits are on their way to the caller while the next ones are computed
+constexpr int kLogSlots = 32;   // at most: steps whose logits are on their way to the caller while the next ones are computed
 
 // Loop state of a batched decode, on the device.
 struct BatchState {
     int pos;              // position of the step being computed
     int token[kMaxBatch];    // input token of every sequence at this position
     int n_prompt[kMaxBatch];
-    float *log;           // null, or kLogSlots x (sequences, vocab): the logits of step pos also go to slot pos % kLogSlots
+    float *log;           // null, or log_slots x (sequences, vocab): the logits of step pos also go to slot pos % log_slots
+    int log_slots;
 };
 
 // x[b] = row token[b] of the embedding table (J/Run.java:72).  As the first kernel of a step it also clears the
@@ -661,7 +662,7 @@ static __global__ void __launch_bounds__(512) k_bnext(const BNext a)
     const int b = blockIdx.y, tid = threadIdx.x;
     const long n = (long)gridDim.y * a.vocab;
     const int pos = a.st->pos;
-    float *log = a.st->log ? a.st->log + (pos % kLogSlots) * n + (long)b * a.vocab : nullptr;
+    float *log = a.st->log ? a.st->log + (pos % a.st->log_slots) * n + (long)b * a.vocab : nullptr;
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
     for (int i = 4 * (tid + 512 * blockIdx.x); i < a.vocab; i += 4 * 512 * kNextParts) {   // (vocab % 16 == 0)

@@ -148,21 +148,32 @@ struct l2j::BatchBufs {
     int h_fault = 0;
     int *h_pin = nullptr;   // pinned: every transfer of a call goes through it, as in the single-sequence loops
     // the logits of every step for a caller that wants them: kept here while later steps are computed, made by the first such call
-    float *log_dev = nullptr, *log_pin = nullptr;   // kLogSlots steps on the device, one pinned
+    float *log_dev = nullptr, *log_pin = nullptr;   // log_slots steps on the device, one pinned
+    int log_slots = 0;
     hipStream_t log_stream = nullptr;
     hipEvent_t log_step[kLogSlots] = {};            // the slot holds its step's logits
     BatchSamplers samplers;   // l2j_decode_sample_batch: a sampler per sequence (made by its first call)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipError_t ensure_log(size_t step_floats)
+    // Slots for a call of `steps` steps: one a step up to kLogSlots, or as many as the device memory suffices for.
+    hipError_t ensure_log(size_t step_floats, int steps)
     {
-        if (log_step[kLogSlots - 1]) return hipSuccess;
         hipError_t e = hipSuccess;
-        if (!log_dev) e = hipMalloc(reinterpret_cast<void **>(&log_dev), kLogSlots * step_floats * sizeof(float));
+        const int want = std::min(steps, kLogSlots);
+        if (log_slots < want) {
+            (void)hipFree(log_dev);   // (no call is under way: nothing uses it)
+            log_dev = nullptr; log_slots = 0;
+            for (int n = want; n > 0; n /= 2) {
+                e = hipMalloc(reinterpret_cast<void **>(&log_dev), n * step_floats * sizeof(float));
+                if (e == hipSuccess) log_slots = n;
+                if (e != hipErrorOutOfMemory) break;
+                (void)hipGetLastError();   // (or the next launch would report it)
+            }
+        }
         if (e == hipSuccess && !log_pin) e = hipHostMalloc(reinterpret_cast<void **>(&log_pin), step_floats * sizeof(float), hipHostMallocDefault);
         if (e == hipSuccess && !log_stream) e = hipStreamCreateWithFlags(&log_stream, hipStreamNonBlocking);
-        for (int i = 0; i < kLogSlots; i++)
+        for (int i = 0; i < log_slots; i++)
             if (e == hipSuccess && !log_step[i]) e = hipEventCreateWithFlags(&log_step[i], hipEventDisableTiming);
         return e;
     }
@@ -472,7 +483,7 @@ public:
     void wait_slot(int pos)
     {
         std::unique_lock<std::mutex> l(mu);
-        cv.wait(l, [&] { return err != hipSuccess || pos - taken < kLogSlots; });
+        cv.wait(l, [&] { return err != hipSuccess || pos - taken < b.log_slots; });
     }
     // log_step of step `pos` has been recorded
     void offer(int pos)
@@ -509,7 +520,7 @@ private:
 
     hipError_t take(int pos)
     {
-        const int slot = pos % kLogSlots;
+        const int slot = pos % b.log_slots;
         hipError_t e = hipEventSynchronize(b.log_step[slot]);
         if (e == hipSuccess) e = hipMemcpyAsync(b.log_pin, b.log_dev + slot * step_floats, step_floats * sizeof(float), hipMemcpyDeviceToHost, b.log_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(b.log_stream);
@@ -575,7 +586,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     if (seeds && (rc = seed_batch_samplers(c, b, seeds))) return rc;
     const size_t step_floats = (size_t)nseq * vocab;
     if (logits_log) {
-        const hipError_t le = b.ensure_log(step_floats);
+        const hipError_t le = b.ensure_log(step_floats, steps);
         if (le != hipSuccess) return hip_rc(le, "logits of every step");
     }
     auto fail_hip = [&](hipError_t e, const char *what) {
@@ -600,6 +611,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     h.pos = known > 0 && !logits_log ? known - 1 : 0;
     for (int i = 0; i < nseq; i++) { h.token[i] = 1; h.n_prompt[i] = n_prompt[i]; }   // BOS first (J/Run.java:612)
     h.log = logits_log ? b.log_dev : nullptr;
+    h.log_slots = std::max(1, b.log_slots);
     memcpy(b.h_pin, &h, sizeof(h));
     memset(b.h_pin + state_ints, 0, (size_t)nseq * pcap * sizeof(int));
     for (int s = 0; s < nseq && prompt_stride > 0; s++)
@@ -616,7 +628,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     // (the sampled token replaces the argmax k_bnext stored)
     auto after_logits = [&](int pos) {
         if (logits_log && e == hipSuccess) {
-            e = hipEventRecord(b.log_step[pos % kLogSlots], c->stream);
+            e = hipEventRecord(b.log_step[pos % b.log_slots], c->stream);
             if (e == hipSuccess) taker.offer(pos);
         }
         if (seeds && e == hipSuccess) {

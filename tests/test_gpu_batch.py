@@ -474,3 +474,28 @@ def test_known_positions_go_through_the_loop_where_the_memory_for_their_pass_is_
         for b in range(32):
             same_until_a_tie(got[b], want[b], logits[:, b], "sequence %d, %d MB" % (b, leave >> 20))
     g.close()
+
+
+def test_the_logits_of_every_step_come_through_as_many_slots_as_there_is_memory_for():
+    """65 MB of logits per step (a vocabulary of 512000, 32 sequences): all slots, a few, one; and a short call keeps no more than it
+    has steps.  The same logits to the bit."""
+    shape = (256, 256, 1, 1, 1, 512000, 64, 1)
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    prompts = [np.array([7 + b, 9], dtype=np.int32) for b in range(32)]
+    want_tokens, want = g.decode_greedy_batch(prompts, 9, n_seq=32, want_logits=True)
+    for leave in (320 << 20, 100 << 20):
+        g.release_batch()
+        g.decode_greedy_batch(prompts, 9, n_seq=32)                  # the step's buffers
+        with FullDevice(leave) as full:
+            got_tokens, got = g.decode_greedy_batch(prompts, 9, n_seq=32, want_logits=True)
+            assert full.free_bytes() < leave - (60 << 20)
+        np.testing.assert_array_equal(got_tokens, want_tokens)
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    g.release_batch()
+    g.decode_greedy_batch(prompts, 2, n_seq=32)
+    before = FullDevice(0).free_bytes()
+    g.decode_greedy_batch(prompts, 2, n_seq=32, want_logits=True)
+    assert before - FullDevice(0).free_bytes() < 3 * 66 << 20        # two slots of 65 MB
+    g.close()
