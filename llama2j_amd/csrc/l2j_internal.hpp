@@ -31,6 +31,7 @@ inline thread_local std::string g_err;
 
 inline int fail(int code, const std::string &msg)
 {
+    if (code == L2J_E_HIP || code == L2J_E_OOM) (void)hipGetLastError();   // (reported here: the next call's launches must not report it again)
     g_err = msg;
     return code;
 }

@@ -499,3 +499,24 @@ def test_the_logits_of_every_step_come_through_as_many_slots_as_there_is_memory_
     g.decode_greedy_batch(prompts, 2, n_seq=32, want_logits=True)
     assert before - FullDevice(0).free_bytes() < 3 * 66 << 20        # two slots of 65 MB
     g.close()
+
+
+def test_a_call_after_one_that_found_no_memory_is_not_blamed_for_it():
+    """The error of a failed allocation stays behind in the runtime: the calls that follow a failed one, of its context and of
+    others, must not take it for their own launches'."""
+    shape = (256, 28672, 1, 1, 1, 512, 64, 1)
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    prompt = np.array([5, 6, 7], dtype=np.int32)
+    want, _ = g.decode_greedy(prompt, 24)
+    with FullDevice(100 << 20):
+        with pytest.raises(L2JError, match="out of memory"):
+            g.decode_greedy_batch([prompt], 24, n_seq=32)
+        g.reset()
+        np.testing.assert_array_equal(g.decode_greedy(prompt, 24)[0], want)
+        with pytest.raises(L2JError, match="out of memory"):
+            l2j.Transformer(l2j.Config(4096, 11008, 4, 32, 32, 512, 64, 0))
+        g.forward(1, 0)
+    np.testing.assert_array_equal(g.decode_greedy_batch([prompt], 24, n_seq=32)[0][0, :len(want)], want)
+    g.close()
