@@ -298,32 +298,44 @@ def main():
         try:
             bsteps = min(steps, 288)
             n0 = min(bsteps, len(tokens))
-            bmean = (bsteps - 1) / 2.0 + 0.5   # mean position of the timed steps 1 .. bsteps - 1
+            # The prompt positions are a pass of their own (n_prompt + 1 of each sequence), so the steps behind them are timed as the
+            # difference of two lengths: b0 steps (the pass and one step) and all bsteps.
+            b0 = min(n_prompt + 2, bsteps - 1)
+            bmean = (b0 + bsteps - 1) / 2.0    # mean position of the steps b0 .. bsteps - 1
             wbytes = g.bytes_per_token(0)      # the weights, read once per step for all sequences
             kvbytes = g.bytes_per_token(int(round(bmean))) - wbytes   # one sequence's cache rows at the mean position
+
+            def timed_steps(run):
+                run(bsteps)                                              # warm: the buffers of the longer call serve both
+                long_toks, long_s = min((run(bsteps) for _ in range(2)), key=lambda r: r[1])
+                short_s = min(run(b0)[1] for _ in range(2))
+                return long_toks, long_s, short_s, (long_s - short_s) / (bsteps - b0)
+
             runs = {}
             for n_seq in (() if a.prefill_only else (32, 16)):
                 prompts = [prompt] + [synth_prompt(seed + 1000 + b, n_prompt, shape[5]) for b in range(1, n_seq)]
                 if n_seq == 32:
                     prompts32 = prompts
-                g.decode_greedy_batch(prompts, min(bsteps, 8), n_seq=n_seq)          # warm
-                btoks, bsec = g.decode_greedy_batch(prompts, bsteps, n_seq=n_seq)
-                per = bsec / (bsteps - 1)
-                runs[n_seq] = {"sequences": n_seq, "steps": bsteps, "tok_s": round(n_seq * (bsteps - 1) / bsec, 1), "ms_per_step": round(per * 1e3, 4),
+                btoks, bsec, bshort, per = timed_steps(lambda n: g.decode_greedy_batch(prompts, n, n_seq=n_seq))
+                prompt_s = bshort - (b0 - n_prompt - 1) * per if b0 > n_prompt else 0.0
+                runs[n_seq] = {"sequences": n_seq, "steps": bsteps - b0, "tok_s": round(n_seq / per, 1), "ms_per_step": round(per * 1e3, 4),
+                               "prompt_pass": {"positions": n_seq * (n_prompt + 1), "ms": round(prompt_s * 1e3, 4),
+                                               "positions_per_s": round(n_seq * (n_prompt + 1) / prompt_s, 1)} if prompt_s > 0 else None,
+                               "whole_run": {"positions": n_seq * bsteps, "ms": round(bsec * 1e3, 3)},
                                "roofline": {"bound": "hbm", "achieved": round((wbytes + n_seq * kvbytes) / per / 1e9, 1), "peak": 8000.0, "unit": "GB/s",
                                             "frac": round((wbytes + n_seq * kvbytes) / per / 8e12, 4),
                                             "bytes_per_step": int(wbytes + n_seq * kvbytes),
                                             "note": "weights once + every sequence's KV cache rows at the mean position, over the whole step time"},
+                               "note": "the steps behind the prompts' pass (positions %d .. %d): difference of two runs" % (b0, bsteps - 1),
                                "sequence_0_equals_the_single_decode": bool(np.array_equal(btoks[0, :n0], tokens[:n0]))}
             if runs:
                 try:   # the same 32 loops with a sampler each, at the reference's default temperature and top-p (J/CommandLine.java:24-25)
-                    stoks32, ssec32 = g.decode_sample_batch(prompts32, bsteps, 0.9, 0.9, np.arange(32, dtype=np.int64) + seed, n_seq=32)
-                    runs[32]["sampled"] = {"temperature": 0.9, "topp": 0.9, "tok_s": round(32 * (bsteps - 1) / ssec32, 1),
-                                           "ms_per_step": round(ssec32 / (bsteps - 1) * 1e3, 4)}
+                    sper = timed_steps(lambda n: g.decode_sample_batch(prompts32, n, 0.9, 0.9, np.arange(32, dtype=np.int64) + seed, n_seq=32))[3]
+                    runs[32]["sampled"] = {"temperature": 0.9, "topp": 0.9, "tok_s": round(32 / sper, 1), "ms_per_step": round(sper * 1e3, 4)}
                 except l2j.L2JError as e:   # a vocabulary above the one-launch sampling step's
                     runs[32]["sampled"] = {"error": str(e)}
                 out["batched_decode"] = runs[32]
-                out["batched_decode"]["sixteen_sequences"] = {k: runs[16][k] for k in ("tok_s", "ms_per_step", "sequence_0_equals_the_single_decode")}
+                out["batched_decode"]["sixteen_sequences"] = {k: runs[16][k] for k in ("tok_s", "ms_per_step", "prompt_pass", "sequence_0_equals_the_single_decode")}
         except l2j.L2JError as e:  # shapes the batched path does not take (rows that are not whole groups of 256)
             out["batched_decode"] = {"error": str(e)}
         # Nor this: the forward passes of 1024 consecutive positions of one sequence, in one pass through the same products
