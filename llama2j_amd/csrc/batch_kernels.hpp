@@ -192,10 +192,8 @@ struct BgWave {
         for (int T = 0; T < TB; T++) cw[slot][T] = load_stream(p + 64 * T);
     }
 
-    // This wave's share of workgroup (bx, by) of a gx-wide grid; first = false: the first codes are not requested yet
-    // (run() does it once the activations are requested: a wave's loads return in order, and behind the codes the
-    // activations would arrive with them).
-    __device__ __forceinline__ void begin(int bx, int by_, int gx_, bool first_codes)
+    // This wave's share of workgroup (bx, by) of a gx-wide grid; requests the first codes.
+    __device__ __forceinline__ void begin(int bx, int by_, int gx_)
     {
         const BGemm &a = *ap;
         const int tid = threadIdx.x;
@@ -223,17 +221,14 @@ struct BgWave {
         ntiles = m0.tiles + m1.tiles + m2.tiles;
         first = bx; gx = gx_;
         cnt = bx < ntiles ? (ntiles - bx + gx - 1) / gx : 0;
-        if (first_codes) {
 #pragma unroll
-            for (int d = 0; d < kBgDepth; d++) request(d, d);
-        }
+        for (int d = 0; d < kBgDepth; d++) request(d, d);
     }
 
-    // requested = begin(.., true) was called.  COH: the activations were written by other workgroups of this launch and
-    // the partial sums are read by other workgroups of it (device-coherent loads, write-through stores).
+    // After begin().  The activations were written by other workgroups of this launch and the partial sums are read by other
+    // workgroups of it (device-coherent loads, write-through stores).
     // lds: bg_lds_bytes(NSEQ, HV) bytes, free when the workgroup's waves get here.
-    template <bool COH>
-    __device__ __forceinline__ void run(float *lds, bool requested)
+    __device__ __forceinline__ void run(float *lds)
     {
         const BGemm &a = *ap;
         v4f32 *raw = reinterpret_cast<v4f32 *>(lds);                      // [tile of the batch][wave][column block][lane]
@@ -248,17 +243,7 @@ struct BgWave {
 #pragma unroll
             for (int T2 = 0; T2 < TB; T2 += 2) {
                 float v[2][16];
-                if (COH) {
-                    ld_coh64x2(xsrc + 64 * T2, xsrc + 64 * (T2 + 1), v[0], v[1]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 2; e++)
-#pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            const float4 f = reinterpret_cast<const float4 *>(xsrc + 64 * (T2 + e))[q];
-                            v[e][4 * q] = f.x; v[e][4 * q + 1] = f.y; v[e][4 * q + 2] = f.z; v[e][4 * q + 3] = f.w;
-                        }
-                }
+                ld_coh64x2(xsrc + 64 * T2, xsrc + 64 * (T2 + 1), v[0], v[1]);
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const float (&w)[16] = v[e];
@@ -284,10 +269,6 @@ struct BgWave {
             t += __shfl_xor(t, 16);
             t += __shfl_xor(t, 32);
             if (s == 0) sxw[wave * NSEQ + 16 * nb + c] = active ? t : 0.0f;
-        }
-        if (!requested) {
-#pragma unroll
-            for (int d = 0; d < kBgDepth; d++) request(d, d);
         }
         __syncthreads();
         for (int i0 = 0; i0 < cnt; i0 += WAVES) {
@@ -350,9 +331,7 @@ struct BgWave {
                             y[3] += fmaf(sc[q][1].z, t[3], sc[q][1].w * sx);
                         }
                     }
-                    float *o = mine.out + (long)(16 * nb + c) * mine.rows + 4 * s;
-                    if (COH) st_coh16(o, y);
-                    else *reinterpret_cast<v4f32 *>(o) = y;
+                    st_coh16(mine.out + (long)(16 * nb + c) * mine.rows + 4 * s, y);
                 }
             }
             __syncthreads();   // (the next batch writes the same LDS)

@@ -289,11 +289,11 @@ __global__ void __launch_bounds__(kBgThreads * NB) k_bstep(const BStep *__restri
     BgWave<NB, NB> w(a.g[BS_QKV]);   // aimed at the four products of the argument in turn (the argument is never copied)
     int S = bg_slices(a.g[BS_QKV].K);
     bool in = wg < a.gx[BS_QKV] * S;
-    if (in) w.begin(wg / S, wg % S, a.gx[BS_QKV], true);
+    if (in) w.begin(wg / S, wg % S, a.gx[BS_QKV]);
     for (int l = 0; l < a.n_layers; l++) {
 #pragma unroll 1
         for (int k = 0; k < 4; k++) {
-            if (in) w.template run<true>(lds, true);
+            if (in) w.run(lds);
             wait_own_stores();
             step_barrier(a.bar, nbar++);
             const bool last = l + 1 == a.n_layers;
@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(kBgThreads * NB) k_bstep(const BStep *__restri
             w.layer = l + (k == BS_W2 ? 1 : 0);
             S = bg_slices(a.g[nk].K);
             in = wg < a.gx[nk] * S;
-            if (in) w.begin(wg / S, wg % S, a.gx[nk], true);   // the first codes travel while the others arrive
+            if (in) w.begin(wg / S, wg % S, a.gx[nk]);   // the first codes travel while the others arrive
             step_barrier(a.bar, nbar++);
         }
     }

@@ -225,7 +225,7 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
         RowAttn t{};
         t.q = b.q; t.kc = k.kc; t.vc = k.vc; t.seq_stride = k.seq_stride; t.head_stride = k.head_stride; t.row_stride = k.row_stride;
         t.out = b.xb; t.nseg = job.nseg; t.T = job.T; t.pos0 = job.pos0; t.n_heads = cf.n_heads; t.kv_mul = c->kv_mul; t.dim = dim;
-        t.dig = b.dig; t.sqrt_hs = sqrtf((float)hs); t.nqb = nqb; t.pf_part = b.pf_part; t.pf_cnt = b.pf_cnt;
+        t.dig = b.dig; t.sqrt_hs = sqrtf((float)hs); t.pf_part = b.pf_part; t.pf_cnt = b.pf_cnt;
         if (shared_keys) {
             const dim3 g(cf.n_heads, nqb, split);
             if (hs == 64) hipLaunchKernelGGL((k_pflash<64, 16>), g, dim3(1024), pflash_lds(64, 16), s, t);

@@ -49,6 +49,7 @@ int ensure_batch_tiles(l2j_ctx *c);   // the tile-ordered copy of every matrix
 // k_pflash (the keys of 16 positions shared by the waves of a workgroup, and from kSplitKeysFrom keys on by several workgroups)
 // where k_rows_attn would have fewer than kSharedKeysBelow waves per compute unit for this many keys or more: 40 positions behind 1000
 // of Llama-2-7B 5.0 against 5.8 ms, 128 behind 1000 7.2 against 7.6, 200 from 0 on 9.2 against 9.0, 400 from 0 on 15.3 against 14.7.
+// (kSplitKeysFrom lies below kSharedKeysFrom: it decides with option prefill_flash = 2 alone.)
 constexpr int kSharedKeysFrom = 512, kSharedKeysBelow = 2, kSplitKeysFrom = 192, kPflashMaxSplit = 4;
 inline size_t pflash_lds(int hs, int waves) { return (size_t)(32 * waves + 16 * waves * hs) * sizeof(float); }
 

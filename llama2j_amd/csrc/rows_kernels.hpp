@@ -169,7 +169,6 @@ struct RowAttn {
     int nseg, T, pos0;       // rows: T positions of nseg sequences
     int n_heads, kv_mul, dim;
     float sqrt_hs;
-    int nqb;                 // blocks of 16 positions (k_pflash)
     int paired;              // k_rows_attn: two blocks per workgroup
     // k_pflash with the keys of a (head, block) pair split over gridDim.z workgroups (nseg = 1):
     float *pf_part;          // (head, block, z) x (16 maxima, 16 sums, 16 x head_size values): what each leaves for the last one
