@@ -520,3 +520,27 @@ def test_a_call_after_one_that_found_no_memory_is_not_blamed_for_it():
         g.forward(1, 0)
     np.testing.assert_array_equal(g.decode_greedy_batch([prompt], 24, n_seq=32)[0][0, :len(want)], want)
     g.close()
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(64, 8), (32, 32), (16, 4)])       # head 64, 128, 256
+@pytest.mark.parametrize("n_seq,shortest", [(16, 19), (16, 40), (16, 70), (32, 16), (32, 40)])
+def test_common_prompt_positions_of_a_wide_model(heads, kv_heads, n_seq, shortest):
+    """4096 wide, the attention of a pass has a workgroup for two blocks of a sequence: 20 positions of 16 sequences are two blocks of
+    16, 41 two of 32 (three of 16 with head size 256), 71 two passes.  The logits of every step and sequence against l2j_forward
+    on the sequence's tokens."""
+    shape = (4096, 1024, 2, heads, kv_heads, 512, 96, 0)
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    rng = np.random.default_rng(heads + shortest)
+    prompts = [rng.integers(2, shape[5], size=shortest + int(rng.integers(0, 3))).astype(np.int32) for _ in range(n_seq)]
+    prompts[n_seq - 1] = prompts[n_seq - 1][:shortest]
+    steps = shortest + 4
+    tokens, logits = g.decode_greedy_batch(prompts, steps, n_seq=n_seq, want_logits=True)
+    for b in range(0, n_seq, 1 if n_seq == 16 else 3):
+        g.reset()
+        for pos in range(steps):
+            want = g.forward(1 if pos == 0 else int(tokens[b, pos - 1]), pos)
+            assert rel_err(logits[pos, b], want.astype(np.float64)) < 2e-5, (b, pos)
+            assert tokens[b, pos] == (prompts[b][pos] if pos < len(prompts[b]) else np.argmax(logits[pos, b])), (b, pos)
+    g.close()

@@ -31,7 +31,7 @@ def caches(g, shape):
     return [np.stack([g.read(which, layer) for layer in range(shape[2])]) for which in (BUFFER.KCACHE, BUFFER.VCACHE)]
 
 
-@pytest.mark.parametrize("flash", [2, 0])    # the attention on the matrix cores at every position / at none (default: from position 64 on)
+@pytest.mark.parametrize("flash", [2, 0])    # the keys of 16 positions shared by the waves of a workgroup: always / never (default: few positions behind 512 keys or more)
 @pytest.mark.parametrize("shape", SHAPES)
 def test_prefill_leaves_what_forward_position_by_position_leaves(orc, shape, flash):
     seq_len, kvd = shape[6], shape[0] // shape[3] * shape[4]
@@ -105,7 +105,7 @@ def test_prefill_refuses_what_it_cannot_take(orc):
 
 @pytest.mark.parametrize("shape,n_prompt", [(SHAPES[0], 40), (SHAPES[1], 65), (SHAPES[2], 33)])
 def test_decode_loops_with_option_prefill_give_the_tokens_they_give_without(orc, shape, n_prompt):
-    """Option prefill: the loops take the first whole steps of 32 prompt positions through l2j_prefill and go on from there.
+    """Option prefill: the loops take a prompt of eight ids or more through l2j_prefill and go on from there.
     Greedy against the CPU oracle's loop as well; sampled with the same seed."""
     steps = shape[6]
     prompt = orc.synth_prompt(5, n_prompt, shape[5])
@@ -124,7 +124,7 @@ def test_decode_loops_with_option_prefill_give_the_tokens_they_give_without(orc,
     cpu, _, _ = m.generate_greedy(prompt, steps)
     np.testing.assert_array_equal(got[:len(cpu)], cpu)
     m.close()
-    # a prompt id 1 among the first 32 ends the loop there, as without the option
+    # a prompt id 1 ends the loop there, as without the option
     stop = prompt.copy()
     stop[7] = 1
     g.reset()
@@ -159,28 +159,31 @@ def test_prefill_at_the_published_widths(orc, shape, n):
 
 
 def test_prefill_and_the_batched_decode_share_their_buffers(orc):
-    """Both run in the context's batch buffers (32 rows for prefill): calls of either kind in any order give what they give alone."""
+    """Both use the context's copy of the matrices, and the prompts of a batch run in prefill's buffers: calls of either kind in any
+    order give what they give alone."""
     shape = SHAPES[1]
     g = model(shape)
     rng = np.random.default_rng(3)
     tokens = np.concatenate([[1], rng.integers(2, shape[5], size=44)]).astype(np.int32)
     prompts = [rng.integers(2, shape[5], size=3).astype(np.int32) for _ in range(16)]
     alone_logits, _ = g.prefill(tokens)
-    alone_tokens, _ = g.decode_greedy_batch(prompts, 24, n_seq=16)        # (buffers for 16 sequences replace prefill's)
+    alone_tokens, _ = g.decode_greedy_batch(prompts, 24, n_seq=16)        # (its prompts' pass in prefill's buffers)
     g.reset()
-    again_logits, _ = g.prefill(tokens)                                   # (and prefill's replace those)
+    again_logits, _ = g.prefill(tokens)
     assert np.array_equal(again_logits.view(np.uint32), alone_logits.view(np.uint32))
     again_tokens, _ = g.decode_greedy_batch(prompts + prompts, 24, n_seq=32)
     np.testing.assert_array_equal(again_tokens[:16], alone_tokens)
     g.reset()
-    third, _ = g.prefill(tokens)                                          # (in the buffers of the 32 sequences)
+    third, _ = g.prefill(tokens)                                          # (in the buffers the 32 sequences' pass has grown)
     assert np.array_equal(third.view(np.uint32), alone_logits.view(np.uint32))
 
 
 def test_prefill_past_the_position_where_the_attention_changes_kernels(orc):
-    """By default the attention of a step runs on the matrix cores from position 64 on, and from position 192 on the keys of a
-    head are split over several workgroups: a prompt that crosses both, against position-by-position forwards and the oracle."""
-    shape = (512, 1024, 2, 8, 2, 1008, 480, 0)
+    """By default a pass of few positions over 512 keys or more shares the keys of 16 positions among the waves of a workgroup, and
+    among up to four workgroups: 470 positions at once stay below; behind 480 cached ones 16, 40 and 100 positions have four
+    workgroups per head and block, 180 two, 300 one.  Against position-by-position forwards and the oracle."""
+    shape = (512, 1024, 2, 8, 2, 1008, 800, 0)
+    kvd = 512 * 2 // 8
     rng = np.random.default_rng(640)
     g = model(shape)
     n = 470
@@ -196,6 +199,26 @@ def test_prefill_past_the_position_where_the_attention_changes_kernels(orc):
     m = oracle_of(orc, shape, 9)
     for i, t in enumerate(tokens):
         cpu = m.forward(int(t), i)
+    assert rel_err(got, cpu.astype(np.float64)) < LOGIT_TOL
+    cached, behind = 480, (16, 40, 100, 180, 300)
+    tokens = np.concatenate([tokens, rng.integers(2, shape[5], size=cached + max(behind) - n)]).astype(np.int32)
+    wants = {}
+    g.reset()
+    for i, t in enumerate(tokens):
+        lg = g.forward(int(t), i)
+        if i + 1 - cached in behind:
+            wants[i + 1 - cached] = lg
+    want_k, want_v = (x.reshape(shape[2], shape[6], kvd) for x in caches(g, shape))
+    for more in behind:
+        end = cached + more
+        g.reset()
+        g.prefill(tokens[:cached], want_logits=False)
+        got, _ = g.prefill(tokens[cached:end], pos0=cached)
+        got_k, got_v = (x.reshape(shape[2], shape[6], kvd) for x in caches(g, shape))
+        assert rel_err(got, wants[more].astype(np.float64)) < CLOSE, more
+        assert rel_err(got_k[:, :end], want_k[:, :end].astype(np.float64)) < CLOSE and rel_err(got_v[:, :end], want_v[:, :end].astype(np.float64)) < CLOSE, more
+    for i in range(n, len(tokens)):
+        cpu = m.forward(int(tokens[i]), i)
     assert rel_err(got, cpu.astype(np.float64)) < LOGIT_TOL
     m.close()
 
@@ -311,4 +334,58 @@ def test_a_prompt_goes_through_in_smaller_passes_where_the_memory_for_a_large_on
         np.testing.assert_array_equal(g.decode_greedy(tokens[1:], 1104)[0], single)
     again, _ = g.prefill(tokens)
     np.testing.assert_array_equal(again.view(np.uint32), want.view(np.uint32))
+    g.close()
+
+
+@pytest.mark.parametrize("n_prompt,steps", [(7, 20), (8, 9), (8, 20), (9, 20), (31, 40), (40, 37), (40, 40), (40, 41)])
+def test_option_prefill_at_its_edges(orc, n_prompt, steps):
+    """Prompts on both sides of the eight ids from which the option takes them at once, of no whole number of tiles, and runs that end
+    inside the prompt, with it, and one step behind it: the tokens of the loop without the option."""
+    shape = SHAPES[0]
+    prompt = orc.synth_prompt(7, n_prompt, shape[5])
+    g = model(shape)
+    want, _ = g.decode_greedy(prompt, steps)
+    g.reset()
+    want_s, _ = g.decode_sample(prompt, steps, 0.9, 0.9, 3)
+    g.set_option("prefill", 1)
+    g.reset()
+    np.testing.assert_array_equal(g.decode_greedy(prompt, steps)[0], want)
+    g.reset()
+    np.testing.assert_array_equal(g.decode_sample(prompt, steps, 0.9, 0.9, 3)[0], want_s)
+    g.close()
+
+
+@pytest.mark.parametrize("shape", [
+    (4096, 11008, 2, 32, 32, 512, 1104, 0),     # head 128, the widths of Llama-2-7B
+    (4096, 1024, 2, 64, 8, 512, 1104, 0),       # head 64, eight heads to a kv head
+    (4096, 1024, 2, 16, 4, 512, 1104, 0),       # head 256
+    (8192, 28672, 2, 64, 8, 512, 600, 0),       # the widths of Llama-2-70B
+])
+def test_wide_passes_where_their_kernels_change(shape):
+    """On 256 compute units the attention of these widths has two blocks per workgroup from 257 positions on (an odd number of blocks:
+    one workgroup has one), blocks of 32 positions from 545 on (head sizes 64 and 128; from 257 at 8192 wide), and the products
+    change between 256 x 32 and 512 x 64 with up to sixteen columns of vectors, the last of them ragged.  Against
+    position-by-position forwards: cache rows and the last position's logits; from position 0, and behind cached rows."""
+    seq_len, kvd = shape[6], shape[0] // shape[3] * shape[4]
+    rng = np.random.default_rng(shape[1] + shape[3])
+    g = model(shape)
+    tokens = np.concatenate([[1], rng.integers(2, shape[5], size=seq_len - 1)]).astype(np.int32)
+    sizes = [n for n in (33, 65, 257, 272, 273, 289, 512, 513, 544, 545, 577, 600, 700, 1000, 1024, 1025) if n <= seq_len]
+    want = {}
+    for i, t in enumerate(tokens):
+        lg = g.forward(int(t), i, want_logits=i + 1 in sizes)
+        if i + 1 in sizes:
+            want[i + 1] = lg
+    want_kv = [x.reshape(shape[2], seq_len, kvd) for x in caches(g, shape)]
+    for n in sizes:
+        for first in (0, 7) if n in (273, 577, 1025) else (0,):
+            g.reset()
+            if first:
+                g.prefill(tokens[:first], want_logits=False)
+            got, _ = g.prefill(tokens[first:n], pos0=first)
+            assert rel_err(got, want[n].astype(np.float64)) < CLOSE, (n, first)
+            for x, y in zip(caches(g, shape), want_kv):
+                x = x.reshape(shape[2], seq_len, kvd)
+                assert np.abs(x[:, :n] - y[:, :n]).max() < CLOSE * np.abs(y[:, :n]).max(), (n, first)
+                assert not x[:, n:].any(), (n, first)
     g.close()
