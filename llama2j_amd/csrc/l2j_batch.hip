@@ -601,11 +601,12 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     if (known < 2 || b.step_grid > 0) known = 0;
     int per = std::min(known, kRowsMax / nseq);
     if (known > 0) {
+        // room for the longest common prompt a call on these buffers may have: the next one allocates nothing
         int got = 0;
-        rc = ensure_rows(c, per * nseq, 2 * nseq, &got);
+        rc = ensure_rows(c, std::min({cap, pcap + 1, kRowsMax / nseq}) * nseq, 2 * nseq, &got);
         if (rc == L2J_E_OOM) known = 0;   // (the loop takes these positions as well)
         else if (rc) return rc;
-        per = got / nseq;
+        per = std::min(per, got / nseq);
     }
     BatchState h{};
     h.pos = known > 0 && !logits_log ? known - 1 : 0;

@@ -544,3 +544,19 @@ def test_common_prompt_positions_of_a_wide_model(heads, kv_heads, n_seq, shortes
             assert rel_err(logits[pos, b], want.astype(np.float64)) < 2e-5, (b, pos)
             assert tokens[b, pos] == (prompts[b][pos] if pos < len(prompts[b]) else np.argmax(logits[pos, b])), (b, pos)
     g.close()
+
+
+def test_a_longer_common_prompt_allocates_nothing_where_the_prompts_fit():
+    """The first call whose prompts all have ids makes room for the longest common prompt its buffers take."""
+    shape = (512, 8192, 1, 8, 8, 512, 96, 1)              # (64 positions of 16 sequences: 270 MB)
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    rng = np.random.default_rng(8)
+    full = [rng.integers(2, shape[5], size=70).astype(np.int32) for _ in range(16)]
+    g.decode_greedy_batch([full[0]] + [p[:2] for p in full[1:]], 80, n_seq=16)
+    before = FullDevice(0).free_bytes()
+    for shortest in (9, 30, 70):
+        g.decode_greedy_batch([full[0]] + [p[:shortest] for p in full[1:]], 80, n_seq=16)
+        assert FullDevice(0).free_bytes() == before, shortest
+    g.close()
