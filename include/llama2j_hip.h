@@ -159,10 +159,14 @@ int l2j_decode_greedy(l2j_ctx *ctx, const int32_t *prompt, int32_t n_prompt, int
  * number relative to the largest of its group of 256 (four signed digits to the base 256), the sums over a group are exact
  * and the groups are added in fp32 with their scales and offsets as in K/MatMul.java:117-151 (the fp32 classifier runs on the
  * fp32 matrix cores); sums are formed in another order than in the single-sequence path, so logits agree to rounding, not
- * bit for bit.  The positions whose input tokens all sequences know (up to the shortest prompt) are taken at once.  The first call makes a second copy of the quantized matrices on the
+ * bit for bit.  The positions whose input tokens all n_seq rows know (up to the shortest prompt) are taken at once; a row without
+ * a prompt, as fewer than n_seq requests leave them, has its first position known only, and the prompts then go through the loop.
+ * The first call makes a second copy of the quantized matrices on the
  * device, in the order this path reads them (as large as the matrices themselves: 6.9 GB at the 7B shape), its
- * activation buffers, a KV cache of n_seq x steps rows per layer and the captured graph of a step; the context keeps
- * them until l2j_destroy, so later calls allocate and capture nothing unless they ask for another n_seq, more steps or
+ * activation buffers, a KV cache of n_seq x steps rows per layer and the captured graph of a step, the first one whose rows all have
+ * prompts also buffers for up to 1024 positions at once (0.45 GB at the 7B shape, 1.2 GB at 70B; less where the device memory does
+ * not suffice for them, none where it does not for two positions: the loop then takes them all); the context keeps
+ * them until l2j_release_batch or l2j_destroy, so later calls allocate and capture nothing unless they ask for another n_seq, more steps or
  * longer prompts (then the set is replaced).  The context's own cache is not touched.  L2J_E_OOM when the device
  * memory does not suffice (n_seq x n_layers x steps x kv_dim x 8 bytes of cache).
  * Needs dim and hidden_dim in whole groups of 256 and head_size 64, 128 or 256.
@@ -259,7 +263,8 @@ int l2j_get_config(l2j_ctx *ctx, l2j_config *cfg);
  * pass).  logits (null: not wanted): the vocab_size logits of the last position; they are also what l2j_sample
  * samples from next.  seconds (null: not wanted): device time of the steps.  The sums are formed in another order than
  * l2j_forward's, so cache rows and logits agree with its to rounding (1e-6 of the largest), not bit for bit.  Shapes as for
- * l2j_decode_greedy_batch (else L2J_E_SIZE: take l2j_forward); its buffers and its copy of the matrices are shared. */
+ * l2j_decode_greedy_batch (else L2J_E_SIZE: take l2j_forward), whose copy of the matrices and row buffers it shares (grown by a
+ * longer prompt up to 1024 positions; where the device memory does not suffice the passes are shorter). */
 int l2j_prefill(l2j_ctx *ctx, const int32_t *tokens, int32_t n, int32_t pos0, float *logits, double *seconds);
 
 /* ======================================================================================================
@@ -291,7 +296,8 @@ int l2j_sum_probe(l2j_ctx *ctx, const float *terms, int32_t n, const float *limi
 int l2j_running_sums_noalloc(l2j_ctx *ctx, const float *terms, int32_t n, float *sums);
 /* Test: l2j_decode_greedy_batch that also returns the logits of every step, (steps, n_seq, vocab_size) floats, so that
  * the batched path's arithmetic can be compared with the single-sequence path's and the CPU's step by step (they pass
- * through a device buffer of that size, allocated for the call). */
+ * through a ring of up to 32 steps on the device and one in pinned host memory, kept with the other buffers: 131 + 4 MB for 32
+ * sequences and a vocabulary of 32000; fewer steps for a shorter call or where the memory does not suffice). */
 int l2j_decode_greedy_batch_logits(l2j_ctx *ctx, const int32_t *prompts, const int32_t *n_prompt, int32_t n_seq,
                                    int32_t prompt_stride, int32_t steps, int32_t *out_tokens, float *logits);
 /* Measurement and test of the matrix-core kernel for several sequences at once (the reference has none: "parallel

@@ -439,7 +439,8 @@ class Transformer:
     def decode_greedy_batch(self, prompts, steps, n_seq=None, want_logits=False):
         """Sixteen or thirty-two greedy token loops at once (l2j_decode_greedy_batch).  prompts: up to n_seq id sequences
         (missing ones run without a prompt; n_seq defaults to 16, or 32 for more than sixteen prompts); returns (tokens of
-        shape (n_seq, steps), seconds after the first step), or with want_logits (tokens, logits of shape (steps, n_seq,
+        shape (n_seq, steps), device seconds after the first step, or from the start of the pass over the prompt positions all rows
+        know), or with want_logits (tokens, logits of shape (steps, n_seq,
         vocab_size)) through l2j_decode_greedy_batch_logits."""
         if n_seq is None:
             n_seq = 16 if len(prompts) <= 16 else 32

@@ -11,9 +11,11 @@ namespace {
 // The two shapes of k_dgemm: 256 rows of the matrix x 32 vectors per workgroup, two of which share a compute unit, and
 // 512 x 64, one per compute unit.  Microseconds per group of 256: the only workgroup of its compute unit (alone), in a round that
 // fills the slots (shared), in the rounds before the last (full); before the first and after the last group (start).  Fitted
-// to 800 launches at the products of Llama-2-7B with 32 to 1024 vectors and 1 to 16 slices (9 % root mean square; the
-// pick is 3 % slower than the best of the launches on average, 11 % at most), the full rounds to the same products inside
-// a forward pass of 1024 positions, where the clock is lower than in a short burst.
+// at the products of Llama-2-7B, the full rounds to the same products inside a forward pass of 1024 positions, where the clock is
+// lower than in a short burst.  The pick against the best of all launches, over the four products with fifteen numbers of vectors
+// from 33 to 1024, mean and largest excess: 110M shape 1.7 and 21 %, 7B 2.4 and 29, 13B 4.7 and 71, 70B widths 1.9 and 77.  (The
+// largest: 700 vectors, where the row tiles are dealt unevenly to the eight XCDs and some take a second round, which the
+// estimate does not see.)
 struct Variant { int pt, nw, per_cu; double alone, shared, full, start; };
 constexpr Variant kVariants[2] = {{1, 4, 2, 2.3, 3.8, 4.2, 4.3}, {2, 8, 1, 4.9, 7.2, 7.2, 7.7}};
 
@@ -158,7 +160,8 @@ hipError_t RowBufs::alloc(l2j_ctx *c, int rows, bool attention)
 // Blocks of 32 positions (the cache rows loaded once for 32) where pairs of blocks of 16 are an eighth more workgroups than compute
 // units: a last round of them costs more than half-filled compute units do.  7B shape, us a launch with blocks of 16 -> 32: 520
 // positions 58.6 -> 71.0 (272 pairs of blocks of 16: just past the 256 units), 560 76.4 -> 69.0 (288), 700 88.2 -> 79.5, 900 110.8 ->
-// 100.1.  Pairs of blocks unless one block per workgroup already leaves compute units idle.
+// 100.1; whole passes of 1024 positions, four layers, ms: 7B 3.81 -> 3.77, 13B 5.91 -> 6.04, 70B widths 13.15 -> 13.10.
+// Pairs of blocks unless one block per workgroup already leaves compute units idle.
 template <int HS>
 static void launch_attn(l2j_ctx *c, RowAttn t)
 {

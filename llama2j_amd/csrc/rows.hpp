@@ -9,7 +9,11 @@
 namespace l2j {
 
 constexpr int kRowsMax = 1024;   // rows of a pass
-constexpr int kTogetherFrom = 256;   // rows from which on the rows of a line of digits share an XCD (together_row): below, too few units of eight rows to keep eight XCDs evenly busy
+// Rows from which on the rows of a line of digits share an XCD (together_row): below, too few units of eight rows to keep eight XCDs evenly
+// busy.  Whole passes, ms in order -> together, 256 and 1024 rows: 110M 0.911 -> 0.895 and 1.840 -> 1.804, 7B (four layers, as the others)
+// 1.189 -> 1.179 and 3.882 -> 3.765, 13B 1.631 -> 1.617 and 6.174 -> 6.040, 70B widths 3.523 -> 3.472 and 13.29 -> 13.10; at 64 and 128
+// rows within 2 % of each other.
+constexpr int kTogetherFrom = 256;
 
 struct DgPlan {
     int variant = 0, gps = 0, slices = 0, nrow = 0, ncol = 0;
@@ -49,6 +53,8 @@ int ensure_batch_tiles(l2j_ctx *c);   // the tile-ordered copy of every matrix
 // k_pflash (the keys of 16 positions shared by the waves of a workgroup, and from kSplitKeysFrom keys on by several workgroups)
 // where k_rows_attn would have fewer than kSharedKeysBelow waves per compute unit for this many keys or more: 40 positions behind 1000
 // of Llama-2-7B 5.0 against 5.8 ms, 128 behind 1000 7.2 against 7.6, 200 from 0 on 9.2 against 9.0, 400 from 0 on 15.3 against 14.7.
+// At other shapes, ms never shared -> by this rule, 40 and 128 positions behind 1000: 110M (12 layers) 1.23 -> 0.70 and 1.33 -> 0.81, 13B
+// (four layers) 0.86 -> 0.76 and 1.14 -> 1.24, 70B widths (four layers) 1.42 -> 1.38 and 2.11 -> 2.15.
 // (kSplitKeysFrom lies below kSharedKeysFrom: it decides with option prefill_flash = 2 alone.)
 constexpr int kSharedKeysFrom = 512, kSharedKeysBelow = 2, kSplitKeysFrom = 192, kPflashMaxSplit = 4;
 inline size_t pflash_lds(int hs, int waves) { return (size_t)(32 * waves + 16 * waves * hs) * sizeof(float); }
