@@ -84,6 +84,9 @@ int fused_splits(const l2j_ctx *c)
     return std::max(1, o != kAuto ? o : c->pk_grid / c->cfg.n_heads);
 }
 
+// Words of cls_part: one for each workgroup of k_token, whose number option "grid" sets, or of k_xtoken's classifier, whose number it does not.
+int cls_slots(const l2j_ctx *c) { return std::max(c->pk_grid, c->n_cu); }
+
 // Marks the activation vectors unwritten: set 0 before a k_token that hands over by value, both sets (and the
 // per-workgroup classifier results) before a self-contained one whose vectors others have written.
 hipError_t launch_fill_unset(const l2j_ctx *c, hipStream_t s)
@@ -92,7 +95,7 @@ hipError_t launch_fill_unset(const l2j_ctx *c, hipStream_t s)
     f.p = c->acts;
     f.n = (long)((c->self_contained & 1) ? 2 * c->set_floats : c->set_floats);
     f.part = c->cls_part;
-    f.nparts = (c->self_contained & 2) ? c->pk_grid : 0;
+    f.nparts = (c->self_contained & 2) ? cls_slots(c) : 0;
     f.p2 = c->xcd_mem;
     f.n2 = c->xcd ? 2 * c->xcd_stride : 0;
     hipLaunchKernelGGL(k_fill_unset, dim3(c->n_cu), dim3(1024), 0, s, f);
@@ -570,7 +573,7 @@ int l2j::setup_forward(l2j_ctx *c)
             for (const void *k : ks) HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
         }
         int rc2;
-        if ((rc2 = dev_alloc(&c->cls_part, c->pk_grid))) return rc2;
+        if ((rc2 = dev_alloc(&c->cls_part, cls_slots(c)))) return rc2;
         if ((rc2 = dev_alloc(&c->attn_part, (uint64_t)c->cfg.n_layers * c->cfg.n_heads * c->attn_nsplit * (c->head_size + 2)))) return rc2;
         c->nbar = 5 * c->cfg.n_layers;
         if ((rc2 = dev_alloc(&c->bar_ctr, (uint64_t)c->nbar * kBarStride))) return rc2;

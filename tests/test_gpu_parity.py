@@ -259,6 +259,22 @@ def test_layers_on_one_xcd_match_oracle(orc, shape):
     np.testing.assert_array_equal(g.decode_greedy(prompt, n)[0], m.generate_greedy(prompt, n)[0])
 
 
+@pytest.mark.parametrize("grid", [1, 64, 223, 256])
+def test_layers_on_one_xcd_with_the_grid_of_the_other_kernel(orc, monkeypatch, grid):
+    # option "grid" sizes k_token; the 224 workgroups of the classifier beside the layers store and wait for a word each all the same
+    monkeypatch.setenv("L2J_ONE_XCD", "1")
+    monkeypatch.setenv("L2J_GRID", str(grid))
+    shape = (64, 96, 2, 4, 2, 900, 60, 1)   # four rows of the classifier a workgroup: every one can hold the maximum
+    m, g = make_pair(orc, shape, seed=35, realistic=True)
+    prompt = orc.synth_prompt(35, 4, shape[5])
+    want = m.generate_greedy(prompt, 60)[0]
+    assert g.forward_argmax(int(prompt[0]), 0) == int(np.argmax(g.forward(int(prompt[0]), 0)))   # (the first token too waits for all of them)
+    for _ in range(2):
+        g.reset()
+        np.testing.assert_array_equal(g.decode_greedy(prompt, 60)[0], want)
+    m.close(); g.close()
+
+
 @pytest.mark.parametrize("one_xcd", [1, 0])
 def test_norm_of_a_vector_whose_squares_overflow_is_zero(one_xcd):
     # K/RootMeanSquare.java:31-33 divides by an infinite root: the layers add nothing, and the logits are zero
