@@ -229,15 +229,22 @@ struct XStage {
 };
 
 // 1 / sqrt(sum x^2 / n + 1e-5) from the stagers' sums (K/RootMeanSquare.java:31-33): rn = 1 / n, and one step of Newton's method
-// behind the instruction's result (eight instructions in every wave instead of some forty for two divisions and a root); where the
-// sum is infinite the step's 1 - a y^2 is no number, and the maximum keeps the instruction's 0
+// behind the instruction's result (eight instructions in every wave instead of some forty for two divisions and a root, and no
+// less exact: against 64 bits 0.52 to 0.65 units of 2^-24, 1.95 at most, for the two divisions and the root 0.64 to 0.67 and 2.3);
+// where the sum is infinite the step's 1 - a y^2 is no number, and the maximum keeps the instruction's 0
 __device__ __forceinline__ float xcd_rms(const float *red, float rn)
 {
     const float a = fmaf(red[0] + red[1], rn, 1e-5f), y = __builtin_amdgcn_rsqf(a);
     return fmaf(0.5f * y, fmaxf(fmaf(-a * y, y, 1.0f), -1.0f), y);
 }
 
-__device__ __forceinline__ float exp_neg(float d) { return __builtin_amdgcn_exp2f(d * 1.44269504088896341f); }   // e^d, d <= 0
+// q / b, r = 1 / b rounded: the quotient's residual folded back in (Markstein 1990).  The same word as the division for every q and the root
+// of every head size up to 64; one that is not finite, which the residual is not either, is a NaN (and with it every score it enters or their sum).
+__device__ __forceinline__ float quotient(float q, float b, float r)
+{
+    const float y = q * r;
+    return fmaf(fmaf(-y, b, q), r, y);
+}
 
 // How the cache rows of a head are split at a length: splits, and rows of each.
 __device__ __forceinline__ int xcd_splits(int len, int most, int &chunk)
@@ -259,7 +266,7 @@ __device__ __forceinline__ void xcd_stage_layers(float *lds, int w, int wl, int 
     const int dim = a->g.dim, hid = a->g.hidden, hs = a->g.head_size, L = a->g.n_layers, nh = a->g.n_heads, nsplit = a->nsplit;
     const long so = set * a->g.set_stride, sd = a->g.sd, skv = a->g.skv, sh = a->g.sh;
     const float *x = a->g.x + so, *xb = a->g.xb + so, *hb = a->g.hb + so, *rmsw = a->g.rmsw;
-    const float rs = __fdiv_rn(1.0f, a->g.sqrt_hs);
+    const float sqrt_hs = a->g.sqrt_hs, rs = __fdiv_rn(1.0f, sqrt_hs);
     int chunk;
     const int nact = xcd_splits(pos + 1, nsplit, chunk), head = w % nh;
     const bool item = w < nh * nact;
@@ -287,7 +294,10 @@ __device__ __forceinline__ void xcd_stage_layers(float *lds, int w, int wl, int 
                 const float *p[1] = {qkv + l * qkv_step};
                 float4 q[1];
                 xwait<1>(p, q, pl);
-                if (which == 0) { q[0].x *= rs; q[0].y *= rs; q[0].z *= rs; q[0].w *= rs; }   // (the scores' division by sqrt(head_size), K/AttentionLoop.java:48)
+                if (which == 0) {   // (the scores' division by sqrt(head_size), K/AttentionLoop.java:48)
+                    q[0].x = quotient(q[0].x, sqrt_hs, rs); q[0].y = quotient(q[0].y, sqrt_hs, rs);
+                    q[0].z = quotient(q[0].z, sqrt_hs, rs); q[0].w = quotient(q[0].w, sqrt_hs, rs);
+                }
                 reinterpret_cast<float4 *>(lds + M::qkv)[16 * which + (wl & 15)] = q[0];
             }
             __syncthreads();
@@ -310,7 +320,7 @@ __device__ __forceinline__ void xcd_stage_layers(float *lds, int w, int wl, int 
                     xwait<4>(p, q, pl);
                     const bool two = s + 1 < nact;
                     const float mb = fmaxf(m, two ? fmaxf(q[0].x, q[2].x) : q[0].x);
-                    const float k = exp_neg(m - mb), k0 = exp_neg(q[0].x - mb), k1 = two ? exp_neg(q[2].x - mb) : 0.0f;
+                    const float k = s > 0 ? expf(m - mb) : 0.0f, k0 = expf(q[0].x - mb), k1 = two ? expf(q[2].x - mb) : 0.0f;
                     sum = fmaf(q[2].y, k1, fmaf(q[0].y, k0, sum * k));
                     o.x = fmaf(q[3].x, k1, fmaf(q[1].x, k0, o.x * k));
                     o.y = fmaf(q[3].y, k1, fmaf(q[1].y, k0, o.y * k));
@@ -489,14 +499,19 @@ __device__ __forceinline__ void xcd_layers(float *lds, int w, int nwork, int t, 
                     mb = fmaxf(mb, sc[u]);
                 }
                 mb = fmaxf(m, max_of_groups<16>(mb));
-                const float k = exp_neg(m - mb);
+                // The four rows' weights and the rescaling factor with one exponential: sixteen lanes hold the same scores, so lanes 0 to 3 of
+                // them take one row each, the others the maximum.
+                const int j = lane & 15;
+                const float w = expf((j == 0 ? sc[0] : j == 1 ? sc[1] : j == 2 ? sc[2] : j == 3 ? sc[3] : m) - mb);
+                const float p4[kXRowsAhead] = {dpp_f<0x150>(w), dpp_f<0x151>(w), dpp_f<0x152>(w), dpp_f<0x153>(w)};   // row_newbcast
+                const float k = readlane_f(w, 4);
                 sum *= k;
                 o *= k;
 #pragma unroll
                 for (int u = 0; u < kXRowsAhead; u++) {
                     if (tb + 4 * kXWaves * u + 4 * wave >= t1) continue;
                     const bool ok = tb + slot + 4 * kXWaves * u < t1;
-                    const float p = ok ? exp_neg(sc[u] - mb) : 0.0f;
+                    const float p = ok ? p4[u] : 0.0f;
                     sum += p;
 #pragma unroll
                     for (int e = 0; e < 4; e++) o[e] = fmaf(p, ok ? v4[u][e] : 0.0f, o[e]);   // K/AccumWeightedValue.java:48-62 (the repeated row may hold infinities)
@@ -516,17 +531,18 @@ __device__ __forceinline__ void xcd_layers(float *lds, int w, int nwork, int t, 
             if (lane == 0) { lds[M::ml + 2 * wave] = m; lds[M::ml + 2 * wave + 1] = sum; }
             __syncthreads();
             if (wave == 0) {
-                float mm[kXWaves], ll[kXWaves], oo[kXWaves], top = -3.402823466e+38f, S = 0.0f, O = 0.0f;
+                float ll[kXWaves], oo[kXWaves], top = -3.402823466e+38f, S = 0.0f, O = 0.0f;
+                const float own = lds[M::ml + 2 * min(lane, kXWaves - 1)];   // the waves' maxima, one per lane
 #pragma unroll
                 for (int i = 0; i < kXWaves; i++) {
-                    mm[i] = lds[M::ml + 2 * i];
                     ll[i] = lds[M::ml + 2 * i + 1];
                     oo[i] = lds[M::acc + 64 * i + lane];
-                    top = fmaxf(top, mm[i]);
+                    top = fmaxf(top, readlane_f(own, i));
                 }
+                const float w = expf(own - top);   // (a wave without rows: 0)
 #pragma unroll
                 for (int i = 0; i < kXWaves; i++) {
-                    const float k = exp_neg(mm[i] - top);   // (a wave without rows: 0)
+                    const float k = readlane_f(w, i);
                     S = fmaf(ll[i], k, S);
                     O = fmaf(oo[i], k, O);
                 }

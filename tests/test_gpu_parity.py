@@ -304,6 +304,47 @@ def test_an_infinite_value_stays_in_its_column(one_xcd, pos):
     g.close()
 
 
+@pytest.mark.parametrize("head", [64, 48])
+@pytest.mark.parametrize("pos", [24, 120])
+@pytest.mark.parametrize("one_xcd", [1, 0])
+def test_weights_of_far_scores_are_exact(one_xcd, pos, head):
+    # Scores of -43 to -86 that are known to the last bit beside others of 0: every key has one element, a power of two, and the token's
+    # own key and value are zero.  At 120 positions the heads' rows are in two splits, and the first has none but far ones, all of one
+    # score.  Every rescaling is by 1 or by the far weight itself, and the weights' sum is that of the ones.  So a column is off by the
+    # exponential (2^-23), the sum of its at most six rows (8 roundings), a product, a sum and the quotient: 13 * 2^-24.
+    dim = 4 * head
+    g = l2j.Transformer(l2j.Config(dim, 512, 1, 4, 4, 40, 128, 0), options={"fuse": 1, "one_xcd": one_xcd})
+    g.fill_synthetic(5, 0.02)
+    for t in (TENSOR.WK, TENSOR.WV):
+        g.upload_f32_quantize(t, np.zeros(dim * dim, dtype=np.float32))
+    g.finalize()
+    g.forward(3, pos)
+    q = g.read(BUFFER.Q).reshape(4, head)
+    k, v = np.zeros((2, pos, 4, head), dtype=np.float32)
+    far = np.arange(0, pos, 2) if pos == 24 else np.arange(0, 61)   # the others keep a zero key
+    want = np.zeros((4, head))
+    root = np.float32(np.sqrt(np.float32(head)))
+    for h in range(4):
+        big = np.argsort(-np.abs(q[h]))
+        weight, value = np.ones(pos + 1), np.zeros((pos + 1, head))
+        for i, t in enumerate(far):
+            e = big[i if pos == 24 else 0]
+            k[t, h, e] = -np.sign(q[h, e]) * np.float32(2.0) ** np.floor(np.log2(86.0 * root / abs(q[h, e])))
+            score = (q[h, e] * k[t, h, e]) / root
+            assert score.dtype == np.float32 and -86.0 <= score < -42.9
+            weight[t] = np.exp(np.float64(score))
+            v[t, h, i % 12] = value[t, i % 12] = np.float32(2.0) ** 100
+        want[h] = weight @ value / weight.sum()
+    g.write_kv(0, 0, k.reshape(pos, dim), v.reshape(pos, dim))
+    g.forward(3, pos)
+    got = g.read(BUFFER.XB).reshape(4, head).astype(np.float64)
+    assert not got[:, 12:].any() and want[:, :12].min() > 0
+    worst = float(np.abs(got[:, :12] / want[:, :12] - 1).max())
+    say("far weights: worst relative error %.2e" % worst)
+    assert worst <= 13 * 2.0 ** -24
+    g.close()
+
+
 def test_kernel_timing_entry_point(orc, launch_mode):
     # every kernel class launches and reports a time, deep enough in the context that attention is split;
     # the measurement leaves the context usable (same tokens before and after)
