@@ -562,9 +562,11 @@ __global__ void __launch_bounds__(16384 / LPR) k_battn(const BAttn a)
     float m = -3.0e38f, l = 0.0f;
     float4 acc = zero;
     if (wave == 0) {   // this position's row: the first slot
-        m = readlane_f(score(kp), 0);
-        l = lane < LPR ? 1.0f : 0.0f;
-        acc.x = lane < LPR ? vp.x : 0.0f; acc.y = lane < LPR ? vp.y : 0.0f; acc.z = lane < LPR ? vp.z : 0.0f; acc.w = lane < LPR ? vp.w : 0.0f;
+        const float s = readlane_f(score(kp), 0);
+        m = fmaxf(s, -3.0e38f);   // (as with the rows below: a maximum of -inf would make the rescaling of later rows NaN)
+        const float p = s < -3.0e38f ? 0.0f : (s - s) + 1.0f;   // (1, and NaN where the score is +inf or NaN)
+        l = lane < LPR ? p : 0.0f;
+        acc.x = lane < LPR ? p * vp.x : 0.0f; acc.y = lane < LPR ? p * vp.y : 0.0f; acc.z = lane < LPR ? p * vp.z : 0.0f; acc.w = lane < LPR ? p * vp.w : 0.0f;
     }
     for (int tb = 0; tb < pos; tb += R * NSLOT) {
         if (tb) rows(tb + slot);

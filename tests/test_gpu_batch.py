@@ -149,6 +149,37 @@ def test_products_of_one_to_four_tiles_per_workgroup(orc, hidden, n_seq):
     test_every_sequence_gets_what_it_gets_alone(orc, (256, hidden, 1, 4, 4, 512, 40, 1), n_seq)
 
 
+@pytest.mark.parametrize("heads", [8, 4, 2])
+def test_scores_of_minus_infinity_weigh_nothing(heads):
+    """A token whose keys are huge in one element of head 0 and whose queries are negative there: it scores -inf against itself and its
+    like, and what is left is the softmax over the other rows, also where the first rows that a wave takes are all of its kind."""
+    shape, head, huge, other = (512, 1024, 1, heads, heads, 64, 80, 0), 512 // heads, 3, 4
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    emb = np.random.default_rng(heads).standard_normal((64, 512), dtype=np.float32)
+    emb[:, 0] = 0
+    emb[[1, huge], 0] = 10.0   # (token 1 comes first)
+    g.upload_f32(TENSOR.TOK_EMB, emb)
+    for t in (TENSOR.RMS_ATT, TENSOR.RMS_FFN, TENSOR.RMS_FINAL):
+        g.upload_f32_quantize(t, np.linspace(0.9, 1.1, 512, dtype=np.float32))
+    for t, w in ((TENSOR.WK, 1e28), (TENSOR.WQ, -1e12)):
+        m = 0.02 * np.random.default_rng(int(t)).standard_normal((512, 512), dtype=np.float32)
+        m[head - 2] = 0   # of the pair that positions turn least
+        m[head - 2, 0] = w
+        g.upload_f32_quantize(t, m.reshape(-1))
+    g.finalize()
+    prompt = np.array([huge] * 51 + [other] * 19 + [huge], dtype=np.int32)
+    pos = len(prompt)
+    _, _, logits = g.decode_sample_batch([prompt] + [prompt[-3:]] * 15, pos + 1, 0.0, 0.0, np.arange(1, 17), want_logits=True)
+    for i, t in enumerate([1] + list(prompt)):
+        want = g.forward(int(t), i)
+        if i == 5:
+            assert np.isnan(want).all()   # every row scores -inf
+    assert np.isfinite(want).all()
+    assert rel_err(logits[pos, 0], want) < 1e-4
+    g.close()
+
+
 @pytest.mark.parametrize("shape,n_seq,steps", [
     ((4096, 11008, 3, 32, 32, 32000, 48, 0), 32, 40),      # the widths of Llama-2-7B: rows of 16 and 43 groups
     ((4096, 11008, 3, 32, 32, 32000, 48, 0), 16, 40),
