@@ -91,8 +91,9 @@ int l2j_device_count(void);
  * "token_special", "graph" (0: launch kernel by kernel instead of replaying captured hipGraphs; a token of one launch has none), "graph_tokens" (tokens per
  * replay in the decode loops), "one_xcd" (small models: 1 or -1, the default: the layers of a token on the compute units of one
  * XCD; 0: on all).  At any time: "sampler_scan", "sampler_exp_wgs", "fallback" (1: when a bounded wait of the
- * whole-token kernel runs out, because something else holds compute units of the GPU, the context switches to one launch
- * per phase for good and repeats the call; 0: the call returns L2J_E_HIP), "batch_fuse" (l2j_decode_greedy_batch: 1 runs the
+ * whole-token kernel runs out, because something else holds compute units of the GPU, the context gives it up for good and repeats
+ * the call: a small model's goes on with the kernel on all compute units where that suits its size, else with one launch per
+ * phase; 0: the call returns L2J_E_HIP), "batch_fuse" (l2j_decode_greedy_batch: 1 runs the
  * layers of a step in one resident kernel with grid barriers instead of eight launches per layer; the same results,
  * slower as measured, 0 by default; a bounded wait of that kernel that runs out is L2J_E_HIP), "sampler_wide" (1, the default: a
  * sampling step of a vocabulary of at most 36864 is one launch of a workgroup per 256 probabilities with grid barriers; a

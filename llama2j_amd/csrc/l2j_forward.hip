@@ -137,6 +137,17 @@ bool xcd_fits(const l2j_ctx *c)
     return 2 * per((dim + 2 * kvd) / 2) <= rows_d && per(hid) <= rows_d && per(dim) <= std::min(rows_d, rows_h);
 }
 
+// A context runs k_token where it does not run k_xtoken.  One launch per token pays off when a hand-over inside the kernel costs less
+// than a kernel boundary of the replayed graph: measured whole-token / one launch per phase, 7B shape (208 MB a layer) 1.44 / 1.96 ms
+// per token, 110M shape (7 MB) 0.241 / 0.278 ms, 15M shape (1 MB) 0.123 / 0.134 ms.  Below half a million weights a layer (test
+// models) the phases stay separate launches.
+bool wants_token_kernel(const l2j_ctx *c)
+{
+    const l2j_config &g = c->cfg;
+    const uint64_t layer_floats = 2ull * g.dim * g.dim + 2ull * g.dim * c->kv_dim + 3ull * g.dim * g.hidden_dim;
+    return c->opt[OPT_FUSE] != kAuto ? c->opt[OPT_FUSE] != 0 : layer_floats >= (1ull << 19);
+}
+
 hipError_t launch_xtoken(const l2j_ctx *c, hipStream_t s, hipEvent_t e0, hipEvent_t e1)
 {
     XcdArgs a{};
@@ -325,8 +336,9 @@ int capture_graphs(l2j_ctx *c)
 
 // After hand_out and a synchronize: a workgroup whose bounded wait ran out has set the flag.  The whole-token kernel needs all its
 // workgroups resident at once; when something else holds compute units (another process on the GPU) its waits run
-// out.  With the "fallback" option the context then gives the whole-token kernel up for good: one launch per phase
-// needs no residency, and the caller repeats what failed (kRepeatToken).
+// out.  With the "fallback" option the context then gives the kernel up for good and the caller repeats what failed (kRepeatToken):
+// k_xtoken for k_token, whose workgroups may run anywhere, where the context would run that without k_xtoken; else for one launch
+// per phase, which needs no residency.
 int l2j::check_barrier_error(l2j_ctx *c)
 {
     if (!c->fused || *c->h_fault == 0) return L2J_OK;
@@ -337,18 +349,16 @@ int l2j::check_barrier_error(l2j_ctx *c)
     HIPCHK(hipMemset(c->counters, 0, ((size_t)c->cfg.n_layers * c->cfg.n_heads + 1) * sizeof(unsigned)));
     c->acts_dirty = true;
     if (c->opt[OPT_FALLBACK] != 0) {
-        if (c->xcd) {   // (k_token next: its workgroups may run anywhere)
-            c->xcd = false;
-            const int rc = capture_graphs(c);
-            return rc ? rc : kRepeatToken;
+        const bool token_next = c->xcd && wants_token_kernel(c);
+        c->xcd = false;
+        if (!token_next) {
+            c->fused = false;
+            c->by_value = false;
+            c->self_contained = 0;
+            c->opt[OPT_FUSE] = 0;
         }
-        c->fused = false;
-        c->by_value = false;
-        c->self_contained = 0;
-        c->opt[OPT_FUSE] = 0;
-        int rc = capture_graphs(c);
-        if (rc) return rc;
-        return kRepeatToken;
+        const int rc = capture_graphs(c);
+        return rc ? rc : kRepeatToken;
     }
     return fail(L2J_E_HIP, "a bounded wait of the whole-token kernel ran out (barrier or input vector; its workgroups were not all resident)");
 }
@@ -581,36 +591,32 @@ int l2j::setup_forward(l2j_ctx *c)
         HIPCHK(hipMemset(c->bar_ctr, 0, (size_t)c->nbar * kBarStride * sizeof(unsigned)));
         HIPCHK(hipMemset(c->fault, 0, sizeof(int)));
         *c->h_fault = 0;
-        // k_token needs its whole grid resident at once (grid barriers): at most what the occupancy allows.
-        // One launch per token pays off when a hand-over inside the kernel costs less than a kernel boundary of the
-        // replayed graph: measured whole-token / one launch per phase, 7B shape (208 MB a layer) 1.44 / 1.96 ms per token,
-        // 110M shape (7 MB) 0.241 / 0.278 ms, 15M shape (1 MB) 0.123 / 0.134 ms.  Below half a million weights a layer
-        // (test models) the phases stay separate launches.
-        const uint64_t layer_floats = 2ull * c->cfg.dim * c->cfg.dim + 2ull * c->cfg.dim * c->kv_dim + 3ull * c->cfg.dim * c->cfg.hidden_dim;
-        // The layers on one XCD (k_xtoken) where the shape is small enough, unless an option asks for a form of k_token.
-        bool one_xcd = c->opt[OPT_ONE_XCD] != 0 && xcd_fits(c);
+        // The layers on one XCD (k_xtoken) where the shape is small enough, unless an option asks for a form of k_token; one that rules
+        // k_xtoken out leaves the context what it would be without it.
+        c->layers_per_launch = std::max(1, std::min(c->cfg.n_layers, c->opt[OPT_LAYERS_PER_LAUNCH] != kAuto ? c->opt[OPT_LAYERS_PER_LAUNCH] : c->cfg.n_layers));
+        const bool may_by_value = c->layers_per_launch == c->cfg.n_layers && c->opt[OPT_BY_VALUE] != 0 && nmax <= 4 * kPollWords * c->pk_threads;
+        bool one_xcd = c->opt[OPT_ONE_XCD] != 0 && may_by_value && (c->opt[OPT_SELF_CONTAINED] & 3) == 3 && xcd_fits(c);
         for (int i : {OPT_THREADS, OPT_GRID, OPT_FUSED_ATTN_ROWS, OPT_FUSED_ATTN_SPLITS, OPT_TOKEN_SPECIAL, OPT_FAST_STEPS})
             one_xcd = one_xcd && (c->opt[OPT_ONE_XCD] == 1 || c->opt[i] == kOptions[i].dflt);
-        c->fused = (c->opt[OPT_FUSE] != kAuto ? c->opt[OPT_FUSE] : one_xcd || layer_floats >= (1ull << 19) ? 1 : 0) != 0;
-        c->layers_per_launch = std::max(1, std::min(c->cfg.n_layers, c->opt[OPT_LAYERS_PER_LAUNCH] != kAuto ? c->opt[OPT_LAYERS_PER_LAUNCH] : c->cfg.n_layers));
-        if (c->fused) {
+        if (one_xcd) {
+            int per_cu = 0;
+            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_xtoken<XSmall>), kXThreads, 0));
+            one_xcd = per_cu >= 1;
+        }
+        c->fused = wants_token_kernel(c) || (one_xcd && c->opt[OPT_FUSE] == kAuto);
+        if (c->fused) {   // (k_token needs its whole grid resident at once: at most what the occupancy allows)
             const void *kl = with_token_kernel(c, [](auto kernel) { return reinterpret_cast<const void *>(kernel); });
             int per_cu = 0;
             HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kl, c->pk_threads, layer_smem(c)));
             if (per_cu < 1 || c->pk_grid > per_cu * c->n_cu) c->fused = false;
         }
-        c->by_value = c->fused && c->layers_per_launch == c->cfg.n_layers && c->opt[OPT_BY_VALUE] != 0 &&
-                      std::max(c->cfg.dim, c->cfg.hidden_dim) <= 4 * kPollWords * c->pk_threads;
+        c->by_value = c->fused && may_by_value;
         c->self_contained = c->by_value ? c->opt[OPT_SELF_CONTAINED] & 3 : 0;
-        c->xcd = c->by_value && c->self_contained == 3 && one_xcd;
+        c->xcd = c->fused && one_xcd;
         if (c->xcd) {
             c->xcd_splits = std::max(1, std::min(kXMaxSplits, 32 / c->cfg.n_heads));
             c->xcd_stride = xcd_part_floats(c->cfg.n_layers, c->cfg.n_heads, c->xcd_splits, c->head_size) + kXcds * (long)c->sd;
             if ((rc2 = dev_alloc(&c->xcd_mem, 2 * (uint64_t)c->xcd_stride))) return rc2;
-            const void *k = reinterpret_cast<const void *>(k_xtoken<XSmall>);
-            int per_cu = 0;
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kXThreads, 0));
-            if (per_cu < 1) c->xcd = false;
         }
         c->acts_dirty = true;  // marked unwritten ahead of the first token
         build_geom(c);
@@ -643,7 +649,7 @@ int l2j_forward(l2j_ctx *c, int32_t token, int32_t pos, float *logits)
         std::lock_guard<std::mutex> forward_lock(g_forward_mu);
         int rc = check_forward_args(c, token, pos);
         if (rc) return rc;
-        do {  // (a second time, phase by phase, when the whole-token kernel's waits ran out)
+        do {  // (again, another way, when the whole-token kernel's waits ran out)
             if ((rc = set_state(c, token, pos, 0))) return rc;
             HIPCHK(launch_one_token(c));
             HIPCHK(hand_out(c, logits != nullptr, 0, 0, 0));
@@ -759,7 +765,7 @@ int l2j_time_kernel(l2j_ctx *c, int kclass, int32_t pos, int32_t rounds, double 
             HIPCHK(hand_out(c, false, 0, 0, 0));
             HIPCHK(hipStreamSynchronize(c->stream));
             if ((rc = check_barrier_error(c)))
-                return rc == kRepeatToken ? fail(L2J_E_HIP, "a bounded wait of the whole-token kernel ran out; the context now launches phase by phase") : rc;
+                return rc == kRepeatToken ? fail(L2J_E_HIP, "a bounded wait of the whole-token kernel ran out; the context now runs its tokens another way") : rc;
             double total = 0.0;
             for (int r = 0; r < rounds; r++) {
                 float ms = 0.f;

@@ -312,7 +312,7 @@ inline uint64_t quant_bytes_of(uint64_t weights) { return (weights / kGroup) * k
 
 // ---- l2j_forward.hip
 extern std::mutex g_forward_mu;   // the whole-token kernel needs every compute unit: forwards of all contexts take turns
-constexpr int kRepeatToken = 1;   // check_barrier_error: the context now launches phase by phase; run the token(s) again
+constexpr int kRepeatToken = 1;   // check_barrier_error: the context now runs its tokens another way; run the token(s) again
 int setup_forward(l2j_ctx *c);    // launch shapes, kernel attributes, scratch of the phases, graph capture (end of l2j_finalize)
 void release_forward(l2j_ctx *c); // what setup_forward allocated
 hipError_t launch_one_token(l2j_ctx *c);

@@ -494,6 +494,26 @@ def test_waits_that_run_out_fall_back_to_one_launch_per_phase(orc, monkeypatch):
         m.close(); g.close()
 
 
+@pytest.mark.parametrize("options", [{}, {"by_value": 0}, {"self_contained": 2}, {"layers_per_launch": 1}, {"one_xcd": 0}])
+def test_a_small_model_that_cannot_run_on_one_xcd_is_what_it_is_without(orc, options):
+    # layers of less than half a million weights: the one-XCD kernel where nothing rules it out, else one launch per phase
+    shape = (64, 96, 2, 4, 2, 40, 32, 1)
+    g = l2j.Transformer(l2j.Config(*shape), options=options)
+    g.fill_synthetic(52, 0.02)
+    g.finalize()
+    if options:
+        with pytest.raises(l2j.L2JError) as e:
+            g.time_kernel(l2j.KERNEL.TOKEN, 5, rounds=1)
+        assert e.value.code == -3
+    else:
+        assert g.time_kernel(l2j.KERNEL.TOKEN, 5, rounds=1)[0] > 0
+    m = orc.Model(dim=64, hidden_dim=96, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=40, seq_len=32, shared_weights=1)
+    m.fill_synth(52, 0.02)
+    prompt = orc.synth_prompt(52, 3, shape[5])
+    np.testing.assert_array_equal(g.decode_greedy(prompt, 24)[0], m.generate_greedy(prompt, 24)[0])
+    m.close(); g.close()
+
+
 def test_two_contexts_decode_from_two_threads(orc, launch_mode):
     # forwards of different contexts take turns on the device: concurrent decodes give the sequential answers
     import threading
