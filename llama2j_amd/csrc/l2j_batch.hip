@@ -406,7 +406,7 @@ int ensure_batch(l2j_ctx *c, int nseq, int steps, int pstride)
     }
     if (e == hipSuccess && b->step_grid > 0) {
         const BStep a = bstep_args(c, *b, steps, nseq);
-        e = hipMemcpy(b->step_args, &a, sizeof(a), hipMemcpyHostToDevice);
+        e = copy_now(c, b->step_args, &a, sizeof(a), hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipEventCreate(&b->e0);
     if (e == hipSuccess) e = hipEventCreate(&b->e1);
@@ -684,7 +684,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     }
     if (seeds) {   // the reference's exceptions, as in l2j_sample
         SamplerState h[kMaxBatch] = {};
-        if ((e = hipMemcpy(h, b.samplers.ss, (size_t)nseq * sizeof(SamplerState), hipMemcpyDeviceToHost)) != hipSuccess) return hip_rc(e, "sampler flags");
+        if ((e = copy_now(c, h, b.samplers.ss, (size_t)nseq * sizeof(SamplerState), hipMemcpyDeviceToHost)) != hipSuccess) return hip_rc(e, "sampler flags");
         int st = 0;
         for (int s = 0; s < nseq; s++) st |= h[s].nan;
         if (st & 1) return fail(L2J_E_ARG, "sampler: NaN among the logits (J/Sampler.java:88-90)");
@@ -692,9 +692,9 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
     }
     if (b.step_grid > 0) {
         int fault = 0;
-        if ((e = hipMemcpy(&fault, b.fault, sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess) return hip_rc(e, "fault flag");
+        if ((e = copy_now(c, &fault, b.fault, sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess) return hip_rc(e, "fault flag");
         if (fault) {
-            (void)hipMemset(b.fault, 0, sizeof(int));
+            (void)hipMemsetAsync(b.fault, 0, sizeof(int), c->stream);
             return fail(L2J_E_HIP, "batched decode: a bounded wait at a grid barrier ran out (is another process using the GPU?); "
                                    "option batch_fuse = 0 runs the same step without grid barriers");
         }

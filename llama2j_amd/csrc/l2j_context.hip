@@ -354,7 +354,7 @@ int l2j_upload_f32(l2j_ctx *c, int tensor, const float *data, uint64_t nfloats)
         if (c->finalized) return fail(L2J_E_STATE, "upload after l2j_finalize");
         HIPCHK(hipSetDevice(c->cfg.device));
         if (tensor == L2J_WCLS && c->cfg.shared_weights) return L2J_OK;  // J/TransformerWeights.java:122
-        HIPCHK(hipMemcpy(tensor == L2J_TOK_EMB ? c->emb : c->wcls, data, nfloats * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(copy_now(c, tensor == L2J_TOK_EMB ? c->emb : c->wcls, data, nfloats * sizeof(float), hipMemcpyHostToDevice));
         (tensor == L2J_TOK_EMB ? c->emb_loaded : c->wcls_loaded) = true;
         return L2J_OK;
     }());
@@ -420,8 +420,7 @@ int l2j_read_quant(l2j_ctx *c, int tensor, uint64_t group0, uint64_t ngroups, ui
             hipLaunchKernelGGL(k_pack_groups, dim3((unsigned)std::min<uint64_t>(ng, 1u << 20)), dim3(64), 0, c->stream, stage, (long)ng,
                                t.codes + (group0 + g) * kGroup, t.mm + group0 + g);
             hipError_t e = hipGetLastError();
-            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-            if (e == hipSuccess) e = hipMemcpy(out + g * kGroupBytes, stage, ng * kGroupBytes, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = copy_now(c, out + g * kGroupBytes, stage, ng * kGroupBytes, hipMemcpyDeviceToHost);
             if (e != hipSuccess) rc = fail(L2J_E_HIP, std::string("read_quant: ") + hipGetErrorString(e));
         }
         (void)hipFree(stage);
@@ -485,14 +484,14 @@ int l2j_finalize(l2j_ctx *c)
                 rope[(size_t)pos * half + k] = make_float2((float)std::cos((double)val), (float)std::sin((double)val));
             }
         }
-        HIPCHK(hipMemcpy(c->rope, rope.data(), rope.size() * sizeof(float2), hipMemcpyHostToDevice));
+        HIPCHK(copy_now(c, c->rope, rope.data(), rope.size() * sizeof(float2), hipMemcpyHostToDevice));
         // sigmoid table (K/Silu.java:47-57)
         std::vector<float> tab(kSiluTable);
         for (int i = 0; i < kSiluTable; i++) {
             const double v = ((double)i / (double)kSiluTable) * 10.0 - 5.0;
             tab[i] = (float)(1.0 / (1.0 + std::exp(-v)));
         }
-        HIPCHK(hipMemcpy(c->silu, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(copy_now(c, c->silu, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice));
 
         // rmsnorm weights dequantized once with the reference's expression
         {
@@ -569,10 +568,8 @@ int l2j_read(l2j_ctx *c, int which, int layer, uint64_t off, float *dst, uint64_
             // the vectors of the last token: set 0, or with a self-contained token kernel the set it picked by the epoch
             uint64_t so = 0;
             if ((c->self_contained & 1) && !c->acts_dirty) {
-                int epoch = 0;
-                HIPCHK(hipStreamSynchronize(c->stream));
-                HIPCHK(hipMemcpy(&epoch, &c->st->epoch, sizeof(int), hipMemcpyDeviceToHost));
-                so = ((epoch - 1) & 1) ? c->set_floats : 0;
+                HIPCHK(copy_now(c, &c->h_st->epoch, &c->st->epoch, sizeof(int), hipMemcpyDeviceToHost));
+                so = ((c->h_st->epoch - 1) & 1) ? c->set_floats : 0;
             }
             switch (which) {
             case L2J_B_X: src = c->x + so + 2ull * g.n_layers * c->sd; len = g.dim; break;  // the last layer's vectors
@@ -588,9 +585,7 @@ int l2j_read(l2j_ctx *c, int which, int layer, uint64_t off, float *dst, uint64_
             src = c->taps[which] + (uint64_t)layer * len;
         }
         if (off + n > len) return fail(L2J_E_SIZE, "read past the end of the buffer");
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(dst, src + off, n * sizeof(float), hipMemcpyDeviceToHost));
-        return L2J_OK;
+        return read_floats(c, dst, src + off, n);
     }());
 }
 
@@ -603,9 +598,8 @@ int l2j_write_kv(l2j_ctx *c, int layer, int32_t pos0, int32_t npos, const float 
         if (pos0 < 0 || npos < 0 || (int64_t)pos0 + npos > c->cfg.seq_len) return fail(L2J_E_ARG, "positions out of range");
         HIPCHK(hipSetDevice(c->cfg.device));
         const uint64_t o = ((uint64_t)layer * c->cfg.seq_len + pos0) * c->kv_dim, n = (uint64_t)npos * c->kv_dim;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipMemcpy(c->kcache + o, k, n * sizeof(float), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(c->vcache + o, v, n * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(copy_now(c, c->kcache + o, k, n * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(copy_now(c, c->vcache + o, v, n * sizeof(float), hipMemcpyHostToDevice));
         return L2J_OK;
     }());
 }

@@ -344,9 +344,9 @@ int l2j::check_barrier_error(l2j_ctx *c)
     if (!c->fused || *c->h_fault == 0) return L2J_OK;
     HIPCHK(hipStreamSynchronize(c->stream));  // (tokens enqueued ahead fall through their waits as well)
     *c->h_fault = 0;
-    HIPCHK(hipMemcpy(c->fault, c->h_fault, sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(c->bar_ctr, 0, (size_t)c->nbar * kBarStride * sizeof(unsigned)));  // leave the context usable
-    HIPCHK(hipMemset(c->counters, 0, ((size_t)c->cfg.n_layers * c->cfg.n_heads + 1) * sizeof(unsigned)));
+    HIPCHK(copy_now(c, c->fault, c->h_fault, sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(hipMemsetAsync(c->bar_ctr, 0, (size_t)c->nbar * kBarStride * sizeof(unsigned), c->stream));  // leave the context usable
+    HIPCHK(hipMemsetAsync(c->counters, 0, ((size_t)c->cfg.n_layers * c->cfg.n_heads + 1) * sizeof(unsigned), c->stream));
     c->acts_dirty = true;
     if (c->opt[OPT_FALLBACK] != 0) {
         const bool token_next = c->xcd && wants_token_kernel(c);
@@ -372,6 +372,24 @@ int l2j::set_state(l2j_ctx *c, int token, int pos, int n_prompt)
     c->h_st->pos = pos;   // (l2j_forward_taps: which cache rows to copy)
     hipLaunchKernelGGL(k_set_state, dim3(1), dim3(64), 0, c->stream, StateArgs{c->st, token, pos, n_prompt});
     HIPCHK(hipGetLastError());
+    return L2J_OK;
+}
+
+// `n` floats of device memory to the host.  Up to as many as there are logits by a kernel into the pinned memory, as a call's results
+// go: behind the kernels of a decode loop a copy on the stream of 128 KB takes 70 us longer than one on the null stream did.
+int l2j::read_floats(l2j_ctx *c, float *dst, const float *src, uint64_t n)
+{
+    if (!c->finalized || n == 0 || n > (uint64_t)c->cfg.vocab_size || reinterpret_cast<uintptr_t>(src) % 16) {
+        HIPCHK(copy_now(c, dst, src, n * sizeof(float), hipMemcpyDeviceToHost));
+        return L2J_OK;
+    }
+    HandOut a{};
+    a.logits = src; a.h_logits = c->h_logits; a.nlogits = (int)n;
+    a.fault = c->fault; a.h_fault = c->h_fault;
+    hipLaunchKernelGGL(k_hand_out, dim3((unsigned)std::max<uint64_t>(1, ((n >> 2) + 255) / 256)), dim3(256), 0, c->stream, a);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));
+    memcpy(dst, c->h_logits, n * sizeof(float));
     return L2J_OK;
 }
 
@@ -588,8 +606,8 @@ int l2j::setup_forward(l2j_ctx *c)
         c->nbar = 5 * c->cfg.n_layers;
         if ((rc2 = dev_alloc(&c->bar_ctr, (uint64_t)c->nbar * kBarStride))) return rc2;
         if ((rc2 = dev_alloc(&c->fault, 1))) return rc2;
-        HIPCHK(hipMemset(c->bar_ctr, 0, (size_t)c->nbar * kBarStride * sizeof(unsigned)));
-        HIPCHK(hipMemset(c->fault, 0, sizeof(int)));
+        HIPCHK(hipMemsetAsync(c->bar_ctr, 0, (size_t)c->nbar * kBarStride * sizeof(unsigned), c->stream));
+        HIPCHK(hipMemsetAsync(c->fault, 0, sizeof(int), c->stream));
         *c->h_fault = 0;
         // The layers on one XCD (k_xtoken) where the shape is small enough, unless an option asks for a form of k_token; one that rules
         // k_xtoken out leaves the context what it would be without it.

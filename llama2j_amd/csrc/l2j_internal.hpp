@@ -308,6 +308,14 @@ int dev_alloc(T **p, uint64_t count)
     return L2J_OK;
 }
 
+// A copy that is done when it returns, over the context's stream (as all fills go): the null stream is refused, and breaks the capture,
+// while any thread of the process captures (another context's l2j_finalize).
+inline hipError_t copy_now(l2j_ctx *c, void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, c->stream), done = hipStreamSynchronize(c->stream);
+    return e != hipSuccess ? e : done;
+}
+
 inline uint64_t quant_bytes_of(uint64_t weights) { return (weights / kGroup) * kGroupBytes + (weights % kGroup ? kGroupBytes : 0); }
 
 // ---- l2j_forward.hip
@@ -318,6 +326,7 @@ void release_forward(l2j_ctx *c); // what setup_forward allocated
 hipError_t launch_one_token(l2j_ctx *c);
 int check_barrier_error(l2j_ctx *c);
 int set_state(l2j_ctx *c, int token, int pos, int n_prompt);
+int read_floats(l2j_ctx *c, float *dst, const float *src, uint64_t n);
 
 // ---- l2j_sampler.hip
 int resolve_scratch(int device);

@@ -108,7 +108,7 @@ int alloc_sampler(l2j_ctx *c)
     HIPCHK(hipHostMalloc((void **)&c->h_ss, sizeof(SamplerState), hipHostMallocDefault));
     if (n <= kSampleMaxVocab) {
         if ((rc = dev_alloc(&c->wide_mem, kWideBytes))) return rc;
-        HIPCHK(hipMemset(c->wide_mem, 0, kWideBytes));
+        HIPCHK(hipMemsetAsync(c->wide_mem, 0, kWideBytes, c->stream));
         HIPCHK(hipFuncSetAttribute((const void *)k_sample_wide, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_lds_bytes(n)));
         HIPCHK(hipFuncSetAttribute((const void *)k_sum_probe, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(WideWalk)));
     }
@@ -310,9 +310,9 @@ int l2j::check_sampler_status(l2j_ctx *c)
     const int st = c->h_ss->nan;
     if (!st) return L2J_OK;
     c->h_ss->nan = 0;
-    HIPCHK(hipMemcpy(&c->ss->nan, &c->h_ss->nan, sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(copy_now(c, &c->ss->nan, &c->h_ss->nan, sizeof(int), hipMemcpyHostToDevice));
     if (st & 4) {   // (the counters of the launch are not where the next one expects them)
-        if (c->wide_mem) HIPCHK(hipMemset(c->wide_mem, 0, sizeof(WideSync)));
+        if (c->wide_mem) HIPCHK(hipMemsetAsync(c->wide_mem, 0, sizeof(WideSync), c->stream));
         c->opt[OPT_SAMPLER_WIDE] = 0;   // (something else holds compute units: from here on one launch per stage, which waits for nobody)
         return fail(L2J_E_HIP, "sampler: a workgroup waited too long for the others (k_sample_wide needs a compute unit per 256 "
                                "probabilities); the step was not completed, the context takes one launch per stage from now on: "

@@ -721,6 +721,79 @@ def test_uploads_run_while_another_thread_captures(orc):
     g.close()
 
 
+def test_reads_of_parts_are_parts_of_the_whole():
+    # through the pinned memory of 101 logits at offsets of whole 16-byte words, by a copy at others and beyond that length
+    g = l2j.Transformer(l2j.Config(64, 176, 2, 4, 4, 101, 8, 0))
+    assert g.read(BUFFER.KCACHE, layer=1).size == 8 * 64   # (before l2j_finalize too)
+    g.fill_synthetic(3, 0.02)
+    g.finalize()
+    g.forward(3, 0)
+    g.forward(4, 1)
+    for which, layer, whole in ((BUFFER.LOGITS, -1, 101), (BUFFER.X, -1, 64), (BUFFER.HB, -1, 176), (BUFFER.KCACHE, 1, 512)):
+        want = np.concatenate([g.read(which, layer=layer, off=i, n=1) for i in range(whole)])
+        assert want.any()
+        for off in (0, 1, 4, 28, 36):
+            for n in (0, 1, 3, 4, whole - off):
+                np.testing.assert_array_equal(g.read(which, layer=layer, off=off, n=n), want[off:off + n])
+    np.testing.assert_array_equal(g.read(BUFFER.LOGITS), g.forward(4, 1))
+    g.close()
+
+
+@pytest.mark.parametrize("call", ["create", "upload_f32", "read_quant", "finalize", "finalize_phases", "forward", "read", "write_kv", "decode_greedy",
+                                  "decode_sample", "sample_separately", "prefill", "batch", "batch_sampled", "fallback", "close"])
+def test_calls_run_while_another_thread_captures(call, monkeypatch):
+    # what one context is asked for neither fails beside l2j_finalize of another, which captures, nor breaks its capture
+    import threading
+    hip = l2j.lib()
+    shape = (512, 1024, 1, 8, 8, 512, 40, 0)   # (head 64: a shape of the passes over many positions and of batches too)
+    ops = {"fuse": 0} if call == "finalize_phases" else {"barrier_spins": 0} if call == "fallback" else {}
+    g = l2j.Transformer(l2j.Config(*shape), options=ops)
+    g.fill_synthetic(3, 0.02)
+    if not call.startswith("finalize") and not call.startswith("upload"):
+        g.finalize()
+    x = np.ones((512, 512), dtype=np.float32)
+    ids, got, errs = [np.arange(2, 8, dtype=np.int32)] * 16, [], []
+    kv = np.ones((3, 512), dtype=np.float32)
+    calls = {
+        "create": lambda: l2j.Transformer(l2j.Config(*shape)).close(),
+        "upload_f32": lambda: g.upload_f32(TENSOR.TOK_EMB, x),
+        "read_quant": lambda: g.read_quant(TENSOR.WQ, 0, 8),
+        "finalize": lambda: g.finalize(),
+        "finalize_phases": lambda: g.finalize(),
+        "forward": lambda: g.forward(3, 0),
+        "read": lambda: g.read(BUFFER.X),
+        "write_kv": lambda: g.write_kv(0, 0, kv, kv),
+        "decode_greedy": lambda: g.decode_greedy(ids[0], 20),
+        "decode_sample": lambda: g.decode_sample(ids[0], 20, 0.9, 0.9, 5),
+        "sample_separately": lambda: (g.sampler_seed(3), g.forward(3, 0), g.sample(0.9, 0.9)),
+        "prefill": lambda: g.prefill(ids[0]),
+        "batch": lambda: g.decode_greedy_batch(ids, 12),
+        "batch_sampled": lambda: g.decode_sample_batch(ids, 12, 0.9, 0.9, np.arange(1, 17)),
+        "fallback": lambda: g.forward(3, 0),
+        "close": lambda: g.close(),
+    }
+
+    def run():
+        try:
+            got.append(calls[call]())
+        except Exception as ex:
+            errs.append(ex)
+    stream, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0   # (non-blocking)
+    assert hip.hipStreamBeginCapture(stream, 1) == 0               # (thread-local)
+    t = threading.Thread(target=run)
+    t.start()
+    t.join()
+    rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert not errs and rc == 0, (errs, rc)
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+    if call != "close":
+        if call.startswith("upload"):
+            g.finalize()
+        assert np.isfinite(g.forward(3, 0)).all()
+        g.close()
+
+
 def test_error_text_is_kept_per_context_across_threads(orc):
     """A failing call on thread A, the message fetched on thread B (a Java virtual thread may be mounted on another
     carrier thread for its second downcall): l2j_ctx_last_error has it, the thread-local l2j_last_error of B does not."""
