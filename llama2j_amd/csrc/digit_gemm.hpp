@@ -402,9 +402,11 @@ template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (s
 // That order, request addresses that need no vector registers and the instantiation without the loop, W1 and W3 / Wq, Wk and Wv /
 // W2 / Wo of the 7B shape: 22.4 -> 20.8, 15.2 -> 14.7, 14.8 -> 13.9, 8.1 -> 8.0 us, those of the 110M shape 5.0 -> 4.6.  Codes two tiles
 // ahead instead: 3 to 5 % slower (the requests past the end, of which a workgroup with two tiles then makes two).
-// ONE: no workgroup has more than one tile (every product of the 110M shape): no codes requested ahead, no copy of the loop to fetch.
+// TILES: the most tiles a workgroup has, 0 for any number.  One (every product of the 110M shape): no codes requested ahead, no copy of the
+// loop to fetch.  Two, up to 16 vectors: no third request, which the loop makes for nothing (Wo of the 7B shape 6.9 -> 6.45 us,
+// 24 steps of 16 sequences 52.5 -> 52.0 ms).
 // Workgroup (blockIdx.x, slice blockIdx.y) of gridDim.x per slice: every gridDim.x-th tile of 32 rows (rows % 32 == 0).
-template <int NB, bool ONE>
+template <int NB, int TILES>
 static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
 {
     constexpr int NT = 2;   // blocks of 64 k per wave
@@ -523,7 +525,7 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     };
     Sums u;
     int t = t0;
-    if constexpr (ONE) {
+    if constexpr (TILES == 1) {
         tile(0, c0);
         __syncthreads();
         read(0, u);
@@ -535,6 +537,19 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     __builtin_amdgcn_sched_barrier(0);   // (not moved behind the products, where it would find its registers free)
     tile(0, c0);
     __syncthreads();
+    if constexpr (TILES == 2) {
+        read(0, u);
+        if (t + step >= ntile) {
+            finish(t, u);
+            return;
+        }
+        tile(1, c1);
+        finish(t, u);
+        __syncthreads();
+        read(1, u);
+        finish(t + step, u);
+        return;
+    }
     while (true) {
         read(0, u);
         if (t + step >= ntile) break;

@@ -92,11 +92,11 @@ int l2j::launch_dgemm(l2j_ctx *c, std::initializer_list<int> tensors, int layer,
         a.gps = (a.ngroups + slices - 1) / slices;
         const dim3 grid((ntile + iters - 1) / iters, slices);
         const dim3 block(64 * kStreamWaves);
-        const bool one = iters == 1;
-        if (rows <= 16 && one) hipLaunchKernelGGL((k_dstream<1, true>), grid, block, dstream_lds<1>(), c->stream, a);
-        else if (rows <= 16) hipLaunchKernelGGL((k_dstream<1, false>), grid, block, dstream_lds<1>(), c->stream, a);
-        else if (one) hipLaunchKernelGGL((k_dstream<2, true>), grid, block, dstream_lds<2>(), c->stream, a);
-        else hipLaunchKernelGGL((k_dstream<2, false>), grid, block, dstream_lds<2>(), c->stream, a);
+        if (rows <= 16 && iters == 1) hipLaunchKernelGGL((k_dstream<1, 1>), grid, block, dstream_lds<1>(), c->stream, a);
+        else if (rows <= 16 && iters == 2) hipLaunchKernelGGL((k_dstream<1, 2>), grid, block, dstream_lds<1>(), c->stream, a);
+        else if (rows <= 16) hipLaunchKernelGGL((k_dstream<1, 0>), grid, block, dstream_lds<1>(), c->stream, a);
+        else if (iters == 1) hipLaunchKernelGGL((k_dstream<2, 1>), grid, block, dstream_lds<2>(), c->stream, a);
+        else hipLaunchKernelGGL((k_dstream<2, 0>), grid, block, dstream_lds<2>(), c->stream, a);
         return slices;
     }
     const DgPlan p = dgemm_plan(c->n_cu, a.ntiles, a.ngroups, rows);
