@@ -652,7 +652,7 @@ __device__ __forceinline__ void xcd_classifier(const XcdArgs &a, float *lds, int
                 g.logits[row] = acc;
                 if (better(acc, row, best_v, best_i)) { best_v = acc; best_i = row; }
             }
-            request(i, p0 + i + NPRE);
+            if (r0 + (p0 + i + NPRE) * NG < r1) request(i, p0 + i + NPRE);   // (uniform)
         }
     }
 #pragma unroll
