@@ -363,10 +363,6 @@ int l2j::check_barrier_error(l2j_ctx *c)
     return fail(L2J_E_HIP, "a bounded wait of the whole-token kernel ran out (barrier or input vector; its workgroups were not all resident)");
 }
 
-namespace {
-
-}  // namespace
-
 int l2j::set_state(l2j_ctx *c, int token, int pos, int n_prompt)
 {
     c->h_st->pos = pos;   // (l2j_forward_taps: which cache rows to copy)

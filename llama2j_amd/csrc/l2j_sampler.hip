@@ -155,10 +155,6 @@ int l2j::seed_sampler(l2j_ctx *c, int64_t rng_seed)
     return L2J_OK;
 }
 
-namespace {
-
-}  // namespace
-
 // ---- a sampler per sequence of the batched decode: the launch-per-stage step with the sequence as grid z ----
 
 void l2j::free_batch_samplers(BatchSamplers *bs)
@@ -300,10 +296,6 @@ hipError_t l2j::launch_sampler(l2j_ctx *c, float temperature, float topp, float 
     return hipGetLastError();
 }
 
-namespace {
-
-}  // namespace
-
 // After a synchronize with h_ss read back: the reference's exceptions as an error return; the flag is cleared.
 int l2j::check_sampler_status(l2j_ctx *c)
 {
@@ -322,20 +314,11 @@ int l2j::check_sampler_status(l2j_ctx *c)
     return fail(L2J_E_ARG, "sampler: no probability reaches the top-p cutoff (ArrayIndexOutOfBoundsException at J/Sampler.java:119)");
 }
 
-namespace {
-
-}  // namespace
-
 int l2j::check_sampler_args(float temperature, float topp)
 {
     if (!(temperature >= 0.0f) || !(topp >= 0.0f && topp <= 1.0f)) return fail(L2J_E_ARG, "temperature must be >= 0 and topp in [0, 1]");
     return L2J_OK;
 }
-
-namespace {
-
-
-}  // namespace
 
 extern "C" {
 

@@ -596,6 +596,7 @@ template <class C>
 __device__ __forceinline__ void xcd_classifier(const XcdArgs &a, float *lds, int id, int ncls, int set)
 {
     constexpr int NG = kXThreads / C::LC, NPRE = 3;
+    static_assert(C::LC == 8, "the sums' exchanges between lanes");
     const TokenGeom &g = a.g;
     const int tid = threadIdx.x, dim = g.dim, n4 = dim >> 2, gc = tid / C::LC, cl = tid % C::LC, xcd = blockIdx.x % kXcds;
     const Poll pl{1, a.maxspin, g.fault};
@@ -641,11 +642,7 @@ __device__ __forceinline__ void xcd_classifier(const XcdArgs &a, float *lds, int
             }
             acc += dpp_f<0xB1>(acc);
             acc += dpp_f<0x4E>(acc);
-            if (C::LC == 8) acc += dpp_f<0x141>(acc);
-            if (C::LC == 16) {
-                acc += dpp_f<0x124>(acc);
-                acc += dpp_f<0x128>(acc);
-            }
+            acc += dpp_f<0x141>(acc);   // (row_half_mirror: eight lanes)
             const int row = r0 + gc + (p0 + i) * NG;
             acc = __fmul_rn(ss, acc);
             if (row < r1 && cl == 0) {
