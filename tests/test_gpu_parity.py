@@ -24,11 +24,13 @@ QT = [TENSOR.RMS_ATT, TENSOR.WQ, TENSOR.WK, TENSOR.WV, TENSOR.WO, TENSOR.RMS_FFN
       TENSOR.W3, TENSOR.RMS_FINAL]
 
 
-@pytest.fixture(params=["token", "phase"])
+@pytest.fixture(params=["token", "token on all units", "phase"])
 def launch_mode(request, monkeypatch):
-    """The forward pass as one whole-token launch (the default for large models) or as one launch per phase
-    (the default for small ones); the library reads the switch when a transformer is finalized."""
-    monkeypatch.setenv("L2J_FUSE", "1" if request.param == "token" else "0")
+    """The forward pass as one whole-token launch (small models, where a test has one that fits: the layers on the compute units of one
+    XCD, the default; and on all, the default for the others) or as one launch per phase (what both fall back to); the library reads
+    the switches when a transformer is made."""
+    monkeypatch.setenv("L2J_FUSE", "0" if request.param == "phase" else "1")
+    monkeypatch.setenv("L2J_ONE_XCD", "0" if request.param == "token on all units" else "-1")
     return request.param
 
 
@@ -355,7 +357,7 @@ def test_kernel_timing_entry_point(orc, launch_mode):
     for k in range(6):
         us, nbytes = g.time_kernel(k, 150, rounds=2)
         assert us > 0.0 and nbytes > 0, k
-    if launch_mode == "token":
+    if launch_mode != "phase":
         us, nbytes = g.time_kernel(l2j.KERNEL.TOKEN, 150, rounds=2)
         assert us > 0.0 and nbytes == g.bytes_per_token(150)
     else:  # no whole-token kernel in this mode
@@ -371,13 +373,15 @@ def test_kernel_timing_entry_point(orc, launch_mode):
 
 @pytest.mark.parametrize("env", [{"L2J_BY_VALUE": "0"}, {"L2J_LAYERS_PER_LAUNCH": "1"}, {"L2J_BY_VALUE": "1"},
                                  {"L2J_SELF_CONTAINED": "0"}, {"L2J_SELF_CONTAINED": "1"}, {"L2J_SELF_CONTAINED": "2"},
-                                 {"L2J_GRAPH_TOKENS": "1"}, {"L2J_GRAPH_TOKENS": "7"}, {"L2J_GRAPH": "0"}])
+                                 {"L2J_SELF_CONTAINED": "0", "L2J_GRAPH_TOKENS": "1"}, {"L2J_SELF_CONTAINED": "0", "L2J_GRAPH_TOKENS": "7"},
+                                 {"L2J_SELF_CONTAINED": "0", "L2J_GRAPH": "0"}])
 def test_whole_token_kernel_hand_over_variants(orc, monkeypatch, env):
     # the whole-token kernel with grid barriers instead of the hand-over by value, with one launch per layer (which
     # implies barriers), by value (the default: the kernel alternates two sets of vectors and steps the token loop
-    # itself), by value with k_fill_unset before and / or k_finish after every token, with other numbers of tokens per
-    # graph replay and without graphs: same tokens as the oracle, deep enough that attention runs in several splits
+    # itself, launched directly), by value with k_fill_unset before and / or k_finish after every token (replayed as graphs), those with
+    # other numbers of tokens per replay and without graphs: same tokens as the oracle, deep enough that attention runs in several splits
     monkeypatch.setenv("L2J_FUSE", "1")
+    monkeypatch.setenv("L2J_ONE_XCD", "0")
     for k, v in env.items():
         monkeypatch.setenv(k, v)
     for shape in ((64, 96, 3, 4, 2, 40, 200, 1), (256, 512, 2, 2, 2, 64, 96, 0)):
@@ -400,12 +404,12 @@ def test_general_token_kernel_on_shapes_that_have_an_instance_of_their_own(orc, 
         assert rel_err(g.forward(int(tok), pos), m.forward(int(tok), pos)) < 1e-4, pos
 
 
-def test_whole_token_kernel_between_other_launches(orc, monkeypatch):
+@pytest.mark.parametrize("shape", [(256, 512, 3, 2, 2, 64, 40, 0), (64, 96, 3, 4, 2, 64, 40, 0)])   # (the second: layers on one XCD)
+def test_whole_token_kernel_between_other_launches(orc, monkeypatch, shape):
     """The self-contained whole-token kernel keeps its own book on which activation vectors read 'unwritten'.  Launches
     that write those vectors behind its back (per-layer taps, phases timed on their own) must not confuse it: tokens
     and logits of forwards mixed with such launches equal the oracle's, and the live taps name the set the last token used."""
     monkeypatch.setenv("L2J_FUSE", "1")
-    shape = (256, 512, 3, 2, 2, 64, 40, 0)
     m, g = make_pair(orc, shape, seed=71, realistic=True)
     m.enable_taps()
     tok = 1
@@ -425,10 +429,13 @@ def test_whole_token_kernel_between_other_launches(orc, monkeypatch):
     m.close(); g.close()
 
 
-def test_decode_stops_inside_a_replayed_batch(orc, monkeypatch):
-    """The decode loop replays several tokens per graph launch and enqueues the next batch before it has looked at
-    this one's tokens; a sequence that emits token 1 in the middle of a batch still ends there (J/Run.java:670-672)."""
-    monkeypatch.setenv("L2J_FUSE", "1")
+@pytest.mark.parametrize("env", [{"L2J_FUSE": "0"}, {"L2J_FUSE": "1", "L2J_SELF_CONTAINED": "0"}, {"L2J_FUSE": "1"}])
+def test_decode_stops_inside_a_replayed_batch(orc, monkeypatch, env):
+    """The decode loop replays several tokens per graph launch (where a token takes more than one launch; else launches as many) and
+    enqueues the next batch before it has looked at this one's tokens; a sequence that emits token 1 in the middle of a batch still
+    ends there (J/Run.java:670-672)."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
     monkeypatch.setenv("L2J_GRAPH_TOKENS", "8")
     shape = (64, 96, 2, 4, 4, 3, 200, 1)   # a vocabulary of three: token 1 comes up within a few steps
     for seed in range(40, 48):
@@ -444,11 +451,13 @@ def test_decode_stops_inside_a_replayed_batch(orc, monkeypatch):
         m.close(); g.close()
 
 
-def test_barrier_time_out_is_reported_not_hung(orc, monkeypatch):
+@pytest.mark.parametrize("one_xcd", ["-1", "0"])
+def test_barrier_time_out_is_reported_not_hung(orc, monkeypatch, one_xcd):
     # a spin limit of zero makes the bounded waits of the whole-token kernel give up at once: every kernel still
     # runs to its end, the call reports the failure, and a context with the normal limit is unaffected
     shape = (64, 96, 2, 4, 2, 40, 32, 1)
     monkeypatch.setenv("L2J_FUSE", "1")
+    monkeypatch.setenv("L2J_ONE_XCD", one_xcd)
     monkeypatch.setenv("L2J_BARRIER_SPINS", "0")
     monkeypatch.setenv("L2J_FALLBACK", "0")
     m, bad = make_pair(orc, shape, seed=50)
@@ -468,16 +477,19 @@ def test_barrier_time_out_is_reported_not_hung(orc, monkeypatch):
     bad.close()
 
 
-def test_waits_that_run_out_fall_back_to_one_launch_per_phase(orc, monkeypatch):
+@pytest.mark.parametrize("fuse,one_xcd", [("1", "-1"), ("1", "0"), ("-1", "-1")])
+def test_waits_that_run_out_fall_back_to_one_launch_per_phase(orc, monkeypatch, fuse, one_xcd):
     """The whole-token kernel needs every workgroup resident; when its bounded waits run out (forced here by a spin limit of
     zero; in the field by another process holding compute units) the context switches to one launch per phase for good
-    and repeats the call: the caller sees correct results, not an error."""
+    and repeats the call: the caller sees correct results, not an error.  From the layers on one XCD (one_xcd -1) by way of the kernel
+    on all units where the context is to have one (fuse 1), else at once."""
     shape = (64, 96, 2, 4, 2, 40, 32, 1)
-    monkeypatch.setenv("L2J_FUSE", "1")
+    monkeypatch.setenv("L2J_FUSE", fuse)
+    monkeypatch.setenv("L2J_ONE_XCD", one_xcd)
     monkeypatch.setenv("L2J_BARRIER_SPINS", "0")
     for entry in ("forward", "forward_argmax", "decode_greedy", "decode_sample"):
         m, g = make_pair(orc, shape, seed=51, realistic=True)
-        assert g.get_option("fuse") == 1 and g.get_option("fallback") == 1
+        assert g.get_option("fuse") == int(fuse) and g.get_option("fallback") == 1
         prompt = orc.synth_prompt(51, 3, shape[5])
         if entry == "forward":
             assert rel_err(g.forward(3, 0), m.forward(3, 0)) < 1e-4
