@@ -391,7 +391,7 @@ def main():
                         "stream); bytes at the mean position %d" % (g.get_option("wall_clock_khz"), done - 1, done - 1, done - 1, pos))
         ct = COUNTER_TRAFFIC.get(a.workload) if dom_name == "token" else None
         out["roofline"] = {"bound": "hbm",
-                           "kernel": "k_token (all phases of all layers + classifier), one launch per token" if dom_name == "token"
+                           "kernel": "the whole-token kernel (k_token, for small models k_xtoken: all phases of all layers + classifier), one launch per token" if dom_name == "token"
                            else "k_matvec<PH_W13> (rmsnorm + W1,W3 matvec + SwiGLU), one launch per layer",
                            "achieved": dom["GBps"], "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": dom["frac"],
                            "algorithmic_bytes_per_launch": dom["bytes"], "us_per_launch": dom["us"], "measured": measured,

@@ -133,7 +133,7 @@ bool xcd_fits(const l2j_ctx *c)
     if (c->n_cu != kXcds * nwork || g.n_heads > nwork || c->head_size > 64 || c->head_size % 4 || dim % 16 || hid % 16) return false;
     if (dim > 16 * C::LD * C::CD || hid > 16 * C::LH * C::CH || dim > 4 * C::LC * C::FC) return false;
     if (dim * dim % 256 || dim * kvd % 256 || dim * hid % 256) return false;   // (a layer's matrices are whole groups)
-    if (g.seq_len > 4096) return false;   // (few workgroups per head: 384 wide, two layers, at position 4090 58 us against 56 of k_token, 31 against 42 at 5)
+    if (g.seq_len > 4096) return false;   // (few workgroups per head: 384 wide, two layers, us at positions 5, 500, 2000 and 4090 24, 34, 45, 59 against 51, 56, 64, 66 of k_token, which 6 us per 1000 positions more overtake near 5400)
     return 2 * per((dim + 2 * kvd) / 2) <= rows_d && per(hid) <= rows_d && per(dim) <= std::min(rows_d, rows_h);
 }
 

@@ -211,7 +211,7 @@ struct l2j_ctx {
     void *blocks[1 + ArrayPlan::kMax];   // the device allocations behind the arrays above
     int nblocks = 0;
     char *pinned = nullptr;       // the one behind the h_ pointers
-    // Staging of an upload that finds it free (Upload); others bring a buffer of their own.
+    // Staging of an upload that finds it free (Staged); others bring a buffer of their own.
     char *stage = nullptr;
     uint64_t stage_bytes = 0;
     std::mutex stage_mu;

@@ -8,8 +8,9 @@
 // the others meanwhile mark the next token's vectors unwritten and load their rows of the classifier into registers.  They
 // get the last vector through one workgroup per XCD, which passes it on inside its own L2.
 //
-// 15M shape (288, 768, six layers), us a token at positions 5 and 255: k_token 112 and 123, this 63 and 74; two layers 50 and 54 -> 29
-// and 31.  What is left of a layer's 8.5 us, by time stamps: the hand-overs 0.5 to 0.6 us each, the stagers 0.3, a phase's
+// 15M shape (288, 768, six layers), us a token at positions 5 and 255: k_token 111 and 122, this 58 and 69; two layers 51 and 54 -> 24
+// and 26.  (5.5 of these more when the classifier's workgroups requested rows past their own behind their last; 1.3 less with the
+// exponentials and the scale of q in one rounding each, at 130 times the error of a far weight.)  What is left of a layer's 8.5 us, by time stamps: the hand-overs 0.5 to 0.6 us each, the stagers 0.3, a phase's
 // multiply-adds and sums 0.45 (one wave per SIMD issues an instruction every five to six cycles), attention 1.0.
 //
 // Nothing depends on where the workgroups really run but the speed: a word that is not seen stays unwritten (kUnset), the
