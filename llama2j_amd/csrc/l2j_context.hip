@@ -367,7 +367,7 @@ int l2j_upload_f32_quantize(l2j_ctx *c, int tensor, uint64_t first, const float 
         if (!is_quant(tensor)) return fail(L2J_E_ARG, "not a quantized tensor");
         QTensor &t = c->qt[tensor];
         if (first % kGroup) return fail(L2J_E_ARG, "first must be a multiple of the group size");
-        if (first + nfloats > t.nfloats) return fail(L2J_E_SIZE, "range exceeds the tensor");
+        if (first > t.nfloats || nfloats > t.nfloats - first) return fail(L2J_E_SIZE, "range exceeds the tensor");
         if (nfloats % kGroup && first + nfloats != t.nfloats) return fail(L2J_E_ARG, "only the tensor's tail may be a partial group");
         std::lock_guard<std::mutex> tensor_lock(t.mu);
         HIPCHK(hipSetDevice(c->cfg.device));
@@ -407,7 +407,7 @@ int l2j_read_quant(l2j_ctx *c, int tensor, uint64_t group0, uint64_t ngroups, ui
         if (!c || !out) return fail(L2J_E_ARG, "null argument");
         if (!is_quant(tensor)) return fail(L2J_E_ARG, "not a quantized tensor");
         QTensor &t = c->qt[tensor];
-        if (group0 + ngroups > t.ngroups) return fail(L2J_E_SIZE, "group range exceeds the tensor");
+        if (group0 > t.ngroups || ngroups > t.ngroups - group0) return fail(L2J_E_SIZE, "group range exceeds the tensor");
         if (ngroups == 0) return L2J_OK;
         std::lock_guard<std::mutex> lock(c->upload_mu);
         HIPCHK(hipSetDevice(c->cfg.device));
@@ -584,7 +584,7 @@ int l2j_read(l2j_ctx *c, int which, int layer, uint64_t off, float *dst, uint64_
             len = which == L2J_B_HB ? g.hidden_dim : (which == L2J_B_K || which == L2J_B_V) ? c->kv_dim : g.dim;
             src = c->taps[which] + (uint64_t)layer * len;
         }
-        if (off + n > len) return fail(L2J_E_SIZE, "read past the end of the buffer");
+        if (off > len || n > len - off) return fail(L2J_E_SIZE, "read past the end of the buffer");
         return read_floats(c, dst, src + off, n);
     }());
 }

@@ -751,6 +751,21 @@ def test_reads_of_parts_are_parts_of_the_whole():
     g.close()
 
 
+def test_ranges_whose_end_wraps_are_refused():
+    # first + count modulo 2^64 lies inside the tensor; nothing is read or written
+    g = l2j.Transformer(l2j.Config(64, 176, 2, 4, 4, 101, 8, 0))
+    g.fill_synthetic(3, 0.02)
+    f, b = np.zeros(1024, dtype=np.float32), np.zeros(1024, dtype=np.uint8)
+    fp, bp = f.ctypes.data_as(C.POINTER(C.c_float)), b.ctypes.data_as(C.POINTER(C.c_uint8))
+    before = g.read_quant(TENSOR.WQ, 0, 32)
+    for back, n in ((1, 2), (4, 8), (2 ** 32, 2 ** 32)):
+        assert l2j.lib().l2j_read(g._h, BUFFER.LOGITS, -1, 2 ** 64 - back, fp, n) == -2
+        assert l2j.lib().l2j_read_quant(g._h, TENSOR.WQ, 2 ** 64 - back, n, bp) == -2
+    assert l2j.lib().l2j_upload_f32_quantize(g._h, TENSOR.WQ, 2 ** 64 - 256, fp, 512) == -2
+    np.testing.assert_array_equal(g.read_quant(TENSOR.WQ, 0, 32), before)
+    g.close()
+
+
 @pytest.mark.parametrize("call", ["create", "upload_f32", "read_quant", "finalize", "finalize_phases", "forward", "read", "write_kv", "decode_greedy",
                                   "decode_sample", "sample_separately", "prefill", "batch", "batch_sampled", "fallback", "close"])
 def test_calls_run_while_another_thread_captures(call, monkeypatch):
