@@ -12,6 +12,8 @@
 
 #include "kernels.hpp"
 
+#include <utility>
+
 namespace l2j {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -173,19 +175,47 @@ constexpr int kDgWaveRows = 64;   // matrix rows per wave
 
 template <int PT> __host__ __device__ constexpr size_t dgemm_lds() { return (size_t)2 * PT * (kDigitBytes + 128); }
 
+// f(0), ..., f(N - 1) with the numbers as constants
+template <class F, int... I> __device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F> __device__ __forceinline__ void unroll(F &&f) { unroll_seq(f, std::make_integer_sequence<int, N>{}); }
+
+// A load at a uniform address plus 32 bits per lane (held as such: the compiler otherwise keeps 64-bit sums in vector registers).
+template <class T> __device__ __forceinline__ T load_at(const void *base, unsigned &off)
+{
+    typedef const __attribute__((address_space(1))) char *P;
+    P p = (P)base;
+    asm volatile("" : "+s"(p), "+v"(off));
+    return *reinterpret_cast<const __attribute__((address_space(1))) T *>(p + off);
+}
+
+// The order in which unit u of NU (16 vectors against the wave's 64 rows) takes its sixteen fragments of digits: step j is digit
+// dg_digit and block of 64 k dg_block.  First and third digits before second and fourth, each pair's sums being shifted in between;
+// the first unit of a group begins, and the last one ends, with the two digits of a block of 64 k next to each other, so that the
+// codes of a block are needed 24 matrix instructions after they were free to be requested instead of 12.
+__device__ constexpr int dg_digit(int u, int nu, int j) { return u == 0 && j < 8 ? 2 * (j & 1) : u == nu - 1 && j >= 8 ? 1 + 2 * (j & 1) : (j >> 2) == 1 ? 2 : (j >> 2) == 2 ? 1 : j >> 2; }
+__device__ constexpr int dg_block(int u, int nu, int j) { return u == 0 && j < 8 ? j >> 1 : u == nu - 1 && j >= 8 ? (j - 8) >> 1 : j & 3; }
+
 // A workgroup takes 64 NW rows of the matrix x 32 PT vectors x one slice of K.  A wave holds the codes of its 64 rows of a
 // group in registers (read once from memory, 1 KB per load) and multiplies them by the digits of the vectors, which the
-// workgroup stages in LDS a group ahead; the digits of an output are summed 256 * first + second in one accumulator, and
-// then third and fourth.  (16 x 16 tiles: on random digits and codes of standard deviation 40, operands in registers, two waves per
-// SIMD, v_mfma_i32_16x16x64_i8 sustains 4.0 POP/s over 40 ms and v_mfma_i32_32x32x32_i8 2.9: the clock drops under the matrix
-// cores' load.)  With 1024 vectors of the 7B shape the matrix cores are busy 54 to 59 % of a launch's cycles, no LDS conflicts,
-// 2.3 other vector instructions per matrix instruction; 2.2 POP/s.
+// workgroup stages in LDS a group ahead (straight from memory: no registers, no writes of its own); the digits of an output are
+// summed 256 * first + second in one accumulator, third and fourth in another.  (16 x 16 tiles: on random digits and codes of standard
+// deviation 40, operands in registers, two waves per SIMD, v_mfma_i32_16x16x64_i8 sustains 4.0 POP/s over 40 ms and
+// v_mfma_i32_32x32x32_i8 2.9: the clock drops under the matrix cores' load.)
+// What a unit of 16 vectors leaves is converted, scaled and added between the matrix instructions of the next one, two vector
+// instructions beside each: alone that many cost it 9 % (9.4 -> 10.2 ns each, two waves per SIMD), in a block of their own behind the
+// matrix instructions, where both waves of a SIMD come at once behind a barrier, their whole time.  Against 64 bits the sums err
+// less: one rounding of a group's sum and one of the running sum, where there were two of the latter (7B widths, 1024 vectors: 0.80 to
+// 1.25e-7 for 1.04 to 1.75e-7).  1024 vectors, four products of the 7B shape, us: 206 67.2 351 169 -> 195 63.5 331 157 (2.2 POP/s); 96
+// vectors 33.1 16.8 60 -> 31.3 16.6 56 (Wq+Wk+Wv, Wo, W1+W3).  A group then takes 10960 cycles at 1.9 GHz, 8192 of them
+// matrix instructions; without the codes' loads 0.9 of the time, without the digits' 0.95.  Tried, no faster: codes a whole group ahead in
+// a second set of registers (32 vectors: 3 % slower, it is bound by the codes' way through L2), workgroups that go on to
+// another tile instead of ending, sums stored four rows at a time by way of LDS.
 template <int PT, int NW>
 __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
 {
     extern __shared__ __align__(16) v4i dg_lds[];
     constexpr int STAGE = PT * kDigitBytes / 16;            // 16-byte words of a group's digits
-    constexpr int NT = 64 * NW, NST = STAGE / NT, NQ = NST / (2 * PT);   // words a thread stages per group, and per half of a tile of vectors
+    constexpr int NT = 64 * NW, NST = STAGE / NT, NU = 2 * PT;   // words a thread stages per group; units of 16 vectors
     float *lsx = reinterpret_cast<float *>(dg_lds + 2 * STAGE);   // [2][32 PT]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
     // The workgroups of an XCD (blockIdx % 8) take the same rows of the matrix against all vectors, one after the other.
@@ -210,37 +240,37 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
         cp[r] = cm + blk * 4096;
         sp[r] = sm + blk * 16;
     }
-    const unsigned co = lane * 16;
+    unsigned co = lane * 16, n8 = n * 8, tid16 = tid * 16;
     const v4i *xd = reinterpret_cast<const v4i *>(a.x.d) + ((size_t)col * PT * a.ngroups + g0) * (kDigitBytes / 16);
     const size_t xstep = (size_t)a.ngroups * (kDigitBytes / 16);   // 16-byte words between two tiles of vectors
     const float *xs = a.x.sx + ((size_t)col * PT * a.ngroups + g0) * 32;
     const int xt = tid & (32 * PT - 1);   // (every wave stages the scales: no branch in the loop)
-    const unsigned xso = (xt >> 5) * a.ngroups * 32 + (xt & 31);
+    unsigned xso = ((xt >> 5) * a.ngroups * 32 + (xt & 31)) * 4;
 
     // codes of the first group
     v4i cw[4][4];
 #pragma unroll
     for (int T = 0; T < 4; T++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) cw[r][T] = *reinterpret_cast<const v4i *>(cp[r] + co + 1024 * T);
-    // digits of the first group
-    float sx0;
+        for (int r = 0; r < 4; r++) cw[r][T] = load_at<v4i>(cp[r] + 1024 * T, co);
+    // digits of the first group, its vectors' and its rows' scales
+    float sx0, rm[4], rmp[4] = {0.f, 0.f, 0.f, 0.f};   // (rmp: the rows' scales of the group before)
     {
         v4i st[NST];
 #pragma unroll
         for (int q = 0; q < NST; q++) st[q] = (xd + (q * NT / 2048) * xstep + q * NT % 2048)[(unsigned)tid];
-        sx0 = xs[xso];
+        sx0 = load_at<float>(xs, xso);
+#pragma unroll
+        for (int r = 0; r < 4; r++) rm[r] = load_at<float>(sp[r], n8);
 #pragma unroll
         for (int q = 0; q < NST; q++) dg_lds[q * NT + tid] = st[q];
     }
     // the groups' offsets times the sums of the activations: fp32 matrix cores, four groups at a time
-    v4f f0[PT][2][4];
+    v4f f0[NU][4];
 #pragma unroll
-    for (int p = 0; p < PT; p++)
+    for (int u = 0; u < NU; u++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) f0[p][mt][r] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < 4; r++) f0[u][r] = v4f{0.f, 0.f, 0.f, 0.f};
     for (int g = g0; g < g1; g += 4) {
         const bool on = g + s4 < g1;
         const int gg = on ? s4 : 0;
@@ -248,32 +278,29 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
 #pragma unroll
         for (int r = 0; r < 4; r++) { const float v = (sp[r] + (size_t)(g - g0) * 16)[gg * 16 + n].y; b[r] = on ? v : 0.0f; }
 #pragma unroll
-        for (int p = 0; p < PT; p++)
+        for (int u = 0; u < NU; u++) {
+            const float v = (a.x.sum + ((size_t)(col * PT + (u >> 1)) * a.ngroups + g) * 32 + 16 * (u & 1))[gg * 32 + n];
+            const float s = on ? v : 0.0f;
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                const float v = (a.x.sum + ((size_t)(col * PT + p) * a.ngroups + g) * 32 + 16 * mt)[gg * 32 + n];
-                const float s = on ? v : 0.0f;
-#pragma unroll
-                for (int r = 0; r < 4; r++) f0[p][mt][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(s, b[r], f0[p][mt][r], 0, 0, 0);
-            }
+            for (int r = 0; r < 4; r++) f0[u][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(s, b[r], f0[u][r], 0, 0, 0);
+        }
     }
-    float f[PT][2][4][4];
+    float f[NU][4][4];
 #pragma unroll
-    for (int p = 0; p < PT; p++)
+    for (int u = 0; u < NU; u++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) f[p][mt][r][e] = f0[p][mt][r][e];
+            for (int e = 0; e < 4; e++) f[u][r][e] = f0[u][r][e];
     // Where 2^-s of some vector is so small that its product with a matrix's scale would lose bits (below 2^-126), all sums are kept
     // times 2^48 from that group on, unless a group of some vector is so large that this might carry its sum past the largest
-    // float.  (2^-s into the sum of digits instead, as k_dstream has it, is one product more behind the matrix cores: W1 and W3
+    // float.  (2^-s into the sum of digits instead, as k_dstream has it, was one product more behind the matrix cores: W1 and W3
     // of the 7B shape with 1024 vectors 330 -> 336 us; the vectors looked through ahead 330 -> 335.)  Every wave holds the 2^-s of all
     // the workgroup's vectors, so all come to the same power.
     const bool live = col * PT * 32 + xt < a.npos;
     float up = 1.0f;
     bool large = false;
+    v4f sxp = {0.f, 0.f, 0.f, 0.f};   // the scales of the unit whose sums are still to be added
     auto keep = [&](float x) {
         x = live ? x : 1.0f;
         if (__any(!(x >= 0x1p-64f && x <= 0x1p20f))) {
@@ -282,111 +309,117 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
             if (k != up) {
                 const float by = k > up ? 0x1p48f : 0x1p-48f;
 #pragma unroll
-                for (int p = 0; p < PT; p++)
+                for (int u = 0; u < NU; u++)
 #pragma unroll
-                    for (int mt = 0; mt < 2; mt++)
+                    for (int r = 0; r < 4; r++)
 #pragma unroll
-                        for (int r = 0; r < 4; r++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) f[p][mt][r][e] *= by;
+                        for (int e = 0; e < 4; e++) f[u][r][e] *= by;
+                sxp *= by;
                 up = k;
             }
         }
         return x * up;
     };
     lsx[xt] = keep(sx0);
-    float rm[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) rm[r] = sp[r][n].x;
     __syncthreads();
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): (a load under way here would be waited for in every round of the loop)
 
+    // The accumulators of two units in turn, and what adding up a unit takes: 80 operations, five for each of four rows' four values.
+    // operation o of unit v, whose vectors' scales are sx and whose rows' are r_m:
+    v4i hi[2][4], lo[2][4];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) { hi[k][r] = v4i{0, 0, 0, 0}; lo[k][r] = v4i{0, 0, 0, 0}; }
+    float eh[4], el[4], em[4];
+    auto add_up = [&](auto oc, auto vc, const v4f &sx, const float (&r_m)[4]) __attribute__((always_inline)) {
+        constexpr int o = oc.value, v = vc.value;
+        if constexpr (o < 80) {
+            constexpr int r = o / 20, what = o % 20 / 4, e = o % 4, k = v & 1;
+            if constexpr (what == 0) eh[e] = (float)hi[k][r][e];
+            else if constexpr (what == 1) el[e] = (float)lo[k][r][e];
+            else if constexpr (what == 2) em[e] = r_m[r] * sx[e];
+            else if constexpr (what == 3) eh[e] = fmaf(eh[e], 65536.0f, el[e]);
+            else f[v][r][e] = fmaf(eh[e], em[e], f[v][r][e]);
+        }
+    };
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) v4i *)dg_lds;
     const int ng = g1 - g0;
     for (int g = 0; g < ng; g++) {
-        const v4i *cur = dg_lds + (g & 1) * STAGE;
-        v4i *nxt = dg_lds + ((g + 1) & 1) * STAGE;
+        const v4i *cur = dg_lds + (g & 1) * STAGE + lane;
         const float *csx = lsx + (g & 1) * 32 * PT;
         const int gn = min(g + 1, ng - 1);                    // (past the last group: that group again, not used)
         const v4i *xn = xd + (size_t)gn * (kDigitBytes / 16);
-        float rm_lo[4], rm_hi[4];
+        // The next group's digits on their way into the other buffer, a KB per wave and instruction (m0: where in LDS; the lanes'
+        // 16 bytes follow each other).  Nothing the compiler counts: they come behind the codes of this group, which it waits for one by one,
+        // and are waited for below.
+        auto stage = [&](int q) __attribute__((always_inline)) {
+            const v4i *from = xn + (q * NT / 2048) * xstep + q * NT % 2048;
+            const unsigned to = lds0 + (((g + 1) & 1) * STAGE + q * NT + wave * 64) * 16;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(tid16), "s"(from) : "memory");
+        };
+        v4i x[4];   // fragments, three ahead of their use
+        auto fragment = [&](int u, int j) __attribute__((always_inline)) {
+            return cur[(u >> 1) * (kDigitBytes / 16) + dg_digit(u, NU, j) * 512 + (2 * dg_block(u, NU, j) + (u & 1)) * 64];
+        };
+        x[0] = fragment(0, 0); x[1] = fragment(0, 1); x[2] = fragment(0, 2);
+        const float nsx = load_at<float>(xs + gn * 32, xso);
+        float rmn[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) { rm_lo[r] = rm[r]; rm_hi[r] = rm[r] * 65536.0f; }
-        const float nsx = (xs + gn * 32)[xso];
+        for (int r = 0; r < 4; r++) rmn[r] = load_at<float>(sp[r] + (size_t)gn * 16, n8);
+        __builtin_amdgcn_sched_barrier(0);
+        unroll<NU>([&](auto uc) __attribute__((always_inline)) {
+            constexpr int u = uc.value, k = u & 1;
+            typedef std::integral_constant<int, (u + NU - 1) % NU> Before;
+            const v4f sx = *reinterpret_cast<const v4f *>(csx + 16 * u + 4 * s4);
+            unroll<16>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = jc.value, d = dg_digit(u, NU, j), T = dg_block(u, NU, j), at = 16 * u + j;
+                constexpr int per = (NST + NU - 2) / (NU - 1);   // words staged in a unit behind the first
+                if constexpr (u > 0 && j < per && (u - 1) * per + j < NST) stage((u - 1) * per + j);
+                if constexpr (at + 3 < 16 * NU) x[(at + 3) & 3] = fragment((at + 3) >> 4, (at + 3) & 15);
+                unroll<4>([&](auto rc) __attribute__((always_inline)) {
+                    constexpr int r = rc.value, i = 4 * j + r;
+                    v4i &acc = (d & 2) ? lo[k][r] : hi[k][r];
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[at & 3], cw[r][T], !(d & 1) && T == 0 ? v4i{0, 0, 0, 0} : acc, 0, 0, 0);
+                    // beside it the unit before, and the shifts between the digits of a pair
+                    constexpr int o = i < 16 ? 2 * i : 16 + i;
+                    add_up(std::integral_constant<int, o>{}, Before{}, sxp, u == 0 ? rmp : rm);
+                    if constexpr (i < 16) add_up(std::integral_constant<int, o + 1>{}, Before{}, sxp, u == 0 ? rmp : rm);
+                    if constexpr (u == 0 && j == 7) hi[k][r] <<= 8;
+                    if constexpr (u != 0 && j >= 4 && j < 8) hi[k][j - 4][r] <<= 8;
+                    if constexpr (u == NU - 1 && j == 8) lo[k][r] <<= 8;
+                    if constexpr (u != NU - 1 && j >= 8 && j < 12) lo[k][j - 8][r] <<= 8;
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                if constexpr (u == NU - 1 && j >= 8 && (j & 1)) {   // (the last use of these codes: the next group's in their place)
 #pragma unroll
-        for (int r = 0; r < 4; r++) rm[r] = (sp[r] + (size_t)gn * 16)[n].x;
-#pragma unroll
-        for (int p = 0; p < PT; p++) {
-#pragma unroll
-            for (int pair = 0; pair < 2; pair++) {
-                v4i st[NQ];
-                const int q0 = (2 * p + pair) * NQ;
-#pragma unroll
-                for (int q = 0; q < NQ; q++) st[q] = (xn + ((q0 + q) * NT / 2048) * xstep + (q0 + q) * NT % 2048)[(unsigned)tid];
-                const v4i *fr = cur + p * (kDigitBytes / 16) + pair * 2 * 512 + lane;
-                v4i acc[2][4];
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[mt][r] = v4i{0, 0, 0, 0};
-#pragma unroll
-                for (int T = 0; T < 4; T++)
-#pragma unroll
-                    for (int mt = 0; mt < 2; mt++) {
-                        const v4i x = fr[(2 * T + mt) * 64];
-#pragma unroll
-                        for (int r = 0; r < 4; r++) acc[mt][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, cw[r][T], acc[mt][r], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[mt][r] <<= 8;
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int T = 0; T < 4; T++) {
-#pragma unroll
-                    for (int mt = 0; mt < 2; mt++) {
-                        const v4i x = fr[512 + (2 * T + mt) * 64];
-#pragma unroll
-                        for (int r = 0; r < 4; r++) acc[mt][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, cw[r][T], acc[mt][r], 0, 0, 0);
-                    }
-                    if (p == PT - 1 && pair == 1) {   // (the last use of these codes: the next group's in their place)
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int r = 0; r < 4; r++) cw[r][T] = *reinterpret_cast<const v4i *>(cp[r] + (size_t)gn * 4096 + co + 1024 * T);
-                    }
+                    for (int r = 0; r < 4; r++) cw[r][T] = load_at<v4i>(cp[r] + (size_t)gn * 4096 + 1024 * T, co);
                 }
+            });
+            sxp = sx;
+            __builtin_amdgcn_sched_barrier(0);
+        });
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++) {
-                    const v4f sx = *reinterpret_cast<const v4f *>(csx + 32 * p + 16 * mt + 4 * s4);
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            f[p][mt][r][e] = fmaf((float)acc[mt][r][e], (pair ? rm_lo[r] : rm_hi[r]) * sx[e], f[p][mt][r][e]);
-                }
-#pragma unroll
-                for (int q = 0; q < NQ; q++) nxt[(q0 + q) * NT + tid] = st[q];
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+        for (int r = 0; r < 4; r++) { rmp[r] = rm[r]; rm[r] = rmn[r]; }
         lsx[((g + 1) & 1) * 32 * PT + xt] = keep(nsx);
+        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // (the staged digits: all but the sixteen loads of codes behind them)
         __syncthreads();
     }
+    unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
     const int ldo = 16 * a.ntiles;
     const float down = up == 1.0f ? 1.0f : 0x1p-48f;
 #pragma unroll
-    for (int p = 0; p < PT; p++)
+    for (int u = 0; u < NU; u++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int e = 0; e < 4; e++) {
+            const int pos = (col * NU + u) * 16 + 4 * s4 + e;
+            if (pos < a.npos) {
+                float *o = a.out + ((size_t)slice * a.npos + pos) * ldo;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int pos = (col * PT + p) * 32 + 16 * mt + 4 * s4 + e;
-                if (pos < a.npos) {
-                    float *o = a.out + ((size_t)slice * a.npos + pos) * ldo;
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[p][mt][r][e] * down;
-                }
+                for (int r = 0; r < 4; r++)
+                    if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[u][r][e] * down;
             }
+        }
 }
 
 // ---- at most 32 vectors: a decode step of a batch ---------------------------------------------------------------------
