@@ -636,7 +636,7 @@ int decode_batch(l2j_ctx *c, const int32_t *prompts, const int32_t *n_prompt, in
             unsigned active = 0;
             for (int s = 0; s < nseq; s++) active |= pos >= n_prompt[s] ? 1u << s : 0u;
             if (active) {
-                e = launch_samplers(c, b.samplers, active, cur, b.logits, temperature, topp, b.st->token, b.out + pos, cap);
+                e = launch_samplers(c, b.samplers, active, cur, b.logits, b.best, kNextParts, temperature, topp, b.st->token, b.out + pos, cap);
                 if ((double)topp <= 0.999) cur ^= active;   // (a top-p step leaves the array in its other copy)
             }
         }

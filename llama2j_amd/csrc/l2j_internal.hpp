@@ -348,9 +348,10 @@ struct BatchSamplers {
 int alloc_batch_samplers(l2j_ctx *c, int nseq, BatchSamplers *bs);
 void free_batch_samplers(BatchSamplers *bs);
 // One sampling step for the sequences whose bit is set in `active` (cur: bit s = the copy of its array that sequence s's last
-// top-p step left), on the rows of logits; the tokens go to token[s] and out[s * out_stride].
-hipError_t launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned active, unsigned cur, float *logits, float temperature,
-                           float topp, int *token, int *out, long out_stride);
+// top-p step left), on the rows of logits, whose largest k_bnext has left in best (nbest words per sequence); the tokens go to
+// token[s] and out[s * out_stride].
+hipError_t launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned active, unsigned cur, float *logits,
+                           const unsigned long long *best, int nbest, float temperature, float topp, int *token, int *out, long out_stride);
 // l2j_rows.hip: l2j_prefill without the lock (the decode loops call it holding it)
 // keep_logits: leave the last position's logits in the context, as l2j_prefill does
 int prefill_positions(l2j_ctx *c, const int32_t *tokens, int32_t n, int32_t pos0, float *logits, double *seconds, bool keep_logits = true);

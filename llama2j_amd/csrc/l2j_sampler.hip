@@ -192,8 +192,8 @@ int l2j::alloc_batch_samplers(l2j_ctx *c, int nseq, BatchSamplers *bs)
     return rc;
 }
 
-hipError_t l2j::launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned active, unsigned cur, float *logits, float temperature,
-                                float topp, int *token, int *out, long out_stride)
+hipError_t l2j::launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned active, unsigned cur, float *logits,
+                                const unsigned long long *best, int nbest, float temperature, float topp, int *token, int *out, long out_stride)
 {
     const int n = c->cfg.vocab_size, nseq = bs.nseq;
     const int npad = (n + kSortRun - 1) / kSortRun * kSortRun;
@@ -207,20 +207,20 @@ hipError_t l2j::launch_samplers(l2j_ctx *c, const BatchSamplers &bs, unsigned ac
     a.pi_prob0 = bs.pi_prob[0]; a.pi_prob1 = bs.pi_prob[1]; a.pi_idx0 = bs.pi_idx[0]; a.pi_idx1 = bs.pi_idx[1];
     a.logits_stride = n; a.pi_stride = (long)bs.pi_stride;
     a.btoken = token; a.bout = out; a.bout_stride = out_stride;
-    // (no k_sample_exp: with the sequences' workgroups side by side the exponentials cost less inside k_sample_probs than
-    // a launch of their own, in which every workgroup reads all of its sequence's logits for the maximum: 81 us measured)
+    a.expbuf = bs.sort_k[0]; a.exp_stride = (long)bs.sort_stride;   // (where the sort's tiles come to lie behind k_sample_probs)
+    hipLaunchKernelGGL(k_sample_exp_b, dim3((n + 1023) / 1024, 1, nseq), dim3(256), 0, c->stream, a, best, nbest);
     const size_t lds = sampler_lds_bytes(n);
     hipLaunchKernelGGL(k_sample_probs<true>, dim3(1, 1, nseq), dim3(1024), lds, c->stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.plain) return e;
     SortBatch sb{};
-    sb.active = active; sb.cur = cur;
+    sb.active = active; sb.cur = cur; sb.ss = bs.ss;
     sb.pi_prob0 = bs.pi_prob[0]; sb.pi_prob1 = bs.pi_prob[1]; sb.pi_idx0 = bs.pi_idx[0]; sb.pi_idx1 = bs.pi_idx[1];
     sb.tiles_k = bs.sort_k[0]; sb.tiles_v = bs.sort_v[0]; sb.runs_k = bs.sort_k[1]; sb.runs_v = bs.sort_v[1];
     sb.pi_stride = (long)bs.pi_stride; sb.sort_stride = (long)bs.sort_stride;
-    hipLaunchKernelGGL(k_sort_tiles_b, dim3(npad / kSortTile, 1, nseq), dim3(kSortTile), 0, c->stream, sb, n);
+    hipLaunchKernelGGL(k_sort_tiles_b, dim3(npad / kSortTile, 1, nseq), dim3(kSortTile), 0, c->stream, sb);
     hipLaunchKernelGGL(k_merge_tiles_b, dim3(npad / kSortRun, 16, nseq), dim3(256), 0, c->stream, sb);
-    hipLaunchKernelGGL(k_merge_far_b, dim3(npad / 256, 1, nseq), dim3(256), 0, c->stream, sb, npad, n);
+    hipLaunchKernelGGL(k_merge_old_b, dim3((n + 255) / 256, 1, nseq), dim3(256), 0, c->stream, sb, n);
     hipLaunchKernelGGL(k_topp_pick<true>, dim3(1, 1, nseq), dim3(1024), lds, c->stream, a);
     return hipGetLastError();
 }

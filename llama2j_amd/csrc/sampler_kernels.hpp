@@ -37,17 +37,16 @@ struct SampleArgs {
     int *out_tokens;         //   that k_finish stored for position st->pos - 1
     unsigned long long *tstamp;   //   and the time that it stored with it
     int scan;                // 1: the running sums by spec_sums, 0: one lane adds them all (vocabularies that fit in LDS only)
-    float *expbuf;           // not null: k_sample_exp has left exp(x / temperature - max) here (n floats)
+    float *expbuf;           // not null: k_sample_exp or k_sample_exp_b has left exp(x / temperature - max) here (n floats)
     int *tok0, *tok1;        // null, or two more places that receive the token
     // Several samplers in one launch (the sequences of the batched decode; nseq 0: one): grid z = sequence.  The fields above
-    // are those of sequence 0 (cand_*, sorted_* unused; expbuf null: k_sample_probs forms the exponentials itself, the
-    // sequences' workgroups side by side); the arrays of the others follow at these strides.
+    // are those of sequence 0 (cand_*, sorted_* unused); the arrays of the others follow at these strides.
     int nseq;
     unsigned active;         // bit s: sequence s samples in this step (the others' workgroups leave at once)
     unsigned cur;            // bit s: the copy of its ProbIndex array that sequence s's last top-p step left
     float *pi_prob0, *pi_prob1;   // the two copies, (sequence, pi_stride); named one by one: a member array indexed by a
     int *pi_idx0, *pi_idx1;       // variable would move the whole argument to scratch memory
-    long logits_stride, pi_stride;
+    long logits_stride, pi_stride, exp_stride;
     int *btoken;             // (sequence): the token goes here (the sequence's next input)
     int *bout;               // and to bout[s * bout_stride]
     long bout_stride;
@@ -73,6 +72,7 @@ __device__ __forceinline__ bool sample_seq(SampleArgs &a)
     if (!((a.active >> s) & 1u)) return false;
     const bool cur = (a.cur >> s) & 1u;
     a.logits += s * a.logits_stride;
+    a.expbuf += s * a.exp_stride;
     a.ss += s;
     a.cand_prob = (cur ? a.pi_prob1 : a.pi_prob0) + s * a.pi_stride;
     a.cand_idx = (cur ? a.pi_idx1 : a.pi_idx0) + s * a.pi_stride;
@@ -259,8 +259,17 @@ __device__ __forceinline__ float spec_uniform(float F)
 // F + p[lo] + ... + p[hi - 1], one after the other (every lane of the wave the same)
 __device__ __forceinline__ float spec_add_terms(float F, const float *p, int lo, int hi)
 {
-#pragma unroll 8
-    for (int i = lo; i < hi; i++) F = __fadd_rn(F, p[i]);
+    const int lane = threadIdx.x & 63;
+    for (int c = lo; c < hi; c += 64) {   // (the terms fetched side by side, then taken from the lanes: no load between two additions)
+        const int m = min(64, hi - c);
+        const float v = p[c + min(lane, m - 1)];
+        auto term = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i)); };
+        int i = 0;
+        for (; i + 8 <= m; i += 8)
+#pragma unroll
+            for (int k = 0; k < 8; k++) F = __fadd_rn(F, term(i + k));
+        for (; i < m; i++) F = __fadd_rn(F, term(i));
+    }
     return spec_uniform(F);
 }
 
@@ -457,6 +466,32 @@ static __global__ void __launch_bounds__(1024) k_sample_exp(const SampleArgs a)
     if (bad && blockIdx.x == 0) atomicOr(&a.ss->nan, 1);
 }
 
+// The same for several sequences (grid z), whose largest logits are known already: best[s * nbest ..] holds those of nbest parts of
+// sequence s (bits of the float in the upper half), and the temperature is positive, so that the largest quotient is the quotient of the
+// largest logit.  grid (n / 1024 rounded up, 1, sequences), 256 threads, four logits each; n % 4 == 0.  (In k_sample_probs, one
+// workgroup per sequence: 16 sequences of 32000 logits 80 us, of which the maximum took 17 to 40 and the exponentials 7.)
+static __global__ void __launch_bounds__(256) k_sample_exp_b(const SampleArgs a0, const unsigned long long *__restrict__ best, int nbest)
+{
+    SampleArgs a = a0;
+    if (!sample_seq(a)) return;
+    const int i = 4 * (blockIdx.x * 256 + threadIdx.x);
+    float mx = -__builtin_inff();
+    for (int p = 0; p < nbest; p++) mx = fmaxf(mx, __fdiv_rn(__uint_as_float((unsigned)(best[blockIdx.z * nbest + p] >> 32)), a.temperature));
+    if (i >= a.n) return;
+    const float4 v = *reinterpret_cast<const float4 *>(a.logits + i);
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    float e[4];
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float t = __fdiv_rn(x[k], a.temperature);
+        bad |= t != t;
+        e[k] = (float)exp((double)__fsub_rn(t, mx));
+    }
+    *reinterpret_cast<float4 *>(a.expbuf + i) = make_float4(e[0], e[1], e[2], e[3]);
+    if (bad) atomicOr(&a.ss->nan, 1);
+}
+
 // dst[0..np) in LDS = src[0..n) followed by zeros; src is 16-byte aligned and readable up to n rounded up to 4, np a
 // multiple of 4.  All threads call.
 __device__ __forceinline__ void stage_terms(float *dst, const float *src, int n, int np)
@@ -532,12 +567,17 @@ __global__ void __launch_bounds__(1024) k_sample_probs(const SampleArgs a0)
     }
     __syncthreads();
     const float sum = s_sum;
-    // if (sum != 0) x /= sum; the probabilities replace the logits
+    // if (sum != 0) x /= sum; the probabilities replace the logits.  Every wave takes a contiguous part of the indices and goes
+    // through it 64 at a time, so that the candidates of a step go out to consecutive addresses; it counts them on the way.
+    const float cutoff = __fdiv_rn(__fsub_rn(1.0f, a.topp), (float)(n - 1));
+    const int per_wave = (((n + nt - 1) / nt) * 64 + 63) & ~63, w_lo = min(n, wave * per_wave), w_hi = min(n, w_lo + per_wave);
+    int c = 0;
 #pragma unroll 4
-    for (int i = tid; i < n; i += nt) {
+    for (int i = w_lo + lane; i < w_hi; i += 64) {
         float v = sp[i];
         if (sum != 0.0f) v = __fdiv_rn(v, sum);
         bad |= v != v;
+        c += v >= cutoff;
         sp[i] = v;
         a.logits[i] = v;
     }
@@ -575,13 +615,6 @@ __global__ void __launch_bounds__(1024) k_sample_probs(const SampleArgs a0)
     }
 
     // J/Sampler.java:85-96: candidates in index order into the front of the ProbIndex array
-    const float cutoff = __fdiv_rn(__fsub_rn(1.0f, a.topp), (float)(n - 1));
-    // every wave takes a contiguous part of the indices and goes through it 64 at a time, so that the candidates of a
-    // step go out to consecutive addresses
-    const int per_wave = (((n + nt - 1) / nt) * 64 + 63) & ~63, w_lo = min(n, wave * per_wave), w_hi = min(n, w_lo + per_wave);
-    int c = 0;
-#pragma unroll 4
-    for (int i = w_lo + lane; i < w_hi; i += 64) c += sp[i] >= cutoff;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
     if (lane == 0) u.cnt[wave] = c;
@@ -593,9 +626,11 @@ __global__ void __launch_bounds__(1024) k_sample_probs(const SampleArgs a0)
         total += cw;
     }
     if (tid == 0) a.ss->n0 = total;
+    float next = sp[max(0, min(w_lo + lane, w_hi - 1))];
     for (int i0 = w_lo; i0 < w_hi; i0 += 64) {
         const int i = i0 + lane;
-        const float v = i < w_hi ? sp[i] : 0.0f;
+        const float v = next;
+        next = sp[min(i + 64, w_hi - 1)];
         const bool is = i < w_hi && v >= cutoff;
         const unsigned long long m = __ballot(is);
         if (is) {
@@ -780,10 +815,14 @@ static __global__ void __launch_bounds__(kSortTile) k_sort_tiles(const float *__
     sort_tiles_of(kin, vin, n, kout, vout);
 }
 
-// The sort for several samplers in one launch (grid z = sequence; SampleArgs says which take part and where their arrays
-// lie): a sequence's ProbIndex array goes from the copy its last step left through its own runs into the other copy.
+// The sort for several samplers (grid z = sequence; SampleArgs says which take part and where their arrays lie): a sequence's
+// ProbIndex array goes from the copy its last step left, whose first n0 pairs are this step's candidates, into the other copy.  What
+// stands behind the candidates the last step left sorted, so the candidates alone go through tiles and runs, and one merge
+// puts the runs and the rest together.  Realistic distributions have a few hundred candidates of 32000 pairs (16 sequences, tiles + runs +
+// merge: 12 + 11 + 41 us when the whole array was sorted).
 struct SortBatch {
     unsigned active, cur;
+    const SamplerState *ss;       // (sequence): n0
     float *pi_prob0, *pi_prob1;   // the two copies of the ProbIndex arrays, (sequence, pi_stride)
     int *pi_idx0, *pi_idx1;
     long pi_stride;
@@ -792,23 +831,30 @@ struct SortBatch {
     long sort_stride;
 };
 
-static __global__ void __launch_bounds__(kSortTile) k_sort_tiles_b(const SortBatch b, int n)
+static __global__ void __launch_bounds__(kSortTile) k_sort_tiles_b(const SortBatch b)
 {
     const int s = blockIdx.z;
     const bool cur = (b.cur >> s) & 1u;
     if (!((b.active >> s) & 1u)) return;
-    sort_tiles_of((cur ? b.pi_prob1 : b.pi_prob0) + s * b.pi_stride, (cur ? b.pi_idx1 : b.pi_idx0) + s * b.pi_stride, n,
+    const int n0 = b.ss[s].n0;
+    if ((int)blockIdx.x * kSortTile >= n0) return;
+    sort_tiles_of((cur ? b.pi_prob1 : b.pi_prob0) + s * b.pi_stride, (cur ? b.pi_idx1 : b.pi_idx0) + s * b.pi_stride, n0,
                   b.tiles_k + s * b.sort_stride, b.tiles_v + s * b.sort_stride);
 }
 
+// nk: the tiles up to there are sorted (a multiple of kSortTile); those behind count as padding.
 __device__ __forceinline__ void merge_tiles_of(const float *__restrict__ kin, const int *__restrict__ vin, float *__restrict__ kout,
-                                               int *__restrict__ vout)
+                                               int *__restrict__ vout, int nk)
 {
     __shared__ __align__(16) float keys[kSortRun];
     const int tid = threadIdx.x, base = blockIdx.x * kSortRun;
 #pragma unroll
-    for (int q = 0; q < 4; q++)
-        *reinterpret_cast<float4 *>(&keys[4 * (tid + 256 * q)]) = *reinterpret_cast<const float4 *>(kin + base + 4 * (tid + 256 * q));
+    for (int q = 0; q < 4; q++) {
+        const int at = 4 * (tid + 256 * q);
+        float4 v = make_float4(-1.0f, -1.0f, -1.0f, -1.0f);
+        if (base + at < nk) v = *reinterpret_cast<const float4 *>(kin + base + at);
+        *reinterpret_cast<float4 *>(&keys[at]) = v;
+    }
     __syncthreads();
     const int i = blockIdx.y * 256 + tid;
     const float k = keys[i];
@@ -840,15 +886,17 @@ __device__ __forceinline__ void merge_tiles_of(const float *__restrict__ kin, co
 static __global__ void __launch_bounds__(256) k_merge_tiles(const float *__restrict__ kin, const int *__restrict__ vin, float *__restrict__ kout,
                                                      int *__restrict__ vout)
 {
-    merge_tiles_of(kin, vin, kout, vout);
+    merge_tiles_of(kin, vin, kout, vout, gridDim.x * kSortRun);
 }
 
 static __global__ void __launch_bounds__(256) k_merge_tiles_b(const SortBatch b)
 {
     const int s = blockIdx.z;
     if (!((b.active >> s) & 1u)) return;
+    const int n0 = b.ss[s].n0;
+    if ((int)(blockIdx.x * kSortRun + blockIdx.y * kSortTile) >= n0) return;
     merge_tiles_of(b.tiles_k + s * b.sort_stride, b.tiles_v + s * b.sort_stride, b.runs_k + s * b.sort_stride,
-                   b.runs_v + s * b.sort_stride);
+                   b.runs_v + s * b.sort_stride, (n0 + kSortTile - 1) & ~(kSortTile - 1));
 }
 
 constexpr int kSortMaxRuns = (kSampleMaxVocab + kSortRun - 1) / kSortRun;
@@ -901,7 +949,6 @@ static __global__ void __launch_bounds__(256) k_merge_runs(const float *__restri
 // grid: padded n / 256 workgroups of 256 threads; run_len and group_len are powers of two, npad a multiple of 256.
 constexpr int kSortFanIn = 16;
 
-template <int FANIN = kSortFanIn>
 __device__ __forceinline__ void merge_far_of(const float *__restrict__ kin, const int *__restrict__ vin, int npad, int nout,
                                              int run_len, int group_len, float *__restrict__ kout, int *__restrict__ vout)
 {
@@ -912,9 +959,9 @@ __device__ __forceinline__ void merge_far_of(const float *__restrict__ kin, cons
     const int off = i - g0, ri = off / run_len;
     const int gend = min(npad, g0 + group_len);
     int rank = g0 + off - ri * run_len;
-    int pos[FANIN], len[FANIN];
+    int pos[kSortFanIn], len[kSortFanIn];
 #pragma unroll
-    for (int u = 0; u < FANIN; u++) {
+    for (int u = 0; u < kSortFanIn; u++) {
         len[u] = max(0, min(run_len, gend - g0 - u * run_len));   // 0: no such run in this group
         pos[u] = 0;
     }
@@ -922,14 +969,14 @@ __device__ __forceinline__ void merge_far_of(const float *__restrict__ kin, cons
     const float kb = sort_below(k);
     for (int st = run_len >> 1; st > 0; st >>= 1) {
 #pragma unroll
-        for (int u = 0; u < FANIN; u++) {
+        for (int u = 0; u < kSortFanIn; u++) {
             const int at = pos[u] + st - 1;
             const float o = run[min(u * run_len + at, gend - g0 - 1)];
             pos[u] += (at < len[u] && o > (u < ri ? kb : k)) ? st : 0;   // runs that stood earlier win ties
         }
     }
 #pragma unroll
-    for (int u = 0; u < FANIN; u++) {
+    for (int u = 0; u < kSortFanIn; u++) {
         const float o = run[min(u * run_len + pos[u], gend - g0 - 1)];
         const int cnt = pos[u] + ((pos[u] < len[u] && o > (u < ri ? kb : k)) ? 1 : 0);
         rank += u != ri ? cnt : 0;
@@ -946,20 +993,84 @@ static __global__ void __launch_bounds__(256) k_merge_far(const float *__restric
     merge_far_of(kin, vin, npad, nout, run_len, group_len, kout, vout);
 }
 
-// The last merge of k_sort_tiles_b's sort (at most kSortFanIn runs of kSortRun pairs: padded n up to 65536): the runs of a
-// sequence into the other copy of its ProbIndex array, the keys read where they lie (32 sequences' keys fit the caches;
-// holding a sequence's keys in LDS as k_merge_runs does would leave one workgroup per compute unit).
-static __global__ void __launch_bounds__(256) k_merge_far_b(const SortBatch b, int npad, int nout)
+// How many of the keys a[0..n), which descend, are greater than k: sixteen parts at a time (n up to 65536), whose probes go out
+// together: four trips to memory instead of sixteen.
+__device__ __forceinline__ int count_greater(const float *__restrict__ a, int n, float k)
 {
-    const int s = blockIdx.z;
+    int pos = 0;
+#pragma unroll
+    for (int st = 4096; st > 0; st >>= 4) {
+        int c = 0;
+#pragma unroll
+        for (int m = 1; m < 16; m++) {
+            const int at = pos + m * st - 1;
+            const float o = a[min(at, n - 1)];
+            c += at < n && o > k ? 1 : 0;
+        }
+        pos += c * st;
+    }
+    return pos;
+}
+
+// The sorted runs of a sequence's candidates and what stood behind them, into the other copy of its ProbIndex array (candidates win
+// ties: they stood earlier).  A workgroup places 256 pairs: a candidate by its rank in its run, what stands before it in the other runs
+// and in the rest; a pair of the rest by how many candidates stand before it.  One run (up to 4096 candidates): its keys
+// in LDS.  grid (n / 256 rounded up, 1, sequences); n <= kSampleMaxVocab.
+static __global__ void __launch_bounds__(256) k_merge_old_b(const SortBatch b, int n)
+{
+    __shared__ __align__(16) float keys[kSortRun];
+    const int s = blockIdx.z, tid = threadIdx.x, i = blockIdx.x * 256 + tid;
     const bool cur = (b.cur >> s) & 1u;
     if (!((b.active >> s) & 1u)) return;
-    const float *kin = b.runs_k + s * b.sort_stride;
-    const int *vin = b.runs_v + s * b.sort_stride;
-    float *kout = (cur ? b.pi_prob0 : b.pi_prob1) + s * b.pi_stride;
-    int *vout = (cur ? b.pi_idx0 : b.pi_idx1) + s * b.pi_stride;
-    if (npad <= 8 * kSortRun) merge_far_of<8>(kin, vin, npad, nout, kSortRun, kSortRun * kSortFanIn, kout, vout);   // (eight searches per pair)
-    else merge_far_of<kSortFanIn>(kin, vin, npad, nout, kSortRun, kSortRun * kSortFanIn, kout, vout);
+    const int n0 = b.ss[s].n0, nruns = (n0 + kSortRun - 1) / kSortRun;
+    const float *old = (cur ? b.pi_prob1 : b.pi_prob0) + s * b.pi_stride, *runs = b.runs_k + s * b.sort_stride;
+    const int *old_idx = (cur ? b.pi_idx1 : b.pi_idx0) + s * b.pi_stride;
+    if (nruns == 1) {
+        for (int j = 4 * tid; j < n0; j += 1024) *reinterpret_cast<float4 *>(keys + j) = *reinterpret_cast<const float4 *>(runs + j);
+        __syncthreads();
+    }
+    if (i >= n) return;
+    const bool cand = i < n0;
+    const float k = cand ? runs[i] : old[i];
+    const int v = cand ? b.runs_v[s * b.sort_stride + i] : old_idx[i];
+    const float kb = sort_below(k);
+    const int ri = cand ? i / kSortRun : nruns;
+    int rank = i - (cand ? ri * kSortRun : n0);
+    if (nruns == 1) {
+        if (!cand) {
+            int pos = 0;
+#pragma unroll
+            for (int st = kSortRun / 2; st > 0; st >>= 1) {
+                const int at = pos + st - 1;
+                pos += at < n0 && keys[min(at, n0 - 1)] > kb ? st : 0;
+            }
+            rank += pos + (pos < n0 && keys[min(pos, n0 - 1)] > kb ? 1 : 0);
+        }
+    } else {
+        int pos[kSortMaxRuns], len[kSortMaxRuns];
+#pragma unroll
+        for (int r = 0; r < kSortMaxRuns; r++) { pos[r] = 0; len[r] = max(0, min(kSortRun, n0 - r * kSortRun)); }
+        for (int st = kSortRun / 2; st > 0; st >>= 1) {
+#pragma unroll
+            for (int r = 0; r < kSortMaxRuns; r++) {
+                if (r < nruns) {
+                    const int at = pos[r] + st - 1;
+                    const float o = runs[r * kSortRun + min(at, len[r] - 1)];
+                    pos[r] += at < len[r] && o > (r < ri ? kb : k) ? st : 0;   // runs that stood earlier win ties
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kSortMaxRuns; r++) {
+            if (r < nruns && r != ri) {
+                const float o = runs[r * kSortRun + min(pos[r], len[r] - 1)];
+                rank += pos[r] + (pos[r] < len[r] && o > (r < ri ? kb : k) ? 1 : 0);
+            }
+        }
+    }
+    if (cand && n0 < n) rank += count_greater(old + n0, n - n0, k);
+    (cur ? b.pi_prob0 : b.pi_prob1)[s * b.pi_stride + rank] = k;
+    (cur ? b.pi_idx0 : b.pi_idx1)[s * b.pi_stride + rank] = v;
 }
 
 // J/Sampler.java:46-57 on an array given by the caller: first index of the strict maximum.  One workgroup.

@@ -305,6 +305,27 @@ def test_sampled_batch_gives_every_sequence_its_own_sampler(orc, n_seq, t, topp,
     g.close()
 
 
+@pytest.mark.parametrize("vocab,spread", [(272, 4.0), (1008, 20.0), (4112, 0.3), (8208, 3.0), (32000, 5.0), (36864, 1.0)])
+def test_sampled_batch_merges_few_and_many_candidates_with_what_earlier_steps_left(orc, vocab, spread):
+    """Top-p steps whose candidates are one tile, one run (4096 pairs) or several of the sort, by the logits' spread: every token the one
+    that the oracle's sampler, which sorts its whole array, takes from the same logits."""
+    shape = SHAPES[0][:5] + (vocab,) + SHAPES[0][6:]
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(23, 0.02)
+    g.upload_f32_quantize(l2j.TENSOR.RMS_FINAL, np.full(shape[0], spread / (0.02 * shape[0] ** 0.5), dtype=np.float32))
+    g.finalize()
+    rng = np.random.default_rng(vocab)
+    prompts = [rng.integers(3, vocab, size=int(rng.integers(0, 5))).astype(np.int32) for _ in range(16)]
+    seeds = rng.integers(-2**40, 2**40, size=16).astype(np.int64)
+    for t, topp in ((0.9, 0.9), (1.4, 0.5)):
+        got, _, logits = g.decode_sample_batch(prompts, 12, t, topp, seeds, want_logits=True)
+        for b in range(16):
+            s = orc.Sampler(int(seeds[b]), vocab)
+            want = [int(prompts[b][pos]) if pos < len(prompts[b]) else s.step(logits[pos, b], t, topp)[0] for pos in range(12)]
+            np.testing.assert_array_equal(got[b], np.array(want, dtype=np.int32), err_msg="sequence %d" % b)
+    g.close()
+
+
 def test_sampled_batch_refuses_what_its_sampling_step_cannot_take():
     g = l2j.Transformer(l2j.Config(*SHAPES[3]))
     g.fill_synthetic(3, 0.02)
