@@ -92,7 +92,7 @@ WideWs wide_ws(l2j_ctx *c)
 size_t wide_lds_bytes(int n)
 {
     const size_t keys = (size_t)((n + kSortRun - 1) / kSortRun * kSortRun) * sizeof(float);
-    return std::max(keys, sizeof(WideWalk));
+    return std::max({keys, sizeof(WideWalk), sizeof(FewSort)});
 }
 
 int alloc_sampler(l2j_ctx *c)

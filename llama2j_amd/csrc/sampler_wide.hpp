@@ -9,6 +9,7 @@
 //      it needs, the sum of what stands before the slice, from fast exponentials of the logits the maximum was taken of)
 //   C  every workgroup walks the slices (the same walk everywhere: nobody waits for a result), divides its slice by
 //      the sum, writes the probabilities over the logits and flags its top-p candidates (J/Sampler.java:85-96)
+//   (with at most 768 candidates the rest is one workgroup's: few_sort, few_pick)
 //   D  the ProbIndex array of this call (candidates in index order, then what the last call left, which is sorted)
 //      taken tile by tile and every tile of 256 sorted by counting
 //   E  runs of 16 tiles merged by counting (binary searches in LDS), F all runs merged: Arrays.sort, stable, descending
@@ -101,13 +102,13 @@ __device__ __forceinline__ void wide_barrier(const WideWs &w, unsigned k)
         const unsigned old = __hip_atomic_fetch_add(&w.sync->group[grp].n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (old + 1u == gsize * (k + 1u)) __hip_atomic_fetch_add(&w.sync->ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned want = (k + 1u) * ng;
-        int spins = 0;
-        while (__hip_atomic_load(&w.sync->ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
-            __builtin_amdgcn_s_sleep(1);
-            if (++spins > w.maxspin || ((spins & 255) == 0 && ld_coh(&w.sync->fault) != 0)) {
+        for (int spins = 0;; spins++) {   // (a limit of 0 gives up before it looks, however close together the workgroups come)
+            if (spins >= w.maxspin || ((spins & 255) == 255 && ld_coh(&w.sync->fault) != 0)) {
                 st_coh(&w.sync->fault, 1);
                 break;
             }
+            if (__hip_atomic_load(&w.sync->ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want) break;
+            __builtin_amdgcn_s_sleep(1);
         }
     }
     __syncthreads();
@@ -590,8 +591,157 @@ __device__ __forceinline__ void wide_load_keys(float *keys, const float *src, in
     }
 }
 
+// ---- few candidates -------------------------------------------------------------------------------------------------------
+// A trained model's distribution leaves a few hundred candidates of 32000, which one workgroup sorts in LDS, puts together with the
+// front of what earlier calls left and picks from; the stages for any number (tiles, runs, all runs, two speculative walks) cost their
+// grid barriers whatever they hold: k_sample_wide with about 400 candidates of 32000 57.5 -> 37.8 us.  Up to 768: with 256, 512 and 1024
+// candidates, nearly all of whose sum the pick needs, 44, 54 and 69 us against 66 (up to 4000) to 76 (20000) for the stages.  (In the
+// batched step, behind k_sample_probs, it saves nothing: the launches for many candidates are made in any case.)
+constexpr int kFewMax = 768;
+
+struct FewSort {
+    float key[kFewMax];   // in: the candidates in index order; out: sorted
+    int val[kFewMax];
+    float tk[kFewMax];    // sorted tiles; then the front of the old array
+    int tv[kFewMax];
+    union {
+        unsigned long long k64[kFewMax];
+        struct { float mk[kFewMax]; int mv[kFewMax]; } m;   // the front of the merged array
+    };
+};
+
+// The candidates 0..n0 (at most kFewMax) sorted as Arrays.sort does, stable by descending probability: tiles of 256 by counting,
+// then every pair's place among the tiles.  All threads of the workgroup call, key and val published.
+__device__ __forceinline__ void few_sort(FewSort &f, int n0)
+{
+    const int tid = threadIdx.x, nt = kWideSlice, ntiles = (n0 + kSortTile - 1) / kSortTile, np = ntiles * kSortTile;
+    for (int c = tid; c < np; c += nt)   // (as sort_tiles_of: padding counts as probability 0 at a position behind all others)
+        f.k64[c] = ((unsigned long long)(c < n0 ? __float_as_uint(f.key[c]) : 0u) << 32) | (unsigned)(kSortTile - 1 - (c & (kSortTile - 1)));
+    __syncthreads();
+    for (int c = tid; c < np; c += nt) {
+        const unsigned long long mine = f.k64[c];
+        const ulonglong2 *k2 = reinterpret_cast<const ulonglong2 *>(&f.k64[c & ~(kSortTile - 1)]);
+        int rank = c & ~(kSortTile - 1);
+#pragma unroll 16
+        for (int j = 0; j < kSortTile / 2; j++) rank += (k2[j].x > mine) + (k2[j].y > mine);
+        f.tk[rank] = c < n0 ? f.key[c] : -1.0f;
+        f.tv[rank] = c < n0 ? f.val[c] : 0;
+    }
+    __syncthreads();
+    for (int c = tid; c < np; c += nt) {
+        const float k = f.tk[c], kb = sort_below(k);
+        const int v = f.tv[c], own = c / kSortTile;
+        int rank = c - own * kSortTile, pos[kFewMax / kSortTile];
+#pragma unroll
+        for (int t = 0; t < kFewMax / kSortTile; t++) pos[t] = 0;
+#pragma unroll
+        for (int st = kSortTile / 2; st > 0; st >>= 1) {
+#pragma unroll
+            for (int t = 0; t < kFewMax / kSortTile; t++)
+                if (t < ntiles) pos[t] += f.tk[t * kSortTile + pos[t] + st - 1] > (t < own ? kb : k) ? st : 0;   // tiles that stood earlier win ties
+        }
+#pragma unroll
+        for (int t = 0; t < kFewMax / kSortTile; t++)
+            if (t < ntiles && t != own) rank += pos[t] + (f.tk[t * kSortTile + pos[t]] > (t < own ? kb : k) ? 1 : 0);
+        if (k >= 0.0f) { f.key[rank] = k; f.val[rank] = v; }   // (the padding, -1, stands behind all candidates)
+    }
+    __syncthreads();
+}
+
+// How many of the n > 0 keys in LDS, which descend, are greater than each k (n up to kFewMax); the searches advance together.
+template <int N>
+__device__ __forceinline__ void few_greater(const float *keys, int n, const float (&k)[N], int (&pos)[N])
+{
+#pragma unroll
+    for (int q = 0; q < N; q++) pos[q] = 0;
+#pragma unroll
+    for (int st = 512; st > 0; st >>= 1) {   // (sums to 1023)
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const int at = pos[q] + st - 1;
+            pos[q] += at < n && keys[min(at, n - 1)] > k[q] ? st : 0;
+        }
+    }
+}
+
+// J/Sampler.java:99-119 behind few_sort: old[n0..n) is what earlier calls left, sorted (candidates win ties: they stood earlier).  The
+// sums of the first n0 pairs of the merged array, added one after the other; the first that exceeds topp, or the last, is the cumulative
+// probability, r = coin * that, the pick the first pair whose sum exceeds r.  All threads call; returns the token (wave 0).
+// coin < 0: the generator draws.
+__device__ __forceinline__ int few_pick(FewSort &f, int n0, const float *old, const int *old_idx, int n, float topp, float coin, unsigned long long *rng)
+{
+    const int tid = threadIdx.x, lane = tid & 63, nold = min(n0, n - n0);   // (an old pair further back stands behind n0 others)
+    for (int j = tid; j < nold; j += kWideSlice) { f.tk[j] = old[n0 + j]; f.tv[j] = old_idx[n0 + j]; }
+    __syncthreads();
+    constexpr int Q = kFewMax / kWideSlice;
+    float kc[Q], ko[Q], kb[Q];
+    int pc[Q], po[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        kc[q] = f.key[min(tid + q * kWideSlice, n0 - 1)];
+        ko[q] = nold > 0 ? f.tk[min(tid + q * kWideSlice, nold - 1)] : 0.0f;
+        kb[q] = sort_below(ko[q]);
+        pc[q] = 0;
+    }
+    if (nold > 0) few_greater<Q>(f.tk, nold, kc, pc);
+    few_greater<Q>(f.key, n0, kb, po);
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int c = tid + q * kWideSlice;
+        if (c < n0 && c + pc[q] < n0) { f.m.mk[c + pc[q]] = kc[q]; f.m.mv[c + pc[q]] = f.val[c]; }
+        if (c < nold && c + po[q] < n0) { f.m.mk[c + po[q]] = ko[q]; f.m.mv[c + po[q]] = f.tv[c]; }
+    }
+    __syncthreads();
+    if (tid >= 64) return 0;
+    // (a block of 64 at a time, its terms taken from the lanes; lane b keeps the sum before block b)
+    auto block = [&](int b) { return 64 * b + lane < n0 ? f.m.mk[64 * b + lane] : 0.0f; };
+    auto term = [](float v, int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i)); };
+    auto sums = [&](float F, float v) {   // the running sum up to and including this lane's term
+        float pre = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 64; i++) {
+            F = __fadd_rn(F, term(v, i));
+            pre = lane == i ? F : pre;
+        }
+        return pre;
+    };
+    float F = 0.0f, starts = __builtin_inff(), cum;
+    int last = n0 - 1, b = 0;
+    while (true) {
+        starts = lane == b ? F : starts;
+        const float v = block(b);
+        float end = F;
+#pragma unroll
+        for (int i = 0; i < 64; i++) end = __fadd_rn(end, term(v, i));
+        if (end > topp) {
+            const float pre = sums(F, v);
+            const int i = __ffsll((long long)__ballot(pre > topp)) - 1;   // (a zero behind the last term exceeds nothing first)
+            last = 64 * b + i;
+            cum = term(pre, i);
+            break;
+        }
+        F = end;
+        if (64 * (b + 1) >= n0) {   // never exceeded: all candidates, cumulative_prob = their sum
+            cum = F;
+            break;
+        }
+        b++;
+    }
+    float c = coin;
+    if (c < 0.0f) {
+        if (lane == 0) c = java_next_float(rng);
+        c = spec_uniform(c);
+    }
+    const float r = __fmul_rn(c, cum);
+    b = __popcll(__ballot(starts <= r)) - 1;   // (the sums never fall: the block in which they pass r; r < 0 does not occur)
+    const float pre = sums(term(starts, b), block(b));
+    const unsigned long long hit = __ballot(64 * b + lane <= last && pre > r);
+    const int pick = hit ? 64 * b + __ffsll((long long)hit) - 1 : last;
+    return f.m.mv[pick];
+}
+
 // grid: ceil(n / 256) workgroups of 256 threads, all resident at once (n <= kSampleMaxVocab: at most 144); dynamic LDS:
-// max(sizeof(WideWalk), 4 bytes per key of the array padded to whole runs of 4096).
+// max(sizeof(WideWalk), sizeof(FewSort), 4 bytes per key of the array padded to whole runs of 4096).
 static __global__ void __launch_bounds__(kWideSlice) k_sample_wide(const WideArgs a)
 {
     extern __shared__ __align__(16) unsigned char wide_lds[];
@@ -733,15 +883,77 @@ static __global__ void __launch_bounds__(kWideSlice) k_sample_wide(const WideArg
         wide_leave(a.w, a.ss);
         return;
     }
+    auto candidate = [&](int c) {   // the token of candidate c
+        int h = 0;   // the slice of candidate c: the last h with cp[h] <= c
+        for (int st = 128; st > 0; st >>= 1)
+            if (h + st < G && cp[h + st] <= c) h += st;
+        const unsigned long long cm[4] = {cmw[4 * h], cmw[4 * h + 1], cmw[4 * h + 2], cmw[4 * h + 3]};
+        return min(h * kWideSlice + wide_kth_bit(cm, c - cp[h]), n - 1);
+    };
+    if (n0 <= kFewMax) {
+        // Few candidates: no stage waits for another from here on.  Every workgroup whose part of the array may move (the first ones)
+        // sorts them for itself and places its part; workgroup 0 has picked before it does.
+        FewSort &f = *reinterpret_cast<FewSort *>(wide_lds);
+        float ko = 0.0f, kmin = __builtin_inff();
+        int vo = 0;
+        if (i >= n0 && i < n) { ko = a.old_prob[i]; vo = a.old_idx[i]; }
+        __syncthreads();   // (the walk's LDS is free)
+        constexpr int Q = kFewMax / kWideSlice;
+        float key[Q];
+        int val[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (q * kWideSlice < n0) val[q] = candidate(min(tid + q * kWideSlice, n0 - 1));
+#pragma unroll
+        for (int q = 0; q < Q; q++)   // (the loads in flight together)
+            if (q * kWideSlice < n0) key[q] = ld_coh(a.logits + val[q]);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int c = tid + q * kWideSlice;
+            if (c < n0) {
+                f.key[c] = key[q]; f.val[c] = val[q];
+                kmin = fminf(kmin, key[q]);
+            }
+        }
+        kmin = -block_max(-kmin, red);
+        const int first = g * kWideSlice;
+        if (first >= n0 && (first >= n || a.old_prob[first] < kmin)) {   // what stands here stands behind all candidates
+            if (i < n) { a.new_prob[i] = ko; a.new_idx[i] = vo; }
+            wide_leave(a.w, a.ss);
+            return;
+        }
+        few_sort(f, n0);
+        if (g == 0) {
+            const int token = few_pick(f, n0, a.old_prob, a.old_idx, n, a.topp, a.coin, &a.ss->rng);
+            if (tid == 0) {
+                a.ss->result = token;
+                loop_result(a, token);
+            }
+        }
+        if (i < n) {
+            const bool cand = i < n0;
+            const float k = cand ? f.key[i] : ko;
+            const int v = cand ? f.val[i] : vo;
+            int rank = i;
+            if (cand) {
+                if (n0 < n) rank += count_greater(a.old_prob + n0, n - n0, k);
+            } else {
+                const float kb[1] = {sort_below(k)};
+                int pos[1];
+                few_greater<1>(f.key, n0, kb, pos);
+                rank += pos[0] - n0;
+            }
+            a.new_prob[rank] = k;
+            a.new_idx[rank] = v;
+        }
+        wide_leave(a.w, a.ss);
+        return;
+    }
     {
         float key = -1.0f;
         int val = 0;
         if (i < n0) {
-            int h = 0;   // the slice of candidate i: the last h with cp[h] <= i
-            for (int st = 128; st > 0; st >>= 1)
-                if (h + st < G && cp[h + st] <= i) h += st;
-            const unsigned long long cm[4] = {cmw[4 * h], cmw[4 * h + 1], cmw[4 * h + 2], cmw[4 * h + 3]};
-            val = min(h * kWideSlice + wide_kth_bit(cm, i - cp[h]), n - 1);
+            val = candidate(i);
             key = ld_coh(a.logits + val);
         } else if (i < n) {
             key = a.old_prob[i];

@@ -112,6 +112,27 @@ def test_vocabularies_at_the_edges_of_slices_tiles_and_runs(orc, monkeypatch, vo
         check_probabilities(g.read(BUFFER.LOGITS), probs)
 
 
+@WIDE
+@pytest.mark.parametrize("vocab", [768, 5000, 36864])
+def test_topp_with_few_candidates_at_the_edges_of_tiles_and_of_what_one_workgroup_takes(orc, monkeypatch, vocab, wide):
+    """Up to 768 candidates are sorted, merged and picked from by one workgroup: one, a tile of 256, one more, the most it takes and one
+    more, with ties among them and with what calls of more and of fewer candidates left."""
+    monkeypatch.setenv("L2J_SAMPLER_WIDE", wide)
+    g = small_transformer(vocab)
+    rng = np.random.default_rng(vocab + 31)
+    g.sampler_seed(9)
+    o = orc.Sampler(9, vocab)
+    for call, k in enumerate([1, 255, 256, 257, 767, 768, 769, 3, 3000, 400, 64, 65, 768, 1, 511, 512, 513, 1024, 130]):
+        k = min(k, vocab)
+        lg = np.full(vocab, -40.0, dtype=np.float32)
+        lg[rng.permutation(vocab)[:k]] = (np.round(rng.random(k) * 16) / 8).astype(np.float32)
+        t, topp = float(rng.choice([0.8, 1.0])), float(rng.choice([0.3, 0.9, 0.99]))
+        want, probs = o.step(lg, t, topp)
+        assert g.sample(t, topp, logits=lg) == want, (call, k, topp)
+        check_probabilities(g.read(BUFFER.LOGITS), probs)
+    g.close()
+
+
 def test_topp_worked_example_with_entries_of_an_earlier_call(orc):
     # the hand-worked case of the oracle's tests, on the device: eight tokens, padded with impossible ones
     vocab = 16
