@@ -210,20 +210,18 @@ __device__ constexpr int dg_block(int u, int nu, int j) { return u == 0 && j < 8
 // matrix instructions; without the codes' loads 0.9 of the time, without the digits' 0.95.  Tried, no faster: codes a whole group ahead in
 // a second set of registers (32 vectors: 3 % slower, it is bound by the codes' way through L2), workgroups that go on to
 // another tile instead of ending, sums stored four rows at a time by way of LDS.
-template <int PT, int NW>
-__global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
+// dgemm_tile: the vectors' tile `col`, rows and slice `tile` of the launch.  NU: units of 16 vectors, 2 PT, or 1 of a tile of 32 whose second
+// half is empty.  (The argument by value: behind a reference the addresses came out in vector registers.)
+template <int PT, int NW, int NU>
+__device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile, int col)
 {
-    extern __shared__ __align__(16) v4i dg_lds[];
     constexpr int STAGE = PT * kDigitBytes / 16;            // 16-byte words of a group's digits
-    constexpr int NT = 64 * NW, NST = STAGE / NT, NU = 2 * PT;   // words a thread stages per group; units of 16 vectors
+    constexpr int NT = 64 * NW, NST = STAGE / NT * NU / (2 * PT);   // words a thread stages per group
     float *lsx = reinterpret_cast<float *>(dg_lds + 2 * STAGE);   // [2][32 PT]
+    constexpr int RUN = NU == 2 * PT ? 64 : 128;             // the wave's q-th run of 64 words begins at (q NW + wave) RUN (one unit: the runs of the tile's first half)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
-    // The workgroups of an XCD (blockIdx % 8) take the same rows of the matrix against all vectors, one after the other.
-    const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
-    const int tile = (i / a.ncol) * 8 + xcd, col = i % a.ncol;    // (tile: of rows and slices)
     const int nslice = (a.ngroups + a.gps - 1) / a.gps;
-    if (tile >= a.nrow * nslice) return;
-    const int rt = tile / nslice, slice = tile % nslice;
+    const int rt = __builtin_amdgcn_readfirstlane(tile / nslice), slice = tile - rt * nslice;
     const int g0 = slice * a.gps, g1 = min(g0 + a.gps, a.ngroups);
     // The wave's 64 rows lie in one matrix (with several matrices: rows % 64 == 0): its address is uniform.  (Rows past the
     // matrix's last tile of 16 repeat that tile and are not stored.)
@@ -240,7 +238,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
         cp[r] = cm + blk * 4096;
         sp[r] = sm + blk * 16;
     }
-    unsigned co = lane * 16, n8 = n * 8, tid16 = tid * 16;
+    unsigned co = lane * 16, n8 = n * 8, stage16 = (wave * RUN + lane) * 16;
     const v4i *xd = reinterpret_cast<const v4i *>(a.x.d) + ((size_t)col * PT * a.ngroups + g0) * (kDigitBytes / 16);
     const size_t xstep = (size_t)a.ngroups * (kDigitBytes / 16);   // 16-byte words between two tiles of vectors
     const float *xs = a.x.sx + ((size_t)col * PT * a.ngroups + g0) * 32;
@@ -258,12 +256,12 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
     {
         v4i st[NST];
 #pragma unroll
-        for (int q = 0; q < NST; q++) st[q] = (xd + (q * NT / 2048) * xstep + q * NT % 2048)[(unsigned)tid];
+        for (int q = 0; q < NST; q++) st[q] = (xd + (q * NW * RUN / 2048) * xstep + q * NW * RUN % 2048)[stage16 / 16];
         sx0 = load_at<float>(xs, xso);
 #pragma unroll
         for (int r = 0; r < 4; r++) rm[r] = load_at<float>(sp[r], n8);
 #pragma unroll
-        for (int q = 0; q < NST; q++) dg_lds[q * NT + tid] = st[q];
+        for (int q = 0; q < NST; q++) dg_lds[(q * NW + wave) * RUN + lane] = st[q];
     }
     // the groups' offsets times the sums of the activations: fp32 matrix cores, four groups at a time
     v4f f0[NU][4];
@@ -354,9 +352,9 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
         // 16 bytes follow each other).  Nothing the compiler counts: they come behind the codes of this group, which it waits for one by one,
         // and are waited for below.
         auto stage = [&](int q) __attribute__((always_inline)) {
-            const v4i *from = xn + (q * NT / 2048) * xstep + q * NT % 2048;
-            const unsigned to = lds0 + (((g + 1) & 1) * STAGE + q * NT + wave * 64) * 16;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(tid16), "s"(from) : "memory");
+            const v4i *from = xn + (q * NW * RUN / 2048) * xstep + q * NW * RUN % 2048;
+            const unsigned to = lds0 + (((g + 1) & 1) * STAGE + q * NW * RUN + wave * RUN) * 16;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(stage16), "s"(from) : "memory");
         };
         v4i x[4];   // fragments, three ahead of their use
         auto fragment = [&](int u, int j) __attribute__((always_inline)) {
@@ -374,15 +372,15 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
             const v4f sx = *reinterpret_cast<const v4f *>(csx + 16 * u + 4 * s4);
             unroll<16>([&](auto jc) __attribute__((always_inline)) {
                 constexpr int j = jc.value, d = dg_digit(u, NU, j), T = dg_block(u, NU, j), at = 16 * u + j;
-                constexpr int per = (NST + NU - 2) / (NU - 1);   // words staged in a unit behind the first
-                if constexpr (u > 0 && j < per && (u - 1) * per + j < NST) stage((u - 1) * per + j);
+                constexpr int u1 = NU > 1 ? 1 : 0, per = (NST + NU - 1 - u1) / (NU - u1);   // words staged in a unit behind the first (of one: in it)
+                if constexpr (u >= u1 && j < per && (u - u1) * per + j < NST) stage((u - u1) * per + j);
                 if constexpr (at + 3 < 16 * NU) x[(at + 3) & 3] = fragment((at + 3) >> 4, (at + 3) & 15);
                 unroll<4>([&](auto rc) __attribute__((always_inline)) {
                     constexpr int r = rc.value, i = 4 * j + r;
                     v4i &acc = (d & 2) ? lo[k][r] : hi[k][r];
                     acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[at & 3], cw[r][T], !(d & 1) && T == 0 ? v4i{0, 0, 0, 0} : acc, 0, 0, 0);
-                    // beside it the unit before, and the shifts between the digits of a pair
-                    constexpr int o = i < 16 ? 2 * i : 16 + i;
+                    // beside it the unit before (one unit: nothing, its sums are added up behind it), and the shifts between the digits of a pair
+                    constexpr int o = NU == 1 ? 80 : i < 16 ? 2 * i : 16 + i;
                     add_up(std::integral_constant<int, o>{}, Before{}, sxp, u == 0 ? rmp : rm);
                     if constexpr (i < 16) add_up(std::integral_constant<int, o + 1>{}, Before{}, sxp, u == 0 ? rmp : rm);
                     if constexpr (u == 0 && j == 7) hi[k][r] <<= 8;
@@ -399,20 +397,21 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
             sxp = sx;
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (NU == 1) unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, 0>{}, sxp, rm); });
 #pragma unroll
         for (int r = 0; r < 4; r++) { rmp[r] = rm[r]; rm[r] = rmn[r]; }
         lsx[((g + 1) & 1) * 32 * PT + xt] = keep(nsx);
         asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // (the staged digits: all but the sixteen loads of codes behind them)
         __syncthreads();
     }
-    unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
+    if constexpr (NU > 1) unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
     const int ldo = 16 * a.ntiles;
     const float down = up == 1.0f ? 1.0f : 0x1p-48f;
 #pragma unroll
     for (int u = 0; u < NU; u++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int pos = (col * NU + u) * 16 + 4 * s4 + e;
+            const int pos = (col * 2 * PT + u) * 16 + 4 * s4 + e;
             if (pos < a.npos) {
                 float *o = a.out + ((size_t)slice * a.npos + pos) * ldo;
 #pragma unroll
@@ -420,6 +419,22 @@ __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
                     if (row0 + 16 * r + n < ldo) o[row0 + 16 * r + n] = f[u][r][e] * down;
             }
         }
+}
+
+// Of a last tile of 32 vectors whose second half is empty only the first unit is multiplied, and staged: a third of the work at 77 vectors
+// had been for padding.  Wq+Wk+Wv, Wo, W1+W3, W2 of the 7B shape, us, 40 vectors 24.7 10.7 37 22.0 -> 22.3 10.2 36 19.5, 77 vectors 28.3 13.7 48.4
+// 27.5 -> 27.1 13.3 44.3 24.9, 144 vectors 37.4 17.5 66.6 37.9 -> 34.4 17.6 59.5 34.6.  (The launches are picked as for whole tiles:
+// within 2.3 % of the best on average; an estimate with half a tile in it does worse.)
+template <int PT, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)
+{
+    extern __shared__ __align__(16) v4i dg_lds[];
+    // The workgroups of an XCD (blockIdx % 8) take the same rows of the matrix against all vectors, one after the other.
+    const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const int row = __builtin_amdgcn_readfirstlane(i / a.ncol), tile = row * 8 + xcd, col = i - row * a.ncol;    // (tile: of rows and slices)
+    if (tile >= a.nrow * ((a.ngroups + a.gps - 1) / a.gps)) return;
+    if (PT == 1 && a.npos - 32 * col <= 16) dgemm_tile<PT, NW, PT == 1 ? 1 : 2 * PT>(a, dg_lds, tile, col);
+    else dgemm_tile<PT, NW, 2 * PT>(a, dg_lds, tile, col);
 }
 
 // ---- at most 32 vectors: a decode step of a batch ---------------------------------------------------------------------
