@@ -457,12 +457,16 @@ template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (s
 template <int NB, int TILES>
 static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
 {
-    constexpr int NT = 2;   // blocks of 64 k per wave
+    // Of 32 vectors and one tile a workgroup (the products of the 110M shape) a wave takes half, against the whole group: half as many sums to
+    // convert and to add up, for codes that two waves request (steps of 24 and 32 sequences of the 110M shape 482 and 476 -> 466 and 462 us; with more tiles, where the
+    // codes' way from memory is the bound, 70B widths 1205 -> 1295).
+    constexpr bool WHOLE = NB == 2 && TILES == 1;
+    constexpr int NT = WHOLE ? 4 : 2, MT = WHOLE ? 1 : NB, PARTS = WHOLE ? kStreamGroups : kStreamWaves;   // blocks of 64 k and of 16 vectors per wave, sums of a tile to be added up
     extern __shared__ __align__(16) float ds_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
     const int slice = blockIdx.y, g0 = slice * a.gps, ng = min(a.gps, a.ngroups - g0);
     const bool on = wave < 2 * ng;       // (a wave without a group multiplies the slice's last one by zero scales: no branch around loads)
-    const int g = g0 + min(wave >> 1, ng - 1), hf = wave & 1, ntile = a.ntiles >> 1, step = gridDim.x;
+    const int g = g0 + min(wave >> 1, ng - 1), hf = WHOLE ? 0 : wave & 1, m0 = WHOLE ? wave & 1 : 0, ntile = a.ntiles >> 1, step = gridDim.x;
     // this wave's k of the first tile of the first matrix, and how far from there the others lie (differences of addresses:
     // a choice between pointers would turn the loads into flat ones)
     const uint8_t *cb = a.codes[0] + (size_t)g * 4096 + 1024 * NT * hf;
@@ -496,33 +500,35 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
         asm volatile("" : "+s"(p0), "+s"(p1), "+v"(lane16));
 #pragma unroll
         for (int T = 0; T < NT; T++) {
-            c.w[0][T] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) v4i *>(p0 + lane16 + 1024 * T));
-            c.w[1][T] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) v4i *>(p1 + lane16 + 1024 * T));
+            typedef const __attribute__((address_space(1))) v4i *Words;
+            const Words w0 = reinterpret_cast<Words>(p0 + lane16 + 1024 * T), w1 = reinterpret_cast<Words>(p1 + lane16 + 1024 * T);
+            c.w[0][T] = WHOLE ? *w0 : __builtin_nontemporal_load(w0);   // (WHOLE: the other wave finds them in the cache)
+            c.w[1][T] = WHOLE ? *w1 : __builtin_nontemporal_load(w1);
         }
     };
 
     Codes c0, c1;
     const int t0 = blockIdx.x;
-    v4i dg[4][NB][NT];
+    v4i dg[4][MT][NT];
     {
-        const v4i *xp = reinterpret_cast<const v4i *>(a.x.d) + (size_t)g * (kDigitBytes / 16) + hf * NT * 128;
+        const v4i *xp = reinterpret_cast<const v4i *>(a.x.d) + (size_t)g * (kDigitBytes / 16) + hf * NT * 128 + m0 * 64;
 #pragma unroll
         for (int d = 0; d < 4; d++)
 #pragma unroll
             for (int T = 0; T < NT; T++)
 #pragma unroll
-                for (int mt = 0; mt < NB; mt++) dg[d][mt][T] = (xp + ((d * 4 + T) * 2 + mt) * 64)[(unsigned)lane];
+                for (int mt = 0; mt < MT; mt++) dg[d][mt][T] = (xp + ((d * 4 + T) * 2 + mt) * 64)[(unsigned)lane];
     }
     // The digits first: a wave's loads return in order, and the first tile needs all of the digits but only its own codes.  (Codes first: a step
     // of 16 and 32 sequences of the 110M shape 440 and 482 us for 411 and 476, of the 7B shape 2406 and 2910 for 2356 and 2885.)
     __builtin_amdgcn_sched_barrier(0);
     request(t0, c0);
     __builtin_amdgcn_sched_barrier(0);
-    v4f sx[NB], sm[NB];
+    v4f sx[MT], sm[MT];
 #pragma unroll
-    for (int mt = 0; mt < NB; mt++) {
-        sx[mt] = *reinterpret_cast<const v4f *>(a.x.sx + (size_t)g * 32 + 16 * mt + 4 * s4);
-        sm[mt] = *reinterpret_cast<const v4f *>(a.x.sum + (size_t)g * 32 + 16 * mt + 4 * s4);
+    for (int mt = 0; mt < MT; mt++) {
+        sx[mt] = *reinterpret_cast<const v4f *>(a.x.sx + (size_t)g * 32 + 16 * (m0 + mt) + 4 * s4);
+        sm[mt] = *reinterpret_cast<const v4f *>(a.x.sum + (size_t)g * 32 + 16 * (m0 + mt) + 4 * s4);
         if (!on) sx[mt] = v4f{0.f, 0.f, 0.f, 0.f};
         if (!on || hf) sm[mt] = v4f{0.f, 0.f, 0.f, 0.f};   // (the group's offset: by the first of its waves)
     }
@@ -530,9 +536,9 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     float *out = a.out + (size_t)slice * a.npos * ldo;
 
     auto tile = [&](int buf, const Codes &c) {
-        float *red = ds_lds + buf * kStreamWaves * NB * 512;
+        float *red = ds_lds + buf * PARTS * NB * 512;
 #pragma unroll
-        for (int mt = 0; mt < NB; mt++)
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 v4i hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
@@ -551,15 +557,15 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
 #pragma unroll
                 for (int e = 0; e < 4; e++)   // (the power of two into the sum, which takes it exactly: times the scale a small one would lose bits)
                     y[e] = fmaf(fmaf((float)hi[e], 65536.0f, (float)lo[e]) * sx[mt][e], c.s[r].x, c.s[r].y * sm[mt][e]);
-                *reinterpret_cast<v4f *>(red + (((wave * NB + mt) * 2 + r) * 64 + lane) * 4) = y;
+                *reinterpret_cast<v4f *>(red + (((wave * MT + mt) * 2 + r) * 64 + lane) * 4) = y;
             }
     };
     // the tile's sums: NB x 2 blocks of 64 lanes x 4: NB values per thread
-    struct Sums { float v[kStreamWaves][NB]; };
+    struct Sums { float v[PARTS][NB]; };
     auto read = [&](int buf, Sums &u) {
-        const float *red = ds_lds + buf * kStreamWaves * NB * 512 + tid * NB;
+        const float *red = ds_lds + buf * PARTS * NB * 512 + tid * NB;
 #pragma unroll
-        for (int w = 0; w < kStreamWaves; w++)
+        for (int w = 0; w < PARTS; w++)
 #pragma unroll
             for (int k = 0; k < NB; k++) u.v[w][k] = red[w * NB * 512 + k];
     };
@@ -571,7 +577,7 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
         for (int k = 0; k < NB; k++) {
             float y = u.v[0][k];
 #pragma unroll
-            for (int w = 1; w < kStreamWaves; w++) y += u.v[w][k];
+            for (int w = 1; w < PARTS; w++) y += u.v[w][k];
             if (row + k < a.npos) o[(size_t)k * ldo] = y;
         }
     };
