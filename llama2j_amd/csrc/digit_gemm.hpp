@@ -42,8 +42,8 @@ __device__ __forceinline__ int digit_shift(unsigned amax, float *inv)
     return s;
 }
 
-// Sixteen consecutive activations of one vector (k = 16 c .. 16 c + 15 of group g) as digits; s: the group's exponent.
-__device__ __forceinline__ void store_digits(const Digits &o, int row, int ngroups, int g, int c, const float (&v)[16], int s)
+// Sixteen consecutive activations of a vector as digits, x[d] their digits d (0: the most significant); s: the group's exponent.
+__device__ __forceinline__ void make_digits(const float (&v)[16], int s, v4i (&x)[4])
 {
     unsigned w[16];
 #pragma unroll
@@ -52,18 +52,25 @@ __device__ __forceinline__ void store_digits(const Digits &o, int row, int ngrou
         const int q = (int)rintf(ldexpf(v[i], s));
         w[i] = ((unsigned)q + 0x80808080u) ^ 0x80808080u;   // byte d: digit d, -128 .. 127
     }
-    uint4 *p = o.d + ((size_t)(row >> 5) * ngroups + g) * (kDigitBytes / 16) + (2 * (c >> 2) + ((row >> 4) & 1)) * 64 + (row & 15) + 16 * (c & 3);
 #pragma unroll
     for (int d = 0; d < 4; d++) {   // byte 3 - d of every word
-        unsigned t[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const unsigned sel = 0x0c0c0400u + (unsigned)((3 - d) * 0x0101u);
             const unsigned lo = __builtin_amdgcn_perm(w[4 * i + 1], w[4 * i], sel), hi = __builtin_amdgcn_perm(w[4 * i + 3], w[4 * i + 2], sel);
-            t[i] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+            x[d][i] = (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
         }
-        p[d * 8 * 64] = make_uint4(t[0], t[1], t[2], t[3]);
     }
+}
+
+// Those of vector `row`, k = 16 c .. 16 c + 15 of group g, to their place.
+__device__ __forceinline__ void store_digits(const Digits &o, int row, int ngroups, int g, int c, const float (&v)[16], int s)
+{
+    v4i x[4];
+    make_digits(v, s, x);
+    v4i *p = reinterpret_cast<v4i *>(o.d) + ((size_t)(row >> 5) * ngroups + g) * (kDigitBytes / 16) + (2 * (c >> 2) + ((row >> 4) & 1)) * 64 + (row & 15) + 16 * (c & 3);
+#pragma unroll
+    for (int d = 0; d < 4; d++) p[d * 8 * 64] = x[d];
 }
 
 // max and sum over the sixteen lanes that hold a group (lanes 16 n .. 16 n + 15)
@@ -169,6 +176,8 @@ struct DGemm {
     int npos;                  // vectors
     float *out;                // (slice, npos, 16 * ntiles)
     int ncol, nrow;            // tiles of the grid: vectors, matrix rows
+    const float *silu;         // k_dstream with SwiGLU: the sigmoid table, and whether to do without it
+    int exact;
 };
 
 constexpr int kDgWaveRows = 64;   // matrix rows per wave
@@ -454,7 +463,9 @@ template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (s
 // loop to fetch.  Two, up to 16 vectors: no third request, which the loop makes for nothing (Wo of the 7B shape 6.9 -> 6.45 us,
 // 24 steps of 16 sequences 52.5 -> 52.0 ms).
 // Workgroup (blockIdx.x, slice blockIdx.y) of gridDim.x per slice: every gridDim.x-th tile of 32 rows (rows % 32 == 0).
-template <int NB, int TILES>
+// SWIGLU (one tile, one slice, matrices W1 and W3): a tile is 16 rows of W1 and the same rows of W3, and out is (npos, hidden):
+// silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74).
+template <int NB, int TILES, bool SWIGLU = false>
 static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
 {
     // Of 32 vectors and one tile a workgroup (the products of the 110M shape) a wave takes half, against the whole group: half as many sums to
@@ -479,11 +490,11 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     struct Codes { v4i w[2][NT]; float2 s[2]; };
     // the codes of this wave's k of tile t (past the end: the last tile again, not used), and the rows' scales
     auto request = [&](int t, Codes &c) {
-        t = 2 * min(t, ntile - 1);
+        t = (SWIGLU ? 1 : 2) * min(t, ntile - 1);
         long cd = 0, sd = 0;
-        if (t >= nt0) { t -= nt0; cd = cd1; sd = sd1; if (t >= nt1) { t -= nt1; cd = cd2; sd = sd2; } }
+        if (!SWIGLU && t >= nt0) { t -= nt0; cd = cd1; sd = sd1; if (t >= nt1) { t -= nt1; cd = cd2; sd = sd2; } }
 #pragma unroll
-        for (int r = 0; r < 2; r++) c.s[r] = (sb + ((long)(t + r) * a.ngroups * 16 + sd))[n];
+        for (int r = 0; r < 2; r++) c.s[r] = (sb + (SWIGLU ? (long)t * a.ngroups * 16 + r * sd1 : (long)(t + r) * a.ngroups * 16 + sd))[n];
         // Up to 16 vectors leave the registers for addresses, and scalar ones take longer to form: W1 and W3, W2, Wq Wk Wv and Wo (mean) of the
         // 7B shape 19.2 -> 18.6, 12.3 -> 11.9, 10.0 -> 9.8 us this way.
         if constexpr (NB == 1) {
@@ -491,12 +502,12 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
             for (int T = 0; T < NT; T++)
 #pragma unroll
                 for (int r = 0; r < 2; r++)
-                    c.w[r][T] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(cb + ((long)(t + r) * a.ngroups * 4096 + cd) + 1024 * T + (unsigned)lane * 16));
+                    c.w[r][T] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(cb + (SWIGLU ? (long)t * a.ngroups * 4096 + r * cd1 : (long)(t + r) * a.ngroups * 4096 + cd) + 1024 * T + (unsigned)lane * 16));
             return;
         }
         // (scalar bases and one register of offsets: addresses formed in vector registers took those of the codes two tiles on, and
         // every request waited for all codes under way)
-        CodePtr p0 = (CodePtr)(cb + ((long)t * a.ngroups * 4096 + cd)), p1 = (CodePtr)(cb + ((long)(t + 1) * a.ngroups * 4096 + cd));
+        CodePtr p0 = (CodePtr)(cb + ((long)t * a.ngroups * 4096 + cd)), p1 = (CodePtr)(cb + (SWIGLU ? (long)t * a.ngroups * 4096 + cd1 : (long)(t + 1) * a.ngroups * 4096 + cd));
         asm volatile("" : "+s"(p0), "+s"(p1), "+v"(lane16));
 #pragma unroll
         for (int T = 0; T < NT; T++) {
@@ -583,6 +594,24 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     };
     Sums u;
     int t = t0;
+    if constexpr (SWIGLU) {
+        static_assert(TILES == 1);
+        tile(0, c0);
+        __syncthreads();
+        // thread: vectors and lane of a block of W1 and of the one of W3 beside it
+        const int row = 16 * (tid >> 8) + 4 * ((tid >> 6) & 3) + (tid & 3), col = (tid >> 2) & 15;
+        if (tid < 256 * NB && row < a.npos) {
+            const float *red = ds_lds + (tid >> 8) * 512 + (tid & 255);
+            float h1 = red[0], h3 = red[256];
+#pragma unroll
+            for (int w = 1; w < PARTS; w++) {
+                h1 += red[w * NB * 512];
+                h3 += red[w * NB * 512 + 256];
+            }
+            a.out[(size_t)row * 16 * ntile + 16 * t + col] = __fmul_rn(h1, __fmul_rn(silu_sigma(a.silu, h1, a.exact), h3));
+        }
+        return;
+    }
     if constexpr (TILES == 1) {
         tile(0, c0);
         __syncthreads();

@@ -350,9 +350,7 @@ void launch_batch_step(l2j_ctx *c, BatchBufs &b)
         n.slices = launch_dgemm(c, {L2J_WO}, l, b.r.dig, nseq, b.r.part);
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, nseq);
-        const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, l, b.r.dig, nseq, b.r.part);
-        launch_swiglu(c, b.r.part, s13, b.r.dig, nseq);
-        n.slices = launch_dgemm(c, {L2J_W2}, l, b.r.dig, nseq, b.r.part);
+        n.slices = launch_ffn(c, l, b.r, nseq);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         n.w = c->rmsw + (l + 1 < L ? (size_t)(l + 1) * dim : (size_t)2 * L * dim);
         n.xn = l + 1 < L ? nullptr : b.r.xn;

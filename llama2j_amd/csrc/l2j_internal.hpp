@@ -110,7 +110,7 @@ struct BatchBufs;   // l2j_batch.hip
 // What a forward pass of up to `cap` rows (positions, sequences) works in (l2j_rows.hip).
 struct RowBufs {
     int cap = 0;
-    float *x = nullptr, *part = nullptr, *q = nullptr, *xb = nullptr, *xn = nullptr;
+    float *x = nullptr, *part = nullptr, *act = nullptr, *q = nullptr, *xb = nullptr, *xn = nullptr;   // act: what k_w2_rows reads
     Digits dig{};
     int *tokens = nullptr;
     float *pf_part = nullptr;      // k_pflash with the keys of a block split over several workgroups: what each leaves for the one

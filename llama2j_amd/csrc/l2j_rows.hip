@@ -121,16 +121,48 @@ void l2j::launch_norm(l2j_ctx *c, const RowNorm &n, int rows)
     hipLaunchKernelGGL(k_rows_norm, dim3(a.together ? together_grid(rows, 1) : rows), dim3(threads), (size_t)n.dim * sizeof(float), c->stream, a);
 }
 
-void l2j::launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows)
+static void launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows)
 {
     const int hidden = c->cfg.hidden_dim, parts = (hidden + 1023) / 1024, together = rows >= kTogetherFrom;
     const dim3 grid = together ? dim3(together_grid(rows, parts)) : dim3(parts, rows);
     hipLaunchKernelGGL(k_rows_swiglu, grid, dim3(256), 0, c->stream, part, slices, o, rows, hidden, c->silu, (c->cfg.flags & L2J_F_EXACT_SILU) ? 1 : 0, together);
 }
 
+// W1 and W3 of the normed rows in b.dig, SwiGLU, W2: the slices in b.part, their number returned.
+int l2j::launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows)
+{
+    const int dim = c->cfg.dim, hidden = c->cfg.hidden_dim;
+    if (!swiglu_in_products(c->n_cu, dim, hidden, rows)) {
+        const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, layer, b.dig, rows, b.part);
+        launch_swiglu(c, b.part, s13, b.dig, rows);
+        return launch_dgemm(c, {L2J_W2}, layer, b.dig, rows, b.part);
+    }
+    const uint64_t off = (uint64_t)layer * dim * hidden;
+    DGemm a{};
+    a.codes[0] = c->bt_codes[L2J_W1] + off; a.codes[1] = c->bt_codes[L2J_W3] + off; a.codes[2] = a.codes[0];
+    a.gs[0] = c->bt_gs[L2J_W1] + off / 256; a.gs[1] = c->bt_gs[L2J_W3] + off / 256; a.gs[2] = a.gs[0];
+    a.tiles[0] = a.tiles[1] = hidden / 16; a.ntiles = 2 * (hidden / 16);
+    a.ngroups = a.gps = dim / 256;
+    a.x = b.dig; a.npos = rows; a.out = b.act;
+    a.silu = c->silu; a.exact = (c->cfg.flags & L2J_F_EXACT_SILU) ? 1 : 0;
+    W2Rows d{};
+    d.x = b.act; d.npos = rows; d.hidden = hidden; d.dim = dim;
+    d.codes = c->bt_codes[L2J_W2] + off; d.gs = c->bt_gs[L2J_W2] + off / 256;
+    d.out = b.part;
+    const dim3 grid(dim / 32, hidden / 256);
+    if (rows <= 16) {
+        hipLaunchKernelGGL((k_dstream<1, 1, true>), dim3(hidden / 16), dim3(64 * kStreamWaves), dstream_lds<1>(), c->stream, a);
+        hipLaunchKernelGGL(k_w2_rows<1>, grid, dim3(256), 0, c->stream, d);
+    } else {
+        hipLaunchKernelGGL((k_dstream<2, 1, true>), dim3(hidden / 16), dim3(64 * kStreamWaves), dstream_lds<2>(), c->stream, a);
+        hipLaunchKernelGGL(k_w2_rows<2>, grid, dim3(512), 0, c->stream, d);
+    }
+    return hidden / 256;
+}
+
 void RowBufs::release()
 {
-    void *ps[] = {x, part, q, xb, xn, dig.d, dig.sx, dig.sum, tokens, pf_part, pf_cnt};
+    void *ps[] = {x, part, act, q, xb, xn, dig.d, dig.sx, dig.sum, tokens, pf_part, pf_cnt};
     for (void *p : ps) (void)hipFree(p);
     *this = RowBufs();
 }
@@ -149,6 +181,7 @@ hipError_t RowBufs::alloc(l2j_ctx *c, int rows, bool attention)
     get(&x, rows * dim);
     get(&xn, rows * dim);
     get(&part, (size_t)max_slice_rows(rows, (int)groups) * std::max(2 * hidden, dim + 2 * kvd));
+    if (swiglu_in_products(c->n_cu, cf.dim, cf.hidden_dim, 1)) get(&act, std::min(rows, kRowTile) * hidden);
     get(&dig.d, tiles * groups * (kDigitBytes / 16));
     get(&dig.sx, tiles * groups * 32);
     get(&dig.sum, tiles * groups * 32);
@@ -270,9 +303,7 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
         n.slices = launch_dgemm(c, {L2J_WO}, l, b.dig, rows, b.part);
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, rows);
-        const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, l, b.dig, rows, b.part);
-        launch_swiglu(c, b.part, s13, b.dig, rows);
-        n.slices = launch_dgemm(c, {L2J_W2}, l, b.dig, rows, b.part);
+        n.slices = launch_ffn(c, l, b, rows);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         if (l + 1 < L) {
             n.w = c->rmsw + (size_t)(l + 1) * dim;

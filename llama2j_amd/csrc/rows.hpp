@@ -30,12 +30,22 @@ inline int max_slices(int rows) { return std::min(16, std::max(4, 1024 / std::ma
 // Most (slice, row) pairs of products of up to `cap` rows with rows of up to `ngroups` groups.
 inline int max_slice_rows(int cap, int ngroups) { return std::max({std::min(16 * cap, 1024), 4 * cap, stream_slices(ngroups) * std::min(cap, kRowTile)}); }
 
+// SwiGLU at the end of the product W1 and W3 and its digits at the beginning of W2 (k_dstream<NB, 1, true>, k_w2_rows) instead of a launch of
+// its own: where W1 and W3 leave one slice, and both products are one round of the compute units: 16 rows of each of W1 and W3 a
+// workgroup, 32 rows of W2 and one group of K, as many groups as k_rows_norm adds up with all loads in flight.
+// 110M shape, ms: 13 sequences sampled over 32 steps 16.41 -> 15.21, 15 greedy over 13 5.65 -> 5.27, 17 sampled over 16 9.47 -> 9.31.  (SwiGLU
+// itself at the beginning of W2, by every tile: 16.18 -> 16.46, the sigmoid table's entries come one lane a cycle.)
+inline bool swiglu_in_products(int n_cu, int dim, int hidden, int rows)
+{
+    return streams(dim / 16, rows) && stream_slices(dim / 256) == 1 && hidden / 16 <= n_cu && hidden / 256 <= 8 && dim / 32 * (hidden / 256) <= n_cu;
+}
+
 DgPlan dgemm_plan(int n_cu, int tiles16, int ngroups, int rows);
 hipError_t prepare_dgemm(l2j_ctx *c);
 int product_slices(l2j_ctx *c, int tiles16, int ngroups, int rows);
 void launch_norm(l2j_ctx *c, const RowNorm &n, int rows);
-void launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows);
 int launch_dgemm(l2j_ctx *c, std::initializer_list<int> tensors, int layer, const Digits &x, int rows, float *part);
+int launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows);
 
 struct RowJob {
     int nseg, T, pos0;                                        // T positions from pos0 on of nseg sequences; b.tokens: their tokens

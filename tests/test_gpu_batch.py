@@ -149,6 +149,14 @@ def test_products_of_one_to_four_tiles_per_workgroup(orc, hidden, n_seq):
     test_every_sequence_gets_what_it_gets_alone(orc, (256, hidden, 1, 4, 4, 512, 40, 1), n_seq)
 
 
+@pytest.mark.parametrize("n_seq", [16, 32])
+@pytest.mark.parametrize("dim,hidden", [(256, 256), (256, 2048), (768, 2048), (1024, 2048), (1024, 2304), (1280, 2048)])
+def test_swiglu_within_the_products_up_to_its_last_shape(orc, dim, hidden, n_seq):
+    # SwiGLU at the end of W1 and W3, its digits at the beginning of W2: up to 4 groups of dim, 8 of hidden, 256 workgroups for W2 (1024, 2048); past
+    # that a launch of its own
+    test_every_sequence_gets_what_it_gets_alone(orc, (dim, hidden, 2, dim // 64, dim // 64, 512, 24, 1), n_seq)
+
+
 @pytest.mark.parametrize("heads", [8, 4, 2])
 def test_scores_of_minus_infinity_weigh_nothing(heads):
     """A token whose keys are huge in one element of head 0 and whose queries are negative there: it scores -inf against itself and its

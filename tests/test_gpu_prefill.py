@@ -81,6 +81,21 @@ def test_the_last_layer_for_the_last_position_alone(shape, n):
     g.close()
 
 
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 31, 32])
+def test_swiglu_within_the_products_with_vectors_missing(n):
+    # up to 16 and up to 32 vectors, whole and not
+    shape = (1024, 2048, 2, 8, 8, 512, 40, 1)
+    tokens = np.random.default_rng(n).integers(2, shape[5], size=n).astype(np.int32)
+    g = model(shape)
+    got, _ = g.prefill(tokens)
+    for i, t in enumerate(tokens):
+        want = g.forward(int(t), i)
+    assert rel_err(got, want.astype(np.float64)) < CLOSE
+    g.close()
+    # an activation that is not finite: its group's scale is a NaN, and no other vector's
+    test_values_that_are_not_finite_stay_behind_the_causal_mask((512, 1024, 2, 8, 2, 1008, 64, 0), max(n, 12), 1, 0)
+
+
 @pytest.mark.parametrize("shape", SHAPES[:2])
 def test_prefill_goes_on_from_a_position_and_decode_goes_on_from_prefill(orc, shape):
     seq_len = shape[6]
