@@ -665,10 +665,12 @@ static __global__ void __launch_bounds__(512) k_bnext(const BNext a)
         if (better(bval[w], bidx[w], bv, bi)) { bv = bval[w]; bi = bidx[w]; }
     unsigned long long *best = a.best + b * kNextParts;
     st_coh(best + blockIdx.x, ((unsigned long long)__float_as_uint(bv) << 32) | (unsigned)bi);
-    __threadfence();
-    if (atomicAdd(a.done + 1 + b, 1u) != kNextParts - 1) return;
+    // Only the word above is for another workgroup of the launch, and it is written through.  (Three __threadfence() in its place, which
+    // write back an L2 full of logits: 16 and 32 rows of 32000 ids 11.3 and 14.6 us for 7.5 and 8.3.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (__hip_atomic_fetch_add(a.done + 1 + b, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kNextParts - 1) return;
+    asm volatile("" ::: "memory");
     a.done[1 + b] = 0u;
-    __threadfence();
     for (int w = 0; w < kNextParts; w++) {
         const unsigned long long o = ld_coh(best + w);
         const float ov = __uint_as_float((unsigned)(o >> 32));
@@ -679,8 +681,7 @@ static __global__ void __launch_bounds__(512) k_bnext(const BNext a)
     const int next = pos < a.st->n_prompt[b] ? a.prompts[(long)b * a.prompt_stride + pos] : bi;
     a.out_tokens[(long)b * a.out_stride + pos] = next;
     a.st->token[b] = next;
-    __threadfence();
-    if (atomicAdd(a.done, 1u) == gridDim.y - 1) {   // every sequence has its token: the step is over
+    if (__hip_atomic_fetch_add(a.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1) {   // every sequence has its token: the step is over
         a.done[0] = 0u;
         a.st->pos = pos + 1;
     }
