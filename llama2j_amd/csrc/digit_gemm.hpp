@@ -463,21 +463,20 @@ template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (s
 // loop to fetch.  Two, up to 16 vectors: no third request, which the loop makes for nothing (Wo of the 7B shape 6.9 -> 6.45 us,
 // 24 steps of 16 sequences 52.5 -> 52.0 ms).
 // Workgroup (blockIdx.x, slice blockIdx.y) of gridDim.x per slice: every gridDim.x-th tile of 32 rows (rows % 32 == 0).
+// A row is added up in the same order at 16 and at 32 vectors: sampling from all of the distribution follows the last bits of the logits.
+// (Waves with 16 of 32 vectors against a whole group, where a workgroup has one tile, convert half as many sums, step of 32
+// sequences of the 110M shape 476 -> 462 us, but round them elsewhere: one plain-sampled batch in fifty got other tokens.)
 // SWIGLU (one tile, one slice, matrices W1 and W3): a tile is 16 rows of W1 and the same rows of W3, and out is (npos, hidden):
 // silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74).
 template <int NB, int TILES, bool SWIGLU = false>
 static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
 {
-    // Of 32 vectors and one tile a workgroup (the products of the 110M shape) a wave takes half, against the whole group: half as many sums to
-    // convert and to add up, for codes that two waves request (steps of 24 and 32 sequences of the 110M shape 482 and 476 -> 466 and 462 us; with more tiles, where the
-    // codes' way from memory is the bound, 70B widths 1205 -> 1295).
-    constexpr bool WHOLE = NB == 2 && TILES == 1;
-    constexpr int NT = WHOLE ? 4 : 2, MT = WHOLE ? 1 : NB, PARTS = WHOLE ? kStreamGroups : kStreamWaves;   // blocks of 64 k and of 16 vectors per wave, sums of a tile to be added up
+    constexpr int NT = 2;   // blocks of 64 k per wave
     extern __shared__ __align__(16) float ds_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
     const int slice = blockIdx.y, g0 = slice * a.gps, ng = min(a.gps, a.ngroups - g0);
     const bool on = wave < 2 * ng;       // (a wave without a group multiplies the slice's last one by zero scales: no branch around loads)
-    const int g = g0 + min(wave >> 1, ng - 1), hf = WHOLE ? 0 : wave & 1, m0 = WHOLE ? wave & 1 : 0, ntile = a.ntiles >> 1, step = gridDim.x;
+    const int g = g0 + min(wave >> 1, ng - 1), hf = wave & 1, ntile = a.ntiles >> 1, step = gridDim.x;
     // this wave's k of the first tile of the first matrix, and how far from there the others lie (differences of addresses:
     // a choice between pointers would turn the loads into flat ones)
     const uint8_t *cb = a.codes[0] + (size_t)g * 4096 + 1024 * NT * hf;
@@ -511,35 +510,33 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
         asm volatile("" : "+s"(p0), "+s"(p1), "+v"(lane16));
 #pragma unroll
         for (int T = 0; T < NT; T++) {
-            typedef const __attribute__((address_space(1))) v4i *Words;
-            const Words w0 = reinterpret_cast<Words>(p0 + lane16 + 1024 * T), w1 = reinterpret_cast<Words>(p1 + lane16 + 1024 * T);
-            c.w[0][T] = WHOLE ? *w0 : __builtin_nontemporal_load(w0);   // (WHOLE: the other wave finds them in the cache)
-            c.w[1][T] = WHOLE ? *w1 : __builtin_nontemporal_load(w1);
+            c.w[0][T] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) v4i *>(p0 + lane16 + 1024 * T));
+            c.w[1][T] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) v4i *>(p1 + lane16 + 1024 * T));
         }
     };
 
     Codes c0, c1;
     const int t0 = blockIdx.x;
-    v4i dg[4][MT][NT];
+    v4i dg[4][NB][NT];
     {
-        const v4i *xp = reinterpret_cast<const v4i *>(a.x.d) + (size_t)g * (kDigitBytes / 16) + hf * NT * 128 + m0 * 64;
+        const v4i *xp = reinterpret_cast<const v4i *>(a.x.d) + (size_t)g * (kDigitBytes / 16) + hf * NT * 128;
 #pragma unroll
         for (int d = 0; d < 4; d++)
 #pragma unroll
             for (int T = 0; T < NT; T++)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) dg[d][mt][T] = (xp + ((d * 4 + T) * 2 + mt) * 64)[(unsigned)lane];
+                for (int mt = 0; mt < NB; mt++) dg[d][mt][T] = (xp + ((d * 4 + T) * 2 + mt) * 64)[(unsigned)lane];
     }
     // The digits first: a wave's loads return in order, and the first tile needs all of the digits but only its own codes.  (Codes first: a step
     // of 16 and 32 sequences of the 110M shape 440 and 482 us for 411 and 476, of the 7B shape 2406 and 2910 for 2356 and 2885.)
     __builtin_amdgcn_sched_barrier(0);
     request(t0, c0);
     __builtin_amdgcn_sched_barrier(0);
-    v4f sx[MT], sm[MT];
+    v4f sx[NB], sm[NB];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        sx[mt] = *reinterpret_cast<const v4f *>(a.x.sx + (size_t)g * 32 + 16 * (m0 + mt) + 4 * s4);
-        sm[mt] = *reinterpret_cast<const v4f *>(a.x.sum + (size_t)g * 32 + 16 * (m0 + mt) + 4 * s4);
+    for (int mt = 0; mt < NB; mt++) {
+        sx[mt] = *reinterpret_cast<const v4f *>(a.x.sx + (size_t)g * 32 + 16 * mt + 4 * s4);
+        sm[mt] = *reinterpret_cast<const v4f *>(a.x.sum + (size_t)g * 32 + 16 * mt + 4 * s4);
         if (!on) sx[mt] = v4f{0.f, 0.f, 0.f, 0.f};
         if (!on || hf) sm[mt] = v4f{0.f, 0.f, 0.f, 0.f};   // (the group's offset: by the first of its waves)
     }
@@ -547,9 +544,9 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
     float *out = a.out + (size_t)slice * a.npos * ldo;
 
     auto tile = [&](int buf, const Codes &c) {
-        float *red = ds_lds + buf * PARTS * NB * 512;
+        float *red = ds_lds + buf * kStreamWaves * NB * 512;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+        for (int mt = 0; mt < NB; mt++)
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 v4i hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
@@ -568,15 +565,15 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
 #pragma unroll
                 for (int e = 0; e < 4; e++)   // (the power of two into the sum, which takes it exactly: times the scale a small one would lose bits)
                     y[e] = fmaf(fmaf((float)hi[e], 65536.0f, (float)lo[e]) * sx[mt][e], c.s[r].x, c.s[r].y * sm[mt][e]);
-                *reinterpret_cast<v4f *>(red + (((wave * MT + mt) * 2 + r) * 64 + lane) * 4) = y;
+                *reinterpret_cast<v4f *>(red + (((wave * NB + mt) * 2 + r) * 64 + lane) * 4) = y;
             }
     };
     // the tile's sums: NB x 2 blocks of 64 lanes x 4: NB values per thread
-    struct Sums { float v[PARTS][NB]; };
+    struct Sums { float v[kStreamWaves][NB]; };
     auto read = [&](int buf, Sums &u) {
-        const float *red = ds_lds + buf * PARTS * NB * 512 + tid * NB;
+        const float *red = ds_lds + buf * kStreamWaves * NB * 512 + tid * NB;
 #pragma unroll
-        for (int w = 0; w < PARTS; w++)
+        for (int w = 0; w < kStreamWaves; w++)
 #pragma unroll
             for (int k = 0; k < NB; k++) u.v[w][k] = red[w * NB * 512 + k];
     };
@@ -588,7 +585,7 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
         for (int k = 0; k < NB; k++) {
             float y = u.v[0][k];
 #pragma unroll
-            for (int w = 1; w < PARTS; w++) y += u.v[w][k];
+            for (int w = 1; w < kStreamWaves; w++) y += u.v[w][k];
             if (row + k < a.npos) o[(size_t)k * ldo] = y;
         }
     };
@@ -604,7 +601,7 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
             const float *red = ds_lds + (tid >> 8) * 512 + (tid & 255);
             float h1 = red[0], h3 = red[256];
 #pragma unroll
-            for (int w = 1; w < PARTS; w++) {
+            for (int w = 1; w < kStreamWaves; w++) {
                 h1 += red[w * NB * 512];
                 h3 += red[w * NB * 512 + 256];
             }

@@ -157,6 +157,23 @@ def test_swiglu_within_the_products_up_to_its_last_shape(orc, dim, hidden, n_seq
     test_every_sequence_gets_what_it_gets_alone(orc, (dim, hidden, 2, dim // 64, dim // 64, 512, 24, 1), n_seq)
 
 
+@pytest.mark.parametrize("shape", [(768, 2048, 2, 12, 12, 1008, 24, 1), (512, 1280, 2, 8, 2, 1008, 24, 0), (1024, 2816, 2, 8, 4, 2000, 24, 0)])
+def test_a_sequence_has_the_same_bits_among_sixteen_and_among_32(shape):
+    """The products of up to sixteen vectors and those of up to 32 add a row up in the same order, so a sequence's logits, and with them
+    what is sampled from them, do not depend on how many others there are."""
+    g = l2j.Transformer(l2j.Config(*shape))
+    g.fill_synthetic(9, 0.02)
+    g.finalize()
+    rng = np.random.default_rng(shape[1])
+    prompts = [rng.integers(2, shape[5], size=b % 7).astype(np.int32) for b in range(32)]   # (the first has none: no prompt positions in common)
+    want_tokens, want = g.decode_greedy_batch(prompts, shape[6], want_logits=True)
+    for first in (0, 14):
+        tokens, logits = g.decode_greedy_batch(prompts[first:first + 16], shape[6], want_logits=True)
+        np.testing.assert_array_equal(tokens, want_tokens[first:first + 16])
+        np.testing.assert_array_equal(logits.view(np.uint32), want[:, first:first + 16].view(np.uint32))
+    g.close()
+
+
 @pytest.mark.parametrize("heads", [8, 4, 2])
 def test_scores_of_minus_infinity_weigh_nothing(heads):
     """A token whose keys are huge in one element of head 0 and whose queries are negative there: it scores -inf against itself and its

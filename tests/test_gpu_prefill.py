@@ -347,6 +347,66 @@ def test_values_that_are_not_finite_stay_behind_the_causal_mask(shape, n, flash,
     g.close()
 
 
+def digit_pairs(x):
+    """fp32 activations (vectors, groups, 256) as the products have them: 256 * first + second digit, 256 * third + fourth, 2^-s."""
+    s = 30 - np.frexp(np.abs(x).max(axis=2, keepdims=True))[1]
+    q = np.rint(np.ldexp(x.astype(np.float64), s)).astype(np.int64)
+    d = (((q + 0x80808080) & 0xffffffff) ^ 0x80808080).astype(np.uint32)
+    d = [(d >> np.uint32(24 - 8 * i)).astype(np.uint8).view(np.int8).astype(np.float64) for i in range(4)]
+    return 256 * d[0] + d[1], 256 * d[2] + d[3], np.ldexp(np.float32(1.0), -s[:, :, 0])
+
+
+@pytest.mark.parametrize("dim,heads,n", [(512, 4, 16), (512, 4, 17), (512, 4, 32), (4096, 32, 32)])
+def test_the_sums_of_a_product_are_formed_in_one_order(dim, heads, n):
+    """Wv on inputs, codes and scales whose products are all exact, so that the value rows show the order of the additions to the bit.  Up
+    to 32 vectors the halves of the groups are converted and added one after the other, above that the high and the low digits of a group go
+    into the running sum one after the other; then the slices of K in their order."""
+    vocab, kvd, ng = 512, dim // heads * 2, dim // 256
+    rng = np.random.default_rng(dim + n)
+    emb = np.ldexp(rng.integers(-8, 9, (vocab, dim)).astype(np.float32), rng.integers(-38, -30, (vocab, 1)))   # (nothing beside the norm's 1e-5)
+    norm = rng.choice([-1.0, 127 / 128], (ng, 256)).astype(np.float32)   # (the least and the greatest code are exact)
+    w = rng.integers(-128, 128, (kvd, ng, 256))
+    w[..., :2] = -128, 127                                               # (a group's scale is 2^-7, its offset 0)
+    g = l2j.Transformer(l2j.Config(dim, 256, 1, heads, 2, vocab, 1008, 0))
+    g.fill_synthetic(9, 0.02)
+    g.upload_f32(TENSOR.TOK_EMB, emb)
+    g.upload_f32_quantize(TENSOR.RMS_ATT, norm)
+    g.upload_f32_quantize(TENSOR.WV, np.ldexp(w, -7))
+    g.finalize()
+    tokens = rng.integers(2, vocab, size=n).astype(np.int32)
+    g.prefill(tokens, want_logits=False)
+    got = g.read(BUFFER.VCACHE, 0).reshape(-1, kvd)[:n]
+    g.close()
+    x = norm.reshape(-1) * (np.float32(1.0) / np.sqrt(np.float32(1e-5)) * emb[tokens])
+    high, low, scale = digit_pairs(x.reshape(n, ng, 256))
+    scale = np.ldexp(scale, -7)
+    part = lambda d, group, k: (d[:, group, k] @ w[:, group, k].T.astype(np.float64)).astype(np.float32)   # (whole numbers: exact up to here)
+
+    def slice_sum(g0, g1):
+        f = np.zeros((n, kvd), dtype=np.float32)
+        for group in range(g0, g1):
+            sx = scale[:, group, None]
+            for k in (slice(0, 128), slice(128, 256)) if n <= 32 else (slice(0, 256),):
+                h, l = part(high, group, k), part(low, group, k)
+                if n <= 32:
+                    f += (h.astype(np.float64) * 65536 + l).astype(np.float32) * sx
+                else:
+                    f += h * (65536 * sx)
+                    f += l * sx
+        return f
+
+    def want(per_slice):
+        t = np.zeros((n, kvd), dtype=np.float32)
+        for g0 in range(0, ng, per_slice):
+            t += slice_sum(g0, min(ng, g0 + per_slice))
+        return t
+
+    if n <= 32:                                                          # (slices of four groups)
+        np.testing.assert_array_equal(got.view(np.uint32), want(4).view(np.uint32))
+    else:                                                                # (as many groups as the estimate for this shape picks)
+        assert any(np.array_equal(got.view(np.uint32), want(per).view(np.uint32)) for per in range(1, ng + 1))
+
+
 def test_a_prompt_goes_through_in_smaller_passes_where_the_memory_for_a_large_one_is_missing():
     """1100 positions with room for passes of 275 instead of 550, the decode loop with option prefill likewise; other calls go on
     as before, and so does the prompt once there is room."""
