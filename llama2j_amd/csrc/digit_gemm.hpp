@@ -467,7 +467,7 @@ template <int NB> __host__ __device__ constexpr size_t dstream_lds() { return (s
 // (Waves with 16 of 32 vectors against a whole group, where a workgroup has one tile, convert half as many sums, step of 32
 // sequences of the 110M shape 476 -> 462 us, but round them elsewhere: one plain-sampled batch in fifty got other tokens.)
 // SWIGLU (one tile, one slice, matrices W1 and W3): a tile is 16 rows of W1 and the same rows of W3, and out is (npos, hidden):
-// silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74).
+// silu(h1) * h3 with the reference's sigmoid table (K/Silu.java:72-74); behind it (npos, hidden / 16): the sums of 16 consecutive ones.
 template <int NB, int TILES, bool SWIGLU = false>
 static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const DGemm a)
 {
@@ -605,7 +605,13 @@ static __global__ void __launch_bounds__(64 * kStreamWaves, 2) k_dstream(const D
                 h1 += red[w * NB * 512];
                 h3 += red[w * NB * 512 + 256];
             }
-            a.out[(size_t)row * 16 * ntile + 16 * t + col] = __fmul_rn(h1, __fmul_rn(silu_sigma(a.silu, h1, a.exact), h3));
+            const float m = silu_sigma(a.silu, h1, a.exact) * h3, y = h1 * m;
+            a.out[(size_t)row * 16 * ntile + 16 * t + col] = y;
+            // the sum of the sixteen, in the order (and with the first of two products unrounded, as the compiler contracts it there) of k_rows_swiglu
+            float sum = fmaf(h1, m, __shfl_xor(y, 4));
+#pragma unroll
+            for (int off = 8; off < 64; off <<= 1) sum += __shfl_xor(sum, off);
+            if (col == 0) a.out[(size_t)(a.npos * 16 + row) * ntile + t] = sum;
         }
         return;
     }

@@ -348,9 +348,10 @@ void launch_batch_step(l2j_ctx *c, BatchBufs &b)
         else if (hs == 128) hipLaunchKernelGGL(k_battn<32>, ag, dim3(512), 0, s, t);
         else hipLaunchKernelGGL(k_battn<64>, ag, dim3(256), 0, s, t);
         n.slices = launch_dgemm(c, {L2J_WO}, l, b.r.dig, nseq, b.r.part);
+        n.per_slice = 0;
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, nseq);
-        n.slices = launch_ffn(c, l, b.r, nseq);
+        launch_ffn(c, l, b.r, nseq, n);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         n.w = c->rmsw + (l + 1 < L ? (size_t)(l + 1) * dim : (size_t)2 * L * dim);
         n.xn = l + 1 < L ? nullptr : b.r.xn;

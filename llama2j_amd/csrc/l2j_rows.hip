@@ -55,7 +55,7 @@ hipError_t l2j::prepare_dgemm(l2j_ctx *c)
     if (c->dgemm_ready) return hipSuccess;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dgemm<1, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)dgemm_lds<1>());
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dgemm<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)dgemm_lds<2>());
-    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_norm), hipFuncAttributeMaxDynamicSharedMemorySize, 128 << 10);
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_norm<false>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 << 10);
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_logits), hipFuncAttributeMaxDynamicSharedMemorySize, 128 << 10);
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<64, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(64, 2));
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rows_attn<128, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)attn_lds(128, 1));
@@ -118,7 +118,9 @@ void l2j::launch_norm(l2j_ctx *c, const RowNorm &n, int rows)
     const int threads = std::min(1024, std::max(64, n.dim / 4));
     RowNorm a = n;
     a.together = rows >= kTogetherFrom && !n.xn ? rows : 0;
-    hipLaunchKernelGGL(k_rows_norm, dim3(a.together ? together_grid(rows, 1) : rows), dim3(threads), (size_t)n.dim * sizeof(float), c->stream, a);
+    const dim3 grid(a.together ? together_grid(rows, 1) : rows);
+    if (n.per_slice > 0) hipLaunchKernelGGL(k_rows_norm<true>, grid, dim3(threads), (size_t)n.dim * sizeof(float), c->stream, a);
+    else hipLaunchKernelGGL(k_rows_norm<false>, grid, dim3(threads), (size_t)n.dim * sizeof(float), c->stream, a);
 }
 
 static void launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digits &o, int rows)
@@ -128,14 +130,16 @@ static void launch_swiglu(l2j_ctx *c, const float *part, int slices, const Digit
     hipLaunchKernelGGL(k_rows_swiglu, grid, dim3(256), 0, c->stream, part, slices, o, rows, hidden, c->silu, (c->cfg.flags & L2J_F_EXACT_SILU) ? 1 : 0, together);
 }
 
-// W1 and W3 of the normed rows in b.dig, SwiGLU, W2: the slices in b.part, their number returned.
-int l2j::launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows)
+// W1 and W3 of the normed rows in b.dig, SwiGLU, W2: the slices in b.part, n.slices and n.per_slice what k_rows_norm then adds up.
+void l2j::launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows, RowNorm &n)
 {
     const int dim = c->cfg.dim, hidden = c->cfg.hidden_dim;
+    n.per_slice = 0;
     if (!swiglu_in_products(c->n_cu, dim, hidden, rows)) {
         const int s13 = launch_dgemm(c, {L2J_W1, L2J_W3}, layer, b.dig, rows, b.part);
         launch_swiglu(c, b.part, s13, b.dig, rows);
-        return launch_dgemm(c, {L2J_W2}, layer, b.dig, rows, b.part);
+        n.slices = launch_dgemm(c, {L2J_W2}, layer, b.dig, rows, b.part);
+        return;
     }
     const uint64_t off = (uint64_t)layer * dim * hidden;
     DGemm a{};
@@ -157,7 +161,9 @@ int l2j::launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows)
         hipLaunchKernelGGL((k_dstream<2, 1, true>), dim3(hidden / 16), dim3(64 * kStreamWaves), dstream_lds<2>(), c->stream, a);
         hipLaunchKernelGGL(k_w2_rows<2>, grid, dim3(512), 0, c->stream, d);
     }
-    return hidden / 256;
+    const int groups = hidden / 256, slices = stream_slices(groups);
+    n.slices = 2 * groups;
+    n.per_slice = 2 * ((groups + slices - 1) / slices);
 }
 
 void RowBufs::release()
@@ -181,7 +187,7 @@ hipError_t RowBufs::alloc(l2j_ctx *c, int rows, bool attention)
     get(&x, rows * dim);
     get(&xn, rows * dim);
     get(&part, (size_t)max_slice_rows(rows, (int)groups) * std::max(2 * hidden, dim + 2 * kvd));
-    if (swiglu_in_products(c->n_cu, cf.dim, cf.hidden_dim, 1)) get(&act, std::min(rows, kRowTile) * hidden);
+    if (swiglu_in_products(c->n_cu, cf.dim, cf.hidden_dim, 1)) get(&act, std::min(rows, kRowTile) * (hidden + hidden / 16));
     get(&dig.d, tiles * groups * (kDigitBytes / 16));
     get(&dig.sx, tiles * groups * 32);
     get(&dig.sum, tiles * groups * 32);
@@ -301,9 +307,10 @@ hipError_t l2j::launch_rows(l2j_ctx *c, RowBufs &b, const RowJob &job)
             launch_attn<256>(c, t);
         }
         n.slices = launch_dgemm(c, {L2J_WO}, l, b.dig, rows, b.part);
+        n.per_slice = 0;
         n.w = c->rmsw + (size_t)(L + l) * dim;
         launch_norm(c, n, rows);
-        n.slices = launch_ffn(c, l, b, rows);
+        launch_ffn(c, l, b, rows, n);
         // the residual, then the norm of what follows: the next layer's attention norm, or the final one (rmsw: att, ffn, final)
         if (l + 1 < L) {
             n.w = c->rmsw + (size_t)(l + 1) * dim;

@@ -32,9 +32,11 @@ inline int max_slice_rows(int cap, int ngroups) { return std::max({std::min(16 *
 
 // SwiGLU at the end of the product W1 and W3 and its digits at the beginning of W2 (k_dstream<NB, 1, true>, k_w2_rows) instead of a launch of
 // its own: where W1 and W3 leave one slice, and both products are one round of the compute units: 16 rows of each of W1 and W3 a
-// workgroup, 32 rows of W2 and one group of K, as many groups as k_rows_norm adds up with all loads in flight.
-// 110M shape, ms: 13 sequences sampled over 32 steps 16.41 -> 15.21, 15 greedy over 13 5.65 -> 5.27, 17 sampled over 16 9.47 -> 9.31.  (SwiGLU
-// itself at the beginning of W2, by every tile: 16.18 -> 16.46, the sigmoid table's entries come one lane a cycle.)
+// workgroup, 32 rows of W2 and one group of K, at most two slices of four groups, whose halves k_rows_norm adds up with all loads in flight.
+// The bits are the same either way.  Step of twelve layers with 16 and 32 sequences, us, launch of its own -> this: 256 wide, hidden 256
+// 334 398 -> 316 377, 256 x 2048 354 418 -> 336 393, 512 x 1536 370 436 -> 352 408, 768 x 2048 393 458 -> 376 437, 1024 x 1024 394 458 ->
+// 376 434, 1024 x 2048 399 464 -> 386 446 (2000 ids).  (SwiGLU itself at the beginning of W2, by every tile, was 1.7 % slower than the
+// launch: the sigmoid table's entries come one lane a cycle.)
 inline bool swiglu_in_products(int n_cu, int dim, int hidden, int rows)
 {
     return streams(dim / 16, rows) && stream_slices(dim / 256) == 1 && hidden / 16 <= n_cu && hidden / 256 <= 8 && dim / 32 * (hidden / 256) <= n_cu;
@@ -45,7 +47,7 @@ hipError_t prepare_dgemm(l2j_ctx *c);
 int product_slices(l2j_ctx *c, int tiles16, int ngroups, int rows);
 void launch_norm(l2j_ctx *c, const RowNorm &n, int rows);
 int launch_dgemm(l2j_ctx *c, std::initializer_list<int> tensors, int layer, const Digits &x, int rows, float *part);
-int launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows);
+void launch_ffn(l2j_ctx *c, int layer, const RowBufs &b, int rows, RowNorm &n);
 
 struct RowJob {
     int nseg, T, pos0;                                        // T positions from pos0 on of nseg sequences; b.tokens: their tokens

@@ -37,6 +37,7 @@ struct RowNorm {
     const int *tokens;
     const float *part;      // else: x += the slices of a product (K/Accum.java:26-30)
     int slices, nrows;      // nrows: rows of the product's output
+    int per_slice;          // 0, or part holds that many sums of each slice (of the last one what is left), `slices` in all (k_w2_rows)
     int together;           // 0: a workgroup per row in order, else the number of rows (together_row)
     float *x;               // (rows, dim)
     const float *w;         // norm weights
@@ -45,12 +46,33 @@ struct RowNorm {
     float *xn;              // or, not null, as floats
 };
 
+// The slices of k_w2_rows: the sums of a slice are added up first, as k_dstream does within a workgroup.  At most 2 slices, n <= N sums, all
+// loads in flight.
+template <int N>
+__device__ __forceinline__ v4f sum_in_slices(const float *__restrict__ part, int n, int per_slice, size_t stride)
+{
+    v4f v[N], t = {}, y;
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = *reinterpret_cast<const v4f *>(part + min(i, n - 1) * stride);
+    y = v[0];
+#pragma unroll
+    for (int i = 1; i < N; i++) {
+        if (i < n) {
+            if (i == per_slice) { t += y; y = v[i]; }
+            else y += v[i];
+        }
+    }
+    return t + y;
+}
+
 // x, then w * (ss * x), ss = 1 / sqrt(sum(x^2) / n + 1e-5) (K/RootMeanSquare.java:25-35, K/WeightNormalizeAndScale.java:73).
 // One workgroup per row, four values per thread and step of 4096, kept in LDS (dim floats, each thread its own): a wave
 // holds whole groups of 256 and writes their digits.  Bound by its chain of latencies (slices, sum over the workgroup,
 // digits): the loads of the slices and of the first weights go out together.  32 rows of 4096 behind 4 or 11 slices
 // 6.7 us, 13 of 768 behind 1 or 2 slices 3.5 (7.4 and 4.0 when sixteen lanes per group wrote the digits behind another barrier
 // and the slices came four at a time).
+// W2ROWS: the slices are those of k_w2_rows.
+template <bool W2ROWS>
 static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
 {
     extern __shared__ __align__(16) float ln[];
@@ -74,7 +96,10 @@ static __global__ void __launch_bounds__(1024) k_rows_norm(const RowNorm a)
             v = e[i];
         } else {
             v = x[i];
-            const v4f t = sum_slices<v4f>(part + 4 * i, a.slices, stride);
+            v4f t;
+            if constexpr (!W2ROWS) t = sum_slices<v4f>(part + 4 * i, a.slices, stride);
+            else if (a.slices <= 8) t = sum_in_slices<8>(part + 4 * i, a.slices, a.per_slice, stride);
+            else t = sum_in_slices<16>(part + 4 * i, a.slices, a.per_slice, stride);
 #pragma unroll
             for (int k = 0; k < 4; k++) v[k] = __fadd_rn(v[k], t[k]);
         }
@@ -164,12 +189,15 @@ static __global__ void __launch_bounds__(256) k_rows_swiglu(const float *__restr
 // in and out, and forming the group's digits once per tile costs less than a launch that stores them.
 // A lane holds 16 consecutive activations of the vector and the k at which the matrix instruction takes them from it, so
 // the digits never leave its registers: wave (T, m) has the 64 k of block T for vectors 16 m .. 16 m + 15, and only the groups' maxima
-// and sums cross the waves.  The blocks' sums meet in LDS as integers (exact over a group) and are scaled once.
-// Bound by its chain of latencies (activations, two barriers, codes).  With SwiGLU at the end of W1 and W3 a layer of the 110M shape takes 3.1 us
-// less at 16 vectors than with a launch in between.
-// grid (rows of W2 / 32, groups), 256 NB threads; out: (group, vector, row of W2); vectors past npos count as zeros.
+// and sums cross the waves.  The blocks' sums meet in LDS as integers.  What leaves are the sums of a group's two halves, each
+// scaled for itself, and k_rows_norm adds them up slice by slice: bit for bit what k_rows_swiglu and k_dstream give, so that no result depends on
+// which of the two ways a shape or a number of rows takes.
+// Bound by its chain of latencies (activations, two barriers, codes); with SwiGLU at the end of W1 and W3 a layer takes 1.1 to 1.7 us less at
+// 16 vectors and 1.5 to 2.3 at 32 than with a launch in between.  (One sum per group, of all 256 k at once, was 1.3 us a layer of the
+// 110M shape less still, but rounded elsewhere: plain-sampled batches got other tokens.)
+// grid (rows of W2 / 32, groups), 256 NB threads; out: (half of a group, vector, row of W2); vectors past npos count as zeros.
 struct W2Rows {
-    const float *x;          // (npos, hidden)
+    const float *x;          // (npos, hidden), behind it the sums of 16 consecutive ones (npos, hidden / 16)
     int npos, hidden, dim;
     const uint8_t *codes;    // W2 of the layer in tile order (DGemm)
     const float2 *gs;
@@ -188,6 +216,7 @@ static __global__ void __launch_bounds__(256 * NB) k_w2_rows(const W2Rows a)
     v4f v[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const v4f *>(p + 4 * i);
+    float sum = a.x[(size_t)a.npos * a.hidden + (size_t)min(row, a.npos - 1) * (a.hidden >> 4) + 16 * g + 4 * T + (lane >> 4)];
     // the codes of the two tiles of 16 rows, on their way while the digits are formed
     const uint8_t *cb = a.codes + ((size_t)2 * tile * ngroups + g) * 4096 + 1024 * T + 16 * lane;
     v4i w[2];
@@ -197,21 +226,18 @@ static __global__ void __launch_bounds__(256 * NB) k_w2_rows(const W2Rows a)
     const float2 rm = a.gs[((size_t)(2 * tile + (blk & 1)) * ngroups + g) * 16 + (l2 & 15)];
     float y[16];
     unsigned mx = 0;
-    float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             y[4 * i + e] = row < a.npos ? v[i][e] : 0.0f;
             mx = max(mx, __float_as_uint(y[4 * i + e]) & 0x7fffffffu);   // (as bits: a NaN is the largest)
         }
-        sum += (y[4 * i] + y[4 * i + 1]) + (y[4 * i + 2] + y[4 * i + 3]);
-    }
+    if (row >= a.npos) sum = 0.0f;
+    sum += __shfl_xor(sum, 48);   // (the order of wave_sum in quantize_wave, where the four stand in a row of sixteen lanes: first and last, the two between)
+    sum += __shfl_xor(sum, 16);
 #pragma unroll
-    for (int off = 16; off < 64; off <<= 1) {
-        mx = max(mx, (unsigned)__shfl_xor((int)mx, off));
-        sum += __shfl_xor(sum, off);
-    }
+    for (int off = 16; off < 64; off <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, off));
     if (lane < 16) { s_max[T][row] = mx; s_sum[T][row] = sum; }
     __syncthreads();
     mx = max(max(s_max[0][row], s_max[1][row]), max(s_max[2][row], s_max[3][row]));
@@ -230,17 +256,17 @@ static __global__ void __launch_bounds__(256 * NB) k_w2_rows(const W2Rows a)
     }
     __syncthreads();
     const int first = 16 * (blk >> 1) + 4 * (l2 >> 4) + e2;
-    float *o = a.out + ((size_t)g * a.npos + first) * a.dim + 32 * tile + 16 * (blk & 1) + (l2 & 15);
+    float *o = a.out + ((size_t)2 * g * a.npos + first) * a.dim + 32 * tile + 16 * (blk & 1) + (l2 & 15);
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        int hi = 0, lo = 0;
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            hi += reinterpret_cast<const int *>(&red[0][t][blk][l2])[e2 + k];
-            lo += reinterpret_cast<const int *>(&red[1][t][blk][l2])[e2 + k];
+        for (int k = 0; k < 2; k++) {
+            auto both = [&](int d) { return reinterpret_cast<const int *>(&red[d][2 * h][blk][l2])[e2 + k] + reinterpret_cast<const int *>(&red[d][2 * h + 1][blk][l2])[e2 + k]; };
+            const int hi = both(0), lo = both(1);
+            // (the power of two into the sum, and the offset with the first half, as k_dstream)
+            if (first + k < a.npos)
+                o[((size_t)h * a.npos + k) * a.dim] = fmaf(fmaf((float)hi, 65536.0f, (float)lo) * s_inv[first + k], rm.x, rm.y * (h ? 0.0f : s_tot[first + k]));
         }
-        // (the power of two into the sum, as k_dstream)
-        if (first + k < a.npos) o[(size_t)k * a.dim] = fmaf(fmaf((float)hi, 65536.0f, (float)lo) * s_inv[first + k], rm.x, rm.y * s_tot[first + k]);
     }
 }
 

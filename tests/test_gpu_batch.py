@@ -174,6 +174,39 @@ def test_a_sequence_has_the_same_bits_among_sixteen_and_among_32(shape):
     g.close()
 
 
+@pytest.mark.parametrize("dim,groups,wider", [(256, 1, 9), (512, 3, 9), (768, 4, 10), (512, 5, 9), (768, 6, 9), (256, 7, 10), (768, 8, 16), (1024, 8, 12)])
+def test_hidden_rows_of_zeros_change_no_bit(dim, groups, wider):
+    """The same layers with further rows of zeros in W1 and W3 and zeros behind the rows of W2, so many that SwiGLU is a launch of its own:
+    the logits of every step have the same bits.  (Both widths cut a row into slices of as many groups.)"""
+    n_layers, vocab, seq_len = 2, 512, 16
+    rng = np.random.default_rng(dim + groups)
+    weights = {t: 0.02 * rng.standard_normal((n_layers, 256 * groups, dim)).astype(np.float32) for t in (TENSOR.W1, TENSOR.W3)}
+    weights[TENSOR.W2] = 0.02 * rng.standard_normal((n_layers, dim, 256 * groups)).astype(np.float32)
+    prompts = [rng.integers(2, vocab, size=b % 5).astype(np.int32) for b in range(32)]
+    want = None
+    for width in (groups, wider):
+        g = l2j.Transformer(l2j.Config(dim, 256 * width, n_layers, dim // 64, dim // 64, vocab, seq_len, 1))
+        g.fill_synthetic(9, 0.02)
+        for t, w in weights.items():
+            pad = [(0, 0)] * 3
+            pad[2 if t == TENSOR.W2 else 1] = (0, 256 * (width - groups))
+            g.upload_f32_quantize(t, np.pad(w, pad))
+        for t in (TENSOR.RMS_ATT, TENSOR.RMS_FFN, TENSOR.RMS_FINAL):
+            g.upload_f32_quantize(t, np.ones(dim * (1 if t == TENSOR.RMS_FINAL else n_layers), dtype=np.float32))
+        for t, rows in ((TENSOR.WQ, dim), (TENSOR.WK, dim), (TENSOR.WV, dim), (TENSOR.WO, dim)):
+            g.upload_f32_quantize(t, 0.02 * np.random.default_rng(int(t)).standard_normal((n_layers, rows, dim)).astype(np.float32))
+        g.upload_f32(TENSOR.TOK_EMB, 0.02 * np.random.default_rng(1).standard_normal((vocab, dim)).astype(np.float32))
+        g.finalize()
+        got = [g.decode_greedy_batch(prompts[:n], seq_len, want_logits=True) for n in (16, 32)]
+        got.append((np.int32(0), g.prefill(np.arange(2, 2 + 11, dtype=np.int32))[0]))
+        g.close()
+        if want is None:
+            want = got
+        for (tokens, logits), (tokens1, logits1) in zip(got, want):
+            np.testing.assert_array_equal(tokens, tokens1)
+            np.testing.assert_array_equal(logits.view(np.uint32), logits1.view(np.uint32))
+
+
 @pytest.mark.parametrize("heads", [8, 4, 2])
 def test_scores_of_minus_infinity_weigh_nothing(heads):
     """A token whose keys are huge in one element of head 0 and whose queries are negative there: it scores -inf against itself and its
