@@ -212,10 +212,10 @@ __device__ constexpr int dg_block(int u, int nu, int j) { return u == 0 && j < 8
 // v_mfma_i32_32x32x32_i8 2.9: the clock drops under the matrix cores' load.)
 // What a unit of 16 vectors leaves is converted, scaled and added between the matrix instructions of the next one, two vector
 // instructions beside each: alone that many cost it 9 % (9.4 -> 10.2 ns each, two waves per SIMD), in a block of their own behind the
-// matrix instructions, where both waves of a SIMD come at once behind a barrier, their whole time.  Against 64 bits the sums err
-// less: one rounding of a group's sum and one of the running sum, where there were two of the latter (7B widths, 1024 vectors: 0.80 to
-// 1.25e-7 for 1.04 to 1.75e-7).  1024 vectors, four products of the 7B shape, us: 206 67.2 351 169 -> 195 63.5 331 157 (2.2 POP/s); 96
-// vectors 33.1 16.8 60 -> 31.3 16.6 56 (Wq+Wk+Wv, Wo, W1+W3).  A group then takes 10960 cycles at 1.9 GHz, 8192 of them
+// matrix instructions, where both waves of a SIMD come at once behind a barrier, their whole time.  Inside passes of the 7B
+// shape, us, Wq+Wk+Wv, Wo, W1+W3, W2: 1024 vectors 183 61.6 341 154 -> 179 60.0 329 148 (2.2 POP/s), 448 95.3 35.7 166 79.5 -> 93.5 35.5
+// 160 78.1, 64 24.6 13.8 40.9 23.2 -> 24.4 14.3 41.3 22.9.  (The digits joined before the running sum, four operations less per row, were
+// 1 to 1.5 % faster still, but rounded elsewhere.)  A group of 64 vectors then takes 11000 cycles at 1.9 GHz, 8192 of them
 // matrix instructions; without the codes' loads 0.9 of the time, without the digits' 0.95.  Tried, no faster: codes a whole group ahead in
 // a second set of registers (32 vectors: 3 % slower, it is bound by the codes' way through L2), workgroups that go on to
 // another tile instead of ending, sums stored four rows at a time by way of LDS.
@@ -307,47 +307,51 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
     const bool live = col * PT * 32 + xt < a.npos;
     float up = 1.0f;
     bool large = false;
-    v4f sxp = {0.f, 0.f, 0.f, 0.f};   // the scales of the unit whose sums are still to be added
-    auto keep = [&](float x) {
+    auto keep = [&](float x, auto pending) {   // pending(): what the sums kept so far still lack
         x = live ? x : 1.0f;
         if (__any(!(x >= 0x1p-64f && x <= 0x1p20f))) {
             large |= __any(x > 0x1p20f) != 0;
             const float k = large ? 1.0f : __any(x < 0x1p-64f) ? 0x1p48f : up;
             if (k != up) {
                 const float by = k > up ? 0x1p48f : 0x1p-48f;
+                pending();
 #pragma unroll
                 for (int u = 0; u < NU; u++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
 #pragma unroll
                         for (int e = 0; e < 4; e++) f[u][r][e] *= by;
-                sxp *= by;
                 up = k;
             }
         }
         return x * up;
     };
-    lsx[xt] = keep(sx0);
+    lsx[xt] = keep(sx0, [] {});
     __syncthreads();
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): (a load under way here would be waited for in every round of the loop)
 
-    // The accumulators of two units in turn, and what adding up a unit takes: 80 operations, five for each of four rows' four values.
-    // operation o of unit v, whose vectors' scales are sx and whose rows' are r_m:
+    // The accumulators of two units in turn, and what adding up a unit takes: 96 operations, six for each of four rows' four values.
+    // The high and the low digits go into the running sum one after the other, the high ones times 65536 r_m: joined first, they would share
+    // a factor sixteen powers of two nearer to 2^-126, and every sum round elsewhere.  Operation o of unit v, whose vectors' scales are sx
+    // and whose rows' are r_m:
     v4i hi[2][4], lo[2][4];
 #pragma unroll
     for (int k = 0; k < 2; k++)
 #pragma unroll
         for (int r = 0; r < 4; r++) { hi[k][r] = v4i{0, 0, 0, 0}; lo[k][r] = v4i{0, 0, 0, 0}; }
-    float eh[4], el[4], em[4];
+    v4f sxp = {0.f, 0.f, 0.f, 0.f};   // the scales of the unit whose sums are still to be added
+    float eh[4], el[4], mh[4], ml[4], rh;
     auto add_up = [&](auto oc, auto vc, const v4f &sx, const float (&r_m)[4]) __attribute__((always_inline)) {
         constexpr int o = oc.value, v = vc.value;
-        if constexpr (o < 80) {
-            constexpr int r = o / 20, what = o % 20 / 4, e = o % 4, k = v & 1;
+        if constexpr (o < 96) {
+            constexpr int r = o / 24, what = o % 24 / 4, e = o % 4, k = v & 1;
+            if constexpr (o % 24 == 0) rh = r_m[r] * 65536.0f;
             if constexpr (what == 0) eh[e] = (float)hi[k][r][e];
-            else if constexpr (what == 1) el[e] = (float)lo[k][r][e];
-            else if constexpr (what == 2) em[e] = r_m[r] * sx[e];
-            else if constexpr (what == 3) eh[e] = fmaf(eh[e], 65536.0f, el[e]);
-            else f[v][r][e] = fmaf(eh[e], em[e], f[v][r][e]);
+            else if constexpr (what == 1) mh[e] = rh * sx[e];
+            else if constexpr (what == 2) el[e] = (float)lo[k][r][e];
+            else if constexpr (what == 3) ml[e] = r_m[r] * sx[e];
+            else if constexpr (what == 4) f[v][r][e] = fmaf(eh[e], mh[e], f[v][r][e]);
+            else f[v][r][e] = fmaf(el[e], ml[e], f[v][r][e]);
         }
     };
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) v4i *)dg_lds;
@@ -388,10 +392,11 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
                     constexpr int r = rc.value, i = 4 * j + r;
                     v4i &acc = (d & 2) ? lo[k][r] : hi[k][r];
                     acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[at & 3], cw[r][T], !(d & 1) && T == 0 ? v4i{0, 0, 0, 0} : acc, 0, 0, 0);
-                    // beside it the unit before (one unit: nothing, its sums are added up behind it), and the shifts between the digits of a pair
-                    constexpr int o = NU == 1 ? 80 : i < 16 ? 2 * i : 16 + i;
+                    // beside it the unit before (one unit: nothing, its sums are added up behind it), and the shifts between the digits of a pair:
+                    // about two vector instructions each
+                    constexpr int o = NU == 1 ? 96 : i < 16 ? 2 * i : i < 48 ? 16 + i : 2 * i - 32;
                     add_up(std::integral_constant<int, o>{}, Before{}, sxp, u == 0 ? rmp : rm);
-                    if constexpr (i < 16) add_up(std::integral_constant<int, o + 1>{}, Before{}, sxp, u == 0 ? rmp : rm);
+                    if constexpr (i < 16 || i >= 48) add_up(std::integral_constant<int, o + 1>{}, Before{}, sxp, u == 0 ? rmp : rm);
                     if constexpr (u == 0 && j == 7) hi[k][r] <<= 8;
                     if constexpr (u != 0 && j >= 4 && j < 8) hi[k][j - 4][r] <<= 8;
                     if constexpr (u == NU - 1 && j == 8) lo[k][r] <<= 8;
@@ -406,14 +411,19 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
             sxp = sx;
             __builtin_amdgcn_sched_barrier(0);
         });
-        if constexpr (NU == 1) unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, 0>{}, sxp, rm); });
+        if constexpr (NU == 1) unroll<96>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, 0>{}, sxp, rm); });
 #pragma unroll
         for (int r = 0; r < 4; r++) { rmp[r] = rm[r]; rm[r] = rmn[r]; }
-        lsx[((g + 1) & 1) * 32 * PT + xt] = keep(nsx);
+        lsx[((g + 1) & 1) * 32 * PT + xt] = keep(nsx, [&] {
+            if constexpr (NU > 1) {
+                unroll<96>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
+                sxp = v4f{0.f, 0.f, 0.f, 0.f};
+            }
+        });
         asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // (the staged digits: all but the sixteen loads of codes behind them)
         __syncthreads();
     }
-    if constexpr (NU > 1) unroll<80>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
+    if constexpr (NU > 1) unroll<96>([&](auto oc) __attribute__((always_inline)) { add_up(oc, std::integral_constant<int, NU - 1>{}, sxp, rmp); });
     const int ldo = 16 * a.ntiles;
     const float down = up == 1.0f ? 1.0f : 0x1p-48f;
 #pragma unroll
@@ -431,8 +441,8 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
 }
 
 // Of a last tile of 32 vectors whose second half is empty only the first unit is multiplied, and staged: a third of the work at 77 vectors
-// had been for padding.  Wq+Wk+Wv, Wo, W1+W3, W2 of the 7B shape, us, 40 vectors 24.7 10.7 37 22.0 -> 22.3 10.2 36 19.5, 77 vectors 28.3 13.7 48.4
-// 27.5 -> 27.1 13.3 44.3 24.9, 144 vectors 37.4 17.5 66.6 37.9 -> 34.4 17.6 59.5 34.6.  (The launches are picked as for whole tiles:
+// had been for padding.  Wq+Wk+Wv, Wo, W1+W3, W2 inside passes of the 7B shape, us, 40 vectors 24.2 13.2 41.5 21.8 -> 21.2 12.2 35.4 19.4, 77 vectors
+// 29.9 17.3 50.7 28.6 -> 27.2 16.4 47.6 25.7, 144 vectors 38.2 19.0 66.6 39.3 -> 35.8 18.5 61.2 36.0.  (The launches are picked as for whole tiles:
 // within 2.3 % of the best on average; an estimate with half a tile in it does worse.)
 template <int PT, int NW>
 __global__ void __launch_bounds__(64 * NW, 2) k_dgemm(const DGemm a)

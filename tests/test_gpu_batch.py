@@ -548,6 +548,25 @@ def test_a_product_keeps_its_precision_at_every_magnitude(shape, tensor, rows, K
     g.close()
 
 
+def test_a_product_keeps_its_precision_where_scales_are_small():
+    """k_dgemm where a vector's 2^-s times a row's scale lies below 2^-126, and no sums are kept times 2^48: a matrix of 2^-68, and vectors of
+    2^-95 that share a tile with one of 2^60.  The bound of the other magnitudes."""
+    shape, rows, K = (768, 512, 1, 48, 3, 512, 40, 0), 48, 768
+    rng = np.random.default_rng(1)
+    normal = rng.standard_normal((16, K))
+    w = 0.02 * rng.standard_normal((rows, K))
+    for power, x in ((-62, np.ldexp(normal, -33)), (0, np.ldexp(normal, np.array([60] + [-95] * 15)[:, None]))):
+        g = l2j.Transformer(l2j.Config(*shape))
+        g.upload_f32_quantize(TENSOR.WK, np.ldexp(w, power))
+        W = dequantized(g, TENSOR.WK, 0, rows, K)
+        x = x.astype(np.float32)
+        want = x.astype(np.float64) @ W.T
+        got, _ = g.batch_matmul(TENSOR.WK, 0, x, rows)
+        g.close()
+        err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() < 3e-7, (power, float(err.max()))
+
+
 class FullDevice:
     """All of the device's free memory but `leave` bytes, held for the duration of a with block."""
 

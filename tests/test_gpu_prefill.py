@@ -7,7 +7,7 @@ import pytest
 
 import llama2j_amd as l2j
 from llama2j_amd.binding import BUFFER, TENSOR, L2JError
-from tests.test_gpu_batch import FullDevice, LOGIT_TOL, oracle_of, rel_err
+from tests.test_gpu_batch import FullDevice, LOGIT_TOL, dequantized, oracle_of, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -356,7 +356,7 @@ def digit_pairs(x):
     return 256 * d[0] + d[1], 256 * d[2] + d[3], np.ldexp(np.float32(1.0), -s[:, :, 0])
 
 
-@pytest.mark.parametrize("dim,heads,n", [(512, 4, 16), (512, 4, 17), (512, 4, 32), (4096, 32, 32)])
+@pytest.mark.parametrize("dim,heads,n", [(512, 4, 16), (512, 4, 17), (512, 4, 32), (4096, 32, 32), (4096, 32, 40), (4096, 32, 64), (4096, 32, 600), (8192, 64, 1000)])
 def test_the_sums_of_a_product_are_formed_in_one_order(dim, heads, n):
     """Wv on inputs, codes and scales whose products are all exact, so that the value rows show the order of the additions to the bit.  Up
     to 32 vectors the halves of the groups are converted and added one after the other, above that the high and the low digits of a group go
@@ -405,6 +405,28 @@ def test_the_sums_of_a_product_are_formed_in_one_order(dim, heads, n):
         np.testing.assert_array_equal(got.view(np.uint32), want(4).view(np.uint32))
     else:                                                                # (as many groups as the estimate for this shape picks)
         assert any(np.array_equal(got.view(np.uint32), want(per).view(np.uint32)) for per in range(1, ng + 1))
+
+
+@pytest.mark.parametrize("n", [40, 64, 600])
+def test_value_rows_of_small_scales_keep_their_precision(n):
+    """A vector's 2^-s times a row's scale below 2^-126, in tiles of 16, 32 and 64 vectors (as for one product in test_gpu_batch.py)."""
+    dim, kvd, vocab = 4096, 256, 512
+    rng = np.random.default_rng(n)
+    g = l2j.Transformer(l2j.Config(dim, 256, 1, 32, 2, vocab, 608, 0))
+    g.fill_synthetic(9, 0.02)
+    emb = np.ldexp(rng.standard_normal((vocab, dim)), -40).astype(np.float32)                 # (nothing beside the norm's 1e-5)
+    g.upload_f32(TENSOR.TOK_EMB, emb)
+    g.upload_f32_quantize(TENSOR.RMS_ATT, np.full(dim, 0.5))
+    g.upload_f32_quantize(TENSOR.WV, np.ldexp(0.02 * rng.standard_normal((kvd, dim)), -62))
+    g.finalize()
+    tokens = rng.integers(2, vocab, size=n).astype(np.int32)
+    g.prefill(tokens, want_logits=False)
+    got = g.read(BUFFER.VCACHE, 0).reshape(-1, kvd)[:n]
+    x = np.float32(0.5) * (np.float32(1.0) / np.sqrt(np.float32(1e-5)) * emb[tokens])
+    want = x.astype(np.float64) @ dequantized(g, TENSOR.WV, 0, kvd, dim).T
+    g.close()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert err.max() < 3e-7, float(err.max())
 
 
 def test_a_prompt_goes_through_in_smaller_passes_where_the_memory_for_a_large_one_is_missing():
