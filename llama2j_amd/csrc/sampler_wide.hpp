@@ -668,6 +668,8 @@ __device__ __forceinline__ void few_greater(const float *keys, int n, const floa
 // sums of the first n0 pairs of the merged array, added one after the other; the first that exceeds topp, or the last, is the cumulative
 // probability, r = coin * that, the pick the first pair whose sum exceeds r.  All threads call; returns the token (wave 0).
 // coin < 0: the generator draws.
+// Behind a barrier that gave up the candidates may be logits not yet replaced, of any sign, infinite or NaN: ranks then collide, places of the
+// merged front stay as they were, and sums fall.  Nothing outside the front is read all the same; what is returned may be any number.
 __device__ __forceinline__ int few_pick(FewSort &f, int n0, const float *old, const int *old_idx, int n, float topp, float coin, unsigned long long *rng)
 {
     const int tid = threadIdx.x, lane = tid & 63, nold = min(n0, n - n0);   // (an old pair further back stands behind n0 others)
@@ -733,12 +735,16 @@ __device__ __forceinline__ int few_pick(FewSort &f, int n0, const float *old, co
         c = spec_uniform(c);
     }
     const float r = __fmul_rn(c, cum);
-    b = __popcll(__ballot(starts <= r)) - 1;   // (the sums never fall: the block in which they pass r; r < 0 does not occur)
+    b = min(max(__popcll(__ballot(starts <= r)) - 1, 0), (n0 - 1) >> 6);   // (the sums never fall: the block in which they pass r)
     const float pre = sums(term(starts, b), block(b));
     const unsigned long long hit = __ballot(64 * b + lane <= last && pre > r);
     const int pick = hit ? 64 * b + __ffsll((long long)hit) - 1 : last;
     return f.m.mv[pick];
 }
+
+// Behind a barrier that gave up a pick's id may be any number (of pairs that nobody has stored, here or in earlier launches), and the loop's next
+// step, enqueued before the host learns of it, reads that row of the table: an id of the vocabulary in any case.
+__device__ __forceinline__ int wide_id(int token, int n) { return (unsigned)token < (unsigned)n ? token : 0; }
 
 // grid: ceil(n / 256) workgroups of 256 threads, all resident at once (n <= kSampleMaxVocab: at most 144); dynamic LDS:
 // max(sizeof(WideWalk), sizeof(FewSort), 4 bytes per key of the array padded to whole runs of 4096).
@@ -924,7 +930,7 @@ static __global__ void __launch_bounds__(kWideSlice) k_sample_wide(const WideArg
         }
         few_sort(f, n0);
         if (g == 0) {
-            const int token = few_pick(f, n0, a.old_prob, a.old_idx, n, a.topp, a.coin, &a.ss->rng);
+            const int token = wide_id(few_pick(f, n0, a.old_prob, a.old_idx, n, a.topp, a.coin, &a.ss->rng), n);
             if (tid == 0) {
                 a.ss->result = token;
                 loop_result(a, token);
@@ -1101,7 +1107,7 @@ static __global__ void __launch_bounds__(kWideSlice) k_sample_wide(const WideArg
         if (tid == 0) {
             int pick = L.hit;
             if (pick < 0 || pick > last) pick = last;
-            const int token = ld_coh(a.new_idx + min(pick, n - 1));
+            const int token = wide_id(ld_coh(a.new_idx + min(pick, n - 1)), n);
             a.ss->result = token;
             loop_result(a, token);
         }

@@ -298,6 +298,32 @@ def test_a_wait_of_the_one_launch_step_that_runs_out_is_an_error_and_the_context
         check_probabilities(g.read(BUFFER.LOGITS), probs)
 
 
+@pytest.mark.parametrize("vocab,topp", [(1008, 0.9), (32000, 0.9), (32000, 0.3), (1008, 1.0)])
+def test_waits_that_run_out_inside_the_token_loop_leave_ids_of_the_vocabulary(orc, vocab, topp):
+    """barrier_spins 0 in a loop that enqueues 32 tokens before it looks: every sampling step works on masks and sums of earlier launches, and what
+    it picks is the next token's row of the table.  The call fails, every kernel having run to its end; the next call, one launch per stage,
+    gives the oracle's tokens."""
+    shape = (64, 128, 2, 4, 4, vocab, 96, 1)
+    g = l2j.Transformer(l2j.Config(*shape), options={"barrier_spins": 0, "fuse": 0})   # (the forward pass waits for nobody)
+    g.fill_synthetic(31, 0.02)
+    g.upload_f32_quantize(l2j.TENSOR.RMS_FINAL, np.full(64, 5.0 / (0.02 * 8.0), dtype=np.float32))   # (logits of standard deviation 5: a few hundred candidates)
+    g.finalize()
+    prompt = np.array([5, 6, 7], dtype=np.int32)
+    with pytest.raises(L2JError):
+        g.decode_sample(prompt, 90, 0.9, topp, 5)
+    assert g.get_option("sampler_wide") == 0
+    g.reset()
+    got, _ = g.decode_sample(prompt, 40, 0.9, topp, 5)
+    g.reset()
+    s = orc.Sampler(5, vocab)
+    tok = 1
+    for pos in range(len(got)):
+        lg = g.forward(tok, pos)
+        tok = int(prompt[pos]) if pos < len(prompt) else s.step(lg, 0.9, topp)[0]
+        assert tok == got[pos], pos
+    g.close()
+
+
 def test_largest_vocabulary_the_sampler_takes(orc):
     vocab = 36864
     g = small_transformer(vocab)
