@@ -225,7 +225,11 @@ template <int PT, int NW, int NU>
 __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile, int col)
 {
     constexpr int STAGE = PT * kDigitBytes / 16;            // 16-byte words of a group's digits
-    constexpr int NT = 64 * NW, NST = STAGE / NT * NU / (2 * PT);   // words a thread stages per group
+    constexpr int NT = 64 * NW, NST = STAGE / NT * NU / (2 * PT);   // words a thread stages per group,
+    constexpr int U1 = NU > 1 ? 1 : 0, PER = (NST + NU - 1 - U1) / (NU - U1);   // in the units behind the first (of one: in it), so many in each, one a step
+    // The wait at a group's end leaves sixteen loads under way and takes them for the next codes, which are requested from the last unit's tenth step on:
+    // every word has to be requested before.
+    static_assert(STAGE % NT == 0 && STAGE / NT * NU % (2 * PT) == 0 && PER <= 9, "digits would be read before they are staged");
     float *lsx = reinterpret_cast<float *>(dg_lds + 2 * STAGE);   // [2][32 PT]
     constexpr int RUN = NU == 2 * PT ? 64 : 128;             // the wave's q-th run of 64 words begins at (q NW + wave) RUN (one unit: the runs of the tile's first half)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), s4 = lane >> 4, n = lane & 15;
@@ -367,7 +371,7 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
         auto stage = [&](int q) __attribute__((always_inline)) {
             const v4i *from = xn + (q * NW * RUN / 2048) * xstep + q * NW * RUN % 2048;
             const unsigned to = lds0 + (((g + 1) & 1) * STAGE + q * NW * RUN + wave * RUN) * 16;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(stage16), "s"(from) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(stage16), "s"(from) : "memory", "m0");
         };
         v4i x[4];   // fragments, three ahead of their use
         auto fragment = [&](int u, int j) __attribute__((always_inline)) {
@@ -385,8 +389,7 @@ __device__ __forceinline__ void dgemm_tile(const DGemm a, v4i *dg_lds, int tile,
             const v4f sx = *reinterpret_cast<const v4f *>(csx + 16 * u + 4 * s4);
             unroll<16>([&](auto jc) __attribute__((always_inline)) {
                 constexpr int j = jc.value, d = dg_digit(u, NU, j), T = dg_block(u, NU, j), at = 16 * u + j;
-                constexpr int u1 = NU > 1 ? 1 : 0, per = (NST + NU - 1 - u1) / (NU - u1);   // words staged in a unit behind the first (of one: in it)
-                if constexpr (u >= u1 && j < per && (u - u1) * per + j < NST) stage((u - u1) * per + j);
+                if constexpr (u >= U1 && j < PER && (u - U1) * PER + j < NST) stage((u - U1) * PER + j);
                 if constexpr (at + 3 < 16 * NU) x[(at + 3) & 3] = fragment((at + 3) >> 4, (at + 3) & 15);
                 unroll<4>([&](auto rc) __attribute__((always_inline)) {
                     constexpr int r = rc.value, i = 4 * j + r;
