@@ -886,6 +886,7 @@ static __global__ void __launch_bounds__(kWideSlice) k_sample_wide(const WideArg
             a.ss->result = 0;
             atomicOr(&a.ss->nan, 2);
         }
+        if (i < n) { a.new_prob[i] = a.old_prob[i]; a.new_idx[i] = a.old_idx[i]; }   // (the array stays as it was, in the copy that the next call reads)
         wide_leave(a.w, a.ss);
         return;
     }

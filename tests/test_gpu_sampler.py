@@ -133,6 +133,44 @@ def test_topp_with_few_candidates_at_the_edges_of_tiles_and_of_what_one_workgrou
     g.close()
 
 
+@WIDE
+@pytest.mark.parametrize("vocab", [1003, 32000])
+def test_a_call_that_fails_leaves_the_array_of_the_call_before(orc, monkeypatch, vocab, wide):
+    """NaN among the logits, and no probability at the cutoff: both fail, and the steps behind them, most of whose pick lies among entries that
+    calls before the failed one left, pick what the oracle picks."""
+    monkeypatch.setenv("L2J_SAMPLER_WIDE", wide)
+    g = small_transformer(vocab)
+    rng = np.random.default_rng(vocab + 3)
+    g.sampler_seed(21)
+    o = orc.Sampler(21, vocab)
+
+    def some(k):
+        """k candidates, of an even number much alike, of an odd one with the first at 0.6 and the others below what an even call leaves"""
+        lg = np.full(vocab, -40.0, dtype=np.float32)
+        at = rng.permutation(vocab)[:k]
+        lg[at] = rng.random(k).astype(np.float32) if k % 2 == 0 else -7.0
+        if k % 2:
+            lg[at[0]] = np.log(1.5 * np.exp(-7.0) * (k - 1))
+        return lg
+
+    for call, what in enumerate([300, 40, "nan", 31, 200, 60, "flat", 51, 40, "nan", "nan", 21, 700, 500, "flat", "nan", 401, 900, 800, "nan", 701]):
+        if isinstance(what, str):
+            lg = np.zeros(vocab, dtype=np.float32)
+            if what == "nan":
+                lg[rng.integers(vocab)] = np.nan
+            topp = 0.9 if what == "nan" else 0.0
+            assert o.step(lg, 1.0, topp)[0] < 0
+            with pytest.raises(L2JError):
+                g.sample(1.0, topp, logits=lg)
+        else:
+            lg, coin = some(what), float(np.float32(rng.uniform(0.9, 0.99)))
+            _, probs = o.step(lg, 1.0, 1.0)
+            want = o.sample_topp(probs, 0.99, coin=coin)
+            assert g.sample(1.0, 0.99, logits=lg, coin=coin) == want, (call, what)
+            check_probabilities(g.read(BUFFER.LOGITS), probs)
+    g.close()
+
+
 def test_topp_worked_example_with_entries_of_an_earlier_call(orc):
     # the hand-worked case of the oracle's tests, on the device: eight tokens, padded with impossible ones
     vocab = 16
