@@ -993,8 +993,9 @@ static __global__ void __launch_bounds__(256) k_merge_far(const float *__restric
     merge_far_of(kin, vin, npad, nout, run_len, group_len, kout, vout);
 }
 
-// How many of the keys a[0..n), which descend, are greater than k: sixteen parts at a time (n up to 65536), whose probes go out
-// together: four trips to memory instead of sixteen.
+// How many of the keys a[0..n), which descend, are greater than k: sixteen parts at a time (n up to 65535: fifteen steps of each size),
+// whose probes go out together: four trips to memory instead of sixteen.
+static_assert(kSampleMaxVocab <= 65535, "count_greater counts no further");
 __device__ __forceinline__ int count_greater(const float *__restrict__ a, int n, float k)
 {
     int pos = 0;
