@@ -363,11 +363,12 @@ def test_sampled_batch_gives_every_sequence_its_own_sampler(orc, n_seq, t, topp,
     g.close()
 
 
-@pytest.mark.parametrize("vocab,spread", [(272, 4.0), (1008, 20.0), (4112, 0.3), (8208, 3.0), (32000, 5.0), (36864, 1.0)])
-def test_sampled_batch_merges_few_and_many_candidates_with_what_earlier_steps_left(orc, vocab, spread):
-    """Top-p steps whose candidates are one tile, one run (4096 pairs) or several of the sort, by the logits' spread: every token the one
-    that the oracle's sampler, which sorts its whole array, takes from the same logits."""
-    shape = SHAPES[0][:5] + (vocab,) + SHAPES[0][6:]
+@pytest.mark.parametrize("vocab,spread,least,most", [(272, 4.0, 1, 256), (1008, 20.0, 1, 256), (4112, 0.3, 4097, 4112), (8208, 3.0, 257, 4096),
+                                                     (32000, 5.0, 1, 4096), (32000, 2.0, 8193, 20480), (36864, 1.0, 24577, 36864)])
+def test_sampled_batch_merges_few_and_many_candidates_with_what_earlier_steps_left(orc, vocab, spread, least, most):
+    """Top-p steps whose candidates are one tile (256 pairs), one run (4096), two, three to five or seven of the sort, by the logits' spread: every
+    token the one that the oracle's sampler, which sorts its whole array, takes from the same logits."""
+    shape = SHAPES[1][:5] + (vocab,) + SHAPES[1][6:]    # (a classifier of its own: with the embedding's a token's own logit stands out)
     g = l2j.Transformer(l2j.Config(*shape))
     g.fill_synthetic(23, 0.02)
     g.upload_f32_quantize(l2j.TENSOR.RMS_FINAL, np.full(shape[0], spread / (0.02 * shape[0] ** 0.5), dtype=np.float32))
@@ -381,7 +382,49 @@ def test_sampled_batch_merges_few_and_many_candidates_with_what_earlier_steps_le
             s = orc.Sampler(int(seeds[b]), vocab)
             want = [int(prompts[b][pos]) if pos < len(prompts[b]) else s.step(logits[pos, b], t, topp)[0] for pos in range(12)]
             np.testing.assert_array_equal(got[b], np.array(want, dtype=np.int32), err_msg="sequence %d" % b)
+        p = np.exp((logits.astype(np.float64) - logits.max(axis=2, keepdims=True)) / t)
+        n0 = (p / p.sum(axis=2, keepdims=True) >= (1 - topp) / (vocab - 1)).sum(axis=2)
+        assert least <= n0.min() and n0.max() <= most, (t, int(n0.min()), int(n0.max()))
     g.close()
+
+
+def test_sampled_batch_reports_what_the_sampler_reports_and_goes_on(orc):
+    """A NaN in the logits of one sequence, and a flat distribution with topp 0, which leaves no candidate: both an error, from top-p and (the NaN)
+    plain sampling, and the next call of the same context gives every sequence the oracle's tokens."""
+    shape = SHAPES[1]
+    vocab, dim, n_seq, steps = shape[5], shape[0], 16, 10
+    rng = np.random.default_rng(8)
+    emb = (0.02 * rng.standard_normal((vocab, dim))).astype(np.float32)
+    emb[5, 7] = np.nan
+    prompts = [rng.integers(6, vocab, size=b % 4).astype(np.int32) for b in range(n_seq)]
+    bad = [np.array([9, 5], dtype=np.int32) if b == 11 else p for b, p in enumerate(prompts)]
+    seeds = np.arange(n_seq) + 70
+
+    def check(g, t, topp):
+        got, _, logits = g.decode_sample_batch(prompts, steps, t, topp, seeds, want_logits=True)
+        for b in range(n_seq):
+            s = orc.Sampler(int(seeds[b]), vocab)
+            want = [int(prompts[b][pos]) if pos < len(prompts[b]) else s.step(logits[pos, b], t, topp)[0] for pos in range(steps)]
+            want = np.array(want, dtype=np.int32)
+            if 5 not in want:                                            # (else the sequence has drawn the NaN itself)
+                np.testing.assert_array_equal(got[b], want, err_msg="sequence %d" % b)
+
+    for spread in (4.0, 0.0):
+        g = l2j.Transformer(l2j.Config(*shape))
+        g.fill_synthetic(23, 0.02)
+        g.upload_f32(TENSOR.TOK_EMB, emb)
+        g.upload_f32_quantize(TENSOR.RMS_FINAL, np.full(dim, spread / (0.02 * dim ** 0.5), dtype=np.float32))
+        g.finalize()
+        if spread:
+            for topp in (0.9, 1.0):
+                with pytest.raises(L2JError, match="NaN"):
+                    g.decode_sample_batch(bad, steps, 0.9, topp, seeds)
+                check(g, 0.5, topp)
+        else:
+            with pytest.raises(L2JError, match="cutoff"):
+                g.decode_sample_batch(prompts, steps, 1.0, 0.0, seeds)
+            check(g, 1.0, 0.9)
+        g.close()
 
 
 def test_sampled_batch_refuses_what_its_sampling_step_cannot_take():
